@@ -285,8 +285,8 @@ int sts_batch_destroy(sts_batch *b);
 int sts_batch_time_step(sts_batch *b, const sts_loop_control *lc, const sts_mixed_control *mc, int *iters32,
                         int *iters64);
 /* Tile shapes of the batched launches: variant v of the cell kernels is
-   64x4, 64x8, 128x2, 32x8 cells, of the fused sweep pass 64x8, 64x4, 128x4,
-   64x16 (v = 0..3).  sts_batch_autotune times each variant `reps` times on
+   64x4, 64x8, 128x2, 32x8 cells, of the fused sweep pass 60x6, 60x4, 60x8,
+   60x10 (v = 0..3).  sts_batch_autotune times each variant `reps` times on
    the current state, keeps the fastest and reports the mean milliseconds per
    variant in ms[8] (cell kernels, then sweeps; may be NULL). */
 int sts_batch_set_tiles(sts_batch *b, int cell_variant, int sweep_variant);

@@ -101,6 +101,25 @@ __device__ __forceinline__ unsigned long long wave_max_last(unsigned long long v
   return v;
 }
 
+// The value of the next (CTRL 0x130, wave_shl:1) or the previous lane
+// (0x138, wave_shr:1) of the wave; the last (first) lane gets 0.  Every lane
+// whose value is asked for must be active.
+template <int CTRL>
+__device__ __forceinline__ float dpp_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_lane(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, true),
+                 hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <typename R>
+__device__ __forceinline__ R lane_east(R v) { return dpp_lane<0x130>(v); }
+template <typename R>
+__device__ __forceinline__ R lane_west(R v) { return dpp_lane<0x138>(v); }
+
 // Destinations of block_max_atomic's NV maxima: value k goes to d[k] and,
 // when set, also to e[k] (the first and the last sweep of a single-sweep
 // loop 3 coincide); null destinations are skipped.
@@ -115,14 +134,17 @@ struct MaxDst {
 // destination.  Every thread leaves its values in LDS, one barrier, then the
 // first wave alone folds the NT / 64 entries of each lane and reduces across
 // its lanes; the other waves are done at the barrier.  Called once per
-// kernel by every thread of the block (its LDS words are not reused).
+// kernel by every thread of the block (its LDS words are not reused);
+// threads NT and up carry no values, they only meet the barrier.
 template <int NV, int NT>
 __device__ __forceinline__ void block_max_atomic(const unsigned long long (&v)[NV], const MaxDst<NV> &dst) {
   static_assert(NT % 64 == 0, "whole waves");
   __shared__ unsigned long long sm[NV][NT];
   const int tid = threadIdx.x + threadIdx.y * blockDim.x;
+  if (tid < NT) {
 #pragma unroll
-  for (int k = 0; k < NV; k++) sm[k][tid] = v[k];
+    for (int k = 0; k < NV; k++) sm[k][tid] = v[k];
+  }
   __syncthreads();
   if (tid >= 64) return;
   const unsigned slot = ((unsigned)blockIdx.x + (unsigned)blockIdx.y * gridDim.x) % (unsigned)NSLOT;
@@ -651,80 +673,83 @@ struct PTStencil {
 };
 
 // The reference's T update (S:3837-3857) then p update (S:3884-3895) of one
-// cell of the update set, with the new T in the p denominator (S:3894).  A
-// body neighbour contributes the fluid temperature on its wall (S:3838-3848:
-// m*T_old + !m*T_wall with T_wall finite, i.e. a select).  The per-cell
-// factors that do not depend on the old p, T are formed once (load) with the
-// reference's operations and kept, so a cell swept twice reads its
+// cell of the update set, with the new T in the p denominator (S:3894).  The
+// per-cell factors that do not depend on the old p, T are formed once (set)
+// with the reference's operations and kept, so a cell swept twice reads its
 // coefficient arrays once; update() then performs the rest of each
-// expression in the reference's order.
+// expression in the reference's order.  What few cells use -- a body
+// neighbour's wall temperature, the given-velocity fluxes -- is read from
+// memory where it is used rather than kept.
 template <typename R>
 struct PTCoef {
   R aT1, aT2, aT3, aT4;  // T neighbour coefficients (S:3959-3962)
-  R X1, X2, X3, X4;      // wall temperature of a body neighbour
   R div, sct, denT;      // velocity divergence term, ScT1, T denominator
-  R a1, a2, a3, a4;      // p neighbour coefficients apx_W, apx_E, apy_S, apy_N
-  R b1, b2, b3, b4;      // bpx_W, bpx_E, bpy_S, bpy_N
-  R gxb, gxe;            // given-velocity flux terms (S:3887-3888)
-  R q, Ap, hh;           // p_pr hx hy / T_pr, ht * sum(a), hx hy
-  R c1, ht;
-  unsigned fluid;  // bit q: neighbour q (W, E, S, N) is fluid
-  bool has_gxb, has_gxe;
+  R a1, a3, a4;          // p neighbour coefficients apx_W, apy_S, apy_N
+  R b1, b3, b4;          // bpx_W, bpy_S, bpy_N
+  R q, hh;               // p_pr hx hy / T_pr, hx hy
 
-  __device__ __forceinline__ void load(const KGridT<R> &g, const KFieldsT<R> &fl, const Nbr &n) {
-    const unsigned ij = n.ij, i1j = n.i1j, ij1 = n.ij1;
-    const R *Fx = FLD(FX), *Fy = FLD(FY), *DTx = FLD(DTX), *DTy = FLD(DTY), *u = FLD(U), *v = FLD(V);
-    const R *apx = FLD(APX), *apy = FLD(APY), *bpx = FLD(BPX), *bpy = FLD(BPY);
-    ht = g.ht;
-    c1 = g.c1;
-    const R hxi = g.hx[n.i], hyj = g.hy[n.j];
-    aT1 = maxi0(Fx[ij]) + DTx[ij];
-    aT2 = maxi0(-Fx[i1j]) + DTx[i1j];
-    aT3 = maxi0(Fy[ij]) + DTy[ij];
-    aT4 = maxi0(-Fy[ij1]) + DTy[ij1];
-    const unsigned nb = g.nb[ij];
-    fluid = ((nb & NB_W) ? 1u : 0u) | ((nb & NB_E) ? 2u : 0u) | ((nb & NB_S) ? 4u : 0u) | ((nb & NB_N) ? 8u : 0u);
-    X1 = (fluid & 1u) ? R(0) : FLD(TW_U)[ij];
-    X2 = (fluid & 2u) ? R(0) : FLD(TW_U)[i1j];
-    X3 = (fluid & 4u) ? R(0) : FLD(TW_V)[ij];
-    X4 = (fluid & 8u) ? R(0) : FLD(TW_V)[ij1];
-    div = (u[i1j] - u[ij]) * hyj + (v[ij1] - v[ij]) * hxi;
-    sct = FLD(SCT1)[ij];
-    denT = ht * (aT1 + aT2 + aT3 + aT4 + Fx[i1j] - Fx[ij] + Fy[ij1] - Fy[ij]) + hxi * hyj * FLD(RHO)[ij];
-    a1 = apx[ij];
-    a2 = apx[i1j];
-    a3 = apy[ij];
-    a4 = apy[ij1];
-    b1 = bpx[ij];
-    b2 = bpx[i1j];
-    b3 = bpy[ij];
-    b4 = bpy[ij1];
-    has_gxb = g.given_xb && (int)n.i == g.Nx_o0;
-    has_gxe = g.given_xe && (int)n.i == g.Nx_o1 - 1;
-    gxb = has_gxb ? Fx[ij] : R(0);
-    gxe = has_gxe ? Fx[i1j] : R(0);
-    q = FLD(P_PR)[ij] * hxi * hyj / (FLD(T_PR)[ij]);
-    Ap = ht * (a1 + a2 + a3 + a4);
+  // The cell's own, east and north values: x0/x1 of Fx, DTx, u, apx, bpx,
+  // y0/y1 of Fy, DTy, v, apy, bpy.  The east apx, bpx are not kept.
+  __device__ __forceinline__ void set(const KGridT<R> &g, unsigned i, unsigned j, const R (&x0)[5], const R (&x1)[5],
+                                      const R (&y0)[5], const R (&y1)[5], R rho, R sc, R p_pr, R T_pr) {
+    const R hxi = g.hx[i], hyj = g.hy[j];
+    aT1 = maxi0(x0[0]) + x0[1];
+    aT2 = maxi0(-x1[0]) + x1[1];
+    aT3 = maxi0(y0[0]) + y0[1];
+    aT4 = maxi0(-y1[0]) + y1[1];
+    div = (x1[2] - x0[2]) * hyj + (y1[2] - y0[2]) * hxi;
+    sct = sc;
+    denT = g.ht * (aT1 + aT2 + aT3 + aT4 + x1[0] - x0[0] + y1[0] - y0[0]) + hxi * hyj * rho;
+    a1 = x0[3];
+    a3 = y0[3];
+    a4 = y1[3];
+    b1 = x0[4];
+    b3 = y0[4];
+    b4 = y1[4];
+    q = p_pr * hxi * hyj / T_pr;
     hh = hxi * hyj;
   }
 
-  __device__ __forceinline__ void update(const PTStencil<R> &x, R &pn, R &tn) const {
-    const R t1 = (fluid & 1u) ? x.Tw : X1, t2 = (fluid & 2u) ? x.Te : X2;
-    const R t3 = (fluid & 4u) ? x.Ts : X3, t4 = (fluid & 8u) ? x.Tn : X4;
-    tn = (ht * (aT1 * t1 + aT2 * t2 + aT3 * t3 + aT4 * t4 + c1 * x.Pc * div) + sct) / denT;
+  // (a2, b2): apx, bpx of the east cell.  k, ke, kn: the cell, its east and
+  // its north neighbour.  A body neighbour contributes the fluid temperature
+  // on its wall (S:3838-3848: m*T_old + !m*T_wall with T_wall finite, i.e. a
+  // select).
+  __device__ __forceinline__ void update(const KGridT<R> &g, const KFieldsT<R> &fl, unsigned nb, unsigned i, unsigned k,
+                                         unsigned ke, unsigned kn, R a2, R b2, const PTStencil<R> &x, R &pn,
+                                         R &tn) const {
+    constexpr unsigned ALL = NB_W | NB_E | NB_S | NB_N;
+    R t1 = x.Tw, t2 = x.Te, t3 = x.Ts, t4 = x.Tn;
+    if ((nb & ALL) != ALL) {
+      if (!(nb & NB_W)) t1 = FLD(TW_U)[k];
+      if (!(nb & NB_E)) t2 = FLD(TW_U)[ke];
+      if (!(nb & NB_S)) t3 = FLD(TW_V)[k];
+      if (!(nb & NB_N)) t4 = FLD(TW_V)[kn];
+    }
+    const R ht = g.ht;
+    tn = (ht * (aT1 * t1 + aT2 * t2 + aT3 * t3 + aT4 * t4 + g.c1 * x.Pc * div) + sct) / denT;
     R s = a1 * x.Pw + a2 * x.Pe + a3 * x.Ps + a4 * x.Pn + b1 - b2 + b3 - b4;
-    if (has_gxb) s = s + gxb;
-    if (has_gxe) s = s - gxe;
-    pn = (ht * s + q) / (Ap + hh / (tn));
+    if (g.given_xb && (int)i == g.Nx_o0) s = s + FLD(FX)[k];       // S:3887
+    if (g.given_xe && (int)i == g.Nx_o1 - 1) s = s - FLD(FX)[ke];  // S:3888
+    pn = (ht * s + q) / (ht * (a1 + a2 + a3 + a4) + hh / (tn));
   }
 };
 
+// The T, p update of one cell with every value read from memory.
 template <typename R>
 __device__ __forceinline__ void pt_update(const KGridT<R> &g, const KFieldsT<R> &fl, const Nbr &n, const PTStencil<R> &x,
                                           R &pn, R &tn) {
+  const int fx[5] = {STS_FX, STS_DTX, STS_U, STS_APX, STS_BPX}, fy[5] = {STS_FY, STS_DTY, STS_V, STS_APY, STS_BPY};
+  R x0[5], x1[5], y0[5], y1[5];
+#pragma unroll
+  for (int q = 0; q < 5; q++) {
+    x0[q] = fl.f[fx[q]][n.ij];
+    x1[q] = fl.f[fx[q]][n.i1j];
+    y0[q] = fl.f[fy[q]][n.ij];
+    y1[q] = fl.f[fy[q]][n.ij1];
+  }
   PTCoef<R> c;
-  c.load(g, fl, n);
-  c.update(x, pn, tn);
+  c.set(g, n.i, n.j, x0, x1, y0, y1, FLD(RHO)[n.ij], FLD(SCT1)[n.ij], FLD(P_PR)[n.ij], FLD(T_PR)[n.ij]);
+  c.update(g, fl, g.nb[n.ij], n.i, n.ij, n.i1j, n.ij1, x1[3], x1[4], x, pn, tn);
 }
 
 template <typename R>
@@ -736,21 +761,6 @@ template <typename R>
 __device__ __forceinline__ PTStencil<R> stencil_global(const R *Po, const R *To, const Nbr &n) {
   return PTStencil<R>{Po[n.ij], To[n.ij], Po[n.i_1j], To[n.i_1j], Po[n.i1j], To[n.i1j],
                    Po[n.ij_1], To[n.ij_1], Po[n.ij1], To[n.ij1]};
-}
-
-// The first-sweep value of one cell from (Po, To): the update set gets the
-// new values, any other cell keeps its old ones.
-template <typename R>
-__device__ __forceinline__ void sweep1_cell(const KGridT<R> &g, const KFieldsT<R> &fl, const R *__restrict__ Po,
-                                            const R *__restrict__ To, int i, int j, R &pn, R &tn) {
-  const unsigned ij = (unsigned)i + (unsigned)j * (unsigned)g.Nx;
-  if (in_pt_set(g, i, j, ij)) {
-    const Nbr n((unsigned)i, (unsigned)j, (unsigned)g.Nx, (unsigned)g.Ny, g.px);
-    pt_update(g, fl, n, stencil_global(Po, To, n), pn, tn);
-  } else {
-    pn = Po[ij];
-    tn = To[ij];
-  }
 }
 
 // One sweep: reads (Po, To), writes (Pn, Tn) on every cell: the update set
@@ -786,133 +796,119 @@ __global__ void __launch_bounds__(BX *BY) k_sweep(KGridT<R> g, KFieldsT<R> fl, c
   if (red_p || red_T || red_p2 || red_T2) block_max_atomic<2, BX * BY>(r, MaxDst<2>{{red_p, red_T}, {red_p2, red_T2}});
 }
 
-// Two sweeps in one pass (temporal blocking): each block first sweeps its
-// tile plus a one-cell halo from (Po, To) into LDS, then sweeps the tile from
-// LDS into (Pn, Tn).  Same arithmetic as two k_sweep launches; the
-// intermediate p and T never go to HBM.  Residual maxima of both sweeps over
-// the tile cells go to (r1p, r1T) and (r2p, r2T).
-constexpr int S2X = 64, S2Y = 8;
+// Two sweeps in one pass (temporal blocking).  Same arithmetic as two k_sweep
+// launches; the intermediate p and T never go to memory.  Residual maxima of
+// both sweeps over the tile's cells go to (r1p, r1T) and (r2p, r2T).
+//
+// A workgroup is SR + 2 waves; wave w holds the 64 cells of row j0 - 1 + w
+// from column i0 - 2 on.  Every lane sweeps its cell once, and the waves of
+// the SR rows of the tile sweep theirs again: an east or west neighbour is the
+// next lane (a DPP move: no load, no LDS), a south or north one the same lane
+// of the next wave (LDS after the first sweep).  The second sweep is good on
+// lanes 2..61, the tile's SWEEP_X columns.  Every cell of the update set has
+// all its neighbours in the grid (the solve boxes leave the outer cells out;
+// periodic about OX, the columns wrap), so no clamped neighbour is ever
+// used; lanes off the grid load a clamped address and are not updated.
+//
+// What bounds it: the latency and the number of its vector loads.  A thread
+// issues 25 (34 with every neighbour loaded), all waves in one phase, where a
+// workgroup of whole-tile threads ran the halo ring first and its own cells
+// after it; each cell's factors stay in registers for the second sweep.
+// Tile of 6 rows at seven waves per SIMD (72 registers), k_sweep2 with the
+// ring phase before: 1920x384 28.8 -> 23.2 us, 3840x768 141.7 -> 118.6,
+// 1280x256 17.6 -> 10.5, 961x193 13.3 -> 10.9, 301x95 9.0 ->
+// 6.5.  Other heights at 1920x384: 2 rows 26.7, 4 26.8, 5 24.9, 8 27.1, 10
+// 24.3, 14 29.4; 64 registers (eight waves) spill, 33.2.
+constexpr int SWEEP_X = 60;
+template <int SR>
+struct SweepTile {
+  static constexpr int THREADS = 64 * (SR + 2);
+};
 
-// r: the thread's residuals of sweep 1 (p, T) and sweep 2 (p, T).
-template <typename R>
-__device__ __forceinline__ void sweep2_tile_body(const KGridT<R> &g, const KFieldsT<R> &fl, const R *__restrict__ Po,
-                                                 const R *__restrict__ To, R *__restrict__ Pn, R *__restrict__ Tn,
-                                                 int i0, int j0, int tx, int ty, int SX, int SY, R *sP, R *sT,
-                                                 unsigned long long (&r)[4]) {
-  const int Nx = g.Nx, Ny = g.Ny;
-  const int RX = SX + 2, RY = SY + 2;
-  const int tid = tx + ty * SX;
-  // Sweep 1 on the one-cell halo ring of the tile (its cells belong to the
-  // neighbouring tiles, which count their residuals).  Periodic about OX, the
-  // ring column left of the first grid column holds the last one, and the
-  // column right of the last grid column holds the first one: if the last
-  // column lies inside the tile, SY extra entries fill that LDS column.
-  const int NR = 2 * RX + 2 * SY;
-  const bool east_extra = g.px && i0 <= Nx - 1 && Nx - 1 < i0 + SX - 1;
-  const int NRx = NR + (east_extra ? SY : 0);
-  for (int q = tid; q < NRx; q += SX * SY) {
-    int rx, ry;
-    if (q >= NR) {
-      rx = Nx - i0 + 1;
-      ry = 1 + (q - NR);
-    } else if (q < RX) {
-      rx = q;
-      ry = 0;
-    } else if (q < 2 * RX) {
-      rx = q - RX;
-      ry = RY - 1;
-    } else if (q < 2 * RX + SY) {
-      rx = 0;
-      ry = 1 + (q - 2 * RX);
-    } else {
-      rx = RX - 1;
-      ry = 1 + (q - 2 * RX - SY);
-    }
-    int hi = i0 - 1 + rx;
-    const int hj = j0 - 1 + ry;
-    if (g.px) hi = (hi == -1) ? Nx - 1 : (hi == Nx) ? 0 : hi;
-    if (hi < 0 || hj < 0 || hi >= Nx || hj >= Ny) continue;
-    R pn, tn;
-    sweep1_cell(g, fl, Po, To, hi, hj, pn, tn);
-    sP[ry * RX + rx] = pn;
-    sT[ry * RX + rx] = tn;
-  }
-  // Sweep 1 on the thread's own cell; its factors stay in registers.
-  const int i = i0 + tx, j = j0 + ty;
-  const bool in = i < Nx && j < Ny;
-  const unsigned ij = in ? (unsigned)i + (unsigned)j * (unsigned)Nx : 0u;
-  const bool upd = in && in_pt_set(g, i, j, ij);
-  const Nbr n((unsigned)(in ? i : 0), (unsigned)(in ? j : 0), (unsigned)Nx, (unsigned)Ny, g.px);
-  const int cx = tx + 1, cy = ty + 1;
-  unsigned long long r1[2] = {0ull, 0ull};
-  PTCoef<R> c;
-  if (upd) {
-    c.load(g, fl, n);
-    const PTStencil<R> x = stencil_global(Po, To, n);
-    R pn, tn;
-    c.update(x, pn, tn);
-    r1[0] = absbits(pn - x.Pc);
-    r1[1] = absbits(tn - x.Tc);
-    sP[cy * RX + cx] = pn;
-    sT[cy * RX + cx] = tn;
-  } else if (in) {
-    sP[cy * RX + cx] = Po[ij];
-    sT[cy * RX + cx] = To[ij];
-  }
-  __syncthreads();
-  // Sweep 2 on the own cell from LDS.
-  unsigned long long r2[2] = {0ull, 0ull};
-  if (upd) {
-    // clamped neighbours map to the cell itself at the domain edge; periodic
-    // about OX, the LDS column beside the seam holds the wrapped neighbour
-    const int wx = cx - (g.px ? 1 : (int)(n.i - n.i_1)), ex = cx + (g.px ? 1 : (int)(n.i1 - n.i));
-    const int sy = cy - (int)((n.ij - n.ij_1) / (unsigned)Nx), ny = cy + (int)((n.ij1 - n.ij) / (unsigned)Nx);
-    const PTStencil<R> x{sP[cy * RX + cx], sT[cy * RX + cx], sP[cy * RX + wx], sT[cy * RX + wx],
-                         sP[cy * RX + ex], sT[cy * RX + ex], sP[sy * RX + cx], sT[sy * RX + cx],
-                         sP[ny * RX + cx], sT[ny * RX + cx]};
-    R pn, tn;
-    c.update(x, pn, tn);
-    Tn[ij] = tn;
-    Pn[ij] = pn;
-    r2[0] = absbits(pn - x.Pc);
-    r2[1] = absbits(tn - x.Tc);
-  } else if (in) {
-    Pn[ij] = sP[cy * RX + cx];
-    Tn[ij] = sT[cy * RX + cx];
-  }
-  r[0] = r1[0];
-  r[1] = r1[1];
-  r[2] = r2[0];
-  r[3] = r2[1];
-}
-
-// Tile (i0, j0) of SX x SY cells with its one-cell halo in LDS.
-template <typename R, int SX, int SY>
+template <typename R, int SR>
 __device__ __forceinline__ void sweep2_tile(const KGridT<R> &g, const KFieldsT<R> &fl, const R *__restrict__ Po,
                                             const R *__restrict__ To, R *__restrict__ Pn, R *__restrict__ Tn, int i0,
-                                            int j0, int tx, int ty, unsigned long long *r1p, unsigned long long *r1T,
+                                            int j0, unsigned long long *r1p, unsigned long long *r1T,
                                             unsigned long long *r2p, unsigned long long *r2T) {
-  __shared__ R sP[(SY + 2) * (SX + 2)], sT[(SY + 2) * (SX + 2)];
-  unsigned long long r[4];
-  sweep2_tile_body(g, fl, Po, To, Pn, Tn, i0, j0, tx, ty, SX, SY, sP, sT, r);
-  if (r1p || r1T || r2p || r2T) block_max_atomic<4, SX * SY>(r, MaxDst<4>{{r1p, r1T, r2p, r2T}, {}});
+  __shared__ R sP[SR + 2][64], sT[SR + 2][64];
+  const int Nx = g.Nx, Ny = g.Ny;
+  const int lane = (int)threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  int i = i0 - 2 + lane;
+  const int j = j0 - 1 + w;
+  const bool mine = lane >= 2 && lane < 2 + SWEEP_X && i < Nx && w >= 1 && w <= SR && j < Ny;  // a cell of the tile
+  if (g.px) {
+    if (i < 0) i += Nx;
+    while (i >= Nx) i -= Nx;
+  }
+  const bool in = i >= 0 && i < Nx && j >= 0 && j < Ny;
+  const unsigned ci = (unsigned)min(max(i, 0), Nx - 1), cj = (unsigned)min(max(j, 0), Ny - 1);
+  const unsigned k = ci + cj * (unsigned)Nx, kn = cj + 1u < (unsigned)Ny ? k + (unsigned)Nx : k,
+                 ks = cj > 0u ? k - (unsigned)Nx : k;
+  const unsigned nb = g.nb[k];
+  const bool upd = in && in_box(i, j, g.Nx_o0, g.Nx_o1, g.Ny_o0, g.Ny_o1) && (nb & NB_C);
+  // the last column's east neighbour wraps (the update set holds it only when periodic)
+  const unsigned ke = ci + 1u < (unsigned)Nx ? k + 1u : k + 1u - (unsigned)Nx;
+  R p = Po[k], T = To[k];  // then the values of the first sweep
+  unsigned long long r[4] = {0ull, 0ull, 0ull, 0ull};
+  PTCoef<R> c;
+  const bool work = __any(upd);
+  if (work) {
+    const int fx[5] = {STS_FX, STS_DTX, STS_U, STS_APX, STS_BPX}, fy[5] = {STS_FY, STS_DTY, STS_V, STS_APY, STS_BPY};
+    R x0[5], x1[5], y0[5], y1[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      x0[q] = fl.f[fx[q]][k];
+      y0[q] = fl.f[fy[q]][k];
+      y1[q] = fl.f[fy[q]][kn];
+    }
+    const R rho = FLD(RHO)[k], sc = FLD(SCT1)[k], p_pr = FLD(P_PR)[k], T_pr = FLD(T_PR)[k];
+    const R Ps = Po[ks], Ts = To[ks], Pnn = Po[kn], Tnn = To[kn];
+#pragma unroll
+    for (int q = 0; q < 5; q++) x1[q] = lane_east(x0[q]);
+    const PTStencil<R> x{p, T, lane_west(p), lane_west(T), lane_east(p), lane_east(T), Ps, Ts, Pnn, Tnn};
+    c.set(g, ci, cj, x0, x1, y0, y1, rho, sc, p_pr, T_pr);
+    if (upd) {
+      c.update(g, fl, nb, ci, k, ke, kn, x1[3], x1[4], x, p, T);
+      if (mine) {
+        r[0] = absbits(p - x.Pc);
+        r[1] = absbits(T - x.Tc);
+      }
+    }
+  }
+  sP[w][lane] = p;
+  sT[w][lane] = T;
+  __syncthreads();
+  if (w >= 1 && w <= SR) {
+    R pn = p, tn = T;
+    if (work) {
+      const R a2 = lane_east(c.a1), b2 = lane_east(c.b1);
+      const PTStencil<R> x{p, T, lane_west(p), lane_west(T), lane_east(p), lane_east(T),
+                           sP[w - 1][lane], sT[w - 1][lane], sP[w + 1][lane], sT[w + 1][lane]};
+      if (upd && mine) {
+        c.update(g, fl, nb, ci, k, ke, kn, a2, b2, x, pn, tn);
+        r[2] = absbits(pn - p);
+        r[3] = absbits(tn - T);
+      }
+    }
+    if (mine) {
+      Tn[k] = tn;
+      Pn[k] = pn;
+    }
+  }
+  if (r1p || r1T || r2p || r2T)
+    block_max_atomic<4, SweepTile<SR>::THREADS>(r, MaxDst<4>{{r1p, r1T, r2p, r2T}, {}});
 }
 
-// Six waves per SIMD (80 registers, three workgroups per CU): the pass is
-// bound by the latency of its two load phases, and the third resident
-// workgroup hides more of it.  Uniform factors come from the grid constants
-// (scalar registers), so nothing spills.
-template <typename R>
-__global__ void __launch_bounds__(S2X *S2Y) __attribute__((amdgpu_waves_per_eu(6, 8))) k_sweep2(KGridT<R> g, KFieldsT<R> fl, const R *__restrict__ Po,
+template <typename R, int SR>
+__global__ void __launch_bounds__((SweepTile<SR>::THREADS)) __attribute__((amdgpu_waves_per_eu(7, 8))) k_sweep2(KGridT<R> g, KFieldsT<R> fl, const R *__restrict__ Po,
                                                      const R *__restrict__ To, R *__restrict__ Pn,
                                                      R *__restrict__ Tn, unsigned long long *r1p,
                                                      unsigned long long *r1T, unsigned long long *r2p,
                                                      unsigned long long *r2T, Gate gate) {
   if (gated_out(gate)) return;
   int i0, j0;
-  tile_origin<S2X, S2Y>(g.Nx, i0, j0);
-  sweep2_tile<R, S2X, S2Y>(g, fl, Po, To, Pn, Tn, i0, j0, (int)threadIdx.x,
-                           (int)threadIdx.y, r1p, r1T, r2p, r2T);
+  tile_origin<SWEEP_X, SR>(g.Nx, i0, j0);
+  sweep2_tile<R, SR>(g, fl, Po, To, Pn, Tn, i0, j0, r1p, r1T, r2p, r2T);
 }
 
 // ---------------------------------------------------------------------------
@@ -2293,14 +2289,49 @@ __global__ void __launch_bounds__(BX *BY) k_continuity(KGrid g, KFields fl, doub
 // work is the same code as the single-case kernels above.  par = 1 selects
 // the p/T partners as the current p, T.
 // ---------------------------------------------------------------------------
+//
+// The pointers of the table are read from memory, where the compiler cannot
+// see that they name device memory and would use flat accesses (which count
+// as LDS accesses too); in_memory says so, as a kernel argument's pointer does
+// by itself.
+template <typename T>
+__device__ __forceinline__ T *in_memory(T *p) {
+  return (T *)(__attribute__((address_space(1))) T *)(uintptr_t)p;
+}
+
 template <typename R>
 __device__ __forceinline__ KFieldsT<R> fields_at(const BatchCase<R> &c, int par) {
-  KFieldsT<R> f = c.f;
+  KFieldsT<R> f;
+#pragma unroll
+  for (int q = 0; q < STS_NFIELDS; q++) f.f[q] = in_memory(c.f.f[q]);
   if (par) {
-    f.f[STS_P] = c.p_alt;
-    f.f[STS_T] = c.T_alt;
+    f.f[STS_P] = in_memory(c.p_alt);
+    f.f[STS_T] = in_memory(c.T_alt);
   }
   return f;
+}
+
+template <typename R>
+__device__ __forceinline__ KGridT<R> grid_of(const BatchCase<R> &c) {
+  KGridT<R> g = c.g;
+  g.hx = in_memory(g.hx);
+  g.hy = in_memory(g.hy);
+  g.m = in_memory(g.m);
+  g.nb = in_memory(g.nb);
+  g.vol = in_memory(g.vol);
+  g.bodies = in_memory(g.bodies);
+  return g;
+}
+
+__device__ __forceinline__ AABuf aa_of(const BatchCase<double> &c) {
+  AABuf a = c.aa;
+  a.gp = in_memory(a.gp);
+  a.D = in_memory(a.D);
+  a.fp = in_memory(a.fp);
+  a.part = in_memory(a.part);
+  a.gram = in_memory(a.gram);
+  a.gam = in_memory(a.gam);
+  return a;
 }
 
 // The assembly forms Gamma and D itself (assemble_inl_tile), except in the
@@ -2311,8 +2342,8 @@ template <typename R, int TX, int TY>
 __global__ void __launch_bounds__(TX *TY) kb_assemble(const BatchCase<R> *C, const BatchTile *T, int k, int par) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k}) || (k == 0 && !c.inline0)) return;
-  assemble_inl_tile<R, TX, TY>(c.g, fields_at(c, par), t.x * TX, t.y * TY, (int)threadIdx.x % TX,
+  if (gated_out(Gate{in_memory(c.ctrl), k}) || (k == 0 && !c.inline0)) return;
+  assemble_inl_tile<R, TX, TY>(grid_of(c), fields_at(c, par), t.x * TX, t.y * TY, (int)threadIdx.x % TX,
                                (int)threadIdx.x / TX);
 }
 
@@ -2320,25 +2351,25 @@ template <typename R, int TX, int TY>
 __global__ void __launch_bounds__(TX *TY) kb_assemble_arr(const BatchCase<R> *C, const BatchTile *T, int k, int par) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k}) || k != 0 || c.inline0) return;
-  assemble_cell(c.g, fields_at(c, par), t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX);
+  if (gated_out(Gate{in_memory(c.ctrl), k}) || k != 0 || c.inline0) return;
+  assemble_cell(grid_of(c), fields_at(c, par), t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX);
 }
 
 // Pass of two fused sweeps from parity par; first/last: whether it holds
-// loop 3's first / last sweep (their residuals go to the loop-2 test).  Six
+// loop 3's first / last sweep (their residuals go to the loop-2 test).  Seven
 // waves per SIMD, as k_sweep2.
-template <typename R, int SX, int SY>
-__global__ void __launch_bounds__(SX *SY) __attribute__((amdgpu_waves_per_eu(6, 8))) kb_sweep2(const BatchCase<R> *C, const BatchTile *T, int k, int par,
+template <typename R, int SR>
+__global__ void __launch_bounds__((SweepTile<SR>::THREADS)) __attribute__((amdgpu_waves_per_eu(7, 8))) kb_sweep2(const BatchCase<R> *C, const BatchTile *T, int k, int par,
                                                     int first, int last) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const KFieldsT<R> f = fields_at(c, par);
-  const R *Pi = par ? c.p_alt : c.f.f[STS_P], *Ti = par ? c.T_alt : c.f.f[STS_T];
-  R *Po = par ? c.f.f[STS_P] : c.p_alt, *To = par ? c.f.f[STS_T] : c.T_alt;
-  sweep2_tile<R, SX, SY>(c.g, f, Pi, Ti, Po, To, t.x * SX, t.y * SY, (int)threadIdx.x % SX, (int)threadIdx.x / SX,
-                         first ? c.lred + 4 : nullptr, first ? c.lred + 5 : nullptr, last ? c.lred + 2 : nullptr,
-                         last ? c.lred + 3 : nullptr);
+  const R *Pi = f.f[STS_P], *Ti = f.f[STS_T];
+  R *Po = in_memory(par ? c.f.f[STS_P] : c.p_alt), *To = in_memory(par ? c.f.f[STS_T] : c.T_alt);
+  unsigned long long *lr = in_memory(c.lred);
+  sweep2_tile<R, SR>(grid_of(c), f, Pi, Ti, Po, To, t.x * SWEEP_X, t.y * SR, first ? lr + 4 : nullptr,
+                     first ? lr + 5 : nullptr, last ? lr + 2 : nullptr, last ? lr + 3 : nullptr);
 }
 
 // Single sweep (odd sweep counts).
@@ -2347,11 +2378,11 @@ __global__ void __launch_bounds__(TX *TY) kb_sweep(const BatchCase<R> *C, const 
                                                    int first, int last) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const KFieldsT<R> fl = fields_at(c, par);
-  const KGridT<R> &g = c.g;
-  const R *Po = par ? c.p_alt : c.f.f[STS_P], *To = par ? c.T_alt : c.f.f[STS_T];
-  R *Pn = par ? c.f.f[STS_P] : c.p_alt, *Tn = par ? c.f.f[STS_T] : c.T_alt;
+  const KGridT<R> g = grid_of(c);
+  const R *Po = fl.f[STS_P], *To = fl.f[STS_T];
+  R *Pn = in_memory(par ? c.f.f[STS_P] : c.p_alt), *Tn = in_memory(par ? c.f.f[STS_T] : c.T_alt);
   const int i = t.x * TX + (int)threadIdx.x % TX, j = t.y * TY + (int)threadIdx.x / TX;
   unsigned long long r[2] = {0ull, 0ull};
   if (i < g.Nx && j < g.Ny) {
@@ -2370,19 +2401,20 @@ __global__ void __launch_bounds__(TX *TY) kb_sweep(const BatchCase<R> *C, const 
       Tn[ij] = To[ij];
     }
   }
-  block_max_atomic<2, TX * TY>(r, MaxDst<2>{{last ? c.lred + 2 : nullptr, last ? c.lred + 3 : nullptr},
-                                         {first ? c.lred + 4 : nullptr, first ? c.lred + 5 : nullptr}});
+  unsigned long long *lr = in_memory(c.lred);
+  block_max_atomic<2, TX * TY>(r, MaxDst<2>{{last ? lr + 2 : nullptr, last ? lr + 3 : nullptr},
+                                         {first ? lr + 4 : nullptr, first ? lr + 5 : nullptr}});
 }
 
 template <typename R, int TX, int TY>
 __global__ void __launch_bounds__(TX *TY) kb_correct(const BatchCase<R> *C, const BatchTile *T, int k, int par) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const KFieldsT<R> f = fields_at(c, par);
   unsigned long long r[2] = {0ull, 0ull};
-  correct_cell(c.g, f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, 1, r);
-  block_max_atomic<2, TX * TY>(r, MaxDst<2>{{c.lred + 0, c.lred + 1}, {}});
+  correct_cell(grid_of(c), f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, 1, r);
+  block_max_atomic<2, TX * TY>(r, MaxDst<2>{{in_memory(c.lred), in_memory(c.lred) + 1}, {}});
 }
 
 template <typename R, int TX, int TY>
@@ -2390,9 +2422,9 @@ __global__ void __launch_bounds__(TX *TY) kb_wall(const BatchCase<R> *C, const B
                                                   int parts) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const KFieldsT<R> f = fields_at(c, par);
-  wall_cell(c.g, f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, parts);
+  wall_cell(grid_of(c), f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, parts);
 }
 
 template <typename R>
@@ -2400,13 +2432,13 @@ __global__ void __launch_bounds__(WALL_OPS_PER_TILE) kb_wall_ops(const BatchCase
                                                                  int par, int parts) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const int q = t.x * WALL_OPS_PER_TILE + (int)threadIdx.x;
   if (q >= c.nwops) return;
-  const WallOp o = c.wops[q];
+  const WallOp o = in_memory(c.wops)[q];
   const unsigned kind = o.kb & 7u;
   const int need = kind == WOP_U ? STS_BC_SLIP_U : kind == WOP_V ? STS_BC_SLIP_V : STS_BC_JUMP;
-  if (parts & need) apply_wall_op(c.g, fields_at(c, par), o);
+  if (parts & need) apply_wall_op(grid_of(c), fields_at(c, par), o);
 }
 
 // The fluxes and thermal coefficients (FLUX_PART); the assembly forms the
@@ -2415,11 +2447,12 @@ template <typename R, int TX, int TY>
 __global__ void __launch_bounds__(TX *TY) kb_flux_diff(const BatchCase<R> *C, const BatchTile *T, int k, int par) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const KFieldsT<R> f = fields_at(c, par);
   FluxIn<R> x;
-  x.template load<true, false>(c.g, f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX);
-  x.apply_flux(c.g, f);
+  const KGridT<R> g = grid_of(c);
+  x.template load<true, false>(g, f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX);
+  x.apply_flux(g, f);
 }
 
 // Batched Anderson steps (FP64): the single-context kernels' code per tile
@@ -2433,8 +2466,8 @@ __device__ __forceinline__ AASel case_sel(const BatchCase<double> &c, const AABa
 #pragma unroll
   for (int j = 0; j < MAX_AA; j++) {
     sel.slot[j] = bs.slot[j];
-    sel.dG[j] = j < bs.n ? c.aa_dG[bs.slot[j]] : nullptr;
-    sel.dF[j] = j < bs.n ? c.aa_dF[bs.slot[j]] : nullptr;
+    sel.dG[j] = in_memory(j < bs.n ? c.aa_dG[bs.slot[j]] : nullptr);
+    sel.dF[j] = in_memory(j < bs.n ? c.aa_dF[bs.slot[j]] : nullptr);
   }
   return sel;
 }
@@ -2453,8 +2486,8 @@ __global__ void __launch_bounds__(TX *TY) kb_aa_begin(const BatchCase<double> *C
   const AAFields s = case_state(c, 0);
   const int k = i + j * c.g.Nx;
   const double g4[4] = {s.x[0][k], s.x[1][k], s.x[2][k], s.x[3][k]}, z[4] = {0.0, 0.0, 0.0, 0.0};
-  store4(c.aa.gp + 4 * (size_t)k, g4);
-  store4(c.aa.D + 4 * (size_t)k, z);
+  store4(in_memory(c.aa.gp) + 4 * (size_t)k, g4);
+  store4(in_memory(c.aa.D) + 4 * (size_t)k, z);
 }
 
 // Partial slot of a tile: its position in the case's row-major tile grid.
@@ -2463,23 +2496,23 @@ __global__ void __launch_bounds__(TX *TY) kb_aa_store(const BatchCase<double> *C
                                                       AABatchSel bs) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<double> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k + 1})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k + 1})) return;
   const AASel sel = case_sel(c, bs);
   const int i = t.x * TX + (int)threadIdx.x % TX, j = t.y * TY + (int)threadIdx.x / TX;
   double acc[2 * NM];
 #pragma unroll
   for (int q = 0; q < 2 * NM; q++) acc[q] = 0.0;
-  if (i < c.g.Nx && j < c.g.Ny) aa_store_cell<NM>(case_state(c, par), c.aa, sel, i + j * c.g.Nx, acc);
-  if (bs.n > 0) aa_store_sums<NM, TX * TY>(acc, c.aa, t.y * ((c.g.Nx + TX - 1) / TX) + t.x, sel.n);
+  if (i < c.g.Nx && j < c.g.Ny) aa_store_cell<NM>(case_state(c, par), aa_of(c), sel, i + j * c.g.Nx, acc);
+  if (bs.n > 0) aa_store_sums<NM, TX * TY>(acc, aa_of(c), t.y * ((c.g.Nx + TX - 1) / TX) + t.x, sel.n);
 }
 
 // One workgroup per case.
 template <int NM>
 __global__ void __launch_bounds__(AA_SOLVE_THREADS) kb_aa_solve(const BatchCase<double> *C, int k, AABatchSel bs) {
   const BatchCase<double> &c = C[blockIdx.x];
-  if (gated_out(Gate{c.ctrl, k + 1})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k + 1})) return;
   __shared__ double gam[NM];
-  aa_solve_group<NM, AA_SOLVE_THREADS>(c.aa, case_sel(c, bs), gam, true);
+  aa_solve_group<NM, AA_SOLVE_THREADS>(aa_of(c), case_sel(c, bs), gam, true);
 }
 
 // The mix without the flux part (the batched flux and diffusion pass follows).
@@ -2488,9 +2521,10 @@ __global__ void __launch_bounds__(TX *TY) kb_aa_mix(const BatchCase<double> *C, 
                                                     AABatchSel bs) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<double> &c = C[t.c];
-  if (gated_out(Gate{c.ctrl, k + 1})) return;
+  if (gated_out(Gate{in_memory(c.ctrl), k + 1})) return;
   __shared__ double sp[TY + 1][TX + 1], sT[TY + 1][TX + 1];
-  aa_mix_tile<NM, TX, TY, false>(c.g, fields_at(c, par), case_state(c, par), c.aa, case_sel(c, bs), c.aa.gam,
+  aa_mix_tile<NM, TX, TY, false>(grid_of(c), fields_at(c, par), case_state(c, par), aa_of(c), case_sel(c, bs),
+                                 in_memory(c.aa.gam),
                                  t.x * TX, t.y * TY, (int)threadIdx.x % TX, (int)threadIdx.x / TX, sp, sT, nullptr);
 }
 
@@ -2501,9 +2535,9 @@ __global__ void __launch_bounds__(EDGE_THREADS) kb_edges(const BatchCase<R> *C, 
   const Gate gate{c.ctrl, k};
   if (gated_out(gate)) return;
   const KFieldsT<R> f = fields_at(c, par);
-  const LoopTest lt{c.ctrl, c.lred, c.log + 6 * (size_t)k, c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w,
+  const LoopTest lt{in_memory(c.ctrl), in_memory(c.lred), in_memory(c.log) + 6 * (size_t)k, c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w,
                     c.stall_ratio};
-  edges_block(c.g, f, parts, c.probe, gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
+  edges_block(grid_of(c), f, parts, in_memory(c.probe), gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
 }
 
 // Opens every case's loop 2: control, log (6 N_I words), slotted words.
@@ -2555,7 +2589,15 @@ template <typename R>
 hipError_t launch_sweep2(const KGridT<R> &g, const KFieldsT<R> &f, const R *Po, const R *To, R *Pn, R *Tn,
                          unsigned long long *r1p, unsigned long long *r1T, unsigned long long *r2p,
                          unsigned long long *r2T, hipStream_t s, Gate gate) {
-  hipLaunchKernelGGL(k_sweep2<R>, (grid_tiles<S2X, S2Y>(g)), dim3(S2X, S2Y), 0, s, g, f, Po, To, Pn, Tn, r1p, r1T, r2p, r2T, gate);
+  // 6 rows per tile; 2 where that leaves most of the 256 CUs without a
+  // workgroup (240x48, 32 tiles of 6 rows: 5.7 against 7.1 us; level from 64
+  // tiles on: 301x95, 96 tiles, 6.3 both)
+  if (grid_tiles<SWEEP_X, 6>(g).x < 64)
+    hipLaunchKernelGGL((k_sweep2<R, 2>), (grid_tiles<SWEEP_X, 2>(g)), dim3(SweepTile<2>::THREADS), 0, s, g, f, Po, To,
+                       Pn, Tn, r1p, r1T, r2p, r2T, gate);
+  else
+    hipLaunchKernelGGL((k_sweep2<R, 6>), (grid_tiles<SWEEP_X, 6>(g)), dim3(SweepTile<6>::THREADS), 0, s, g, f, Po, To,
+                       Pn, Tn, r1p, r1T, r2p, r2T, gate);
   return hipGetLastError();
 }
 template <typename R>
@@ -2737,7 +2779,7 @@ hipError_t launch_continuity(const KGrid &g, const KFields &f, double *cs, doubl
 // Batched launches; tile shape variants (the autotuner's choices)
 // ---------------------------------------------------------------------------
 const int CELL_TILES[NVARIANT][2] = {{64, 4}, {64, 8}, {128, 2}, {32, 8}};
-const int SWEEP_TILES[NVARIANT][2] = {{64, 8}, {64, 4}, {128, 4}, {64, 16}};
+const int SWEEP_TILES[NVARIANT][2] = {{SWEEP_X, 6}, {SWEEP_X, 4}, {SWEEP_X, 8}, {SWEEP_X, 10}};
 
 #define CELL_SWITCH(v, KERNEL, ...)                                                                   \
   switch (v) {                                                                                        \
@@ -2746,6 +2788,9 @@ const int SWEEP_TILES[NVARIANT][2] = {{64, 8}, {64, 4}, {128, 4}, {64, 16}};
     case 2: hipLaunchKernelGGL((KERNEL<R, 128, 2>), dim3(ntiles), dim3(256), 0, s, __VA_ARGS__); break; \
     default: hipLaunchKernelGGL((KERNEL<R, 32, 8>), dim3(ntiles), dim3(256), 0, s, __VA_ARGS__); break; \
   }
+
+#define SWEEP_LAUNCH(SR) \
+  hipLaunchKernelGGL((kb_sweep2<R, SR>), dim3(ntiles), dim3(SweepTile<SR>::THREADS), 0, s, C, T, k, par, a, b)
 
 #define AA_SWITCH(v, NM, KERNEL, ...)                                                                 \
   switch (v) {                                                                                        \
@@ -2809,12 +2854,10 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
     case BK_FLUX_DIFF: CELL_SWITCH(variant, kb_flux_diff, C, T, k, par); break;
     case BK_SWEEP2:
       switch (variant) {
-        case 0: hipLaunchKernelGGL((kb_sweep2<R, 64, 8>), dim3(ntiles), dim3(512), 0, s, C, T, k, par, a, b); break;
-        case 1: hipLaunchKernelGGL((kb_sweep2<R, 64, 4>), dim3(ntiles), dim3(256), 0, s, C, T, k, par, a, b); break;
-        case 2: hipLaunchKernelGGL((kb_sweep2<R, 128, 4>), dim3(ntiles), dim3(512), 0, s, C, T, k, par, a, b); break;
-        default:
-          hipLaunchKernelGGL((kb_sweep2<R, 64, 16>), dim3(ntiles), dim3(1024), 0, s, C, T, k, par, a, b);
-          break;
+        case 0: SWEEP_LAUNCH(6); break;
+        case 1: SWEEP_LAUNCH(4); break;
+        case 2: SWEEP_LAUNCH(8); break;
+        default: SWEEP_LAUNCH(10); break;
       }
       break;
     case BK_EDGES:
@@ -2826,6 +2869,7 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
   return hipGetLastError();
 }
 #undef CELL_SWITCH
+#undef SWEEP_LAUNCH
 template hipError_t launch_batch<double>(int, int, const BatchCase<double> *, int, const BatchTile *, int, int, int,
                                          int, int, hipStream_t);
 template hipError_t launch_batch<float>(int, int, const BatchCase<float> *, int, const BatchTile *, int, int, int,
