@@ -816,8 +816,8 @@ __global__ void __launch_bounds__(BX *BY) k_sweep(KGridT<R> g, KFieldsT<R> fl, c
 // after it; each cell's factors stay in registers for the second sweep.
 // Tile of 6 rows at seven waves per SIMD (72 registers), k_sweep2 with the
 // ring phase before: 1920x384 28.8 -> 23.2 us, 3840x768 141.7 -> 118.6,
-// 1280x256 17.6 -> 10.5, 961x193 13.3 -> 10.9, 301x95 9.0 ->
-// 6.5.  Other heights at 1920x384: 2 rows 26.7, 4 26.8, 5 24.9, 8 27.1, 10
+// 1500x375 24.7 -> 19.5, 1280x256 17.6 -> 13.4, 961x193 13.3 -> 10.5, 301x95
+// 9.0 -> 6.6.  Other heights at 1920x384: 2 rows 26.7, 4 26.8, 5 24.9, 8 27.1, 10
 // 24.3, 14 29.4; 64 registers (eight waves) spill, 33.2.
 constexpr int SWEEP_X = 60;
 template <int SR>
@@ -2590,8 +2590,8 @@ hipError_t launch_sweep2(const KGridT<R> &g, const KFieldsT<R> &f, const R *Po, 
                          unsigned long long *r1p, unsigned long long *r1T, unsigned long long *r2p,
                          unsigned long long *r2T, hipStream_t s, Gate gate) {
   // 6 rows per tile; 2 where that leaves most of the 256 CUs without a
-  // workgroup (240x48, 32 tiles of 6 rows: 5.7 against 7.1 us; level from 64
-  // tiles on: 301x95, 96 tiles, 6.3 both)
+  // workgroup (240x48, 32 tiles of 6 rows: 5.7 against 6.6 us; 301x95, 96
+  // tiles: 6.3 against 6.6; 512x128, 198 tiles: 7.3 against 6.6)
   if (grid_tiles<SWEEP_X, 6>(g).x < 64)
     hipLaunchKernelGGL((k_sweep2<R, 2>), (grid_tiles<SWEEP_X, 2>(g)), dim3(SweepTile<2>::THREADS), 0, s, g, f, Po, To,
                        Pn, Tn, r1p, r1T, r2p, r2T, gate);
