@@ -752,7 +752,7 @@ extern "C" int sts_correct(sts_ctx *c, double *res) {
   if (int e = diff_inputs_change(c)) return e;
   HIP_OK(hipMemsetAsync(c->red, 0, sizeof(unsigned long long) * NSLOT * SLOT_STRIDE, c->stream));
   const int t = timed_begin(c, STS_K_CORRECT);
-  HIP_OK(launch_correct(c->g, c->fields(), c->red, c->red + 1, 1, c->stream));
+  HIP_OK(launch_correct(c->g, c->fields(), c->red, c->red + 1, 1, false, c->stream));
   timed_end(c, t);
   int rc = read_red(c, 2, false);
   if (rc) return rc;
@@ -789,7 +789,7 @@ static int enqueue_bcs(sts_ctx *c, int parts, bool probe) {
   }
   if (edge || probe) {
     const int t = timed_begin(c, STS_K_EDGES);
-    HIP_OK(launch_edges(c->g, c->fields(), edge, probe ? c->probe : nullptr, c->stream));
+    HIP_OK(launch_edges(c->g, c->fields(), edge, false, probe ? c->probe : nullptr, c->stream));
     timed_end(c, t);
   }
   return STS_OK;
@@ -872,22 +872,26 @@ extern "C" int sts_continuity(sts_ctx *c, double *cont_stat, double *cont, doubl
 extern "C" int sts_outer_iteration(sts_ctx *c, int n_pc, double *res, double *res_p0T0, double *p_probe) {
   if (!c || n_pc < 1 || n_pc > MAX_SWEEPS) return fail(STS_ERR_ARG, "N_I_p_c must be 1..62");
   const int nslots = 2 + 2 * n_pc;
-  if (int e = refresh_diff(c)) return e;
   HIP_OK(hipMemsetAsync(c->red, 0, sizeof(unsigned long long) * NSLOT * SLOT_STRIDE, c->stream));
-  int t = timed_begin(c, STS_K_ASSEMBLE);
-  HIP_OK(launch_assemble(c->g, c->fields(), c->stream));
+  // as the device-side loops: Gamma and D formed in the assembly where that
+  // gives what the arrays hold, and the arrays themselves written on demand
+  const bool inl = c->diff_inline_ok;
+  int t = timed_begin(c, inl ? STS_K_ASSEMBLE_INL : STS_K_ASSEMBLE);
+  HIP_OK(launch_assemble(c->g, c->fields(), c->stream, Gate{nullptr, 0}, inl));
   timed_end(c, t);
   int rc = run_sweeps(c, n_pc);
   if (rc) return rc;
+  const KFields kf = c->fields();
   t = timed_begin(c, STS_K_CORRECT);
-  HIP_OK(launch_correct(c->g, c->fields(), c->red, c->red + 1, 1, c->stream));
+  HIP_OK(launch_correct(c->g, kf, c->red, c->red + 1, 1, true, c->stream));
   timed_end(c, t);
-  if ((rc = enqueue_bcs(c, STS_BC_ALL, true))) return rc;
-  t = timed_begin(c, STS_K_FLUX_DIFF);
-  HIP_OK(launch_flux_diff(c->g, c->fields(), c->stream));
+  t = timed_begin(c, STS_K_WALL);
+  HIP_OK(launch_wall_ops(c->g, kf, c->wall_ops, c->n_wall_ops, true, c->stream));
   timed_end(c, t);
-  c->diff_inline_ok = true;
-  c->diff_stale = false;
+  t = timed_begin(c, STS_K_EDGES);
+  HIP_OK(launch_edges(c->g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, true, c->probe, c->stream));
+  timed_end(c, t);
+  c->diff_inline_ok = c->diff_stale = true;
   if ((rc = read_red(c, nslots, true))) return rc;
   if (res) {
     res[0] = bits_to_double(c->h_red[0]);
@@ -1007,9 +1011,9 @@ static int enqueue_outer(sts_ctx *c, const Loop2State<R> &st, int k, int n, Loop
     return kf;
   };
   int par = (int)(((long long)k * sweep_passes(c, n)) & 1);
-  // after the loop's first flux pass the assembly forms the diffusion
-  // coefficients from the inputs that pass saw; the pass itself writes only
-  // the fluxes and thermal coefficients
+  // after the loop's first iteration the assembly forms the diffusion
+  // coefficients from the inputs its correction pass saw; that pass itself
+  // writes only the fluxes and thermal coefficients
   const bool inl = k > 0 || st.inline0;
   int t = timed_begin(c, st.kid + (inl ? STS_K_ASSEMBLE_INL : STS_K_ASSEMBLE), k);
   HIP_OK(launch_assemble(g, fields_at(par), c->stream, gate, inl));
@@ -1037,31 +1041,23 @@ static int enqueue_outer(sts_ctx *c, const Loop2State<R> &st, int k, int n, Loop
   const bool aa = st.aa_m > 0 && (k + 1) % st.aa_every == 0;
   AASel sel{};
   if (aa) sel = anderson_select(c, k, st.aa_m, st.aa_every);
+  // the correction pass forms the fluxes, unless an Anderson mix does: then
+  // run_loop2 runs the flux pass for the loop's last iteration (where the
+  // mix, gated on k + 1, does not run)
+  const bool flux = !(aa && sel.n > 0);
   t = timed_begin(c, st.kid + STS_K_CORRECT, k);
-  HIP_OK(launch_correct(g, kf, lr + 0, lr + 1, 1, c->stream, gate));
+  HIP_OK(launch_correct(g, kf, lr + 0, lr + 1, 1, flux, c->stream, gate));
   timed_end(c, t);
   t = timed_begin(c, st.kid + STS_K_WALL, k);
-  HIP_OK(launch_wall(g, kf, STS_BC_SLIP_U | STS_BC_SLIP_V | STS_BC_JUMP, c->stream, gate, c->wall_ops,
-                     k == 0 ? c->n_wall_ops : c->n_wall_var));
+  HIP_OK(launch_wall_ops(g, kf, c->wall_ops, k == 0 ? c->n_wall_ops : c->n_wall_var, flux, c->stream, gate));
   timed_end(c, t);
   lt.lred = lr;
   lt.log_k += 6 * (size_t)k;
   t = timed_begin(c, st.kid + STS_K_EDGES, k);
-  HIP_OK(launch_edges(g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, c->probe, c->stream, gate,
-                      lt));
+  HIP_OK(launch_edges(g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, flux, c->probe, c->stream,
+                      gate, lt));
   timed_end(c, t);
-  if (aa) {
-    int r;
-    if ((r = enqueue_anderson(c, st, kf, k, sel))) return r;
-  }
-  // an Anderson mix forms the fluxes itself, and for the loop's last
-  // iteration (where the mix, gated on k + 1, does not run) run_loop2 runs
-  // the pass once the loop has stopped
-  if (aa && sel.n > 0) return STS_OK;
-  t = timed_begin(c, st.kid + STS_K_FLUX_DIFF, k);
-  HIP_OK(launch_flux_diff(g, kf, c->stream, gate, FLUX_PART));
-  timed_end(c, t);
-  return STS_OK;
+  return aa ? enqueue_anderson(c, st, kf, k, sel) : STS_OK;
 }
 
 // Runs one loop 2 on the device: outer iterations are enqueued in batches
@@ -1133,7 +1129,7 @@ static int ensure_loop_buffers(sts_ctx *c, int n_iter) {
 
 // Copies n_iter iterations of the residual log and the probe to the host.
 // With neither asked for the step returns without waiting for its last
-// launches (the loop's flux pass, iterations gated out past the stop): the
+// launches (an Anderson loop's flux pass, iterations gated out past the stop): the
 // next step's launches queue behind them on the context's stream, and every
 // call that hands device data back waits for the stream.
 static int finish_step(sts_ctx *c, int n_iter, double *res_log, double *p_probe) {
@@ -1276,11 +1272,9 @@ static constexpr unsigned long long WIDEN_MASK =
 // of an outer iteration builds it (after a new start of loop 2).
 static int rebuild_derived(sts_ctx *c, hipStream_t s) {
   const KFields kf = c->fields();
-  HIP_OK(launch_correct(c->g, kf, nullptr, nullptr, 0, s));
-  HIP_OK(launch_wall(c->g, kf, STS_BC_SLIP_U | STS_BC_SLIP_V | STS_BC_JUMP, s, Gate{nullptr, 0}, c->wall_ops,
-                     c->n_wall_ops));
-  HIP_OK(launch_edges(c->g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, nullptr, s));
-  HIP_OK(launch_flux_diff(c->g, kf, s, Gate{nullptr, 0}, FLUX_PART));
+  HIP_OK(launch_correct(c->g, kf, nullptr, nullptr, 0, true, s));
+  HIP_OK(launch_wall_ops(c->g, kf, c->wall_ops, c->n_wall_ops, true, s));
+  HIP_OK(launch_edges(c->g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, true, nullptr, s));
   c->diff_inline_ok = c->diff_stale = true;
   return STS_OK;
 }
@@ -1959,8 +1953,7 @@ static int run_batch_loop2(sts_batch *b, BatchCase<R> *C, int n_pc, int N_I, int
         par ^= 1;
       }
       HIP_OK(launch_batch<R>(BK_CORRECT, cv, C, n, L.cell, L.n_cell, k, par, 0, 0, s));
-      HIP_OK(launch_batch<R>(BK_WALL_OPS, 0, C, n, L.wall, L.n_wall, k, par,
-                             STS_BC_SLIP_U | STS_BC_SLIP_V | STS_BC_JUMP, 0, s));
+      HIP_OK(launch_batch<R>(BK_WALL_OPS, 0, C, n, L.wall, L.n_wall, k, par, 0, 0, s));
       HIP_OK(launch_batch<R>(BK_EDGES, 0, C, n, nullptr, 0, k, par,
                              STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, 0, s));
       if constexpr (sizeof(R) == sizeof(double))
@@ -1978,7 +1971,6 @@ static int run_batch_loop2(sts_batch *b, BatchCase<R> *C, int n_pc, int N_I, int
             HIP_OK(launch_batch_aa(BKA_MIX, cv, C, n, L.cell, L.n_cell, k, par, bs, s));
           }
         }
-      HIP_OK(launch_batch<R>(BK_FLUX_DIFF, cv, C, n, L.cell, L.n_cell, k, par, 0, 0, s));
       if (k == check) {
         HIP_OK(hipMemcpyAsync(b->h_ctrl, b->ctrl, sizeof(LoopCtrl) * n, hipMemcpyDeviceToHost, s));
         HIP_OK(hipEventRecord(b->ev_ctrl, s));
@@ -2130,8 +2122,7 @@ extern "C" int sts_batch_time_step(sts_batch *b, const sts_loop_control *lc, con
 
 // Times the bulk kernels of each tile variant on the current state (the
 // timed launches only rewrite what the next outer iteration recomputes before
-// reading it: assembly outputs, fluxes from unchanged inputs, and the p/T
-// partners), then keeps the fastest.  The assembly is timed in the form the
+// reading it: assembly outputs and the p/T partners), then keeps the fastest.  The assembly is timed in the form the
 // loops use after their first iteration (Gamma and D formed in the tile).
 extern "C" int sts_batch_autotune(sts_batch *b, int reps, int *cell_variant, int *sweep_variant, double *ms) {
   if (!b || reps < 1) return fail(STS_ERR_ARG, "bad autotune arguments");
@@ -2145,10 +2136,8 @@ extern "C" int sts_batch_autotune(sts_batch *b, int reps, int *cell_variant, int
   for (int v = 0; v < NVARIANT; v++) {
     for (int pass = 0; pass < 2; pass++) {  // pass 0 warms up
       HIP_OK(hipEventRecord(b->ev0, s));
-      for (int r = 0; r < reps; r++) {
+      for (int r = 0; r < reps; r++)
         HIP_OK(launch_batch<double>(BK_ASSEMBLE, v, b->C64, n, b->cell_t[v], b->n_cell[v], 0, 0, 0, 0, s));
-        HIP_OK(launch_batch<double>(BK_FLUX_DIFF, v, b->C64, n, b->cell_t[v], b->n_cell[v], 0, 0, 0, 0, s));
-      }
       HIP_OK(hipEventRecord(b->ev1, s));
       HIP_OK(hipEventSynchronize(b->ev1));
       float f = 0;

@@ -917,57 +917,20 @@ __global__ void __launch_bounds__((SweepTile<SR>::THREADS)) __attribute__((amdgp
 // ij needs rho of the west/south cell; it is recomputed here from p and T
 // with the same operations, so no second pass is needed.
 // ---------------------------------------------------------------------------
-template <typename R>
-__device__ __forceinline__ R rho_of(const uint8_t *m, const R *p, const R *T, unsigned c) {
-  return m[c] ? p[c] / T[c] : R(0.0);
-}
-
-template <typename R>
-__device__ __forceinline__ void correct_cell(const KGridT<R> &g, const KFieldsT<R> &fl, int i, int j, int do_correct,
-                                             unsigned long long (&r)[2]) {
-  if (i < g.Nx && j < g.Ny) {
-    const Nbr n((unsigned)i, (unsigned)j, (unsigned)g.Nx, (unsigned)g.Ny, g.px);
-    const uint8_t *m = g.m;
-    const unsigned ij = n.ij, i_1j = n.i_1j, ij_1 = n.ij_1;
-    const R *p = FLD(P), *T = FLD(T);
-    R uf = FLD(U)[ij], vf = FLD(V)[ij];
-    if (do_correct) {
-      if (in_box(i, j, g.Nx_u0, g.Nx_u1, g.Ny_u0, g.Ny_u1) && m[i_1j] && m[ij]) {
-        R un = FLD(U_PSEUDO)[ij] - (p[ij] - p[i_1j]) * FLD(D_P_C_12)[ij];
-        r[0] = absbits(un - uf);
-        uf = un;
-        FLD(U)[ij] = un;
-      }
-      if (in_box(i, j, g.Nx_v0, g.Nx_v1, g.Ny_v0, g.Ny_v1) && m[ij_1] && m[ij]) {
-        R vn = FLD(V_PSEUDO)[ij] - (p[ij] - p[ij - (unsigned)g.Nx]) * FLD(D_P_C_34)[ij];
-        r[1] = absbits(vn - vf);
-        vf = vn;
-        FLD(V)[ij] = vn;
-      }
-    }
-    const R rij = rho_of(m, p, T, ij);
-    FLD(SQRT_T)[ij] = sqrt(T[ij]);
-    FLD(RHO)[ij] = rij;
-    R ru, rv;
-    if (m[i_1j] && m[ij]) ru = upwind_rho(rho_of(m, p, T, i_1j), rij, uf);
-    else if (m[i_1j] != m[ij]) ru = m[i_1j] ? rho_of(m, p, T, i_1j) : rij;
-    else ru = R(0.0);
-    if (m[ij_1] && m[ij]) rv = upwind_rho(rho_of(m, p, T, ij_1), rij, vf);
-    else if (m[ij_1] != m[ij]) rv = m[ij_1] ? rho_of(m, p, T, ij_1) : rij;
-    else rv = R(0.0);
-    FLD(RHO_U)[ij] = ru;
-    FLD(RHO_V)[ij] = rv;
-  }
-}
-
-// correct_cell in two phases, so that a thread can issue the loads of
-// several cells before it computes any of them.
-template <typename R>
+// The pass in two phases, so that a thread can issue the loads of several
+// cells before it computes any of them.  FLUX: with it the fluxes and thermal
+// diffusion coefficients (S:10440-10618) of the corrected state, whose
+// inputs at the cell and its west and south neighbours are all here.  What
+// the wall and edge conditions change after it (u, v at wall faces and box
+// edges, wall temperatures), they set right themselves (apply_wall_op,
+// edges_block).
+template <typename R, bool FLUX = false>
 struct CorrectIn {
   unsigned ij, i_1j, ij_1;
   bool in, cu, cv;                    // cell in grid; u, v corrected
   bool mc, mw, ms;                    // fluid: cell, west, south
   R uf, vf, ups, vps, d12, d34, pc, pw, ps, Tc, Tw, Ts;
+  R hxi, hxw, hyj, hys, twu, twv;     // FLUX: mesh steps (cell, west; cell, south), wall temperatures
   __device__ __forceinline__ void load(const KGridT<R> &g, const KFieldsT<R> &fl, int i, int j, int do_correct) {
     in = i < g.Nx && j < g.Ny;
     if (!in) return;
@@ -994,10 +957,24 @@ struct CorrectIn {
     Tc = T[ij];
     Tw = T[i_1j];
     Ts = T[ij_1];
+    if (FLUX) {
+      hxi = g.hx[i];
+      hxw = g.hx[n.i_1];
+      hyj = g.hy[j];
+      hys = g.hy[j - 1 * (0 < j)];
+      load_walls(fl);
+    }
+  }
+  // A wall temperature enters DTx (DTy) only where exactly one of the cell
+  // and its west (south) neighbour is fluid: with both fluid its term is
+  // 0 * sqrt(Tw), +0 for every wall temperature the state holds (finite,
+  // >= 0) as for 0, and with neither DTx is 0; those loads are left out.
+  __device__ __forceinline__ void load_walls(const KFieldsT<R> &fl) {
+    twu = mc == mw ? R(0) : FLD(TW_U)[ij];
+    twv = mc == ms ? R(0) : FLD(TW_V)[ij];
   }
   // S:4170-4305 (u, v), S:4323-4330 (sqrt_T, rho), S:10382-10437 (face densities)
-  // rr (optional): the face densities rho_u, rho_v written
-  __device__ __forceinline__ void apply(const KFieldsT<R> &fl, unsigned long long (&r)[2], R *rr = nullptr) const {
+  __device__ __forceinline__ void apply(const KGridT<R> &g, const KFieldsT<R> &fl, unsigned long long (&r)[2]) const {
     if (!in) return;
     R u = uf, v = vf;
     if (cu) {
@@ -1014,8 +991,13 @@ struct CorrectIn {
       v = vn;
       FLD(V)[ij] = vn;
     }
+    derive(g, fl, u, v, sqrt(Tc), FLUX ? sqrt(Tw) : R(0), FLUX ? sqrt(Ts) : R(0));
+  }
+  // What the cell derives from its u, v and the p, T around it; sc, sw, ss:
+  // sqrt(T) of the cell, west and south.
+  __device__ __forceinline__ void derive(const KGridT<R> &g, const KFieldsT<R> &fl, R u, R v, R sc, R sw, R ss) const {
     const R rij = mc ? pc / Tc : R(0.0);
-    FLD(SQRT_T)[ij] = sqrt(Tc);
+    FLD(SQRT_T)[ij] = sc;
     FLD(RHO)[ij] = rij;
     const R rw = mw ? pw / Tw : R(0.0), rs = ms ? ps / Ts : R(0.0);
     R ru, rv;
@@ -1027,29 +1009,49 @@ struct CorrectIn {
     else rv = R(0.0);
     FLD(RHO_U)[ij] = ru;
     FLD(RHO_V)[ij] = rv;
-    if (rr) {
-      rr[0] = ru;
-      rr[1] = rv;
-    }
+    if (!FLUX) return;
+    FluxIn<R> f;
+    f.in = true;
+    f.ij = ij;
+    f.hxi = hxi;
+    f.hxw = hxw;
+    f.hyj = hyj;
+    f.hys = hys;
+    f.ru = ru;
+    f.u = u;
+    f.rv = rv;
+    f.v = v;
+    f.m10 = ms;
+    f.m01 = mw;
+    f.m11 = mc;
+    f.s10 = ss;
+    f.s01 = sw;
+    f.s11 = sc;
+    f.twu11 = twu;
+    f.twv11 = twv;
+    f.apply_flux(g, fl);
   }
 };
 
-// CORRECT_ROWS cells per thread, rows BY apart, all loads issued first.
+// CORRECT_ROWS cells per thread, rows BY apart, all loads issued first.  Bound
+// by its memory traffic: with the fluxes it reads 8 arrays and writes 10 (107
+// MB at 1920x384: 20.0 us, 5.3 TB/s), where the correction and a flux pass of
+// its own took 15.7 + 11.8 us there and 5.5 + 4.4 us on 240x48 (now 7.0).
 constexpr int CORRECT_ROWS = 2;
 
-template <typename R>
+template <typename R, bool FLUX>
 __global__ void __launch_bounds__(BX *BY) k_correct(KGridT<R> g, KFieldsT<R> fl, unsigned long long *red_u,
                                                     unsigned long long *red_v, int do_correct, Gate gate) {
   if (gated_out(gate)) return;
   unsigned long long r[2] = {0ull, 0ull};
   int i0, j0;
   tile_origin<BX, BY * CORRECT_ROWS>(g.Nx, i0, j0);
-  CorrectIn<R> c[CORRECT_ROWS];
+  CorrectIn<R, FLUX> c[CORRECT_ROWS];
 #pragma unroll
   for (int q = 0; q < CORRECT_ROWS; q++)
     c[q].load(g, fl, i0 + (int)threadIdx.x, j0 + (int)threadIdx.y + q * BY, do_correct);
 #pragma unroll
-  for (int q = 0; q < CORRECT_ROWS; q++) c[q].apply(fl, r);
+  for (int q = 0; q < CORRECT_ROWS; q++) c[q].apply(g, fl, r);
   if (do_correct) block_max_atomic<2, BX * BY>(r, MaxDst<2>{{red_u, red_v}, {}});
 }
 
@@ -1266,19 +1268,51 @@ __device__ __forceinline__ void plan_wall_cell(const KGridT<R> &g, int i, int j,
 
 // Value of one planned write; every value read is a face or cell that no
 // write of the pass modifies, so the writes are independent.
-template <typename R>
+// FLUX: the one flux or thermal coefficient that depends on the written
+// value is formed again, as the correction pass formed it before the write.
+template <bool FLUX = false, typename R>
 __device__ __forceinline__ void apply_wall_op(const KGridT<R> &g, const KFieldsT<R> &fl, const WallOp &o) {
   const unsigned kind = o.kb & 7u;
   if (kind == WOP_NONE) return;
   const DevBody *b = &g.bodies[o.kb >> 3];
+  R x;
   if (kind == WOP_U)
-    FLD(U)[o.dst] = slip_value(g, b, R(b->u_body), FLD(U)[o.src], FLD(RHO_U)[o.src], g.hy[o.h]);
+    FLD(U)[o.dst] = x = slip_value(g, b, R(b->u_body), FLD(U)[o.src], FLD(RHO_U)[o.src], g.hy[o.h]);
   else if (kind == WOP_V)
-    FLD(V)[o.dst] = slip_value(g, b, R(b->v_body), FLD(V)[o.src], FLD(RHO_V)[o.src], g.hx[o.h]);
+    FLD(V)[o.dst] = x = slip_value(g, b, R(b->v_body), FLD(V)[o.src], FLD(RHO_V)[o.src], g.hx[o.h]);
   else if (kind == WOP_TWU)
-    FLD(TW_U)[o.dst] = wall_T(g, b, FLD(T)[o.src], FLD(RHO)[o.src], R(0.5) * g.hx[o.h]);
+    FLD(TW_U)[o.dst] = x = wall_T(g, b, FLD(T)[o.src], FLD(RHO)[o.src], R(0.5) * g.hx[o.h]);
   else
-    FLD(TW_V)[o.dst] = wall_T(g, b, FLD(T)[o.src], FLD(RHO)[o.src], R(0.5) * g.hy[o.h]);
+    FLD(TW_V)[o.dst] = x = wall_T(g, b, FLD(T)[o.src], FLD(RHO)[o.src], R(0.5) * g.hy[o.h]);
+  if (!FLUX) return;
+  const unsigned Nx = (unsigned)g.Nx, ij = o.dst, j = ij / Nx, i = ij - j * Nx;
+  FluxIn<R> f;
+  f.hxi = g.hx[i];
+  f.hyj = g.hy[j];
+  if (kind == WOP_U) {
+    f.ru = FLD(RHO_U)[ij];
+    f.u = x;
+    FLD(FX)[ij] = f.fx();
+  } else if (kind == WOP_V) {
+    f.rv = FLD(RHO_V)[ij];
+    f.v = x;
+    FLD(FY)[ij] = f.fy();
+  } else {
+    const Nbr n(i, j, Nx, (unsigned)g.Ny, g.px);
+    const unsigned nb = g.nb[ij];
+    const R *sT = FLD(SQRT_T);
+    f.hxw = g.hx[n.i_1];
+    f.hys = g.hy[j - (0u < j)];
+    f.m10 = (nb & NB_S) != 0;
+    f.m01 = (nb & NB_W) != 0;
+    f.m11 = (nb & NB_C) != 0;
+    f.s10 = sT[n.ij_1];
+    f.s01 = sT[n.i_1j];
+    f.s11 = sT[ij];
+    f.twu11 = f.twv11 = x;
+    if (kind == WOP_TWU) FLD(DTX)[ij] = f.dtx(g);
+    else FLD(DTY)[ij] = f.dty(g);
+  }
 }
 
 template <typename R>
@@ -1286,28 +1320,27 @@ __device__ __forceinline__ void wall_cell(const KGridT<R> &g, const KFieldsT<R> 
   WallOp op[4];
   plan_wall_cell(g, i, j, parts, op);
 #pragma unroll
-  for (int q = 0; q < 4; q++) apply_wall_op(g, fl, op[q]);
+  for (int q = 0; q < 4; q++) apply_wall_op<false>(g, fl, op[q]);
 }
 
 template <typename R>
-__global__ void __launch_bounds__(BX *BY) k_wall(KGridT<R> g, KFieldsT<R> fl, int parts, Gate gate) {
-  if (gated_out(gate)) return;
+__global__ void __launch_bounds__(BX *BY) k_wall(KGridT<R> g, KFieldsT<R> fl, int parts) {
   int i0, j0;
   tile_origin<BX, BY>(g.Nx, i0, j0);
   wall_cell(g, fl, i0 + (int)threadIdx.x, j0 + (int)threadIdx.y, parts);
 }
 
-// The planned writes of a case (built once from its mask), one per thread.
+// The planned writes of a case (built once from its mask), one per thread,
+// all kinds; flux: after a correction pass that formed the fluxes.
 template <typename R>
 __global__ void __launch_bounds__(256) k_wall_ops(KGridT<R> g, KFieldsT<R> fl, const WallOp *__restrict__ ops, int n,
-                                                  int parts, Gate gate) {
+                                                  bool flux, Gate gate) {
   if (gated_out(gate)) return;
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (t >= n) return;
   const WallOp o = ops[t];
-  const unsigned kind = o.kb & 7u;
-  const int need = kind == WOP_U ? STS_BC_SLIP_U : kind == WOP_V ? STS_BC_SLIP_V : STS_BC_JUMP;
-  if (parts & need) apply_wall_op(g, fl, o);
+  if (flux) apply_wall_op<true>(g, fl, o);
+  else apply_wall_op<false>(g, fl, o);
 }
 
 // Planning pass: the four planned writes of each listed cell (out[4 t + q]).
@@ -1429,8 +1462,8 @@ __device__ __forceinline__ void loop_test_wave(const Gate &gate, const LoopTest 
 constexpr int EDGE_GROUPS = 4;
 
 template <typename R>
-__device__ void edges_block(const KGridT<R> &g, const KFieldsT<R> &fl, int parts, double *probe, const Gate &gate,
-                            const LoopTest &lt, int group) {
+__device__ void edges_block(const KGridT<R> &g, const KFieldsT<R> &fl, int parts, bool flux, double *probe,
+                            const Gate &gate, const LoopTest &lt, int group) {
   // The velocity, temperature and pressure conditions touch disjoint arrays
   // (u, v read rho and the face densities, which none of them writes), and
   // the loop test reads only the residual words, so four workgroups run them
@@ -1512,6 +1545,25 @@ __device__ void edges_block(const KGridT<R> &g, const KFieldsT<R> &fl, int parts
     __syncthreads();
     edge_y(g, u, g.Ny_u0, g.Ny_u1, false, bc & BC_DUDY_YE);
     __syncthreads();
+    if (flux) {  // the fluxes of the cells whose u, v the conditions above may have changed
+      auto strip = [&](R *F, const R *rho_f, const R *vel, bool x, int c0, int c1, int r0, int r1) {
+        const int w = c1 - c0;
+        for (int t = threadIdx.x; t < w * (r1 - r0); t += EDGE_THREADS) {
+          const int dj = t / w, i = c0 + (t - dj * w), j = r0 + dj, k = i + j * Nx;
+          F[k] = (x ? hy[j] : hx[i]) * rho_f[k] * vel[k];
+        }
+      };
+      R *Fx = FLD(FX), *Fy = FLD(FY);
+      if (bc & (BC_DUDX_XB | BC_DURHODX_XB | BC_DRHODT_XB)) strip(Fx, rho_u, u, true, 0, g.Nx_u0, 0, Ny);
+      if (bc & (BC_DUDX_XE | BC_DURHODX_XE | BC_DRHODT_XE | BC_UMINMOUT_XE))
+        strip(Fx, rho_u, u, true, g.Nx_u1, Nx, 0, Ny);
+      if (bc & BC_DUDY_YB) strip(Fx, rho_u, u, true, 0, Nx, 0, g.Ny_u0);
+      if (bc & BC_DUDY_YE) strip(Fx, rho_u, u, true, 0, Nx, g.Ny_u1, Ny);
+      if (bc & BC_DVDX_XB) strip(Fy, rho_v, v, false, 0, g.Nx_v0, 0, Ny);
+      if (bc & BC_DVDX_XE) strip(Fy, rho_v, v, false, g.Nx_v1, Nx, 0, Ny);
+      if (bc & BC_DVDY_YB) strip(Fy, rho_v, v, false, 0, Nx, 0, g.Ny_v0);
+      if (bc & BC_DVDY_YE) strip(Fy, rho_v, v, false, 0, Nx, g.Ny_v1, Ny);
+    }
   }
   if (parts & STS_BC_TEMPERATURE) {
     R *T = FLD(T);
@@ -1543,17 +1595,20 @@ __device__ void edges_block(const KGridT<R> &g, const KFieldsT<R> &fl, int parts
 }
 
 template <typename R>
-__global__ void __launch_bounds__(EDGE_THREADS) k_edges(KGridT<R> g, KFieldsT<R> fl, int parts, double *probe,
-                                                        Gate gate, LoopTest lt) {
+__global__ void __launch_bounds__(EDGE_THREADS) k_edges(KGridT<R> g, KFieldsT<R> fl, int parts, bool flux,
+                                                        double *probe, Gate gate, LoopTest lt) {
   if (gated_out(gate)) return;
-  edges_block(g, fl, parts, probe, gate, lt, (int)blockIdx.x);
+  edges_block(g, fl, parts, flux, probe, gate, lt, (int)blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
 // A10 + A11: fluxes (S:10440-10454) and diffusion coefficients
 // (S:10457-10618) over all cells.
 // ---------------------------------------------------------------------------
-// FLUX_ROWS cells per thread, rows BY apart, all loads issued first.
+// Stage calls, the Gamma and D arrays where they are asked for, and the
+// fluxes after the last iteration of an Anderson loop; every other loop
+// iteration gets its fluxes from the correction pass.  FLUX_ROWS cells per
+// thread, rows BY apart, all loads issued first.
 constexpr int FLUX_ROWS = 2;
 
 // PARTS: FLUX_PART (Fx, Fy, DTx, DTy) and/or DIFF_PART (Gamma, D_ux, D_uy,
@@ -1995,15 +2050,13 @@ __device__ __forceinline__ void aa_mixed(const AABuf &ab, const AASel &sel, cons
 
 // The next start x of a TX x TY tile (origin i0, j0; this thread tx, ty)
 // into the state arrays (and D = x - gp when sel.write_D), and, from it,
-// what the correction pass derives without correcting: sqrt_T, rho and the
-// face densities
-// (CorrectIn::apply on the mixed p, T of the cell and of its west and south
-// neighbours); with FLUX also what the loop's flux pass writes (Fx, Fy, DTx,
-// DTy; FluxIn::apply_flux).  The mixed p, T of the tile and of its west
-// column and south row (formed by the first threads) meet in LDS (sp, sT:
-// [1 + row][1 + column], row 0 and column 0 the halo); with FLUX their
-// sqrt(T) too (ss), each formed once.
-template <int NM, int TX, int TY, bool FLUX, typename R>
+// what the correction pass derives without correcting: sqrt_T, rho, the face
+// densities, the fluxes and thermal coefficients (CorrectIn::derive on the
+// mixed p, T of the cell and of its west and south neighbours).  The mixed
+// p, T of the tile and of its west column and south row (formed by the first
+// threads) meet in LDS (sp, sT: [1 + row][1 + column], row 0 and column 0
+// the halo), their sqrt(T) too (ss), each formed once.
+template <int NM, int TX, int TY, typename R>
 __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R> &fl, const AAFieldsT<R> &s,
                                             const AABuf &ab, const AASel &sel, const double *gsrc, int i0, int j0,
                                             int tx, int ty, double (*sp)[TX + 1], double (*sT)[TX + 1],
@@ -2023,7 +2076,7 @@ __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R
     for (int q = 0; q < 4; q++) x[q] = (double)(R)x[q];
     sp[ty + 1][tx + 1] = x[2];
     sT[ty + 1][tx + 1] = x[3];
-    if constexpr (FLUX) ss[ty + 1][tx + 1] = (double)sqrt((R)x[3]);
+    ss[ty + 1][tx + 1] = (double)sqrt((R)x[3]);
   }
   // halo: thread (t, 0) the cell south of column t, thread (t < TY, 1) the
   // cell west of row t (the clamped or wrapped neighbour of the reference)
@@ -2032,35 +2085,34 @@ __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R
     aa_mixed<NM>(ab, sel, gam, nb.ij_1, h, hg);
     sp[0][tx + 1] = (double)(R)h[2];
     sT[0][tx + 1] = (double)(R)h[3];
-    if constexpr (FLUX) ss[0][tx + 1] = (double)sqrt((R)h[3]);
+    ss[0][tx + 1] = (double)sqrt((R)h[3]);
   }
   if (ty == 1 && tx < TY && i0 < Nx && j0 + tx < Ny) {
     const Nbr w((unsigned)i0, (unsigned)(j0 + tx), (unsigned)Nx, (unsigned)Ny, g.px);
     aa_mixed<NM>(ab, sel, gam, w.i_1j, h, hg);
     sp[tx + 1][0] = (double)(R)h[2];
     sT[tx + 1][0] = (double)(R)h[3];
-    if constexpr (FLUX) ss[tx + 1][0] = (double)sqrt((R)h[3]);
+    ss[tx + 1][0] = (double)sqrt((R)h[3]);
   }
   __syncthreads();
   if (!in) return;
-  CorrectIn<R> ci;
-  ci.in = true;
-  ci.cu = ci.cv = false;
+  CorrectIn<R, true> ci;
   ci.ij = nb.ij;
-  ci.i_1j = nb.i_1j;
-  ci.ij_1 = nb.ij_1;
   const unsigned bits = g.nb[nb.ij];
   ci.mc = (bits & NB_C) != 0;
   ci.mw = (bits & NB_W) != 0;
   ci.ms = (bits & NB_S) != 0;
-  ci.uf = (R)x[0];
-  ci.vf = (R)x[1];
   ci.pc = (R)x[2];
   ci.Tc = (R)x[3];
   ci.pw = (R)sp[ty + 1][tx];
   ci.Tw = (R)sT[ty + 1][tx];
   ci.ps = (R)sp[ty][tx + 1];
   ci.Ts = (R)sT[ty][tx + 1];
+  ci.hxi = g.hx[i];
+  ci.hxw = g.hx[nb.i_1];
+  ci.hyj = g.hy[j];
+  ci.hys = g.hy[j - 1 * (0 < j)];
+  ci.load_walls(fl);
   double d[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
@@ -2068,39 +2120,7 @@ __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R
     d[q] = x[q] - gp[q];
   }
   if (sel.write_D) store4(ab.D + 4 * (size_t)nb.ij, d);
-  KFieldsT<R> kf = fl;
-  kf.f[STS_P] = s.x[2];
-  kf.f[STS_T] = s.x[3];
-  unsigned long long rr[2] = {0ull, 0ull};
-  R rho_uv[2];
-  ci.apply(kf, rr, rho_uv);
-  if (!FLUX) return;
-  // the loop's flux pass on the mixed state (fluxes, thermal coefficients):
-  // its inputs at this cell and the west and south sqrt_T are all here
-  FluxIn<R> fi;
-  fi.in = true;
-  fi.ij = nb.ij;
-  fi.hxi = g.hx[i];
-  fi.hxw = g.hx[nb.i_1];
-  fi.hyj = g.hy[j];
-  fi.hys = g.hy[j - 1 * (0 < j)];
-  fi.ru = rho_uv[0];
-  fi.u = (R)x[0];
-  fi.rv = rho_uv[1];
-  fi.v = (R)x[1];
-  fi.m10 = ci.ms;
-  fi.m01 = ci.mw;
-  fi.m11 = ci.mc;
-  fi.s10 = (R)ss[ty][tx + 1];
-  fi.s01 = (R)ss[ty + 1][tx];
-  fi.s11 = (R)ss[ty + 1][tx + 1];
-  // a wall temperature enters DTx (DTy) only where exactly one of the cell
-  // and its west (south) neighbour is fluid: with both fluid its term is
-  // 0 * sqrt(Tw), +0 for every wall temperature the state holds (finite,
-  // >= 0) as for 0, and with neither DTx is 0; those loads are left out
-  fi.twu11 = ci.mc == ci.mw ? R(0) : FLD(TW_U)[nb.ij];
-  fi.twv11 = ci.mc == ci.ms ? R(0) : FLD(TW_V)[nb.ij];
-  fi.apply_flux(g, kf);
+  ci.derive(g, fl, (R)x[0], (R)x[1], (R)ss[ty + 1][tx + 1], (R)ss[ty + 1][tx], (R)ss[ty][tx + 1]);
 }
 
 // The weights and the mix in one launch: every workgroup folds the store
@@ -2120,7 +2140,7 @@ __global__ void __launch_bounds__(AA_MIX_TX *AA_MIX_TY) k_aa_mix(KGridT<R> g, KF
   const int ntx = (g.Nx + AA_MIX_TX - 1) / AA_MIX_TX, ntiles = ntx * ((g.Ny + AA_MIX_TY - 1) / AA_MIX_TY);
   const int tx = (int)threadIdx.x % AA_MIX_TX, ty = (int)threadIdx.x / AA_MIX_TX;
   for (int t = (int)blockIdx.x; t < ntiles; t += (int)gridDim.x) {
-    aa_mix_tile<NM, AA_MIX_TX, AA_MIX_TY, true, R>(g, fl, s, ab, sel, gam, (t % ntx) * AA_MIX_TX,
+    aa_mix_tile<NM, AA_MIX_TX, AA_MIX_TY, R>(g, fl, s, ab, sel, gam, (t % ntx) * AA_MIX_TX,
                                                   (t / ntx) * AA_MIX_TY, tx, ty, sp, sT, ss);
     __syncthreads();  // the next tile reuses sp, sT, ss
   }
@@ -2413,46 +2433,22 @@ __global__ void __launch_bounds__(TX *TY) kb_correct(const BatchCase<R> *C, cons
   if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const KFieldsT<R> f = fields_at(c, par);
   unsigned long long r[2] = {0ull, 0ull};
-  correct_cell(grid_of(c), f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, 1, r);
+  const KGridT<R> g = grid_of(c);
+  CorrectIn<R, true> x;
+  x.load(g, f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, 1);
+  x.apply(g, f, r);
   block_max_atomic<2, TX * TY>(r, MaxDst<2>{{in_memory(c.lred), in_memory(c.lred) + 1}, {}});
-}
-
-template <typename R, int TX, int TY>
-__global__ void __launch_bounds__(TX *TY) kb_wall(const BatchCase<R> *C, const BatchTile *T, int k, int par,
-                                                  int parts) {
-  const BatchTile t = T[blockIdx.x];
-  const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
-  const KFieldsT<R> f = fields_at(c, par);
-  wall_cell(grid_of(c), f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, parts);
 }
 
 template <typename R>
 __global__ void __launch_bounds__(WALL_OPS_PER_TILE) kb_wall_ops(const BatchCase<R> *C, const BatchTile *T, int k,
-                                                                 int par, int parts) {
+                                                                 int par) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
   if (gated_out(Gate{in_memory(c.ctrl), k})) return;
   const int q = t.x * WALL_OPS_PER_TILE + (int)threadIdx.x;
   if (q >= c.nwops) return;
-  const WallOp o = in_memory(c.wops)[q];
-  const unsigned kind = o.kb & 7u;
-  const int need = kind == WOP_U ? STS_BC_SLIP_U : kind == WOP_V ? STS_BC_SLIP_V : STS_BC_JUMP;
-  if (parts & need) apply_wall_op(grid_of(c), fields_at(c, par), o);
-}
-
-// The fluxes and thermal coefficients (FLUX_PART); the assembly forms the
-// diffusion coefficients itself.
-template <typename R, int TX, int TY>
-__global__ void __launch_bounds__(TX *TY) kb_flux_diff(const BatchCase<R> *C, const BatchTile *T, int k, int par) {
-  const BatchTile t = T[blockIdx.x];
-  const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
-  const KFieldsT<R> f = fields_at(c, par);
-  FluxIn<R> x;
-  const KGridT<R> g = grid_of(c);
-  x.template load<true, false>(g, f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX);
-  x.apply_flux(g, f);
+  apply_wall_op<true>(grid_of(c), fields_at(c, par), in_memory(c.wops)[q]);
 }
 
 // Batched Anderson steps (FP64): the single-context kernels' code per tile
@@ -2515,17 +2511,16 @@ __global__ void __launch_bounds__(AA_SOLVE_THREADS) kb_aa_solve(const BatchCase<
   aa_solve_group<NM, AA_SOLVE_THREADS>(aa_of(c), case_sel(c, bs), gam, true);
 }
 
-// The mix without the flux part (the batched flux and diffusion pass follows).
 template <int TX, int TY, int NM>
 __global__ void __launch_bounds__(TX *TY) kb_aa_mix(const BatchCase<double> *C, const BatchTile *T, int k, int par,
                                                     AABatchSel bs) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<double> &c = C[t.c];
   if (gated_out(Gate{in_memory(c.ctrl), k + 1})) return;
-  __shared__ double sp[TY + 1][TX + 1], sT[TY + 1][TX + 1];
-  aa_mix_tile<NM, TX, TY, false>(grid_of(c), fields_at(c, par), case_state(c, par), aa_of(c), case_sel(c, bs),
-                                 in_memory(c.aa.gam),
-                                 t.x * TX, t.y * TY, (int)threadIdx.x % TX, (int)threadIdx.x / TX, sp, sT, nullptr);
+  __shared__ double sp[TY + 1][TX + 1], sT[TY + 1][TX + 1], ss[TY + 1][TX + 1];
+  aa_mix_tile<NM, TX, TY>(grid_of(c), fields_at(c, par), case_state(c, par), aa_of(c), case_sel(c, bs),
+                          in_memory(c.aa.gam), t.x * TX, t.y * TY, (int)threadIdx.x % TX, (int)threadIdx.x / TX, sp,
+                          sT, ss);
 }
 
 // Edge conditions and the loop-2 test: one workgroup per case.
@@ -2537,7 +2532,7 @@ __global__ void __launch_bounds__(EDGE_THREADS) kb_edges(const BatchCase<R> *C, 
   const KFieldsT<R> f = fields_at(c, par);
   const LoopTest lt{in_memory(c.ctrl), in_memory(c.lred), in_memory(c.log) + 6 * (size_t)k, c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w,
                     c.stall_ratio};
-  edges_block(grid_of(c), f, parts, in_memory(c.probe), gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
+  edges_block(grid_of(c), f, parts, true, in_memory(c.probe), gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
 }
 
 // Opens every case's loop 2: control, log (6 N_I words), slotted words.
@@ -2602,27 +2597,29 @@ hipError_t launch_sweep2(const KGridT<R> &g, const KFieldsT<R> &f, const R *Po, 
 }
 template <typename R>
 hipError_t launch_correct(const KGridT<R> &g, const KFieldsT<R> &f, unsigned long long *ru, unsigned long long *rv,
-                          int do_correct, hipStream_t s, Gate gate) {
-  hipLaunchKernelGGL(k_correct<R>, (grid_tiles<BX, BY * CORRECT_ROWS>(g)), dim3(BX, BY), 0, s, g, f, ru, rv, do_correct,
-                     gate);
+                          int do_correct, bool flux, hipStream_t s, Gate gate) {
+  const dim3 gr = grid_tiles<BX, BY * CORRECT_ROWS>(g);
+  if (flux) hipLaunchKernelGGL((k_correct<R, true>), gr, dim3(BX, BY), 0, s, g, f, ru, rv, do_correct, gate);
+  else hipLaunchKernelGGL((k_correct<R, false>), gr, dim3(BX, BY), 0, s, g, f, ru, rv, do_correct, gate);
   return hipGetLastError();
 }
 template <typename R>
-hipError_t launch_wall(const KGridT<R> &g, const KFieldsT<R> &f, int parts, hipStream_t s, Gate gate,
-                       const WallOp *ops, int nops) {
-  if (ops) {
-    if (nops > 0)
-      hipLaunchKernelGGL(k_wall_ops<R>, dim3((nops + 255) / 256), dim3(256), 0, s, g, f, ops, nops, parts, gate);
-  } else {
-    hipLaunchKernelGGL(k_wall<R>, (grid_tiles<BX, BY>(g)), dim3(BX, BY), 0, s, g, f, parts, gate);
-  }
+hipError_t launch_wall(const KGridT<R> &g, const KFieldsT<R> &f, int parts, hipStream_t s) {
+  hipLaunchKernelGGL(k_wall<R>, (grid_tiles<BX, BY>(g)), dim3(BX, BY), 0, s, g, f, parts);
   return hipGetLastError();
 }
 template <typename R>
-hipError_t launch_edges(const KGridT<R> &g, const KFieldsT<R> &f, int parts, double *probe, hipStream_t s,
+hipError_t launch_wall_ops(const KGridT<R> &g, const KFieldsT<R> &f, const WallOp *ops, int nops, bool flux,
+                           hipStream_t s, Gate gate) {
+  if (nops == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_wall_ops<R>, dim3((nops + 255) / 256), dim3(256), 0, s, g, f, ops, nops, flux, gate);
+  return hipGetLastError();
+}
+template <typename R>
+hipError_t launch_edges(const KGridT<R> &g, const KFieldsT<R> &f, int parts, bool flux, double *probe, hipStream_t s,
                         Gate gate, LoopTest lt) {
   hipLaunchKernelGGL(k_edges<R>, dim3(lt.ctrl ? EDGE_GROUPS : EDGE_GROUPS - 1), dim3(EDGE_THREADS), 0, s, g, f, parts,
-                     probe, gate, lt);
+                     flux, probe, gate, lt);
   return hipGetLastError();
 }
 template <typename R>
@@ -2648,15 +2645,16 @@ hipError_t launch_flux_diff(const KGridT<R> &g, const KFieldsT<R> &f, hipStream_
                                        unsigned long long *, unsigned long long *, unsigned long long *,       \
                                        unsigned long long *, hipStream_t, Gate);                               \
   template hipError_t launch_correct<R>(const KGridT<R> &, const KFieldsT<R> &, unsigned long long *,          \
-                                        unsigned long long *, int, hipStream_t, Gate);                         \
-  template hipError_t launch_wall<R>(const KGridT<R> &, const KFieldsT<R> &, int, hipStream_t, Gate,           \
-                                     const WallOp *, int);                                                    \
-  template hipError_t launch_edges<R>(const KGridT<R> &, const KFieldsT<R> &, int, double *, hipStream_t, Gate, \
-                                      LoopTest);                                                               \
+                                        unsigned long long *, int, bool, hipStream_t, Gate);                   \
+  template hipError_t launch_wall_ops<R>(const KGridT<R> &, const KFieldsT<R> &, const WallOp *, int, bool,    \
+                                         hipStream_t, Gate);                                                   \
+  template hipError_t launch_edges<R>(const KGridT<R> &, const KFieldsT<R> &, int, bool, double *, hipStream_t, \
+                                      Gate, LoopTest);                                                         \
   template hipError_t launch_flux_diff<R>(const KGridT<R> &, const KFieldsT<R> &, hipStream_t, Gate, int);
 STS_INSTANTIATE(double)
 STS_INSTANTIATE(float)
 #undef STS_INSTANTIATE
+template hipError_t launch_wall<double>(const KGrid &, const KFields &, int, hipStream_t);
 
 hipError_t launch_properties(const KGrid &g, const KFields &f, hipStream_t s) {
   hipLaunchKernelGGL(k_properties<double>, grid2d(g), dim3(BX, BY), 0, s, g, f);
@@ -2846,12 +2844,10 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
     case BK_ASSEMBLE_ARR: CELL_SWITCH(variant, kb_assemble_arr, C, T, k, par); break;
     case BK_SWEEP: CELL_SWITCH(variant, kb_sweep, C, T, k, par, a, b); break;
     case BK_CORRECT: CELL_SWITCH(variant, kb_correct, C, T, k, par); break;
-    case BK_WALL: CELL_SWITCH(variant, kb_wall, C, T, k, par, a); break;
     case BK_WALL_OPS:
       if (ntiles > 0)
-        hipLaunchKernelGGL(kb_wall_ops<R>, dim3(ntiles), dim3(WALL_OPS_PER_TILE), 0, s, C, T, k, par, a);
+        hipLaunchKernelGGL(kb_wall_ops<R>, dim3(ntiles), dim3(WALL_OPS_PER_TILE), 0, s, C, T, k, par);
       break;
-    case BK_FLUX_DIFF: CELL_SWITCH(variant, kb_flux_diff, C, T, k, par); break;
     case BK_SWEEP2:
       switch (variant) {
         case 0: SWEEP_LAUNCH(6); break;

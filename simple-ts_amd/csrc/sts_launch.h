@@ -20,17 +20,23 @@ template <typename R>
 hipError_t launch_sweep2(const KGridT<R> &g, const KFieldsT<R> &f, const R *Po, const R *To, R *Pn, R *Tn,
                          unsigned long long *r1p, unsigned long long *r1T, unsigned long long *r2p,
                          unsigned long long *r2T, hipStream_t s, Gate gate = Gate{nullptr, 0});
+// flux: the pass forms the fluxes and thermal diffusion coefficients too, and
+// the wall writes and edge conditions that follow it (their own flux set)
+// form again what they change of them.
 template <typename R>
 hipError_t launch_correct(const KGridT<R> &g, const KFieldsT<R> &f, unsigned long long *ru, unsigned long long *rv,
-                          int do_correct, hipStream_t s, Gate gate = Gate{nullptr, 0});
-// cells: list of the cells next to a body/fluid interface (or null: all cells)
+                          int do_correct, bool flux, hipStream_t s, Gate gate = Gate{nullptr, 0});
+// The wall conditions `parts` over all cells (stage calls), or all planned
+// writes of a case (every kind).
 template <typename R>
-hipError_t launch_wall(const KGridT<R> &g, const KFieldsT<R> &f, int parts, hipStream_t s,
-                       Gate gate = Gate{nullptr, 0}, const WallOp *ops = nullptr, int nops = 0);
+hipError_t launch_wall(const KGridT<R> &g, const KFieldsT<R> &f, int parts, hipStream_t s);
+template <typename R>
+hipError_t launch_wall_ops(const KGridT<R> &g, const KFieldsT<R> &f, const WallOp *ops, int nops, bool flux,
+                           hipStream_t s, Gate gate = Gate{nullptr, 0});
 // The planned writes of the listed cells: out[4 t + q], q = U, V, TW_U, TW_V.
 hipError_t launch_wall_plan(const KGrid &g, const unsigned *cells, int n, WallOp *out, hipStream_t s);
 template <typename R>
-hipError_t launch_edges(const KGridT<R> &g, const KFieldsT<R> &f, int parts, double *probe, hipStream_t s,
+hipError_t launch_edges(const KGridT<R> &g, const KFieldsT<R> &f, int parts, bool flux, double *probe, hipStream_t s,
                         Gate gate = Gate{nullptr, 0},
                         LoopTest lt = LoopTest{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0});
 // parts: FLUX_PART (Fx, Fy, DTx, DTy) and/or DIFF_PART (Gamma_*, D_*).
@@ -83,7 +89,7 @@ hipError_t launch_continuity(const KGrid &g, const KFields &f, double *cs, doubl
 // Batched loop-2 launches over the tiles T[0..ntiles) of the cases
 // C[0..ncases).  kernel: BK_*; variant: index into CELL_TILES (cell
 // kernels) or SWEEP_TILES (BK_SWEEP2).  (a, b) = (first, last) for the
-// sweeps, a = parts for BK_WALL and BK_EDGES.
+// sweeps, a = parts for BK_EDGES.
 // BK_ASSEMBLE forms Gamma and D in the tile; BK_ASSEMBLE_ARR (first outer
 // iteration only) assembles the cases whose arrays are to be read instead.
 enum {
@@ -91,9 +97,7 @@ enum {
   BK_SWEEP2,
   BK_SWEEP,
   BK_CORRECT,
-  BK_WALL,
   BK_EDGES,
-  BK_FLUX_DIFF,
   BK_LOOP_OPEN,
   BK_WALL_OPS,
   BK_ASSEMBLE_ARR
