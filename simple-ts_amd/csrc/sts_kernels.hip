@@ -7,6 +7,8 @@
 // body mask; inside a set the reference's "bc" formula is used, which is
 // bit-identical to its "nch" formula where all masks are 1.  Built with
 // -ffp-contract=off so each a*b+c rounds twice, as the reference's SSE2 build.
+#include <algorithm>
+
 #include "sts_device.h"
 
 #define FLD(name) fl.f[STS_##name]
@@ -1778,10 +1780,10 @@ __device__ __forceinline__ double wave_sum_last(double v) {
 }
 
 // Sums acc[0..NV) over a workgroup of NT threads (fixed order: lanes, then
-// waves in turn); thread t < NV gets sum t in out[t].  Only the sums j with
-// live(j) are formed, the others are 0 (their acc is unused).
+// waves in turn); every thread gets them in acc.  Only the sums j with live(j)
+// are formed, the others are 0 (their acc is unused).
 template <int NV, int NT, typename Live>
-__device__ __forceinline__ void block_sums(const double (&acc)[NV], double *out, Live live) {
+__device__ __forceinline__ void block_sums(double (&acc)[NV], Live live) {
   static_assert(NT % 64 == 0, "whole waves");
   __shared__ double sm[NV][NT / 64];
   const int lane = (int)threadIdx.x & 63, wid = (int)threadIdx.x >> 6;
@@ -1791,11 +1793,14 @@ __device__ __forceinline__ void block_sums(const double (&acc)[NV], double *out,
     if (lane == 63) sm[j][wid] = w;
   }
   __syncthreads();
-  if ((int)threadIdx.x < NV) {
-    double s = 0.0;
 #pragma unroll
-    for (int q = 0; q < NT / 64; q++) s += sm[threadIdx.x][q];
-    out[threadIdx.x] = s;
+  for (int j = 0; j < NV; j++) {
+    double s = 0.0;
+    if (live(j)) {
+#pragma unroll
+      for (int q = 0; q < NT / 64; q++) s += sm[j][q];
+    }
+    acc[j] = s;
   }
 }
 
@@ -1911,12 +1916,11 @@ __device__ __forceinline__ void aa_store_cell(const AAFieldsT<R> &s, const AABuf
 // The workgroup's (NT threads) sums of acc into partial slot idx:
 // part[j nb + idx] (a_j) and part[(MAX_AA + j) nb + idx] (b_j).
 template <int NM, int NT>
-__device__ __forceinline__ void aa_store_sums(const double (&acc)[2 * NM], const AABuf &ab, int idx, int n) {
-  __shared__ double sums[2 * NM];
-  block_sums<2 * NM, NT>(acc, sums, [n](int j) { return j % NM < n; });
-  __syncthreads();
-  const int j = (int)threadIdx.x;
-  if (j < 2 * NM) ab.part[(size_t)(j < NM ? j : MAX_AA + j - NM) * ab.nb + idx] = sums[j];
+__device__ __forceinline__ void aa_store_sums(double (&acc)[2 * NM], const AABuf &ab, int idx, int n) {
+  block_sums<2 * NM, NT>(acc, [n](int j) { return j % NM < n; });
+#pragma unroll
+  for (int j = 0; j < 2 * NM; j++)
+    if ((int)threadIdx.x == j) ab.part[(size_t)(j < NM ? j : MAX_AA + j - NM) * ab.nb + idx] = acc[j];
 }
 
 // AA_STORE_CELLS cells per thread (AA_THREADS apart), so that the partial
@@ -1940,13 +1944,19 @@ __global__ void __launch_bounds__(AA_THREADS) k_aa_store(AAFieldsT<R> s, AABuf a
 // completes the Gram matrix of the differences in use (the newest row from
 // the sums; the rest as stored), and solves (Gram + 1e-12 trace I) gamma = b
 // by Gaussian elimination with partial pivoting.  A singular or non-finite
-// solve gives gamma = 0 (the next start is g).  The weights go to gam_out
-// (shared memory of the workgroup, valid after a barrier); a leader
-// workgroup also stores the newest Gram row, for the next steps, and the
-// weights in ab.gam.  Workgroups that solve the same system concurrently
-// read only rows other than the newest, which the leader alone writes.
+// solve gives gamma = 0 (the next start is g).  Every thread gets the weights
+// in gam; a leader workgroup also stores the newest Gram row, for the next
+// steps, and the weights in ab.gam.  Workgroups that solve the same system
+// concurrently read only rows other than the newest, which the leader alone
+// writes.
+//
+// Every workgroup of a mix starts with this chain (load latency, reduction,
+// solve), so it is kept short: one barrier, and for up to two differences the
+// elimination in every thread's registers (a one-thread elimination with its
+// matrix in LDS and two more barriers took 0.7 us longer of the mix's 13.0 on
+// 301x95).
 template <int NM, int NT>
-__device__ __forceinline__ void aa_solve_group(const AABuf &ab, const AASel &sel, double *gam_out, bool leader) {
+__device__ __forceinline__ void aa_solve_group(const AABuf &ab, const AASel &sel, double (&gam)[NM], bool leader) {
   const int n = sel.n;
   double acc[2 * NM];
 #pragma unroll
@@ -1969,61 +1979,102 @@ __device__ __forceinline__ void aa_solve_group(const AABuf &ab, const AASel &sel
 #pragma unroll
       for (int j = 0; j < 2 * NM; j++) acc[j] += v[r][j];
   }
-  __shared__ double dots[2 * NM];
+  double g00 = 0.0;  // two differences: the stored part of the Gram matrix
+  if (NM == 2 && n == 2) g00 = ab.gram[sel.slot[0] * MAX_AA + sel.slot[0]];
   __shared__ double A[NM][NM + 1];
-  double *gam = gam_out;
-  if ((int)threadIdx.x < NM * NM) {  // the stored part of the Gram matrix
+  if (NM > 2 && (int)threadIdx.x < NM * NM) {
     const int a = (int)threadIdx.x / NM, b = (int)threadIdx.x % NM;
     if (a < n - 1 && b < n - 1) A[a][b] = ab.gram[sel.slot[a] * MAX_AA + sel.slot[b]];
   }
-  block_sums<2 * NM, NT>(acc, dots, [n](int j) { return j % NM < n; });
-  __syncthreads();
-  if (leader && (int)threadIdx.x < n) {  // the newest row, kept for the next steps
-    const int kn = sel.slot[n - 1], sa = sel.slot[threadIdx.x];
-    ab.gram[sa * MAX_AA + kn] = dots[threadIdx.x];
-    ab.gram[kn * MAX_AA + sa] = dots[threadIdx.x];
-  }
-  if (threadIdx.x != 0) return;
-  double tr = 0.0;
-  for (int a = 0; a < n; a++) {
-    A[a][n - 1] = dots[a];
-    A[n - 1][a] = dots[a];
-  }
-  for (int a = 0; a < n; a++) {
-    A[a][n] = dots[NM + a];
-    tr += A[a][a];
-  }
-  for (int a = 0; a < n; a++) A[a][a] += 1e-12 * tr;
-  bool ok = true;
-  for (int col = 0; col < n && ok; col++) {
-    int piv = col;
-    for (int r = col + 1; r < n; r++)
-      if (fabs(A[r][col]) > fabs(A[piv][col])) piv = r;
-    if (!(fabs(A[piv][col]) > 0.0)) {
-      ok = false;
-      break;
-    }
-    if (piv != col)
-      for (int q = col; q <= n; q++) {
-        const double t = A[col][q];
-        A[col][q] = A[piv][q];
-        A[piv][q] = t;
+  block_sums<2 * NM, NT>(acc, [n](int j) { return j % NM < n; });
+  if (leader) {  // the newest row, kept for the next steps
+    const int kn = sel.slot[n - 1];
+#pragma unroll
+    for (int j = 0; j < NM; j++)
+      if (j < n && (int)threadIdx.x == j) {
+        ab.gram[sel.slot[j] * MAX_AA + kn] = acc[j];
+        ab.gram[kn * MAX_AA + sel.slot[j]] = acc[j];
       }
-    for (int r = col + 1; r < n; r++) {
-      const double l = A[r][col] / A[col][col];
-      for (int q = col; q <= n; q++) A[r][q] -= l * A[col][q];
+  }
+  if constexpr (NM <= 2) {
+    bool ok = true;
+    if (NM == 1 || n == 1) {
+      const double a = acc[0] + 1e-12 * acc[0], t = acc[NM] / a;
+      ok = fabs(a) > 0.0 && isfinite(t);
+      gam[0] = ok ? t : 0.0;
+      if (NM == 2) gam[NM - 1] = 0.0;
+    } else {
+      const double tr = g00 + acc[1 % NM], e = 1e-12 * tr;
+      double a00 = g00 + e, a01 = acc[0], b0 = acc[NM], a10 = acc[0], a11 = acc[1 % NM] + e, b1 = acc[NM + 1 % NM];
+      if (fabs(a10) > fabs(a00)) {
+        const double p = a00, q = a01, t = b0;
+        a00 = a10;
+        a01 = a11;
+        b0 = b1;
+        a10 = p;
+        a11 = q;
+        b1 = t;
+      }
+      const double l = a10 / a00;
+      ok = fabs(a00) > 0.0;
+      a11 -= l * a01;
+      b1 -= l * b0;
+      ok = ok && fabs(a11) > 0.0;
+      const double g1 = b1 / a11, g0 = (b0 - a01 * g1) / a00;
+      ok = ok && isfinite(g1) && isfinite(g0);
+      gam[0] = ok ? g0 : 0.0;
+      gam[NM - 1] = ok ? g1 : 0.0;
     }
+  } else {
+    __shared__ double sg[NM];
+    if (threadIdx.x == 0) {
+      double tr = 0.0;
+#pragma unroll
+      for (int a = 0; a < NM; a++)
+        if (a < n) {
+          A[a][n - 1] = acc[a];
+          A[n - 1][a] = acc[a];
+          A[a][n] = acc[NM + a];
+        }
+      for (int a = 0; a < n; a++) tr += A[a][a];
+      for (int a = 0; a < n; a++) A[a][a] += 1e-12 * tr;
+      bool ok = true;
+      for (int col = 0; col < n && ok; col++) {
+        int piv = col;
+        for (int r = col + 1; r < n; r++)
+          if (fabs(A[r][col]) > fabs(A[piv][col])) piv = r;
+        if (!(fabs(A[piv][col]) > 0.0)) {
+          ok = false;
+          break;
+        }
+        if (piv != col)
+          for (int q = col; q <= n; q++) {
+            const double t = A[col][q];
+            A[col][q] = A[piv][q];
+            A[piv][q] = t;
+          }
+        for (int r = col + 1; r < n; r++) {
+          const double l = A[r][col] / A[col][col];
+          for (int q = col; q <= n; q++) A[r][q] -= l * A[col][q];
+        }
+      }
+      for (int a = n - 1; a >= 0 && ok; a--) {
+        double t = A[a][n];
+        for (int q = a + 1; q < n; q++) t -= A[a][q] * sg[q];
+        sg[a] = t / A[a][a];
+        ok = isfinite(sg[a]);
+      }
+      for (int a = 0; a < NM; a++)
+        if (!ok || a >= n) sg[a] = 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NM; j++) gam[j] = sg[j];
   }
-  for (int a = n - 1; a >= 0 && ok; a--) {
-    double t = A[a][n];
-    for (int q = a + 1; q < n; q++) t -= A[a][q] * gam[q];
-    gam[a] = t / A[a][a];
-    ok = isfinite(gam[a]);
+  if (leader && threadIdx.x == 0) {
+#pragma unroll
+    for (int a = 0; a < MAX_AA; a++) ab.gam[a] = a < NM ? gam[a < NM ? a : 0] : 0.0;
   }
-  for (int a = 0; a < n; a++)
-    if (!ok) gam[a] = 0.0;
-  if (leader)
-    for (int a = 0; a < MAX_AA; a++) ab.gam[a] = a < n ? gam[a] : 0.0;
 }
 
 // Mixed state of cell k: x = gp - sum_j gamma_j dG_j (gp = the newest
@@ -2058,12 +2109,9 @@ __device__ __forceinline__ void aa_mixed(const AABuf &ab, const AASel &sel, cons
 // the halo), their sqrt(T) too (ss), each formed once.
 template <int NM, int TX, int TY, typename R>
 __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R> &fl, const AAFieldsT<R> &s,
-                                            const AABuf &ab, const AASel &sel, const double *gsrc, int i0, int j0,
-                                            int tx, int ty, double (*sp)[TX + 1], double (*sT)[TX + 1],
+                                            const AABuf &ab, const AASel &sel, const double (&gam)[NM], int i0,
+                                            int j0, int tx, int ty, double (*sp)[TX + 1], double (*sT)[TX + 1],
                                             double (*ss)[TX + 1]) {
-  double gam[NM];
-#pragma unroll
-  for (int j = 0; j < NM; j++) gam[j] = gsrc[j];
   const int Nx = g.Nx, Ny = g.Ny;
   const int i = i0 + tx, j = j0 + ty;
   const bool in = i < Nx && j < Ny;
@@ -2125,16 +2173,23 @@ __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R
 
 // The weights and the mix in one launch: every workgroup folds the store
 // pass's partial sums itself (the same sums in the same order, so the same
-// weights; workgroup 0 stores the Gram row), then mixes AA_MIX_TILES tiles
-// of AA_MIX_TX x AA_MIX_TY cells in turn.
-constexpr int AA_MIX_TX = 64, AA_MIX_TY = 8, AA_MIX_TILES = 3;
+// weights; workgroup 0 stores the Gram row), then mixes its tiles of
+// AA_MIX_TX x AA_MIX_TY cells in turn (launch_aa_mix: how many).
+constexpr int AA_MIX_TX = 64, AA_MIX_TY = 8;
+// Tiles per workgroup: one while the tiles fit the workgroups the GPU holds at
+// once (256 CUs x 3), so that small grids spread over the CUs and no tile
+// waits for another (three tiles each before: 301x95 12.4 against 6.6 us,
+// 961x193 14.8 against 10.5); then as few as give about one such round, at
+// most 4, to fold the partial sums less often (1920x384, 1440 tiles: 21.6,
+// 21.4, 22.0 us with 1, 2, 3, at depth 2 27.6 against 30.4 with 2 and 3;
+// 3840x768, 5760 tiles: 117.8, 102.0, 100.2, 99.0 us with 1, 2, 3, 4).
+constexpr int AA_MIX_ROUND = 768, AA_MIX_MOST = 4;
 template <int NM, typename R>
 __global__ void __launch_bounds__(AA_MIX_TX *AA_MIX_TY) k_aa_mix(KGridT<R> g, KFieldsT<R> fl, AAFieldsT<R> s,
                                                                  AABuf ab, AASel sel, Gate gate) {
   if (gated_out(gate)) return;
-  __shared__ double gam[NM];
+  double gam[NM];
   aa_solve_group<NM, AA_MIX_TX * AA_MIX_TY>(ab, sel, gam, blockIdx.x == 0);
-  __syncthreads();
   __shared__ double sp[AA_MIX_TY + 1][AA_MIX_TX + 1], sT[AA_MIX_TY + 1][AA_MIX_TX + 1],
       ss[AA_MIX_TY + 1][AA_MIX_TX + 1];
   const int ntx = (g.Nx + AA_MIX_TX - 1) / AA_MIX_TX, ntiles = ntx * ((g.Ny + AA_MIX_TY - 1) / AA_MIX_TY);
@@ -2507,7 +2562,7 @@ template <int NM>
 __global__ void __launch_bounds__(AA_SOLVE_THREADS) kb_aa_solve(const BatchCase<double> *C, int k, AABatchSel bs) {
   const BatchCase<double> &c = C[blockIdx.x];
   if (gated_out(Gate{in_memory(c.ctrl), k + 1})) return;
-  __shared__ double gam[NM];
+  double gam[NM];
   aa_solve_group<NM, AA_SOLVE_THREADS>(aa_of(c), case_sel(c, bs), gam, true);
 }
 
@@ -2518,9 +2573,12 @@ __global__ void __launch_bounds__(TX *TY) kb_aa_mix(const BatchCase<double> *C, 
   const BatchCase<double> &c = C[t.c];
   if (gated_out(Gate{in_memory(c.ctrl), k + 1})) return;
   __shared__ double sp[TY + 1][TX + 1], sT[TY + 1][TX + 1], ss[TY + 1][TX + 1];
-  aa_mix_tile<NM, TX, TY>(grid_of(c), fields_at(c, par), case_state(c, par), aa_of(c), case_sel(c, bs),
-                          in_memory(c.aa.gam), t.x * TX, t.y * TY, (int)threadIdx.x % TX, (int)threadIdx.x / TX, sp,
-                          sT, ss);
+  const AABuf ab = aa_of(c);
+  double gam[NM];
+#pragma unroll
+  for (int j = 0; j < NM; j++) gam[j] = ab.gam[j];
+  aa_mix_tile<NM, TX, TY>(grid_of(c), fields_at(c, par), case_state(c, par), ab, case_sel(c, bs), gam, t.x * TX,
+                          t.y * TY, (int)threadIdx.x % TX, (int)threadIdx.x / TX, sp, sT, ss);
 }
 
 // Edge conditions and the loop-2 test: one workgroup per case.
@@ -2708,7 +2766,8 @@ hipError_t launch_aa_mix(const KGridT<R> &g, const KFieldsT<R> &fl, const AAFiel
   const int Na = g.Nx * g.Ny;
   if (sel.n < 1 || sel.n > MAX_AA || ab.nb != aa_store_blocks(Na)) return hipErrorInvalidValue;
   const int ntiles = ((g.Nx + AA_MIX_TX - 1) / AA_MIX_TX) * ((g.Ny + AA_MIX_TY - 1) / AA_MIX_TY);
-  const dim3 gm((ntiles + AA_MIX_TILES - 1) / AA_MIX_TILES);
+  const int per = std::min(AA_MIX_MOST, (ntiles + AA_MIX_ROUND - 1) / AA_MIX_ROUND);
+  const dim3 gm((ntiles + per - 1) / per);
   if (sel.n <= 1)
     hipLaunchKernelGGL((k_aa_mix<1, R>), gm, dim3(AA_MIX_TX * AA_MIX_TY), 0, s, g, fl, f, ab, sel, gate);
   else if (sel.n <= 2)

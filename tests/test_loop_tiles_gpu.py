@@ -59,3 +59,28 @@ def test_loop_of_outer_iterations(sts, oracle, size, kind):
     bad = _same(sts, ctx, ora, sts.FIELDS)
     ctx.close()
     assert it == 3 and np.array_equal(log[:, :4], ro) and not bad, (log, ro, bad)
+
+
+@pytest.mark.parametrize("depth", [1, 2, 3])
+@pytest.mark.parametrize("size", [(130, 27), (1601, 257)], ids=["one_tile_each", "two_tiles_each"])
+def test_anderson_mix_tiles(sts, size, depth, tmp_path):
+    """Anderson steps on grids whose mix gives a workgroup one tile and two:
+    both end on the reference's test, so the fields are the plain path's to
+    the tolerance (1e-8) times the slow modes' amplification, as the other
+    acceleration tests allow (1e-5 relative L2)."""
+    import importlib
+
+    ws = importlib.import_module("simple-ts_amd.warmstart")
+    prm = dict(Ma=1.2, Kn=0.01, Re=1.2 / (0.01 * ws.SQ), side=0.25, xc=4.0)
+    runs = [ws.Run(ws.write_case(str(tmp_path / n), *size, prm, 3, dt_over_tin=0.005 * 240 / size[0]))
+            for n in ("plain", "aa")]
+    n_plain = n_aa = 0
+    for _ in range(2):
+        n_plain += runs[0].step()
+        n_aa += runs[1].ctx.time_step_mixed(*runs[1].loop, 0, (1e-7,) * 3, anderson=depth)[1]
+    assert n_aa < n_plain, (n_aa, n_plain)
+    for k in ("u", "v", "p", "Temper"):
+        a, b = runs[0].ctx.get(k), runs[1].ctx.get(k)
+        assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(a), k
+    for r in runs:
+        r.close()
