@@ -286,7 +286,7 @@ int sts_batch_time_step(sts_batch *b, const sts_loop_control *lc, const sts_mixe
                         int *iters64);
 /* Tile shapes of the batched launches: variant v of the cell kernels is
    64x4, 64x8, 128x2, 32x8 cells, of the fused sweep pass 60x6, 60x4, 60x8,
-   60x10 (v = 0..3).  sts_batch_autotune times each variant `reps` times on
+   60x5 (v = 0..3).  sts_batch_autotune times each variant `reps` times on
    the current state, keeps the fastest and reports the mean milliseconds per
    variant in ms[8] (cell kernels, then sweeps; may be NULL). */
 int sts_batch_set_tiles(sts_batch *b, int cell_variant, int sweep_variant);

@@ -2836,7 +2836,7 @@ hipError_t launch_continuity(const KGrid &g, const KFields &f, double *cs, doubl
 // Batched launches; tile shape variants (the autotuner's choices)
 // ---------------------------------------------------------------------------
 const int CELL_TILES[NVARIANT][2] = {{64, 4}, {64, 8}, {128, 2}, {32, 8}};
-const int SWEEP_TILES[NVARIANT][2] = {{SWEEP_X, 6}, {SWEEP_X, 4}, {SWEEP_X, 8}, {SWEEP_X, 10}};
+const int SWEEP_TILES[NVARIANT][2] = {{SWEEP_X, 6}, {SWEEP_X, 4}, {SWEEP_X, 8}, {SWEEP_X, 5}};
 
 #define CELL_SWITCH(v, KERNEL, ...)                                                                   \
   switch (v) {                                                                                        \
@@ -2912,7 +2912,7 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
         case 0: SWEEP_LAUNCH(6); break;
         case 1: SWEEP_LAUNCH(4); break;
         case 2: SWEEP_LAUNCH(8); break;
-        default: SWEEP_LAUNCH(10); break;
+        default: SWEEP_LAUNCH(5); break;
       }
       break;
     case BK_EDGES:
