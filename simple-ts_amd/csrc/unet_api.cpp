@@ -54,8 +54,11 @@ struct sts_unet {
   // activations
   float *xin = nullptr, *y = nullptr, *dy = nullptr, *tg = nullptr;
   uint8_t *mask = nullptr;
-  u16 *x = nullptr, *act[NCONV] = {}, *pl[3] = {}, *cat[3] = {};  // cat[0] = c1 (level 0) .. cat[2] = c3
-  u16 *dz = nullptr, *gA = nullptr, *gB = nullptr, *gP = nullptr, *dc[3] = {};
+  u16 *x = nullptr, *act[NCONV] = {}, *pl[3] = {};
+  u16 *gA = nullptr, *gB = nullptr, *gP = nullptr, *dc[3] = {};
+  float *part = nullptr, *bpart = nullptr;  // partial sums of the parameter gradients
+  double *carry = nullptr;                  // and their running sums, where one part does not hold them all;
+  size_t carry_n = 0;                       // behind those, 2 zeros
   double *loss = nullptr;
   int *slots_dev = nullptr;
   // training set
@@ -83,14 +86,14 @@ void free_all(sts_unet *u) {
     (void)hipFree(c.Wb);
   }
   for (void *p : {(void *)u->P, (void *)u->G, (void *)u->Mo, (void *)u->Vo, (void *)u->xin, (void *)u->y,
-                  (void *)u->dy, (void *)u->tg, (void *)u->mask, (void *)u->x, (void *)u->dz, (void *)u->gA,
+                  (void *)u->dy, (void *)u->tg, (void *)u->mask, (void *)u->x, (void *)u->part,
+                  (void *)u->bpart, (void *)u->carry, (void *)u->gA,
                   (void *)u->gB, (void *)u->gP, (void *)u->loss, (void *)u->slots_dev, (void *)u->ds_x,
                   (void *)u->ds_t, (void *)u->ds_m})
     (void)hipFree(p);
   for (int k = 0; k < NCONV; k++) (void)hipFree(u->act[k]);
   for (int k = 0; k < 3; k++) {
     (void)hipFree(u->pl[k]);
-    (void)hipFree(u->cat[k]);
     (void)hipFree(u->dc[k]);
   }
   if (u->stream) (void)hipStreamDestroy(u->stream);
@@ -98,16 +101,15 @@ void free_all(sts_unet *u) {
 
 // Re-derives the BF16 weight layouts from the FP32 master parameters.
 int pack_weights(sts_unet *u) {
+  static_assert(NCONV <= PACK_MAX, "table");
+  PackArgs a{};
+  a.P = u->P;
+  a.n = NCONV;
   for (int k = 0; k < NCONV; k++) {
-    Conv &c = u->L[k];
-    const float *W = u->P + c.w_off;
-    if (k == HEAD) {
-      U_OK(unet_pack_head(W, c.Cin * c.Cout, c.Wt, u->stream));
-      continue;
-    }
-    U_OK(unet_pack_fwd(W, 9, c.Cin, c.Cx, c.Cout, c.Kp, c.Wt, u->stream));
-    if (c.Wb) U_OK(unet_pack_bwd(W, 9, c.Cin, c.Cout, c.Kpb, c.Wb, u->stream));
+    const Conv &c = u->L[k];
+    a.c[k] = PackConv{c.w_off, c.ks * c.ks, c.Cin, c.Cx, c.Cout, k == HEAD ? c.Cin : c.Kp, c.Kpb, c.Wt, c.Wb};
   }
+  U_OK(unet_pack(a, u->stream));
   return STS_OK;
 }
 
@@ -118,36 +120,25 @@ int conv_fwd(sts_unet *u, int k, const u16 *X, int n, u16 *Y, const u16 *skip = 
   return STS_OK;
 }
 
-// Decoder conv on [nearest-up(half), skip]: materialised (training keeps the
-// concatenation for the backward pass) or read in place by the convolution.
-int conv_cat(sts_unet *u, int k, const u16 *half, int Cb, const u16 *skip, int Cs, int n, u16 *cat, bool keep,
-             u16 *Y) {
-  const int l = u->L[k].level;
-  if (!keep) return conv_fwd(u, k, half, n, Y, skip, Cb);
-  U_OK(unet_upcat(half, Cb, skip, Cs, n, u->h(l), u->w(l), cat, u->stream));
-  return conv_fwd(u, k, cat, n, Y);
-}
-
-// Backward of conv k + ReLU: g = dL/d(output) (BF16); writes the parameter
-// gradients and, if dX, the input gradient (BF16).
-int conv_back(sts_unet *u, int k, const u16 *Xin, int n, const u16 *g, u16 *dX) {
+// Backward of conv k: dz = dL/d(output before the ReLU) (BF16); writes the
+// parameter gradients and, if dX, the input gradient (BF16), passed on through
+// the ReLU of that input when act is given.  The decoder's first convolutions
+// read [nearest-up(X), skip] in place (Cb channels of X).
+int conv_back(sts_unet *u, int k, const u16 *X, int n, const u16 *dz, u16 *dX, const u16 *act = nullptr,
+              const u16 *skip = nullptr, int Cb = 0) {
   const Conv &c = u->L[k];
   const int Hh = u->h(c.level), Ww = u->w(c.level);
-  const size_t np = u->npix(n, c.level);
-  U_OK(unet_relu_mask(g, u->act[k], np * c.Cout, u->dz, u->stream));
-  WgradArgs wa{Xin, c.Cx, c.Cin, n, Hh, Ww, 3, u->dz, c.Cout, u->G + c.w_off, 2048};
-  U_OK(unet_wgrad(wa, u->stream));
-  U_OK(unet_bgrad(u->dz, (int)np, c.Cout, u->G + c.b_off, u->stream));
+  U_OK(unet_wgrad(WgradArgs{X, c.Cx, c.Cin, n, Hh, Ww, dz, c.Cout, u->part, u->bpart, u->carry + u->carry_n, skip, Cb}, u->carry, u->G + c.w_off,
+                  u->G + c.b_off, u->stream));
   if (dX) {
-    ConvArgs a{u->dz, c.Cout, n, Hh, Ww, 3, c.Wb, c.Kpb, nullptr, c.Cx, dX, 0};
+    ConvArgs a{dz, c.Cout, n, Hh, Ww, 3, c.Wb, c.Kpb, nullptr, c.Cx, dX, 0, nullptr, 0, act};
     U_OK(unet_conv(a, u->stream));
   }
   return STS_OK;
 }
 
-// Forward of the batch already in u->x; result in u->y.  keep: materialise
-// the concatenations the backward pass reads.
-int forward_dev(sts_unet *u, int n, bool keep = true) {
+// Forward of the batch already in u->x; result in u->y.
+int forward_dev(sts_unet *u, int n) {
   int rc;
   const int B = u->base;
   if ((rc = conv_fwd(u, E1A, u->x, n, u->act[E1A])) || (rc = conv_fwd(u, E1B, u->act[E1A], n, u->act[E1B])))
@@ -161,13 +152,14 @@ int forward_dev(sts_unet *u, int n, bool keep = true) {
   U_OK(unet_pool(u->act[E3B], n, u->h(2), u->w(2), 4 * B, u->pl[2], u->stream));
   if ((rc = conv_fwd(u, BA, u->pl[2], n, u->act[BA])) || (rc = conv_fwd(u, BB, u->act[BA], n, u->act[BB])))
     return rc;
-  if ((rc = conv_cat(u, D3A, u->act[BB], 8 * B, u->act[E3B], 4 * B, n, u->cat[2], keep, u->act[D3A])) ||
+  // decoder convolutions on [nearest-up(half), skip], read in place
+  if ((rc = conv_fwd(u, D3A, u->act[BB], n, u->act[D3A], u->act[E3B], 8 * B)) ||
       (rc = conv_fwd(u, D3B, u->act[D3A], n, u->act[D3B])))
     return rc;
-  if ((rc = conv_cat(u, D2A, u->act[D3B], 4 * B, u->act[E2B], 2 * B, n, u->cat[1], keep, u->act[D2A])) ||
+  if ((rc = conv_fwd(u, D2A, u->act[D3B], n, u->act[D2A], u->act[E2B], 4 * B)) ||
       (rc = conv_fwd(u, D2B, u->act[D2A], n, u->act[D2B])))
     return rc;
-  if ((rc = conv_cat(u, D1A, u->act[D2B], 2 * B, u->act[E1B], B, n, u->cat[0], keep, u->act[D1A])) ||
+  if ((rc = conv_fwd(u, D1A, u->act[D2B], n, u->act[D1A], u->act[E1B], 2 * B)) ||
       (rc = conv_fwd(u, D1B, u->act[D1A], n, u->act[D1B])))
     return rc;
   const Conv &hd = u->L[HEAD];
@@ -175,40 +167,48 @@ int forward_dev(sts_unet *u, int n, bool keep = true) {
   return STS_OK;
 }
 
-// Backward from u->dy (FP32) after forward_dev of the same batch.
+// Backward from u->dy (FP32) after forward_dev of the same batch.  Every
+// gradient that reaches a convolution has passed its ReLU in the kernel that
+// wrote it.
 int backward_dev(sts_unet *u, int n) {
   const int B = u->base;
-  U_OK(hipMemsetAsync(u->G, 0, sizeof(float) * u->nparams, u->stream));
   const Conv &hd = u->L[HEAD];
-  U_OK(unet_head_back(u->dy, u->act[D1B], B, hd.Wt, u->cout, (int)u->npix(n, 0), u->gA, u->G + hd.w_off,
-                      u->G + hd.b_off, u->stream));
+  U_OK(unet_head_back(u->dy, u->act[D1B], B, hd.Wt, u->cout, (int)u->npix(n, 0), u->gA, u->part, u->G + hd.w_off,
+                      u->stream));
   int rc;
   // decoder level 0
-  if ((rc = conv_back(u, D1B, u->act[D1A], n, u->gA, u->gB)) || (rc = conv_back(u, D1A, u->cat[0], n, u->gB, u->dc[0])))
+  if ((rc = conv_back(u, D1B, u->act[D1A], n, u->gA, u->gB, u->act[D1A])) ||
+      (rc = conv_back(u, D1A, u->act[D2B], n, u->gB, u->dc[0], nullptr, u->act[E1B], 2 * B)))
     return rc;
-  U_OK(unet_up_back(u->dc[0], 3 * B, 2 * B, n, u->h(0), u->w(0), u->gA, u->stream));
+  U_OK(unet_up_back(u->dc[0], 3 * B, 2 * B, u->act[D2B], n, u->h(0), u->w(0), u->gA, u->stream));
   // decoder level 1
-  if ((rc = conv_back(u, D2B, u->act[D2A], n, u->gA, u->gB)) || (rc = conv_back(u, D2A, u->cat[1], n, u->gB, u->dc[1])))
+  if ((rc = conv_back(u, D2B, u->act[D2A], n, u->gA, u->gB, u->act[D2A])) ||
+      (rc = conv_back(u, D2A, u->act[D3B], n, u->gB, u->dc[1], nullptr, u->act[E2B], 4 * B)))
     return rc;
-  U_OK(unet_up_back(u->dc[1], 6 * B, 4 * B, n, u->h(1), u->w(1), u->gA, u->stream));
+  U_OK(unet_up_back(u->dc[1], 6 * B, 4 * B, u->act[D3B], n, u->h(1), u->w(1), u->gA, u->stream));
   // decoder level 2
-  if ((rc = conv_back(u, D3B, u->act[D3A], n, u->gA, u->gB)) || (rc = conv_back(u, D3A, u->cat[2], n, u->gB, u->dc[2])))
+  if ((rc = conv_back(u, D3B, u->act[D3A], n, u->gA, u->gB, u->act[D3A])) ||
+      (rc = conv_back(u, D3A, u->act[BB], n, u->gB, u->dc[2], nullptr, u->act[E3B], 8 * B)))
     return rc;
-  U_OK(unet_up_back(u->dc[2], 12 * B, 8 * B, n, u->h(2), u->w(2), u->gA, u->stream));
+  U_OK(unet_up_back(u->dc[2], 12 * B, 8 * B, u->act[BB], n, u->h(2), u->w(2), u->gA, u->stream));
   // bottleneck (level 3)
-  if ((rc = conv_back(u, BB, u->act[BA], n, u->gA, u->gB)) || (rc = conv_back(u, BA, u->pl[2], n, u->gB, u->gP)))
+  if ((rc = conv_back(u, BB, u->act[BA], n, u->gA, u->gB, u->act[BA])) ||
+      (rc = conv_back(u, BA, u->pl[2], n, u->gB, u->gP)))
     return rc;
-  U_OK(unet_pool_back_add(u->gP, u->dc[2], 12 * B, 8 * B, n, u->h(2), u->w(2), 4 * B, u->gA, u->stream));
+  U_OK(unet_pool_back_add(u->gP, u->dc[2], 12 * B, 8 * B, u->act[E3B], n, u->h(2), u->w(2), 4 * B, u->gA, u->stream));
   // encoder level 2
-  if ((rc = conv_back(u, E3B, u->act[E3A], n, u->gA, u->gB)) || (rc = conv_back(u, E3A, u->pl[1], n, u->gB, u->gP)))
+  if ((rc = conv_back(u, E3B, u->act[E3A], n, u->gA, u->gB, u->act[E3A])) ||
+      (rc = conv_back(u, E3A, u->pl[1], n, u->gB, u->gP)))
     return rc;
-  U_OK(unet_pool_back_add(u->gP, u->dc[1], 6 * B, 4 * B, n, u->h(1), u->w(1), 2 * B, u->gA, u->stream));
+  U_OK(unet_pool_back_add(u->gP, u->dc[1], 6 * B, 4 * B, u->act[E2B], n, u->h(1), u->w(1), 2 * B, u->gA, u->stream));
   // encoder level 1
-  if ((rc = conv_back(u, E2B, u->act[E2A], n, u->gA, u->gB)) || (rc = conv_back(u, E2A, u->pl[0], n, u->gB, u->gP)))
+  if ((rc = conv_back(u, E2B, u->act[E2A], n, u->gA, u->gB, u->act[E2A])) ||
+      (rc = conv_back(u, E2A, u->pl[0], n, u->gB, u->gP)))
     return rc;
-  U_OK(unet_pool_back_add(u->gP, u->dc[0], 3 * B, 2 * B, n, u->h(0), u->w(0), B, u->gA, u->stream));
+  U_OK(unet_pool_back_add(u->gP, u->dc[0], 3 * B, 2 * B, u->act[E1B], n, u->h(0), u->w(0), B, u->gA, u->stream));
   // encoder level 0
-  if ((rc = conv_back(u, E1B, u->act[E1A], n, u->gA, u->gB)) || (rc = conv_back(u, E1A, u->x, n, u->gB, nullptr)))
+  if ((rc = conv_back(u, E1B, u->act[E1A], n, u->gA, u->gB, u->act[E1A])) ||
+      (rc = conv_back(u, E1A, u->x, n, u->gB, nullptr)))
     return rc;
   return STS_OK;
 }
@@ -297,10 +297,20 @@ extern "C" int sts_unet_create(int cin, int cout, int base, int max_n, int H, in
   }
   for (int l = 0; l < 3; l++) {
     A_OK(hipMalloc(&u->pl[l], sizeof(u16) * u->npix(max_n, l + 1) * (B << l)));
-    A_OK(hipMalloc(&u->cat[l], sizeof(u16) * u->npix(max_n, l) * 3 * (B << l)));
     A_OK(hipMalloc(&u->dc[l], sizeof(u16) * u->npix(max_n, l) * 3 * (B << l)));
   }
-  A_OK(hipMalloc(&u->dz, sizeof(u16) * big));
+  size_t part = ((n0 + 255) / 256) * (size_t)(B + 1) * cout, bpart = 0;
+  for (int k = 0; k < HEAD; k++) {
+    const Conv &c = u->L[k];
+    const size_t np = u->npix(max_n, c.level), P = (size_t)9 * c.Cin * c.Cout;
+    part = std::max(part, std::max(P, std::min(UNET_PART_FLOATS, (np + 2047) / 2048 * P)));
+    bpart = std::max(bpart, (np + 1023) / 1024 * (size_t)c.Cout);
+    u->carry_n = std::max(u->carry_n, (P + 1) / 2 * 2);
+  }
+  A_OK(hipMalloc(&u->part, sizeof(float) * part));
+  A_OK(hipMalloc(&u->bpart, sizeof(float) * bpart));
+  A_OK(hipMalloc(&u->carry, sizeof(double) * (u->carry_n + 2)));
+  A_OK(hipMemsetAsync(u->carry + u->carry_n, 0, 2 * sizeof(double), u->stream));
   A_OK(hipMalloc(&u->gA, sizeof(u16) * big));
   A_OK(hipMalloc(&u->gB, sizeof(u16) * big));
   A_OK(hipMalloc(&u->gP, sizeof(u16) * big));
@@ -365,7 +375,7 @@ extern "C" int sts_unet_infer(sts_unet *u, int n, const float *x, float *y) {
   const size_t np = u->npix(n, 0);
   U_OK(hipMemcpyAsync(u->xin, x, sizeof(float) * np * u->cin, hipMemcpyHostToDevice, u->stream));
   U_OK(unet_to_bf16(u->xin, u->cin, u->Cx0, np, u->x, u->stream));
-  if ((rc = forward_dev(u, n, false))) return rc;
+  if ((rc = forward_dev(u, n))) return rc;
   U_OK(hipMemcpyAsync(y, u->y, sizeof(float) * np * u->cout, hipMemcpyDeviceToHost, u->stream));
   U_OK(hipStreamSynchronize(u->stream));
   return STS_OK;
@@ -381,13 +391,24 @@ extern "C" int sts_unet_backward(sts_unet *u, int n, const float *dy) {
   return STS_OK;
 }
 
-// Loss + dy on the device, then backward; count = masked cells.
-static int loss_backward_dev(sts_unet *u, int n, long long count, double *loss, bool backward) {
+// One Adam step and the BF16 weights that follow from it.
+static int adam_dev(sts_unet *u, float lr, float b1, float b2, float eps) {
+  u->adam_t++;
+  const float c1 = 1.0f - (float)std::pow((double)b1, u->adam_t), c2 = 1.0f - (float)std::pow((double)b2, u->adam_t);
+  U_OK(unet_adam(u->P, u->G, u->Mo, u->Vo, u->nparams, lr, b1, b2, eps, c1, c2, u->stream));
+  return pack_weights(u);
+}
+
+// Loss + dy on the device, then backward; count = masked cells.  adam_lr: then
+// one Adam step (the loss is read back behind its launches).
+static int loss_backward_dev(sts_unet *u, int n, long long count, double *loss, bool backward,
+                             const float *adam_lr = nullptr) {
   U_OK(hipMemsetAsync(u->loss, 0, sizeof(double), u->stream));
   const float inv = 1.0f / (float)((double)(count > 0 ? count : 1) * u->cout);
   U_OK(unet_mse(u->y, u->tg, u->mask, u->cout, (int)u->npix(n, 0), inv, u->dy, u->loss, u->stream));
   int rc;
   if (backward && (rc = backward_dev(u, n))) return rc;
+  if (adam_lr && (rc = adam_dev(u, *adam_lr, 0.9f, 0.999f, 1e-8f))) return rc;
   if (loss) U_OK(hipMemcpyAsync(loss, u->loss, sizeof(double), hipMemcpyDeviceToHost, u->stream));
   U_OK(hipStreamSynchronize(u->stream));
   return STS_OK;
@@ -407,10 +428,7 @@ extern "C" int sts_unet_backward_mse(sts_unet *u, int n, const float *t, const u
 
 extern "C" int sts_unet_adam(sts_unet *u, float lr, float b1, float b2, float eps) {
   if (!u) return ufail(STS_ERR_ARG, "null argument");
-  u->adam_t++;
-  const float c1 = 1.0f - (float)std::pow((double)b1, u->adam_t), c2 = 1.0f - (float)std::pow((double)b2, u->adam_t);
-  U_OK(unet_adam(u->P, u->G, u->Mo, u->Vo, u->nparams, lr, b1, b2, eps, c1, c2, u->stream));
-  int rc = pack_weights(u);
+  int rc = adam_dev(u, lr, b1, b2, eps);
   if (rc) return rc;
   U_OK(hipStreamSynchronize(u->stream));
   return STS_OK;
@@ -506,9 +524,7 @@ static int batch_loss(sts_unet *u, const int *slots, int n, double *loss, bool t
   U_OK(hipMemcpyAsync(u->slots_dev, slots, sizeof(int) * n, hipMemcpyHostToDevice, u->stream));
   U_OK(unet_gather(u->ds_x, u->ds_t, u->ds_m, u->slots_dev, n, np, u->Cx0, u->cout, u->x, u->tg, u->mask, u->stream));
   if ((rc = forward_dev(u, n))) return rc;
-  if ((rc = loss_backward_dev(u, n, count, loss, train))) return rc;
-  if (train) return sts_unet_adam(u, lr, 0.9f, 0.999f, 1e-8f);
-  return STS_OK;
+  return loss_backward_dev(u, n, count, loss, train, train ? &lr : nullptr);
 }
 
 extern "C" int sts_unet_train_step(sts_unet *u, const int *slots, int n, float lr, double *loss) {
@@ -528,7 +544,7 @@ int sts_internal_unet_correct(sts_unet *u, const StsView &v, const sts_unet_corr
   const CorrFields xe{{v.xe[0], v.xe[1], v.xe[2], v.xe[3]}};
   U_OK(unet_pack_corr_in(state_fields(v, true), xe, v.mask, np, u->Cx0, 1.0 / nrm->u_ref, 1.0 / nrm->p_ref,
                          1.0 / nrm->step, u->x, u->stream));
-  if ((rc = forward_dev(u, 1, false))) return rc;
+  if ((rc = forward_dev(u, 1))) return rc;
   CorrBoxes bx{v.Nx, v.px, {}, {}, {}};
   for (int q = 0; q < 4; q++) {
     bx.u[q] = v.box_u[q];
@@ -550,7 +566,7 @@ int sts_internal_unet_predict(sts_unet *u, const StsView &v, const sts_unet_norm
   const double *const *f = v.f;
   U_OK(unet_pack_state(f[STS_U], f[STS_V], f[STS_P], f[STS_T], v.mask, np, u->Cx0, 1.0 / nrm->u_ref, 1.0 / nrm->p_ref,
                        u->x, u->stream));
-  if ((rc = forward_dev(u, 1, false))) return rc;
+  if ((rc = forward_dev(u, 1))) return rc;
   U_OK(unet_apply_pred(u->y, f[STS_P], f[STS_T], v.mask, v.Nx, np, v.box_o, nrm->p_ref * nrm->dp_scale,
                        nrm->dT_scale, pw, Tw, u->stream));
   U_OK(hipStreamSynchronize(u->stream));

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "unet_launch.h"
 
 namespace {
@@ -115,7 +117,8 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
         if (p >= npix) continue;
         float v = acc[x][y][q] + bias;
         if (a.relu) v = fmaxf(v, 0.f);
-        a.Y[(size_t)p * a.Cout + co] = f2bf(v);
+        const size_t o = (size_t)p * a.Cout + co;
+        a.Y[o] = (a.act && !(bf2f(a.act[o]) > 0.f)) ? (u16)0 : f2bf(v);
       }
   }
 }
@@ -243,145 +246,355 @@ __global__ void __launch_bounds__(256) k_conv_lds(ConvArgs a) {
         if (i >= a.W) continue;
         float v = acc[x][y][q] + bias;
         if (a.relu) v = fmaxf(v, 0.f);
-        a.Y[((size_t)(n * a.H + j) * a.W + i) * a.Cout + co] = f2bf(v);
+        const size_t o = ((size_t)(n * a.H + j) * a.W + i) * a.Cout + co;
+        a.Y[o] = (a.act && !(bf2f(a.act[o]) > 0.f)) ? (u16)0 : f2bf(v);
       }
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient dW[t][ci][co] += sum_p X[p + off(t)][ci] * dZ[p][co]:
-// GEMM with M = co, N = k = t*Cx + ci, reduced over pixels.  Wave w of block
-// (bx, by, bz) owns k tile [64 bx + 16 w, +16), co tile [16 by, +16), pixels
-// [bz * chunk, +chunk); partial sums go to dW with atomicAdd.  W (row length)
-// is a multiple of 8, so the 8 pixels of a lane are one row segment.
+// Weight gradient of a 3x3 convolution, dW[t][ci][co] = sum_p X[p + off(t)][ci] *
+// dZ[p][co]: a GEMM with M = co, N = ci for each of the 9 taps, reduced over
+// pixels.
+//
+// A workgroup takes one run of WG_RUN consecutive pixels for 16 WCI input
+// channels x 16 MT WCO output channels x 9 taps; a wave owns 16 x 16 MT of them
+// for five or four of the taps.  Per step of 64 pixels (8 groups of 8, each
+// within an image row; 32 pixels with 4 waves) a wave stages one group: dZ and
+// the 3 x 10 pixels of X that the taps read, as they lie in memory, in one of two
+// LDS buffers, the loads of the next AHEAD steps in flight in registers: one
+// barrier per step.  Both operands need 8 consecutive pixels of one channel per
+// lane: ds_read_b64_tr_b16 reads them transposed (lane i of 16 gets channel i of
+// 4 pixels), and a tap's shift is then only another pixel address.  The workgroup
+// leaves its sums in its own slot of `part` (laid out as the gradient is);
+// k_sum_parts adds the slots in FP64: no atomics, and the same gradients on every
+// run.  The runs' length and the order within them, for the bias too, are those
+// the sums always had: each slot holds the same bits as before.
+//
+// The bound is the chain of a step (LDS write, barrier, transposed reads, MFMA):
+// a layer with one workgroup per CU takes 27 us whatever its size.  At 8 x 512 x
+// 128, base 32: 590 us per training step for the 14 convolutions, biases
+// included.  The kernels before took 3,484 us (one wave per 16 x 16 of one tap,
+// channel-strided 2-byte loads, atomics) and 2,958 us for the biases.  Loads
+// under an exec mask had to be waited for at each branch's end (73 us per layer);
+// the bias summed by a wave of the tile's own added 13 us to each layer: it has
+// workgroups of its own.  Pixel strides of 96 and 160 bytes put 4 pixels x 32
+// bytes on distinct banks.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_wgrad(WgradArgs a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int npix = a.N * a.H * a.W;
-  const int kk = blockIdx.x * 64 + wave * 16 + r;  // B column of this lane
-  const int co = blockIdx.y * 16 + r;              // A row of this lane
-  const int rad = a.ks / 2, taps = a.ks * a.ks;
-  const int t = kk / a.Cx, ci = kk - t * a.Cx;
-  const bool kv = t < taps && ci < a.Cin;
-  const int dy = kv ? t / a.ks - rad : 0, dx = kv ? t % a.ks - rad : 0;
-  const bool cv = co < a.Cout;
-  const int pbeg = blockIdx.z * a.chunk, pend = min(npix, pbeg + a.chunk);
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int pc = pbeg; pc < pend; pc += 32) {
-    const int p = pc + 8 * g;  // 8 pixels p..p+7, one row segment
-    U16x8 av{}, bv{};
-    if (p < pend) {
-      const int i0 = p % a.W, tt = p / a.W, j = tt % a.H, n = tt / a.H;
-      if (cv) {
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+
+// Channels c0 .. c0 + 15 (lane i = channel i) of 8 pixels of a row, as MFMA
+// operand: base = LDS address of channel c0 + 4 (lane & 3) of pixel (lane & 15)
+// / 4 of them.
+__device__ __forceinline__ bf16x8 load_tr(const unsigned char *base, int stride) {
+  typedef __attribute__((address_space(3))) s16x4 *Lp;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lp)(base));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lp)(base + 4 * stride));
+  return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+constexpr int WG_RUN = 2048, WG_BIAS = 1024;  // pixels per slot of the weights and of the bias
+
+template <int WCI, int WCO, int MT, int AHEAD, bool CAT>
+__global__ void __launch_bounds__(128 * WCI * WCO, MT == 4 ? 2 : 4) k_wgrad(WgradArgs a, int run0) {
+  constexpr int NW = 2 * WCI * WCO, CI = 16 * WCI, CO = 16 * MT * WCO;
+  static_assert((NW == 4 || NW == 8) && CI <= 64 && CO <= 64, "tile");
+  constexpr int SX = CI == 64 ? 160 : 96, SZ = CO == 64 ? 160 : 96;  // bytes per pixel
+  constexpr int VX = CI / 8, VZ = CO / 8;                            // 16-byte vectors per pixel
+  // A step takes NW groups, one staged by each wave: vectors per lane, and the
+  // pixels that the lanes then write (those past 30 and 8 are not read: no branch
+  // around a store to LDS either).
+  constexpr int STEP = 8 * NW, RX = 32 * VX / 64, NX = 32, NZ = 64 / VZ;
+  static_assert(AHEAD % 2 == 0 && VX >= 2, "buffers, vectors");
+  __shared__ alignas(16) unsigned char Xs[2][NW][NX * SX], Zs[2][NW][NZ * SZ];
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  const int wci = wave % WCI, wco = wave / WCI % WCO, wt = wave / (WCI * WCO);
+  const int ci0 = blockIdx.x * CI, co0 = blockIdx.y * CO, H = a.H, W = a.W;
+  const int npix = a.N * H * W, run = run0 + (int)blockIdx.z;
+  const int pbeg = run * WG_RUN, pend = min(npix, pbeg + WG_RUN);
+  if (blockIdx.x == gridDim.x - 1) {  // the bias: a lane takes a channel of one of the two runs
+    const int co = co0 + (int)threadIdx.x % CO, p0 = pbeg + (int)threadIdx.x / CO * WG_BIAS;
+    const int p1 = min(npix, p0 + WG_BIAS);
+    if ((int)threadIdx.x >= WG_RUN / WG_BIAS * CO || co >= a.Cout || p0 >= p1) return;
+    const u16 *z = a.dZ + (size_t)p0 * a.Cout + co;
+    const int C = a.Cout;
+    float s = 0.f;
+    int p = 0;
+    const int n = p1 - p0;  // a multiple of 8
+    if (n >= 32) {          // two batches of pixels, one in flight (at the end the last one again)
+      u16 v0[32], v1[32];
+      auto load = [&](u16 (&d)[32], int at) {
+        const u16 *q0 = z + (size_t)min(at, n - 32) * C;
 #pragma unroll
-        for (int q = 0; q < 8; q++) av.v[q] = a.dZ[(size_t)(p + q) * a.Cout + co];
+        for (int q = 0; q < 32; q++) d[q] = *q0, q0 += C;
+      };
+      auto add = [&](const u16 (&d)[32]) {
+#pragma unroll
+        for (int q = 0; q < 32; q++) s += bf2f(d[q]);
+      };
+      load(v0, 0);
+      for (; p + 64 <= n; p += 64) {
+        load(v1, p + 32);
+        add(v0);
+        load(v0, p + 64);
+        add(v1);
       }
-      const int jj = j + dy;
-      if (kv && jj >= 0 && jj < a.H) {
-        const size_t rowb = (size_t)(n * a.H + jj) * a.W;
+      if (p + 32 <= n) add(v0), p += 32;
+    }
+    for (; p < n; p += 8) {
+      float d[8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-          const int ii = i0 + q + dx;
-          bv.v[q] = (ii >= 0 && ii < a.W) ? a.X[(rowb + ii) * a.Cx + ci] : (u16)0;
+      for (int q = 0; q < 8; q++) d[q] = bf2f(z[(size_t)(p + q) * C]);
+#pragma unroll
+      for (int q = 0; q < 8; q++) s += d[q];
+    }
+    a.bpart[(size_t)(p0 / WG_BIAS) * a.Cout + co] = s;
+    return;
+  }
+  floatx4 acc[5][MT];  // taps 5 wt ..
+#pragma unroll
+  for (int m = 0; m < MT; m++)
+#pragma unroll
+    for (int q = 0; q < 5; q++) acc[q][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  u32x4 qx[AHEAD][RX], qz[AHEAD];
+  // first pixel (fp), column, row and image of the wave's group in the next
+  // step to fetch
+  int fp = pbeg + 8 * wave, fi = fp % W, fn = fp / W / H, fj = fp / W - fn * H;
+  // Per vector: its address, and where it lies outside the image: bit 0 / 1 in
+  // the first / last row's group, 2 / 3 in the first / last column's, 4 past the
+  // run's end, 5 always.  A vector outside is loaded from a.zero: no branch around
+  // a load, which would have to be waited for at the branch's end.
+  // bu: in the half-size image, less the group's first pixel's address and for an
+  // even row (in an odd one the rows above and below are one row further down).
+  typedef unsigned long long U64;
+  U64 bx[RX], bu[CAT ? RX : 1];
+  int ox[RX];
+  bool up[RX];
+  const int Cs = CAT ? a.Cx - a.Cb : a.Cx;
+#pragma unroll
+  for (int k = 0; k < RX; k++) {
+    const int e = lane + 64 * k, px = e / VX, ci = ci0 + 8 * (e % VX);
+    const int dy = px / 10 - 1, dx = px % 10 - 1;
+    up[k] = CAT && ci < a.Cb;
+    bx[k] = (U64)(CAT ? a.X2 : a.X) + 2ll * ((fp + (long long)dy * W + dx) * Cs + (CAT ? ci - a.Cb : ci));
+    if (CAT) bu[k] = (U64)a.X + 2ll * (((long long)(dy >> 1) * (W / 2) + (dx >> 1)) * a.Cb + ci);
+    ox[k] = (dy < 0) | (dy > 0) << 1 | (dx < 0) << 2 | (dx > 7) << 3 | 16 | (e >= 30 * VX || ci >= a.Cx) << 5;
+  }
+  const int zpx = lane / VZ, zco = co0 + 8 * (lane % VZ);
+  U64 bz = (U64)a.dZ + 2ll * (((long long)fp + zpx) * a.Cout + zco);
+  const int oz = 16 | (zpx >= 8 || zco >= a.Cout) << 5;
+  typedef const __attribute__((address_space(1))) u32x4 *Gp;
+  auto fetch = [&](u32x4 (&x)[RX], u32x4 &z) {
+    const int i = fi, j = fj;
+    const int out = (j == 0 ? 1 : 0) + (j == H - 1 ? 2 : 0) + (i == 0 ? 4 : 0) + (i + 8 == W ? 8 : 0) +
+                    (fp >= pend ? 16 : 0) + 32;
+    const U64 su = CAT ? 2ull * ((U64)(fn * (H / 2) + j / 2) * (U64)(W / 2) + (U64)(i / 2)) * (U64)a.Cb : 0;
+    const U64 su1 = CAT && (j & 1) ? su + 2ull * (U64)(W / 2) * (U64)a.Cb : su;
+#pragma unroll
+    for (int k = 0; k < RX; k++) {
+      U64 at = bx[k];
+      if (CAT) {
+        const U64 half = bu[k] + (ox[k] & 3 ? su1 : su);
+        at = up[k] ? half : at;
+      }
+      x[k] = *(Gp)(ox[k] & out ? (U64)a.zero : at);
+      bx[k] += 2ull * STEP * (U64)Cs;
+    }
+    z = *(Gp)(oz & out ? (U64)a.zero : bz);
+    bz += 2ull * STEP * (U64)a.Cout;
+    fp += STEP;
+    for (fi += STEP; fi >= W; fi -= W)
+      if (++fj == H) fj = 0, fn++;
+  };
+#pragma unroll
+  for (int k = 0; k < AHEAD; k++) fetch(qx[k], qz[k]);
+  for (int p0 = pbeg; p0 < pend; p0 += STEP * AHEAD) {  // (zeros past the end)
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) {
+      const int buf = k & 1;  // its readers are past the last barrier
+#pragma unroll
+      for (int v = 0; v < RX; v++) {
+        const int e = lane + 64 * v;
+        *reinterpret_cast<u32x4 *>(&Xs[buf][wave][(e / VX) * SX + 16 * (e % VX)]) = qx[k][v];
+      }
+      *reinterpret_cast<u32x4 *>(&Zs[buf][wave][zpx * SZ + 16 * (lane % VZ)]) = qz[k];
+      __syncthreads();
+      fetch(qx[k], qz[k]);
+#pragma unroll
+      for (int h = 0; h < NW; h += 4) {
+        const int x = r >> 2;
+        const unsigned char *zb = &Zs[buf][h + g][x * SZ + 2 * (16 * MT * wco + 4 * (r & 3))];
+        const unsigned char *xb = &Xs[buf][h + g][(11 + x) * SX + 2 * (16 * wci + 4 * (r & 3))];
+        bf16x8 A[MT];
+#pragma unroll
+        for (int m = 0; m < MT; m++) A[m] = load_tr(zb + 32 * m, SZ);
+        auto tap = [&](int t, floatx4 (&d)[MT]) {
+          const bf16x8 B = load_tr(xb + ((t / 3 - 1) * 10 + t % 3 - 1) * SX, SX);
+#pragma unroll
+          for (int m = 0; m < MT; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], B, d[m], 0, 0, 0);
+        };
+        if (wt == 0) {
+#pragma unroll
+          for (int q = 0; q < 5; q++) tap(q, acc[q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; q++) tap(5 + q, acc[q]);
         }
       }
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv), acc,
-                                                  0, 0, 0);
   }
-  // D rows = co (4g + q of the tile), column = k tile entry r
-  const int col_k = blockIdx.x * 64 + wave * 16 + r;
-  const int tc = col_k / a.Cx, cc = col_k - tc * a.Cx;
-  if (tc >= taps || cc >= a.Cin) return;
+  // D rows = co (4 g + q of the tile), column = ci
+  float *out = a.part + (size_t)blockIdx.z * (9 * a.Cin) * a.Cout;
+  const int ci = ci0 + 16 * wci + r;
+  if (ci >= a.Cin) return;
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int c = blockIdx.y * 16 + 4 * g + q;
-    if (c < a.Cout) atomicAdd(&a.dW[((size_t)tc * a.Cin + cc) * a.Cout + c], acc[q]);
+  for (int m = 0; m < MT; m++) {
+    const int co = co0 + 16 * (MT * wco + m) + 4 * g;
+    if (co >= a.Cout) continue;
+#pragma unroll
+    for (int q = 0; q < 5; q++)
+      if (5 * wt + q < 9) *reinterpret_cast<floatx4 *>(out + ((size_t)(5 * wt + q) * a.Cin + ci) * a.Cout + co) = acc[q][m];
   }
 }
 
-// db[co] += sum_p dZ[p][co]; block = 256 threads over a pixel chunk.
-__global__ void __launch_bounds__(256) k_bgrad(const u16 *dZ, int npix, int Cout, int chunk, float *db) {
-  const int pbeg = blockIdx.x * chunk, pend = min(npix, pbeg + chunk);
-  for (int co = threadIdx.x; co < Cout; co += blockDim.x) {
-    float s = 0.f;
-    for (int p = pbeg; p < pend; p++) s += bf2f(dZ[(size_t)p * Cout + co]);
-    atomicAdd(&db[co], s);
+// Sums of slots of FP32 partial sums, in FP64 and a fixed order (each addition
+// of the many is then as good as exact): over part[s * P + e], s < S, for every
+// e < P (a multiple of 4) -- 8 runs of slots side by side, then the runs in
+// turn -- onto carry[e] unless `first`, into out[e] (rounded) if `last`, else
+// into carry[e].
+constexpr int SUM_RUNS = 8;
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// The same for one e of few, by one wave: lane l adds slots l, l + 64, .., then
+// the lanes in a fixed tree.
+__device__ __forceinline__ void sum_row(const float *part, int S, int P, int e, float *out) {
+  const int lane = threadIdx.x & 63;
+  if (e >= P) return;
+  double v = 0.0;
+  for (int q = lane; q < S; q += 64) v += (double)part[(size_t)q * P + e];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if (lane == 0) out[e] = (float)v;
+}
+
+__global__ void __launch_bounds__(256) k_sum_rows(const float *part, int S, int P, float *out) {
+  sum_row(part, S, P, (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), out);
+}
+
+struct SumArgs {
+  const float *part;
+  int S;
+  size_t P;
+  double *carry;
+  bool first, last;
+  float *out;
+  // workgroups past the first `groups`: rpart[rS][rP] by rows into rout
+  int groups;
+  const float *rpart;
+  int rS, rP;
+  float *rout;
+};
+__global__ void __launch_bounds__(64 * SUM_RUNS) k_sum_parts(SumArgs a) {
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+  if ((int)blockIdx.x >= a.groups) {
+    sum_row(a.rpart, a.rS, a.rP, ((int)blockIdx.x - a.groups) * SUM_RUNS + y, a.rout);
+    return;
   }
+  const size_t e = 4 * ((size_t)blockIdx.x * 64 + x);
+  const int per = (a.S + SUM_RUNS - 1) / SUM_RUNS, s1 = min(a.S, (y + 1) * per);
+  doublex4 v = {0.0, 0.0, 0.0, 0.0};
+  if (e < a.P) {
+#pragma unroll 4
+    for (int q = y * per; q < s1; q++)
+      v += __builtin_convertvector(*reinterpret_cast<const floatx4 *>(a.part + (size_t)q * a.P + e), doublex4);
+  }
+  __shared__ doublex4 sm[SUM_RUNS][64];
+  sm[y][x] = v;
+  __syncthreads();
+  if (y != 0 || e >= a.P) return;
+  if (!a.first) v += *reinterpret_cast<const doublex4 *>(a.carry + e);
+#pragma unroll
+  for (int q = 1; q < SUM_RUNS; q++) v += sm[q][x];
+  if (a.last) *reinterpret_cast<floatx4 *>(a.out + e) = __builtin_convertvector(v, floatx4);
+  else *reinterpret_cast<doublex4 *>(a.carry + e) = v;
 }
 
 // ---------------------------------------------------------------------------
 // Element-wise and layout kernels
 // ---------------------------------------------------------------------------
-// 2x2 average pool: X [N][H][W][C] -> Y [N][H/2][W/2][C]
-__global__ void k_pool(const u16 *X, int N, int H, int W, int C, u16 *Y) {
-  const size_t n_out = (size_t)N * (H / 2) * (W / 2) * C;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n_out) return;
-  const int c = (int)(e % C);
-  size_t q = e / C;
-  const int i = (int)(q % (W / 2));
-  q /= (W / 2);
-  const int j = (int)(q % (H / 2));
-  const int n = (int)(q / (H / 2));
+// Channel counts are multiples of 8: a thread moves 8 channels (16 bytes) of
+// one output pixel.
+__device__ __forceinline__ void load8f(const u16 *p, float (&v)[8]) {
+  const U16x8 q = *reinterpret_cast<const U16x8 *>(p);
+#pragma unroll
+  for (int k = 0; k < 8; k++) v[k] = bf2f(q.v[k]);
+}
+
+// Sum of the 2x2 children (row pitch W) of output pixel (n, j, i), channels
+// c .. c + 7 of a tensor of stride C: (00 + 01) + (10 + 11), as before.
+__device__ __forceinline__ void sum4(const u16 *X, int H, int W, int C, int n, int j, int i, int c, float (&s)[8]) {
   const size_t b = ((size_t)(n * H + 2 * j) * W + 2 * i) * C + c;
-  const float s = (bf2f(X[b]) + bf2f(X[b + C])) + (bf2f(X[b + (size_t)W * C]) + bf2f(X[b + (size_t)W * C + C]));
-  Y[e] = f2bf(s * 0.25f);
+  float x[4][8];
+  load8f(X + b, x[0]);
+  load8f(X + b + C, x[1]);
+  load8f(X + b + (size_t)W * C, x[2]);
+  load8f(X + b + (size_t)W * C + C, x[3]);
+#pragma unroll
+  for (int k = 0; k < 8; k++) s[k] = (x[0][k] + x[1][k]) + (x[2][k] + x[3][k]);
 }
 
-// concat [nearest-up(B), S]: B [N][H/2][W/2][Cb], S [N][H][W][Cs] -> O [N][H][W][Cb+Cs]
-__global__ void k_upcat(const u16 *B, int Cb, const u16 *S, int Cs, int N, int H, int W, u16 *O) {
-  const int C = Cb + Cs;
-  const size_t n_out = (size_t)N * H * W * C;
+// 2x2 average pool: X [N][H][W][C] -> Y [N][H/2][W/2][C]
+__global__ void __launch_bounds__(256) k_pool(const u16 *X, int N, int H, int W, int C, u16 *Y) {
+  const int V = C / 8, h = H / 2, w = W / 2;
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n_out) return;
-  const int c = (int)(e % C);
-  const size_t p = e / C;
-  const int i = (int)(p % W);
-  const size_t t = p / W;
-  const int j = (int)(t % H), n = (int)(t / H);
-  O[e] = (c < Cb) ? B[((size_t)(n * (H / 2) + j / 2) * (W / 2) + i / 2) * Cb + c] : S[p * Cs + (c - Cb)];
+  if (e >= (size_t)N * h * w * V) return;
+  const int v = (int)(e % V), p = (int)(e / V), i = p % w, j = (p / w) % h, n = p / (w * h);
+  float s[8];
+  sum4(X, H, W, C, n, j, i, 8 * v, s);
+  U16x8 o;
+#pragma unroll
+  for (int k = 0; k < 8; k++) o.v[k] = f2bf(s[k] * 0.25f);
+  *reinterpret_cast<U16x8 *>(Y + 8 * e) = o;
 }
 
-// dZ = G * (Act > 0)
-__global__ void k_relu_mask(const u16 *G, const u16 *Act, size_t n, u16 *dZ) {
+// Backward of nearest-up on channels [0, Cu) of D [N][H][W][Cd], through the
+// ReLU of the upsampled tensor Act: O [N][H/2][W/2][Cu] = round(sum of the 4
+// children) where Act > 0, else 0
+__global__ void __launch_bounds__(256) k_up_back(const u16 *D, int Cd, int Cu, const u16 *Act, int N, int H, int W,
+                                                 u16 *O) {
+  const int V = Cu / 8, h = H / 2, w = W / 2;
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  dZ[e] = (bf2f(Act[e]) > 0.f) ? G[e] : (u16)0;
+  if (e >= (size_t)N * h * w * V) return;
+  const int v = (int)(e % V), p = (int)(e / V), i = p % w, j = (p / w) % h, n = p / (w * h);
+  float s[8], m[8];
+  sum4(D, H, W, Cd, n, j, i, 8 * v, s);
+  load8f(Act + 8 * e, m);
+  U16x8 o;
+#pragma unroll
+  for (int k = 0; k < 8; k++) o.v[k] = m[k] > 0.f ? f2bf(s[k]) : (u16)0;
+  *reinterpret_cast<U16x8 *>(O + 8 * e) = o;
 }
 
-// Backward of nearest-up on channels [0, Cu) of D [N][H][W][Cd]:
-// O [N][H/2][W/2][Cu] = round(sum of the 4 children)
-__global__ void k_up_back(const u16 *D, int Cd, int Cu, int N, int H, int W, u16 *O) {
-  const size_t n_out = (size_t)N * (H / 2) * (W / 2) * Cu;
+// Backward of the pool plus the skip branch, through the ReLU of the pooled
+// tensor Act: O [N][H][W][C] = round(round(P[parent] / 4) + Skip[p][off + c])
+// where Act > 0, else 0, with Skip of stride Cs.
+__global__ void __launch_bounds__(256) k_pool_back_add(const u16 *P, const u16 *Skip, int Cs, int off, const u16 *Act,
+                                                       int N, int H, int W, int C, u16 *O) {
+  const int V = C / 8;
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n_out) return;
-  const int c = (int)(e % Cu);
-  size_t q = e / Cu;
-  const int i = (int)(q % (W / 2));
-  q /= (W / 2);
-  const int j = (int)(q % (H / 2)), n = (int)(q / (H / 2));
-  const size_t b = ((size_t)(n * H + 2 * j) * W + 2 * i) * Cd + c;
-  const size_t rw = (size_t)W * Cd;
-  const float s = (bf2f(D[b]) + bf2f(D[b + Cd])) + (bf2f(D[b + rw]) + bf2f(D[b + rw + Cd]));
-  O[e] = f2bf(s);
-}
-
-// Backward of the pool plus the skip branch: O [N][H][W][C] =
-// round(round(P[parent] / 4) + Skip[p][off + c]) with Skip of stride Cs.
-__global__ void k_pool_back_add(const u16 *P, const u16 *Skip, int Cs, int off, int N, int H, int W, int C, u16 *O) {
-  const size_t n_out = (size_t)N * H * W * C;
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n_out) return;
-  const int c = (int)(e % C);
-  const size_t p = e / C;
-  const int i = (int)(p % W);
-  const size_t t = p / W;
-  const int j = (int)(t % H), n = (int)(t / H);
-  const float pb = bf2f(f2bf(bf2f(P[((size_t)(n * (H / 2) + j / 2) * (W / 2) + i / 2) * C + c]) * 0.25f));
-  O[e] = f2bf(pb + bf2f(Skip[p * Cs + off + c]));
+  if (e >= (size_t)N * H * W * V) return;
+  const int v = (int)(e % V), p = (int)(e / V), i = p % W, j = (p / W) % H, n = p / (W * H);
+  float q[8], s[8], m[8];
+  load8f(P + ((size_t)(n * (H / 2) + j / 2) * (W / 2) + i / 2) * C + 8 * v, q);
+  load8f(Skip + (size_t)p * Cs + off + 8 * v, s);
+  load8f(Act + 8 * e, m);
+  U16x8 o;
+#pragma unroll
+  for (int k = 0; k < 8; k++) o.v[k] = m[k] > 0.f ? f2bf(bf2f(f2bf(q[k] * 0.25f)) + s[k]) : (u16)0;
+  *reinterpret_cast<U16x8 *>(O + 8 * e) = o;
 }
 
 // Head (1x1 conv, linear): Y[p][o] = sum_c X[p][c] * Wb[c][o] + b[o], FP32 out.
@@ -415,48 +628,89 @@ __global__ void __launch_bounds__(256) k_head(const u16 *X, int C, const u16 *Wb
     if (o < Co) Y[(size_t)p * Co + o] = s[o] + b[o];
 }
 
-// Head backward: dX[p][c] = round(sum_o dY[p][o] Wb[c][o]); dW[c][o] and
-// db[o] accumulate per block, then atomically.
+// Head backward, through the ReLU of its input: dX[p][c] = round(sum_o
+// dY[p][o] Wb[c][o]) where X > 0, else 0; and per workgroup of 256 pixels one
+// slot of partial sums of dW[c][o] = sum_p dY[p][o] X[p][c] and (behind them)
+// db[o] = sum_p dY[p][o].  A workgroup's sum is the pairwise tree over its
+// threads (t + 128, t + 64, .. t + 1); the products of 8 channels at a time meet
+// in LDS and the 4 waves share the sums, 4 at once: the levels 32 and 16 put two
+// sums into one register each, the rest are moves within 16 lanes.  8 x 512 x 128,
+// 32 -> 2: 40 us (64 MB of X and dX: 10 us); 759 us with a tree through LDS and
+// barriers per sum and atomics.
+template <int CO>
 __global__ void __launch_bounds__(256) k_head_back(const float *dY, const u16 *X, int C, const u16 *Wb, int Co,
-                                                   int npix, u16 *dX, float *dW, float *db) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+                                                   int npix, u16 *dX, float *part) {
+  __shared__ float Ws[HEAD_MAX_W], red[8 * CO][256];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, p = (int)blockIdx.x * 256 + t;
   const bool ok = p < npix;
-  for (int c = 0; c < C; c++) {
-    float s = 0.f;
-    if (ok)
-      for (int o = 0; o < Co; o++) s += dY[(size_t)p * Co + o] * bf2f(Wb[c * Co + o]);
-    if (ok) dX[(size_t)p * C + c] = f2bf(s);
-  }
-  __shared__ float red[256];
-  for (int q = 0; q < C * Co; q++) {  // dW[c][o], one block reduction each
-    const int c = q / Co, o = q - c * Co;
-    red[threadIdx.x] = ok ? dY[(size_t)p * Co + o] * bf2f(X[(size_t)p * C + c]) : 0.f;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-      if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-      __syncthreads();
+  for (int e = t; e < C * Co; e += 256) Ws[e] = bf2f(Wb[e]);
+  float dy[CO];
+#pragma unroll
+  for (int o = 0; o < CO; o++) dy[o] = ok && o < Co ? dY[(size_t)p * Co + o] : 0.f;
+  float *out = part + (size_t)blockIdx.x * (C + 1) * Co;
+  // sums of rows q, q + 1, .. q + 3: in lanes 0, 32, 16, 48
+  auto trees = [&](int q) {
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      v[k] = (red[q + k][lane] + red[q + k][lane + 128]) + (red[q + k][lane + 64] + red[q + k][lane + 192]);
+    auto swap = [](float &x, float &y, auto f) {
+      const auto z = f(__float_as_uint(x), __float_as_uint(y));
+      x = __uint_as_float(z[0]), y = __uint_as_float(z[1]);
+    };
+    auto p32 = [](unsigned x, unsigned y) { return __builtin_amdgcn_permlane32_swap(x, y, false, false); };
+    auto p16 = [](unsigned x, unsigned y) { return __builtin_amdgcn_permlane16_swap(x, y, false, false); };
+    swap(v[0], v[1], p32);
+    swap(v[2], v[3], p32);
+    v[0] += v[1], v[2] += v[3];
+    swap(v[0], v[2], p16);
+    float t = v[0] + v[2];
+    t += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(t), 0x128, 0xf, 0xf, true));  // row_ror:8
+    t += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(t), 0x124, 0xf, 0xf, true));
+    t += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(t), 0x122, 0xf, 0xf, true));
+    t += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(t), 0x121, 0xf, 0xf, true));
+    return t;
+  };
+  const int mine = (lane >> 4 & 1) * 2 + (lane >> 5);  // the row of this lane's 16
+  for (int c0 = 0; c0 < C; c0 += 8) {
+    __syncthreads();  // Ws; the last channels' sums have been read
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (ok) load8f(X + (size_t)p * C + c0, x);
+    U16x8 d;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      float s = 0.f;
+#pragma unroll
+      for (int o = 0; o < CO; o++) {
+        red[k * CO + o][t] = dy[o] * x[k];
+        if (o < Co) s += dy[o] * Ws[(c0 + k) * Co + o];
+      }
+      d.v[k] = x[k] > 0.f ? f2bf(s) : (u16)0;
     }
-    if (threadIdx.x == 0) atomicAdd(&dW[q], red[0]);
+    if (ok) *reinterpret_cast<U16x8 *>(dX + (size_t)p * C + c0) = d;
     __syncthreads();
-  }
-  for (int o = 0; o < Co; o++) {
-    red[threadIdx.x] = ok ? dY[(size_t)p * Co + o] : 0.f;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-      if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-      __syncthreads();
+#pragma unroll
+    for (int q = 4 * wave; q < 8 * CO; q += 16) {
+      const float v = trees(q);
+      const int k = (q + mine) / CO, o = (q + mine) % CO;
+      if ((lane & 15) == 0 && o < Co) out[(size_t)(c0 + k) * Co + o] = v;
     }
-    if (threadIdx.x == 0) atomicAdd(&db[o], red[0]);
-    __syncthreads();
+  }
+  __syncthreads();
+#pragma unroll
+  for (int o = 0; o < CO; o++) red[o][t] = dy[o];
+  __syncthreads();
+  if (4 * wave < CO) {
+    const float v = trees(4 * wave);  // (rows past CO: not kept)
+    if ((lane & 15) == 0 && 4 * wave + mine < Co) out[(size_t)C * Co + 4 * wave + mine] = v;
   }
 }
 
 // Masked MSE: dY = (Y - T) * m / count; loss += sum((Y - T)^2 m) / (2 count)
 __global__ void __launch_bounds__(256) k_mse(const float *Y, const float *T, const uint8_t *M, int Co, int npix,
                                              float inv_count, float *dY, double *loss) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
   double s = 0.0;
-  if (p < npix) {
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < npix; p += gridDim.x * blockDim.x) {
     const float m = M[p] ? 1.f : 0.f;
     for (int o = 0; o < Co; o++) {
       const float e = (Y[(size_t)p * Co + o] - T[(size_t)p * Co + o]) * m;
@@ -492,23 +746,28 @@ __global__ void k_adam(float *P, const float *G, float *m, float *v, size_t n, f
 //   Wt[co][t*Cx + ci]       forward (zero for ci >= Cin and k >= taps*Cx)
 //   Wb[ci][t'*Co + co] = W[taps-1-t'][ci][co]   backward data (flipped taps)
 //   Wh[ci][co]              1x1 head
-__global__ void k_pack_fwd(const float *W, int taps, int Cin, int Cx, int Co, int Kp, u16 *Wt) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (size_t)Co * Kp) return;
-  const int co = (int)(e / Kp), k = (int)(e % Kp);
-  const int t = k / Cx, ci = k - t * Cx;
-  Wt[e] = (t < taps && ci < Cin) ? f2bf(W[((size_t)t * Cin + ci) * Co + co]) : (u16)0;
-}
-__global__ void k_pack_bwd(const float *W, int taps, int Cin, int Co, int Kpb, u16 *Wb) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (size_t)Cin * Kpb) return;
-  const int ci = (int)(e / Kpb), k = (int)(e % Kpb);
-  const int t = k / Co, co = k - t * Co;
-  Wb[e] = (t < taps) ? f2bf(W[((size_t)(taps - 1 - t) * Cin + ci) * Co + co]) : (u16)0;
-}
-__global__ void k_pack_head(const float *W, int n, u16 *Wh) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) Wh[e] = f2bf(W[e]);
+// All convolutions of the network in one launch: workgroup b works on the
+// convolution c with first[c] <= b < first[c + 1].
+__global__ void __launch_bounds__(256) k_pack(PackArgs a) {
+  int c = 0;
+  while (c + 1 < a.n && (int)blockIdx.x >= a.first[c + 1]) c++;
+  const PackConv &L = a.c[c];
+  const size_t e = (size_t)((int)blockIdx.x - a.first[c]) * 256 + threadIdx.x;
+  const float *W = a.P + L.w_off;
+  const size_t nf = (size_t)L.Cout * L.Kp;
+  if (e < nf) {  // forward layout (head: W as it is, Kp = Cin)
+    if (L.taps == 1) {
+      L.Wt[e] = f2bf(W[e]);
+      return;
+    }
+    const int co = (int)(e / L.Kp), k = (int)(e % L.Kp), t = k / L.Cx, ci = k - t * L.Cx;
+    L.Wt[e] = (t < L.taps && ci < L.Cin) ? f2bf(W[((size_t)t * L.Cin + ci) * L.Cout + co]) : (u16)0;
+    return;
+  }
+  const size_t q = e - nf;  // backward-data layout
+  if (!L.Wb || q >= (size_t)L.Cin * L.Kpb) return;
+  const int ci = (int)(q / L.Kpb), k = (int)(q % L.Kpb), t = k / L.Cout, co = k - t * L.Cout;
+  L.Wb[q] = (t < L.taps) ? f2bf(W[((size_t)(L.taps - 1 - t) * L.Cin + ci) * L.Cout + co]) : (u16)0;
 }
 
 // FP32 NHWC [n][C] -> BF16 with channel stride Cx (zero padding channels).
@@ -653,40 +912,52 @@ hipError_t unet_conv(const ConvArgs &a, hipStream_t s) {
     hipLaunchKernelGGL((k_conv<4, 2>), dim3(nblk(npix, 256), nblk(a.Cout, 32)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
-hipError_t unet_wgrad(const WgradArgs &a, hipStream_t s) {
-  const size_t npix = (size_t)a.N * a.H * a.W;
-  const int Kp = ((a.ks * a.ks * a.Cx + 31) / 32) * 32;
-  hipLaunchKernelGGL(k_wgrad, dim3(nblk(Kp, 64), nblk(a.Cout, 16), nblk(npix, a.chunk)), dim3(256), 0, s, a);
-  return hipGetLastError();
-}
-hipError_t unet_bgrad(const uint16_t *dZ, int npix, int Cout, float *db, hipStream_t s) {
-  const int chunk = 1024;
-  hipLaunchKernelGGL(k_bgrad, dim3(nblk(npix, chunk)), dim3(256), 0, s, dZ, npix, Cout, chunk, db);
+// Tiles of the weight gradient: the widest (64 x 64 channels; it reads least from
+// LDS per MFMA) that leaves a workgroup per CU, else 32 x 64, else 32 x 32 (16 x
+// 32 for a narrow input): a workgroup takes as long however few there are (64
+// workgroups of 64 x 64: 86 us per layer, 256 of 32 x 32: 27 us).
+constexpr long WGRAD_FULL = 256;
+
+hipError_t unet_wgrad(const WgradArgs &a, double *carry, float *dW, float *db, hipStream_t s) {
+  if (a.W % 8 || a.Cx % 8 || a.Cout % 8 || (a.X2 && a.Cb % 8)) return hipErrorInvalidValue;
+  const int npix = a.N * a.H * a.W, S = (int)nblk(npix, WG_RUN);
+  auto groups = [&](int CI, int CO) { return (long)nblk(a.Cx, CI) * nblk(a.Cout, CO) * S; };
+  const int CI = a.Cx <= 16 && !a.X2 ? 16 : a.Cx % 64 == 0 && a.Cout % 64 == 0 && groups(64, 64) >= WGRAD_FULL ? 64 : 32;
+  const int CO = CI == 64 || (CI == 32 && a.Cout % 64 == 0 && groups(32, 64) >= WGRAD_FULL) ? 64 : 32;
+  // as many slots at a time as the workspace holds
+  const size_t P = (size_t)9 * a.Cin * a.Cout;
+  const int most = (int)std::min<size_t>(std::max<size_t>(1, UNET_PART_FLOATS / P), 65535);
+  for (int q = 0; q < S; q += most) {
+    const int n = std::min(most, S - q), nsum = (int)nblk(P, 256);
+    const bool last = q + n == S;
+    const dim3 gr(nblk(a.Cx, CI) + 1, nblk(a.Cout, CO), n);  // + the bias
+    if (CI == 64 && a.X2) hipLaunchKernelGGL((k_wgrad<4, 1, 4, 2, true>), gr, dim3(512), 0, s, a, q);
+    else if (CI == 64) hipLaunchKernelGGL((k_wgrad<4, 1, 4, 2, false>), gr, dim3(512), 0, s, a, q);
+    else if (CO == 64 && a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 2, 2, true>), gr, dim3(512), 0, s, a, q);
+    else if (CO == 64) hipLaunchKernelGGL((k_wgrad<2, 2, 2, 2, false>), gr, dim3(512), 0, s, a, q);
+    else if (a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, true>), gr, dim3(512), 0, s, a, q);
+    else if (CI == 32) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, false>), gr, dim3(512), 0, s, a, q);
+    else hipLaunchKernelGGL((k_wgrad<1, 2, 1, 4, false>), gr, dim3(256), 0, s, a, q);
+    const SumArgs b{a.part, n, P, carry, q == 0, last, dW, nsum, a.bpart, (int)nblk(npix, WG_BIAS), a.Cout, db};
+    hipLaunchKernelGGL(k_sum_parts, dim3(nsum + (last ? nblk(a.Cout, SUM_RUNS) : 0)), dim3(64 * SUM_RUNS), 0, s, b);
+  }
   return hipGetLastError();
 }
 hipError_t unet_pool(const uint16_t *X, int N, int H, int W, int C, uint16_t *Y, hipStream_t s) {
-  hipLaunchKernelGGL(k_pool, dim3(nblk((size_t)N * (H / 2) * (W / 2) * C, 256)), dim3(256), 0, s, X, N, H, W, C, Y);
+  hipLaunchKernelGGL(k_pool, dim3(nblk((size_t)N * (H / 2) * (W / 2) * (C / 8), 256)), dim3(256), 0, s, X, N, H, W, C,
+                     Y);
   return hipGetLastError();
 }
-hipError_t unet_upcat(const uint16_t *B, int Cb, const uint16_t *S, int Cs, int N, int H, int W, uint16_t *O,
-                      hipStream_t s) {
-  hipLaunchKernelGGL(k_upcat, dim3(nblk((size_t)N * H * W * (Cb + Cs), 256)), dim3(256), 0, s, B, Cb, S, Cs, N, H, W,
-                     O);
+hipError_t unet_up_back(const uint16_t *D, int Cd, int Cu, const uint16_t *Act, int N, int H, int W, uint16_t *O,
+                        hipStream_t s) {
+  hipLaunchKernelGGL(k_up_back, dim3(nblk((size_t)N * (H / 2) * (W / 2) * (Cu / 8), 256)), dim3(256), 0, s, D, Cd, Cu,
+                     Act, N, H, W, O);
   return hipGetLastError();
 }
-hipError_t unet_relu_mask(const uint16_t *G, const uint16_t *Act, size_t n, uint16_t *dZ, hipStream_t s) {
-  hipLaunchKernelGGL(k_relu_mask, dim3(nblk(n, 256)), dim3(256), 0, s, G, Act, n, dZ);
-  return hipGetLastError();
-}
-hipError_t unet_up_back(const uint16_t *D, int Cd, int Cu, int N, int H, int W, uint16_t *O, hipStream_t s) {
-  hipLaunchKernelGGL(k_up_back, dim3(nblk((size_t)N * (H / 2) * (W / 2) * Cu, 256)), dim3(256), 0, s, D, Cd, Cu, N, H,
-                     W, O);
-  return hipGetLastError();
-}
-hipError_t unet_pool_back_add(const uint16_t *P, const uint16_t *Skip, int Cs, int off, int N, int H, int W, int C,
-                              uint16_t *O, hipStream_t s) {
-  hipLaunchKernelGGL(k_pool_back_add, dim3(nblk((size_t)N * H * W * C, 256)), dim3(256), 0, s, P, Skip, Cs, off, N, H,
-                     W, C, O);
+hipError_t unet_pool_back_add(const uint16_t *P, const uint16_t *Skip, int Cs, int off, const uint16_t *Act, int N,
+                              int H, int W, int C, uint16_t *O, hipStream_t s) {
+  hipLaunchKernelGGL(k_pool_back_add, dim3(nblk((size_t)N * H * W * (C / 8), 256)), dim3(256), 0, s, P, Skip, Cs, off,
+                     Act, N, H, W, C, O);
   return hipGetLastError();
 }
 hipError_t unet_head(const uint16_t *X, int C, const uint16_t *Wh, const float *b, int Co, int npix, float *Y,
@@ -696,13 +967,21 @@ hipError_t unet_head(const uint16_t *X, int C, const uint16_t *Wh, const float *
   return hipGetLastError();
 }
 hipError_t unet_head_back(const float *dY, const uint16_t *X, int C, const uint16_t *Wh, int Co, int npix,
-                          uint16_t *dX, float *dW, float *db, hipStream_t s) {
-  hipLaunchKernelGGL(k_head_back, dim3(nblk(npix, 256)), dim3(256), 0, s, dY, X, C, Wh, Co, npix, dX, dW, db);
+                          uint16_t *dX, float *part, float *grads, hipStream_t s) {
+  if (Co > HEAD_MAX_CO || C * Co > HEAD_MAX_W || C % 8) return hipErrorInvalidValue;
+  const int groups = (int)nblk(npix, 256);
+  if (Co <= 2) hipLaunchKernelGGL(k_head_back<2>, dim3(groups), dim3(256), 0, s, dY, X, C, Wh, Co, npix, dX, part);
+  else if (Co <= 4) hipLaunchKernelGGL(k_head_back<4>, dim3(groups), dim3(256), 0, s, dY, X, C, Wh, Co, npix, dX, part);
+  else hipLaunchKernelGGL(k_head_back<8>, dim3(groups), dim3(256), 0, s, dY, X, C, Wh, Co, npix, dX, part);
+  hipLaunchKernelGGL(k_sum_rows, dim3(nblk((size_t)(C + 1) * Co, 4)), dim3(256), 0, s, part, groups, (C + 1) * Co,
+                     grads);
   return hipGetLastError();
 }
 hipError_t unet_mse(const float *Y, const float *T, const uint8_t *M, int Co, int npix, float inv_count, float *dY,
                     double *loss, hipStream_t s) {
-  hipLaunchKernelGGL(k_mse, dim3(nblk(npix, 256)), dim3(256), 0, s, Y, T, M, Co, npix, inv_count, dY, loss);
+  // a workgroup per CU (one atomic each: with a thread per pixel the 2,048
+  // atomics on one word took 29 us at 8 x 512 x 128)
+  hipLaunchKernelGGL(k_mse, dim3(std::min(256u, nblk(npix, 256))), dim3(256), 0, s, Y, T, M, Co, npix, inv_count, dY, loss);
   return hipGetLastError();
 }
 hipError_t unet_adam(float *P, const float *G, float *m, float *v, size_t n, float lr, float b1, float b2, float eps,
@@ -710,16 +989,15 @@ hipError_t unet_adam(float *P, const float *G, float *m, float *v, size_t n, flo
   hipLaunchKernelGGL(k_adam, dim3(nblk(n, 256)), dim3(256), 0, s, P, G, m, v, n, lr, b1, b2, eps, c1, c2);
   return hipGetLastError();
 }
-hipError_t unet_pack_fwd(const float *W, int taps, int Cin, int Cx, int Co, int Kp, uint16_t *Wt, hipStream_t s) {
-  hipLaunchKernelGGL(k_pack_fwd, dim3(nblk((size_t)Co * Kp, 256)), dim3(256), 0, s, W, taps, Cin, Cx, Co, Kp, Wt);
-  return hipGetLastError();
-}
-hipError_t unet_pack_bwd(const float *W, int taps, int Cin, int Co, int Kpb, uint16_t *Wb, hipStream_t s) {
-  hipLaunchKernelGGL(k_pack_bwd, dim3(nblk((size_t)Cin * Kpb, 256)), dim3(256), 0, s, W, taps, Cin, Co, Kpb, Wb);
-  return hipGetLastError();
-}
-hipError_t unet_pack_head(const float *W, int n, uint16_t *Wh, hipStream_t s) {
-  hipLaunchKernelGGL(k_pack_head, dim3(nblk(n, 256)), dim3(256), 0, s, W, n, Wh);
+hipError_t unet_pack(PackArgs a, hipStream_t s) {
+  int blocks = 0;
+  for (int c = 0; c < a.n; c++) {
+    a.first[c] = blocks;
+    const PackConv &L = a.c[c];
+    blocks += (int)nblk((size_t)L.Cout * L.Kp + (L.Wb ? (size_t)L.Cin * L.Kpb : 0), 256);
+  }
+  a.first[a.n] = blocks;
+  hipLaunchKernelGGL(k_pack, dim3(blocks), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 hipError_t unet_to_bf16(const float *X, int C, int Cx, size_t npix, uint16_t *Y, hipStream_t s) {

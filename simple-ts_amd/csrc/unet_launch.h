@@ -21,41 +21,60 @@ struct ConvArgs {
   // Cx - Cb).  X2 == null: X is one tensor of stride Cx.
   const uint16_t *X2 = nullptr;
   int Cb = 0;
+  // Optional: Y is the gradient of a ReLU's output act (same layout), passed
+  // on through it: 0 where act is not positive.
+  const uint16_t *act = nullptr;
 };
 
-// Weight gradient dW[t][ci][co] += sum_p X[p+off(t)][ci] dZ[p][co].
+// Weight gradient dW[t][ci][co] = sum_p X[p+off(t)][ci] dZ[p][co] of a 3x3
+// convolution, and its bias gradient db[co] = sum_p dZ[p][co].
 struct WgradArgs {
-  const uint16_t *X;  // layer input [N][H][W][Cx]
+  const uint16_t *X;  // layer input [N][H][W][Cx] (X2, Cb: as in ConvArgs)
   int Cx, Cin;
   int N, H, W;  // W a multiple of 8
-  int ks;
-  const uint16_t *dZ;  // [N][H][W][Cout]
+  const uint16_t *dZ;  // [N][H][W][Cout], Cout a multiple of 8
   int Cout;
-  float *dW;  // [ks*ks][Cin][Cout]
-  int chunk;  // pixels per block (multiple of 32)
+  float *part, *bpart;  // workspaces: slots of the weights' sums, of the bias's (per 1024 pixels)
+  const void *zero;      // 16 bytes of zeros
+  const uint16_t *X2 = nullptr;
+  int Cb = 0;
 };
+// Workspace of the gradients' partial sums: the weight gradients use as many
+// slots at a time as fit UNET_PART_FLOATS (64 MB; one at least).
+constexpr size_t UNET_PART_FLOATS = (size_t)16 << 20;
 
 hipError_t unet_conv(const ConvArgs &a, hipStream_t s);
-hipError_t unet_wgrad(const WgradArgs &a, hipStream_t s);
-hipError_t unet_bgrad(const uint16_t *dZ, int npix, int Cout, float *db, hipStream_t s);
+// carry: 9 Cin Cout doubles.
+hipError_t unet_wgrad(const WgradArgs &a, double *carry, float *dW, float *db, hipStream_t s);
 hipError_t unet_pool(const uint16_t *X, int N, int H, int W, int C, uint16_t *Y, hipStream_t s);
-hipError_t unet_upcat(const uint16_t *B, int Cb, const uint16_t *S, int Cs, int N, int H, int W, uint16_t *O,
-                      hipStream_t s);
-hipError_t unet_relu_mask(const uint16_t *G, const uint16_t *Act, size_t n, uint16_t *dZ, hipStream_t s);
-hipError_t unet_up_back(const uint16_t *D, int Cd, int Cu, int N, int H, int W, uint16_t *O, hipStream_t s);
-hipError_t unet_pool_back_add(const uint16_t *P, const uint16_t *Skip, int Cs, int off, int N, int H, int W, int C,
-                              uint16_t *O, hipStream_t s);
+hipError_t unet_up_back(const uint16_t *D, int Cd, int Cu, const uint16_t *Act, int N, int H, int W, uint16_t *O,
+                        hipStream_t s);
+hipError_t unet_pool_back_add(const uint16_t *P, const uint16_t *Skip, int Cs, int off, const uint16_t *Act, int N,
+                              int H, int W, int C, uint16_t *O, hipStream_t s);
 hipError_t unet_head(const uint16_t *X, int C, const uint16_t *Wh, const float *b, int Co, int npix, float *Y,
                      hipStream_t s);
+// part: workspace of (C + 1) Co floats per 256 pixels; grads: the head's
+// weights' gradients, the bias's behind them.
 hipError_t unet_head_back(const float *dY, const uint16_t *X, int C, const uint16_t *Wh, int Co, int npix,
-                          uint16_t *dX, float *dW, float *db, hipStream_t s);
+                          uint16_t *dX, float *part, float *grads, hipStream_t s);
 hipError_t unet_mse(const float *Y, const float *T, const uint8_t *M, int Co, int npix, float inv_count, float *dY,
                     double *loss, hipStream_t s);
 hipError_t unet_adam(float *P, const float *G, float *m, float *v, size_t n, float lr, float b1, float b2, float eps,
                      float c1, float c2, hipStream_t s);
-hipError_t unet_pack_fwd(const float *W, int taps, int Cin, int Cx, int Co, int Kp, uint16_t *Wt, hipStream_t s);
-hipError_t unet_pack_bwd(const float *W, int taps, int Cin, int Co, int Kpb, uint16_t *Wb, hipStream_t s);
-hipError_t unet_pack_head(const float *W, int n, uint16_t *Wh, hipStream_t s);
+// BF16 weight layouts of every convolution from the FP32 parameters P.
+struct PackConv {
+  size_t w_off;
+  int taps, Cin, Cx, Cout, Kp, Kpb;  // taps 1: the head (Kp = Cin, as it is)
+  uint16_t *Wt, *Wb;                 // Wb null: no backward-data layout
+};
+constexpr int PACK_MAX = 16;
+struct PackArgs {
+  const float *P;
+  int n;
+  PackConv c[PACK_MAX];
+  int first[PACK_MAX + 1];  // set by unet_pack
+};
+hipError_t unet_pack(PackArgs a, hipStream_t s);
 hipError_t unet_to_bf16(const float *X, int C, int Cx, size_t npix, uint16_t *Y, hipStream_t s);
 hipError_t unet_pack_state(const double *u, const double *v, const double *p, const double *T, const uint8_t *m,
                            int npix, int Cx, double inv_u, double inv_p, uint16_t *X, hipStream_t s);
