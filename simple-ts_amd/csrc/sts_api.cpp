@@ -376,6 +376,23 @@ static std::vector<uint16_t> neighbour_bits(const std::vector<uint8_t> &mask, in
   return out;
 }
 
+// The mesh steps of one direction and behind them the reciprocals that the
+// assembly's quotients are formed from (TileMesh): of h[k], 3 h[k] and h[k - 1] +
+// h[k], the one before the first being the last when periodic, else the first
+// (and the one after the last the last).
+template <typename R>
+static std::vector<R> mesh_plan(const double *h, int N, bool periodic) {
+  std::vector<R> out(4 * (size_t)N + 1);
+  for (int k = 0; k < N; k++) out[k] = (R)h[k];
+  for (int k = 0; k < N; k++) {
+    out[N + k] = R(1) / out[k];
+    out[2 * N + k] = R(1) / (out[k] * R(3));
+    out[3 * N + k] = R(1) / (out[k > 0 ? k - 1 : (periodic ? N - 1 : 0)] + out[k]);
+  }
+  out[4 * N] = R(1) / (out[N - 1] + out[N - 1]);
+  return out;
+}
+
 static int alloc_state(sts_ctx *c, const sts_grid *gi, const std::vector<uint8_t> &mask) {
   const size_t Na = (size_t)c->Na;
   const size_t bytes = Na * sizeof(double);
@@ -386,8 +403,10 @@ static int alloc_state(sts_ctx *c, const sts_grid *gi, const std::vector<uint8_t
   }
   HIP_OK(hipMalloc(&c->p_alt, bytes));
   HIP_OK(hipMalloc(&c->T_alt, bytes));
-  HIP_OK(hipMalloc(&c->hx, sizeof(double) * gi->Nx));
-  HIP_OK(hipMalloc(&c->hy, sizeof(double) * gi->Ny));
+  const std::vector<double> hx = mesh_plan<double>(gi->hx, gi->Nx, gi->periodic_x != 0),
+                            hy = mesh_plan<double>(gi->hy, gi->Ny, false);
+  HIP_OK(hipMalloc(&c->hx, sizeof(double) * hx.size()));
+  HIP_OK(hipMalloc(&c->hy, sizeof(double) * hy.size()));
   HIP_OK(hipMalloc(&c->m, Na));
   HIP_OK(hipMalloc(&c->vol, sizeof(uint32_t) * Na));
   const size_t nb = (size_t)(gi->nbodies > 0 ? gi->nbodies : 1);
@@ -401,8 +420,8 @@ static int alloc_state(sts_ctx *c, const sts_grid *gi, const std::vector<uint8_t
   HIP_OK(hipHostMalloc(&c->h_red, sizeof(unsigned long long) * (NRED + 1), hipHostMallocDefault));
   HIP_OK(hipHostMalloc(&c->h_ctrl, sizeof(LoopCtrl), hipHostMallocDefault));
   HIP_OK(hipEventCreateWithFlags(&c->ev_ctrl, hipEventDisableTiming));
-  HIP_OK(hipMemcpyAsync(c->hx, gi->hx, sizeof(double) * gi->Nx, hipMemcpyHostToDevice, c->stream));
-  HIP_OK(hipMemcpyAsync(c->hy, gi->hy, sizeof(double) * gi->Ny, hipMemcpyHostToDevice, c->stream));
+  HIP_OK(hipMemcpyAsync(c->hx, hx.data(), sizeof(double) * hx.size(), hipMemcpyHostToDevice, c->stream));
+  HIP_OK(hipMemcpyAsync(c->hy, hy.data(), sizeof(double) * hy.size(), hipMemcpyHostToDevice, c->stream));
   HIP_OK(hipMemcpyAsync(c->m, mask.data(), Na, hipMemcpyHostToDevice, c->stream));
   const std::vector<uint16_t> nbits = neighbour_bits(mask, gi->Nx, gi->Ny, gi->periodic_x != 0);
   HIP_OK(hipMalloc(&c->nb, sizeof(uint16_t) * Na));
@@ -432,7 +451,6 @@ static void narrow_grid(sts_ctx *c) {
   h.cT1 = (float)g.cT1; h.cT2 = (float)g.cT2; h.cPch = (float)g.cPch; h.c_Fr_v = (float)g.c_Fr_v;
   h.rht = 1.0f / h.ht;  // IEEE single division on the host: RN(1/ht) in FP32
   h.c1 = 1.0f - h.gamma1;  // single subtraction in FP32, as the kernels formed it
-  h.rht_one = std::fabs(std::fma(-h.rht, h.ht, 1.0f)) <= 0x1p-25f;
   h.given_xb = g.given_xb; h.given_xe = g.given_xe; h.kn_local = g.kn_local;
   h.bc = g.bc;
   h.px = g.px;
@@ -446,11 +464,12 @@ static int alloc_fp32(sts_ctx *c, const sts_grid *gi) {
   }
   HIP_OK(hipMalloc(&c->p_alt32, bytes));
   HIP_OK(hipMalloc(&c->T_alt32, bytes));
-  HIP_OK(hipMalloc(&c->hx32, sizeof(float) * gi->Nx));
-  HIP_OK(hipMalloc(&c->hy32, sizeof(float) * gi->Ny));
-  std::vector<float> hx(gi->hx, gi->hx + gi->Nx), hy(gi->hy, gi->hy + gi->Ny);
-  HIP_OK(hipMemcpyAsync(c->hx32, hx.data(), sizeof(float) * gi->Nx, hipMemcpyHostToDevice, c->stream));
-  HIP_OK(hipMemcpyAsync(c->hy32, hy.data(), sizeof(float) * gi->Ny, hipMemcpyHostToDevice, c->stream));
+  const std::vector<float> hx = mesh_plan<float>(gi->hx, gi->Nx, gi->periodic_x != 0),
+                           hy = mesh_plan<float>(gi->hy, gi->Ny, false);
+  HIP_OK(hipMalloc(&c->hx32, sizeof(float) * hx.size()));
+  HIP_OK(hipMalloc(&c->hy32, sizeof(float) * hy.size()));
+  HIP_OK(hipMemcpyAsync(c->hx32, hx.data(), sizeof(float) * hx.size(), hipMemcpyHostToDevice, c->stream));
+  HIP_OK(hipMemcpyAsync(c->hy32, hy.data(), sizeof(float) * hy.size(), hipMemcpyHostToDevice, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   narrow_grid(c);
   return STS_OK;
@@ -576,8 +595,7 @@ extern "C" int sts_create(const sts_grid *gi, int precision, sts_ctx **out) {
   g.Nx_v0 = gi->Nx_v[0]; g.Nx_v1 = gi->Nx_v[1]; g.Ny_v0 = gi->Ny_v[0]; g.Ny_v1 = gi->Ny_v[1];
   g.Nx_o0 = gi->Nx_o[0]; g.Nx_o1 = gi->Nx_o[1]; g.Ny_o0 = gi->Ny_o[0]; g.Ny_o1 = gi->Ny_o[1];
   g.ht = gi->ht;
-  g.rht = 1.0 / g.ht;  // RN(1/ht); 1 - rht ht is exact in an fma
-  g.rht_one = std::fabs(std::fma(-g.rht, g.ht, 1.0)) <= 0x1p-54;
+  g.rht = 1.0 / g.ht;  // RN(1/ht)
   g.gamma1 = gi->gamma1;
   g.c1 = 1.0 - g.gamma1;
   g.Kn = gi->Kn;

@@ -40,7 +40,7 @@ enum : unsigned {
 template <typename R>
 struct KGridT {
   int Nx, Ny;
-  const R *hx, *hy;
+  const R *hx, *hy;       // mesh steps, and behind them the reciprocals of TileMesh
   const uint8_t *m;       // vol_inf_fb_bool
   const uint16_t *nb;     // neighbour fluid bits (NB_*)
   const uint32_t *vol;    // vol_inf_fb
@@ -50,7 +50,6 @@ struct KGridT {
   R ht, gamma1, Kn, cT, cT1, cT2, cPch, c_Fr_v;
   R rht;      // 1/ht rounded to nearest in R
   R c1;       // 1 - gamma1 in R, formed on the host (a uniform kernel argument, no vector register)
-  int rht_one;  // |1 - rht ht| <= 2^-(p+1): a rht is within an ulp of a/ht for every a (quot1)
   int given_xb, given_xe, kn_local;
   unsigned bc;
   int px;  // periodic about OX: x neighbours wrap, box-edge conditions off

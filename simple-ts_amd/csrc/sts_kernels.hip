@@ -41,17 +41,32 @@ __device__ __forceinline__ bool in_box(int i, int j, int x0, int x1, int y0, int
   return i >= x0 && i < x1 && j >= y0 && j < y1;
 }
 
+__device__ __forceinline__ double div_fixup(double q, double b, double a) {
+  return __builtin_amdgcn_div_fixup(q, b, a);
+}
+__device__ __forceinline__ float div_fixup(float q, float b, float a) { return __builtin_amdgcn_div_fixupf(q, b, a); }
+
 // a / b, correctly rounded, from y = RN(1/b) when RN(a y) is within one ulp
 // of a/b -- Markstein's theorem: then r = a - b q is exact in an fma and
 // RN(q + r y) = RN(a/b), barring underflow and overflow.  RN(a y) is that
 // close for every a when |1 - b y| <= 2^-(p+1) (half the unit roundoff).
-// r = 0 (an exact quotient, a = +-0) or NaN (a infinite or NaN) keeps q, so
-// signed zeros and non-finite quotients are those of a / b.
+// The fixup gives zeros, infinities and NaN as a / b does.
+template <typename R>
+__device__ __forceinline__ R quot1_from(R q, R a, R b, R y) {
+  return div_fixup(fma(fma(-q, b, a), y, q), b, a);
+}
 template <typename R>
 __device__ __forceinline__ R quot1(R a, R b, R y) {
+  return quot1_from(a * y, a, b, y);
+}
+
+// The same for any b: RN(a y) is within 1.5 ulp of a/b, one correction brings
+// it within one.  6 instructions at the full rate; a division takes 10 and a
+// reciprocal at a quarter of it.
+template <typename R>
+__device__ __forceinline__ R quot2(R a, R b, R y) {
   const R q = a * y;
-  const R r = fma(-q, b, a);
-  return (fabs(r) > R(0)) ? fma(r, y, q) : q;
+  return quot1_from(fma(fma(-q, b, a), y, q), a, b, y);
 }
 
 // a / 3: RN(1/3) = (1/3)(1 - 2^-(p+1)) meets quot1's condition.
@@ -326,18 +341,44 @@ struct GlobalStencil {
   __device__ __forceinline__ R hx(int di) const { return hx_[di < 0 ? n.i_1 : (di > 0 ? n.i1 : n.i)]; }
   __device__ __forceinline__ R hy(int dj) const { return hy_[dj < 0 ? n.j - (0u < n.j) : n.j]; }  // dj = -1, 0
   __device__ __forceinline__ R div_ht(R a, const KGridT<R> &g) const { return a / g.ht; }
+  // a over hx, 3 hx of column di; over hy, 3 hy of row dj
+  __device__ __forceinline__ R over_hx(R a, int di) const { return a / hx(di); }
+  __device__ __forceinline__ R over_hy(R a, int dj) const { return a / hy(dj); }
+  __device__ __forceinline__ R over_hx3(R a, int di) const { return a / (hx(di) * R(3.0)); }
+  __device__ __forceinline__ R over_hy3(R a, int dj) const { return a / (hy(dj) * R(3.0)); }
+};
+
+// The mesh steps of a tile's columns (or rows) with their one-cell ring, and
+// the correctly rounded reciprocals of the divisors made of them alone, for
+// quot2: entry e is of column e; rs: of hx(e - 1) + hx(e), e > 0.  They lie
+// behind the mesh steps in memory: N steps, their reciprocals, those of three
+// times them, and N + 1 of a step and the one before it (the last: of two
+// last steps, beside a clamped neighbour).
+template <typename R, int N>
+struct TileMesh {
+  R h[N], r1[N], r3[N], rs[N];
+  __device__ __forceinline__ void load(int e, const R *mesh, int n, int k, int ks) {
+    h[e] = mesh[k];
+    r1[e] = mesh[n + k];
+    r3[e] = mesh[2 * n + k];
+    rs[e] = mesh[3 * n + ks];
+  }
+  __device__ __forceinline__ R over(R a, int e) const { return quot2(a, h[e], r1[e]); }
+  __device__ __forceinline__ R over3(R a, int e) const { return quot2(a, h[e] * R(3.0), r3[e]); }
+  __device__ __forceinline__ R over_sum(R a, int e) const { return quot2(a, h[e - 1] + h[e], rs[e]); }
 };
 
 // LDS tile [TY + 2][TX + 2] of each field: entry [y][x] holds the field at
 // cell (i0 + x - 1, j0 + y - 1) with the coordinates clamped (x wrapped when
 // periodic) as Nbr clamps a neighbour, so that the neighbour (di, dj) of the
-// tile's cell (tx, ty) is entry [ty + 1 + dj][tx + 1 + di].  HT1: the grid's
-// 1/ht meets quot1's condition (rht_one), quotients by ht are formed from it.
-template <typename R, int TX, int TY, bool HT1>
+// tile's cell (tx, ty) is entry [ty + 1 + dj][tx + 1 + di] (Fx, rho and rho_pr,
+// which no cell reads to the north, have no row TY + 1).
+template <typename R, int TX, int TY>
 struct TileStencil {
   const R (*Fx_)[TX + 2], (*Fy_)[TX + 2], (*u_)[TX + 2], (*v_)[TX + 2], (*sT_)[TX + 2], (*rho_)[TX + 2],
       (*rho_pr_)[TX + 2];
-  const R *hx_, *hy_;  // [TX + 2], [TY + 2]: the tile's columns and rows with their one-cell ring
+  const TileMesh<R, TX + 2> &X;
+  const TileMesh<R, TY + 2> &Y;
   int tx, ty;
   __device__ __forceinline__ R Fx(int di, int dj) const { return Fx_[ty + 1 + dj][tx + 1 + di]; }
   __device__ __forceinline__ R Fy(int di, int dj) const { return Fy_[ty + 1 + dj][tx + 1 + di]; }
@@ -346,24 +387,27 @@ struct TileStencil {
   __device__ __forceinline__ R sT(int di, int dj) const { return sT_[ty + 1 + dj][tx + 1 + di]; }
   __device__ __forceinline__ R rho(int di, int dj) const { return rho_[ty + 1 + dj][tx + 1 + di]; }
   __device__ __forceinline__ R rho_pr(int di, int dj) const { return rho_pr_[ty + 1 + dj][tx + 1 + di]; }
-  __device__ __forceinline__ R hx(int di) const { return hx_[tx + 1 + di]; }
-  __device__ __forceinline__ R hy(int dj) const { return hy_[ty + 1 + dj]; }
-  __device__ __forceinline__ R div_ht(R a, const KGridT<R> &g) const {
-    if constexpr (HT1) return quot1(a, g.ht, g.rht);
-    else return a / g.ht;
-  }
+  __device__ __forceinline__ R hx(int di) const { return X.h[tx + 1 + di]; }
+  __device__ __forceinline__ R hy(int dj) const { return Y.h[ty + 1 + dj]; }
+  __device__ __forceinline__ R over_hx(R a, int di) const { return X.over(a, tx + 1 + di); }
+  __device__ __forceinline__ R over_hy(R a, int dj) const { return Y.over(a, ty + 1 + dj); }
+  __device__ __forceinline__ R over_hx3(R a, int di) const { return X.over3(a, tx + 1 + di); }
+  __device__ __forceinline__ R over_hy3(R a, int dj) const { return Y.over3(a, ty + 1 + dj); }
+  // a over hx(di - 1) + hx(di), hy(dj - 1) + hy(dj)
+  __device__ __forceinline__ R over_sx(R a, int di) const { return X.over_sum(a, tx + 1 + di); }
+  __device__ __forceinline__ R over_sy(R a, int dj) const { return Y.over_sum(a, ty + 1 + dj); }
+  __device__ __forceinline__ R div_ht(R a, const KGridT<R> &g) const { return quot2(a, g.ht, g.rht); }
 };
 
 template <typename R, typename St>
 __device__ __forceinline__ void cell_assemble_u(const KGridT<R> &g, const KFieldsT<R> &fl, const Nbr &n,
-                                                const CellDiff<R> &df, unsigned nb, const St &S) {
-  const R *u_pr = FLD(U_PR), *rho_u = FLD(RHO_U);
+                                                const CellDiff<R> &df, unsigned nb, const St &S, R u_pr, R rho_u) {
   const unsigned ij = n.ij;
   const R cT = g.cT;
   R F_xu1 = R(0.5) * (S.Fx(-1, 0) + S.Fx(0, 0));
   R F_xu2 = R(0.5) * (S.Fx(0, 0) + S.Fx(1, 0));
-  R Scu = cT * (R((nb & NB_E) != 0) * S.u(1, 0) * S.sT(0, 0) * S.hy(0) / (S.hx(0) * R(3.0))
-                     + R((nb & NB_WW) != 0) * S.u(-1, 0) * S.sT(-1, 0) * S.hy(0) / (S.hx(-1) * R(3.0))
+  R Scu = cT * (S.over_hx3(R((nb & NB_E) != 0) * S.u(1, 0) * S.sT(0, 0) * S.hy(0), 0)
+                     + S.over_hx3(R((nb & NB_WW) != 0) * S.u(-1, 0) * S.sT(-1, 0) * S.hy(0), -1)
                      + df.Gy1 * (S.v(0, 1) * R((nb & NB_N) != 0) - S.v(-1, 1) * R((nb & NB_NW) != 0))
                      - df.Gy0 * (S.v(0, 0) * R((nb & NB_S) != 0) - S.v(-1, 0) * R((nb & NB_SW) != 0))
                      - third(S.sT(0, 0) * (S.v(0, 1) * R((nb & NB_N) != 0) - S.v(0, 0) * R((nb & NB_S) != 0)) * R(2.0))
@@ -373,12 +417,12 @@ __device__ __forceinline__ void cell_assemble_u(const KGridT<R> &g, const KField
   R au2 = maxi0(-F_xu2) + df.Dux1;
   R au3 = R(0.5) * (maxi0(S.Fy(-1, 0)) + maxi0(S.Fy(0, 0))) + df.Duy0;
   R au4 = R(0.5) * (maxi0(-S.Fy(-1, 1)) + maxi0(-S.Fy(0, 1))) + df.Duy1;
-  R bu3 = S.div_ht((S.rho_pr(-1, 0) * S.hx(-1) + S.rho_pr(0, 0) * S.hx(0)) * u_pr[ij] * S.hy(0) * R(0.5), g) + Scu;
+  R bu3 = S.div_ht((S.rho_pr(-1, 0) * S.hx(-1) + S.rho_pr(0, 0) * S.hx(0)) * u_pr * S.hy(0) * R(0.5), g) + Scu;
   R au0 = au1 + au2 + au3 + au4 + R(0.5) * (-S.Fy(-1, 0) - S.Fy(0, 0) + S.Fy(-1, 1) + S.Fy(0, 1)) + F_xu2 - F_xu1 - Spu
                + S.div_ht((S.rho(-1, 0) * S.hx(-1) + S.rho(0, 0) * S.hx(0)) * S.hy(0) * R(0.5), g);
   R ups = (au1 * R((nb & NB_E) != 0) * S.u(-1, 0) + au2 * R((nb & NB_WW) != 0) * S.u(1, 0) + au3 * S.u(0, -1) + au4 * S.u(0, 1) + bu3) / au0;
   R dpc = g.cPch * S.hy(0) / au0;
-  R h = S.hy(0) * rho_u[ij];
+  R h = S.hy(0) * rho_u;
   FLD(U_PSEUDO)[ij] = ups;
   FLD(D_P_C_12)[ij] = dpc;
   FLD(APX)[ij] = dpc * h;
@@ -387,8 +431,7 @@ __device__ __forceinline__ void cell_assemble_u(const KGridT<R> &g, const KField
 
 template <typename R, typename St>
 __device__ __forceinline__ void cell_assemble_v(const KGridT<R> &g, const KFieldsT<R> &fl, const Nbr &n,
-                                                const CellDiff<R> &df, unsigned nb, const St &S) {
-  const R *v_pr = FLD(V_PR), *rho_v = FLD(RHO_V);
+                                                const CellDiff<R> &df, unsigned nb, const St &S, R v_pr, R rho_v) {
   const unsigned ij = n.ij;
   const R cT = g.cT;
   // S:3399 the mask at ij_1 - Nx*(0 <= (int)(j-2)) (NB_SS); S:3399, S:3404 hy[j - 1*(0 <= (int)(j-1))],
@@ -396,8 +439,8 @@ __device__ __forceinline__ void cell_assemble_v(const KGridT<R> &g, const KField
   const R hyjm = S.hy(-1);
   R F_yv3 = R(0.5) * (S.Fy(0, -1) + S.Fy(0, 0));
   R F_yv4 = R(0.5) * (S.Fy(0, 0) + S.Fy(0, 1));
-  R Scv = cT * (R((nb & NB_N) != 0) * S.v(0, 1) * S.sT(0, 0) * S.hx(0) / (S.hy(0) * R(3.0))
-                     + R((nb & NB_SS) != 0) * S.v(0, -1) * S.sT(0, -1) * S.hx(0) / (hyjm * R(3.0))
+  R Scv = cT * (S.over_hy3(R((nb & NB_N) != 0) * S.v(0, 1) * S.sT(0, 0) * S.hx(0), 0)
+                     + S.over_hy3(R((nb & NB_SS) != 0) * S.v(0, -1) * S.sT(0, -1) * S.hx(0), -1)
                      + df.Gx1 * (S.u(1, 0) * R((nb & NB_E) != 0) - S.u(1, -1) * R((nb & NB_SE) != 0))
                      - df.Gx0 * (S.u(0, 0) * R((nb & NB_W) != 0) - S.u(0, -1) * R((nb & NB_SW) != 0))
                      - third(S.sT(0, 0) * (S.u(1, 0) * R((nb & NB_E) != 0) - S.u(0, 0) * R((nb & NB_W) != 0)) * R(2.0))
@@ -408,43 +451,55 @@ __device__ __forceinline__ void cell_assemble_v(const KGridT<R> &g, const KField
   R av2 = R(0.5) * (maxi0(-S.Fx(1, 0)) + maxi0(-S.Fx(1, -1))) + df.Dvx1;
   R av3 = maxi0(F_yv3) + df.Dvy0;
   R av4 = maxi0(-F_yv4) + df.Dvy1;
-  R bv3 = S.div_ht((S.rho_pr(0, -1) * S.hy(-1) + S.rho_pr(0, 0) * S.hy(0)) * v_pr[ij] * S.hx(0) * R(0.5), g) + Scv;
+  R bv3 = S.div_ht((S.rho_pr(0, -1) * S.hy(-1) + S.rho_pr(0, 0) * S.hy(0)) * v_pr * S.hx(0) * R(0.5), g) + Scv;
   R av0 = av1 + av2 + av3 + av4 + R(0.5) * (S.Fx(1, 0) - S.Fx(0, 0) + S.Fx(1, -1) - S.Fx(0, -1)) + F_yv4 - F_yv3 - Spv
                + S.div_ht((S.rho(0, -1) * S.hy(-1) + S.rho(0, 0) * S.hy(0)) * S.hx(0) * R(0.5), g);
   R vps = (av1 * S.v(-1, 0) + av2 * S.v(1, 0) + av3 * R((nb & NB_SS) != 0) * S.v(0, -1) + av4 * R((nb & NB_N) != 0) * S.v(0, 1) + bv3) / av0;
   R dpc = g.cPch * S.hx(0) / av0;
-  R h = S.hx(0) * rho_v[ij];
+  R h = S.hx(0) * rho_v;
   FLD(V_PSEUDO)[ij] = vps;
   FLD(D_P_C_34)[ij] = dpc;
   FLD(APY)[ij] = dpc * h;
   FLD(BPY)[ij] = R((nb & NB_S) != 0 && (nb & NB_C) != 0) * h * vps;
 }
 
-template <typename R, typename St>
+// S:3729-3740: the upper neighbour row is guarded by j < Nx-1; the lower is
+// clamped.
+template <typename R>
+__device__ __forceinline__ unsigned energy_row_above(const KGridT<R> &g, unsigned j) {
+  return j + 1 * (j < (unsigned)g.Nx - 1);
+}
+
+// FLUID: nb has every bit (as a constant) and the row above is S's.
+template <bool FLUID = false, typename R, typename St>
 __device__ __forceinline__ void cell_energy_source(const KGridT<R> &g, const KFieldsT<R> &fl, const Nbr &n,
-                                                   unsigned nb, const St &S) {
-  const unsigned Nx = (unsigned)g.Nx;
-  const R *p_pr = FLD(P_PR);
+                                                   unsigned nb, const St &S, R p_pr) {
   const unsigned j = n.j, ij = n.ij;
-  // S:3729-3740: the upper neighbour row is guarded by j < Nx-1 (from global
-  // memory: that row may lie past the grid's last one); the lower is clamped
-  const unsigned jp = j + 1 * (j < (Nx - 1));
-  const R hyp = g.hy[jp];
-  R dudx_T = (R(((nb & NB_E) != 0)) * S.u(1, 0) - R(((nb & NB_W) != 0)) * S.u(0, 0)) / S.hx(0);
-  R dvdy_T = (R(((nb & NB_N) != 0)) * S.v(0, 1) - R(((nb & NB_S) != 0)) * S.v(0, 0)) / S.hy(0);
-  R s0 = ((S.u(0, 0) - S.u(0, -1)) / (R(((nb & NB_SW) != 0) && ((nb & NB_S) != 0)) * S.hy(-1) + S.hy(0)))
+  R dudx_T = S.over_hx(R(((nb & NB_E) != 0)) * S.u(1, 0) - R(((nb & NB_W) != 0)) * S.u(0, 0), 0);
+  R dvdy_T = S.over_hy(R(((nb & NB_N) != 0)) * S.v(0, 1) - R(((nb & NB_S) != 0)) * S.v(0, 0), 0);
+  R s0, s1, s2, s3;
+  if constexpr (FLUID) {
+    s0 = S.over_sy(S.u(0, 0) - S.u(0, -1), 0) + S.over_sx(S.v(0, 0) - S.v(-1, 0), 0);
+    s1 = S.over_sy(S.u(1, 0) - S.u(1, -1), 0) + S.over_sx(S.v(1, 0) - S.v(0, 0), 1);
+    s2 = S.over_sy(S.u(0, 1) - S.u(0, 0), 1) + S.over_sx(S.v(0, 1) - S.v(-1, 1), 0);
+    s3 = S.over_sy(S.u(1, 1) - S.u(1, 0), 1) + S.over_sx(S.v(1, 1) - S.v(0, 1), 1);
+  } else {
+    // from global memory: the row above may lie past the grid's last one
+    const R hyp = g.hy[energy_row_above(g, j)];
+    s0 = ((S.u(0, 0) - S.u(0, -1)) / (R(((nb & NB_SW) != 0) && ((nb & NB_S) != 0)) * S.hy(-1) + S.hy(0)))
               + ((S.v(0, 0) - S.v(-1, 0)) / (R(((nb & NB_SW) != 0) && ((nb & NB_W) != 0)) * S.hx(-1) + S.hx(0)));
-  R s1 = ((S.u(1, 0) - S.u(1, -1)) / (R(((nb & NB_S) != 0) && ((nb & NB_SE) != 0)) * S.hy(-1) + S.hy(0)))
+    s1 = ((S.u(1, 0) - S.u(1, -1)) / (R(((nb & NB_S) != 0) && ((nb & NB_SE) != 0)) * S.hy(-1) + S.hy(0)))
               + ((S.v(1, 0) - S.v(0, 0)) / (S.hx(0) + R(((nb & NB_SE) != 0) && ((nb & NB_E) != 0)) * S.hx(1)));
-  R s2 = ((S.u(0, 1) - S.u(0, 0)) / (S.hy(0) + R(((nb & NB_NW) != 0) && ((nb & NB_N) != 0)) * hyp))
+    s2 = ((S.u(0, 1) - S.u(0, 0)) / (S.hy(0) + R(((nb & NB_NW) != 0) && ((nb & NB_N) != 0)) * hyp))
               + ((S.v(0, 1) - S.v(-1, 1)) / (R(((nb & NB_W) != 0) && ((nb & NB_NW) != 0)) * S.hx(-1) + S.hx(0)));
-  R s3 = ((S.u(1, 1) - S.u(1, 0)) / (S.hy(0) + R(((nb & NB_N) != 0) && ((nb & NB_NE) != 0)) * hyp))
+    s3 = ((S.u(1, 1) - S.u(1, 0)) / (S.hy(0) + R(((nb & NB_N) != 0) && ((nb & NB_NE) != 0)) * hyp))
               + ((S.v(1, 1) - S.v(0, 1)) / (S.hx(0) + R(((nb & NB_E) != 0) && ((nb & NB_NE) != 0)) * S.hx(1)));
+  }
   R dsum = dudx_T + dvdy_T;
   FLD(SCT1)[ij] = g.ht * S.sT(0, 0) * g.cT2 * S.hx(0) * S.hy(0)
                       * (R(2.0) * (dudx_T * dudx_T + dvdy_T * dvdy_T) + s0 * s0 + s1 * s1 + s2 * s2 + s3 * s3
                          - third(dsum * dsum * R(2.0)))
-                  + p_pr[ij] * S.hx(0) * S.hy(0);
+                  + p_pr * S.hx(0) * S.hy(0);
 }
 
 // The assembly of cell (i, j) with Gamma and D read from their arrays (stage
@@ -463,11 +518,11 @@ __device__ __forceinline__ void assemble_cell(const KGridT<R> &g, const KFieldsT
     const CellDiff<R> df{Gyf[n.ij], Gyf[n.ij1], Gxf[n.ij], Gxf[n.i1j], Dux[n.ij], Dux[n.i1j],
                          Duy[n.ij], Duy[n.ij1], Dvx[n.ij], Dvx[n.i1j], Dvy[n.ij], Dvy[n.ij1]};
     const GlobalStencil<R> S(g, fl, n);
-    if (du) cell_assemble_u(g, fl, n, df, nb, S);
-    if (dv) cell_assemble_v(g, fl, n, df, nb, S);
+    if (du) cell_assemble_u(g, fl, n, df, nb, S, FLD(U_PR)[n.ij], FLD(RHO_U)[n.ij]);
+    if (dv) cell_assemble_v(g, fl, n, df, nb, S, FLD(V_PR)[n.ij], FLD(RHO_V)[n.ij]);
   }
   if (in_box(i, j, g.Nx_o0, g.Nx_o1, g.Ny_o0, g.Ny_o1) && c)
-    cell_energy_source(g, fl, n, nb, GlobalStencil<R>(g, fl, n));
+    cell_energy_source(g, fl, n, nb, GlobalStencil<R>(g, fl, n), FLD(P_PR)[n.ij]);
 }
 
 template <typename R>
@@ -490,20 +545,37 @@ struct FaceDiff {
 // as face_diff forms them, with sqrt_T and the mesh steps taken from a
 // workgroup's LDS tile: (cx, cy) is the face cell's position in the tile
 // (entry [cy + 1][cx + 1] of sT holds its sqrt_T, [cy][cx] that of its
-// clamped or wrapped south-west neighbour; Shx[cx + 1], Shx[cx] its hx and
-// the west one, Shy likewise in y), b its neighbour fluid bits.  The wall
+// clamped or wrapped south-west neighbour; X.h[cx + 1], X.h[cx] its hx and
+// the west one, Y likewise), b its neighbour fluid bits.  The wall
 // temperatures are read only where some but not all of the four cells are
 // fluid, the one case gamma() uses them.
-template <typename R, int TX>
+// FLUID: all four cells are, for which every divisor is the mesh's alone.
+constexpr unsigned NB_FACE = NB_SW | NB_S | NB_W | NB_C;
+constexpr unsigned NB_ALL = NB_FACE | NB_E | NB_WW | NB_N | NB_SE | NB_NW | NB_NE | NB_SS;
+
+template <bool FLUID, typename R, int TX, int TY>
 __device__ __forceinline__ FaceDiff<R> face_diff_tile(const KGridT<R> &g, const KFieldsT<R> &fl, unsigned fi,
-                                                      unsigned fj, unsigned b, const R (*sT)[TX + 2], const R *Shx,
-                                                      const R *Shy, int cx, int cy) {
+                                                      unsigned fj, unsigned b, const R (*sT)[TX + 2],
+                                                      const TileMesh<R, TX + 2> &X, const TileMesh<R, TY + 2> &Y,
+                                                      int cx, int cy) {
+  FaceDiff<R> d;
+  if constexpr (FLUID) {
+    const R s00 = sT[cy][cx], s10 = sT[cy][cx + 1], s01 = sT[cy + 1][cx], s11 = sT[cy + 1][cx + 1];
+    const R hxi = X.h[cx + 1], hxw = X.h[cx], hyj = Y.h[cy + 1], hys = Y.h[cy];
+    d.Gy = R(0.5) * (Y.over_sum(s00 * hyj + s01 * hys, cy + 1) + Y.over_sum(s10 * hyj + s11 * hys, cy + 1));
+    d.Gx = R(0.5) * (X.over_sum(s00 * hxi + s10 * hxw, cx + 1) + X.over_sum(s01 * hxi + s11 * hxw, cx + 1));
+    d.Dux = g.cT * s01 * X.over(hyj, cx);
+    d.Duy = g.cT * d.Gy * Y.over_sum(hxi + hxw, cy + 1);
+    d.Dvx = g.cT * d.Gx * X.over_sum(hyj + hys, cx + 1);
+    d.Dvy = g.cT * s10 * Y.over(hxi, cy);
+    return d;
+  }
   FluxIn<R> f;
   f.in = true;
-  f.hxi = Shx[cx + 1];
-  f.hxw = Shx[cx];
-  f.hyj = Shy[cy + 1];
-  f.hys = Shy[cy];
+  f.hxi = X.h[cx + 1];
+  f.hxw = X.h[cx];
+  f.hyj = Y.h[cy + 1];
+  f.hys = Y.h[cy];
   f.m00 = (b & NB_SW) != 0;
   f.m10 = (b & NB_S) != 0;
   f.m01 = (b & NB_W) != 0;
@@ -520,7 +592,6 @@ __device__ __forceinline__ FaceDiff<R> face_diff_tile(const KGridT<R> &g, const 
     f.twv01 = FLD(TW_V)[n.i_1j];
     f.twv11 = FLD(TW_V)[n.ij];
   }
-  FaceDiff<R> d;
   f.gamma(d.Gy, d.Gx);
   d.Dux = f.d_ux(g);
   d.Duy = f.d_uy(g, d.Gy);
@@ -539,20 +610,28 @@ __device__ __forceinline__ FaceDiff<R> face_diff_tile(const KGridT<R> &g, const 
 // own face and the east one: when a tile row lies within one wave (64 % TX
 // == 0) the east cell's come from the next lane and only the ring column's
 // from LDS (a quarter less LDS per workgroup, so more workgroups per CU);
-// otherwise they are all kept in LDS.  (tx, ty): the thread's cell in the
-// tile; the workgroup has TX * TY >= TX + TY + 4 threads, the linear thread
-// index tx + TX ty.
-template <typename R, int TX, int TY, bool HT1 = false>
-__device__ __forceinline__ void assemble_inl_tile(const KGridT<R> &g, const KFieldsT<R> &fl, int i0, int j0, int tx,
-                                                  int ty) {
+// otherwise they are all kept in LDS.  t: the linear thread index of TX * TY
+// >= TX + TY + 4, cell (t % TX, t / TX).
+//
+// SPLIT: three threads per cell (TX TY multiple of 64: three sets of waves),
+// one of which assembles u, one v and one the energy source; the second and
+// third form the ring's faces while the first forms the cells' own.  What a
+// thread reads of its cell alone is loaded with the tile.
+template <typename R, int TX, int TY, bool SPLIT = false>
+__device__ __forceinline__ void assemble_inl_tile(const KGridT<R> &g, const KFieldsT<R> &fl, int i0, int j0, int t) {
   static_assert(TX * TY >= TX + TY + 4, "the face ring and the mesh steps need TX + TY + 4 threads");
-  constexpr bool XL = 64 % TX == 0;      // x-face values of the east cell by lane exchange
+  static_assert(!SPLIT || TX * TY % 64 == 0, "whole waves");
+  constexpr int CELLS = TX * TY, THREADS = SPLIT ? 3 * CELLS : CELLS;
+  constexpr bool XL = !SPLIT && 64 % TX == 0;  // x-face values of the east cell by lane exchange
   constexpr int LXW = XL ? 1 : TX + 1;  // x-face arrays: the ring column only, or every face
   constexpr int LXR = XL ? 0 : TX;      // their ring column
   __shared__ R Lgy[TY + 1][TX], Luy[TY + 1][TX], Lvy[TY + 1][TX], Lgx[TY][LXW], Lux[TY][LXW], Lvx[TY][LXW];
-  __shared__ R SFx[TY + 2][TX + 2], SFy[TY + 2][TX + 2], Su[TY + 2][TX + 2], Sv[TY + 2][TX + 2],
-      SsT[TY + 2][TX + 2], Srho[TY + 2][TX + 2], Srho_pr[TY + 2][TX + 2], Shx[TX + 2], Shy[TY + 2];
-  const int Nx = g.Nx, Ny = g.Ny, t = tx + ty * TX;
+  __shared__ R SFx[TY + 1][TX + 2], SFy[TY + 2][TX + 2], Su[TY + 2][TX + 2], Sv[TY + 2][TX + 2],
+      SsT[TY + 2][TX + 2], Srho[TY + 1][TX + 2], Srho_pr[TY + 1][TX + 2];
+  __shared__ TileMesh<R, TX + 2> X;
+  __shared__ TileMesh<R, TY + 2> Y;
+  const int role = SPLIT ? t / CELLS : 0, tx = t % CELLS % TX, ty = t % CELLS / TX;
+  const int Nx = g.Nx, Ny = g.Ny;
   // column x - 1 and row y - 1 of the tile, clamped (x wrapped when periodic)
   // as Nbr takes a neighbour; x - 1 >= -1, and x - 1 < Nx + TX
   auto col = [&](int x) {
@@ -568,28 +647,57 @@ __device__ __forceinline__ void assemble_inl_tile(const KGridT<R> &g, const KFie
   // the tile's neighbourhood of the fields the cells and faces read
   // (TileStencil, face_diff_tile); the entries past the grid's last tile
   // column are never read, only kept in it
-  for (int e = t; e < (TX + 2) * (TY + 2); e += TX * TY) {
+  for (int e = t; e < (TX + 2) * (TY + 2); e += THREADS) {
     const int x = e % (TX + 2), y = e / (TX + 2);
     const unsigned k = (unsigned)col(x) + (unsigned)row(y) * (unsigned)Nx;
-    SFx[y][x] = FLD(FX)[k];
     SFy[y][x] = FLD(FY)[k];
     Su[y][x] = FLD(U)[k];
     Sv[y][x] = FLD(V)[k];
     SsT[y][x] = FLD(SQRT_T)[k];
-    Srho[y][x] = FLD(RHO)[k];
-    Srho_pr[y][x] = FLD(RHO_PR)[k];
+    if (y <= TY) {
+      SFx[y][x] = FLD(FX)[k];
+      Srho[y][x] = FLD(RHO)[k];
+      Srho_pr[y][x] = FLD(RHO_PR)[k];
+    }
   }
-  if (t < TX + 2) Shx[t] = g.hx[col(t)];
-  else if (t < TX + TY + 4) Shy[t - (TX + 2)] = g.hy[row(t - (TX + 2))];
+  if (t < TX + 2) {
+    X.load(t, g.hx, Nx, col(t), g.px ? col(t) : min(max(i0 + t - 1, 0), Nx));
+  } else if (t < TX + TY + 4) {
+    const int y = t - (TX + 2);
+    Y.load(y, g.hy, Ny, row(y), min(max(j0 + y - 1, 0), Ny));
+  }
   const int i = i0 + tx, j = j0 + ty;
   const int il = min(i0 + TX, Nx) - 1, jl = min(j0 + TY, Ny) - 1;  // last cell of the tile in x, y
   const bool in = i < Nx && j < Ny;
   const unsigned ij = (unsigned)i + (unsigned)j * (unsigned)Nx, nb = in ? g.nb[ij] : 0u;
+  // The ring's face of this thread: north, of column rt's last cell (jl itself on
+  // the grid's top row), or east, of row rt - TX's last cell (Nbr's i1 of il).
+  const int rt = SPLIT ? t - CELLS : t;
+  const bool north = rt >= 0 && rt < TX && i0 + rt < Nx;
+  const bool east = rt >= TX && rt < TX + TY && j0 + rt - TX < Ny;
+  const int ri = north ? i0 + rt : g.px ? (il == Nx - 1 ? 0 : il + 1) : il + (il < Nx - 1 ? 1 : 0);
+  const int rj = north ? jl + (jl < Ny - 1 ? 1 : 0) : j0 + rt - TX;
+  unsigned rb = 0;
+  R own0 = R(0), own1 = R(0);
+  if constexpr (SPLIT) {
+    if (north || east) rb = g.nb[(unsigned)ri + (unsigned)rj * (unsigned)Nx];
+    if (in) {
+      own0 = (role == 0 ? FLD(U_PR) : role == 1 ? FLD(V_PR) : FLD(P_PR))[ij];
+      if (role < 2) own1 = (role == 0 ? FLD(RHO_U) : FLD(RHO_V))[ij];
+    }
+  }
   __syncthreads();
+  // the face of cell (fi, fj), at (cx, cy) of the tile; waves without a wall
+  // take the fluid form
+  auto face = [&](int fi, int fj, unsigned b, int cx, int cy) {
+    if (__all((b & NB_FACE) == NB_FACE))
+      return face_diff_tile<true, R, TX, TY>(g, fl, (unsigned)fi, (unsigned)fj, b, SsT, X, Y, cx, cy);
+    return face_diff_tile<false, R, TX, TY>(g, fl, (unsigned)fi, (unsigned)fj, b, SsT, X, Y, cx, cy);
+  };
   // the cell's own face
   R gx = R(0), ux = R(0), vx = R(0);
-  if (in) {
-    const FaceDiff<R> d = face_diff_tile<R, TX>(g, fl, (unsigned)i, (unsigned)j, nb, SsT, Shx, Shy, tx, ty);
+  if (in && role == 0) {
+    const FaceDiff<R> d = face(i, j, nb, tx, ty);
     Lgy[ty][tx] = d.Gy;
     Luy[ty][tx] = d.Duy;
     Lvy[ty][tx] = d.Dvy;
@@ -602,67 +710,96 @@ __device__ __forceinline__ void assemble_inl_tile(const KGridT<R> &g, const KFie
       Lvx[ty][tx] = vx;
     }
   }
-  if (t < TX) {  // north: the ij1 face of column t's last cell (jl itself on the grid's top row); its y-face values
-    const int fj = jl + (jl < Ny - 1 ? 1 : 0);
-    if (i0 + t < Nx) {
-      const FaceDiff<R> d = face_diff_tile<R, TX>(g, fl, (unsigned)(i0 + t), (unsigned)fj,
-                                                  g.nb[(unsigned)(i0 + t) + (unsigned)fj * (unsigned)Nx], SsT, Shx,
-                                                  Shy, t, fj - j0);
-      Lgy[TY][t] = d.Gy;
-      Luy[TY][t] = d.Duy;
-      Lvy[TY][t] = d.Dvy;
-    }
-  } else if (t < TX + TY) {  // east: the i1j face of row t - TX's last cell (Nbr's i1 of il); its x-face values
-    const int r = t - TX;
-    const int fi = g.px ? (il == Nx - 1 ? 0 : il + 1) : il + (il < Nx - 1 ? 1 : 0);
-    if (j0 + r < Ny) {
-      const FaceDiff<R> d = face_diff_tile<R, TX>(g, fl, (unsigned)fi, (unsigned)(j0 + r),
-                                                  g.nb[(unsigned)fi + (unsigned)(j0 + r) * (unsigned)Nx], SsT, Shx,
-                                                  Shy, il - i0 + (fi != il ? 1 : 0), r);
-      Lgx[r][LXR] = d.Gx;
-      Lux[r][LXR] = d.Dux;
-      Lvx[r][LXR] = d.Dvx;
-    }
+  if constexpr (!SPLIT) {
+    if (north || east) rb = g.nb[(unsigned)ri + (unsigned)rj * (unsigned)Nx];
   }
+  if (north) {  // its y-face values
+    const FaceDiff<R> d = face(ri, rj, rb, rt, rj - j0);
+    Lgy[TY][rt] = d.Gy;
+    Luy[TY][rt] = d.Duy;
+    Lvy[TY][rt] = d.Dvy;
+  } else if (east) {  // its x-face values
+    const FaceDiff<R> d = face(ri, rj, rb, il - i0 + (ri != il ? 1 : 0), rt - TX);
+    Lgx[rt - TX][LXR] = d.Gx;
+    Lux[rt - TX][LXR] = d.Dux;
+    Lvx[rt - TX][LXR] = d.Dvx;
+  }
+  __syncthreads();
   // the next lane's own x-face values (lanes of one wave, every lane active)
   R egx = R(0), eux = R(0), evx = R(0);
   if constexpr (XL) {
-    egx = __shfl_down(gx, 1);
-    eux = __shfl_down(ux, 1);
-    evx = __shfl_down(vx, 1);
+    egx = lane_east(gx);
+    eux = lane_east(ux);
+    evx = lane_east(vx);
   }
-  __syncthreads();
   if (!in) return;
   const Nbr n((unsigned)i, (unsigned)j, (unsigned)Nx, (unsigned)Ny, g.px);
   const bool c = (nb & NB_C) != 0;
   const bool du = in_box(i, j, g.Nx_u0, g.Nx_u1, g.Ny_u0, g.Ny_u1) && (nb & NB_W) && c;
   const bool dv = in_box(i, j, g.Nx_v0, g.Nx_v1, g.Ny_v0, g.Ny_v1) && (nb & NB_S) && c;
-  const TileStencil<R, TX, TY, HT1> S{SFx, SFy, Su, Sv, SsT, Srho, Srho_pr, Shx, Shy, tx, ty};
-  if (du || dv) {
-    const int ny = (j == jl) ? TY : ty + 1;
-    const bool last = i == il;  // the east face is the ring column's
-    const R gx1 = last ? Lgx[ty][LXR] : XL ? egx : Lgx[ty][tx + 1];
-    const R ux1 = last ? Lux[ty][LXR] : XL ? eux : Lux[ty][tx + 1];
-    const R vx1 = last ? Lvx[ty][LXR] : XL ? evx : Lvx[ty][tx + 1];
-    const CellDiff<R> df{Lgy[ty][tx], Lgy[ny][tx], gx, gx1, ux, ux1,
-                         Luy[ty][tx], Luy[ny][tx], vx, vx1, Lvy[ty][tx], Lvy[ny][tx]};
-    if (du) cell_assemble_u(g, fl, n, df, nb, S);
-    if (dv) cell_assemble_v(g, fl, n, df, nb, S);
-  }
-  if (in_box(i, j, g.Nx_o0, g.Nx_o1, g.Ny_o0, g.Ny_o1) && c) cell_energy_source(g, fl, n, nb, S);
+  const TileStencil<R, TX, TY> S{SFx, SFy, Su, Sv, SsT, Srho, Srho_pr, X, Y, tx, ty};
+  // (of the lanes left) every cell the assembly looks at is fluid, and the
+  // energy source's row above the clamped one
+  const bool fluid = __all((nb & NB_ALL) == NB_ALL && energy_row_above(g, (unsigned)j) == (unsigned)min(j + 1, Ny - 1));
+  const int ny = (j == jl) ? TY : ty + 1;
+  const bool last = i == il;  // the east face is the ring column's
+  auto diff = [&]() {
+    const R gx0 = SPLIT ? Lgx[ty][XL ? 0 : tx] : gx, gx1 = last ? Lgx[ty][LXR] : XL ? egx : Lgx[ty][XL ? 0 : tx + 1];
+    const R ux0 = SPLIT ? Lux[ty][XL ? 0 : tx] : ux, ux1 = last ? Lux[ty][LXR] : XL ? eux : Lux[ty][XL ? 0 : tx + 1];
+    const R vx0 = SPLIT ? Lvx[ty][XL ? 0 : tx] : vx, vx1 = last ? Lvx[ty][LXR] : XL ? evx : Lvx[ty][XL ? 0 : tx + 1];
+    return CellDiff<R>{Lgy[ty][tx], Lgy[ny][tx], gx0, gx1, ux0, ux1,
+                       Luy[ty][tx], Luy[ny][tx], vx0, vx1, Lvy[ty][tx], Lvy[ny][tx]};
+  };
+  const bool en = in_box(i, j, g.Nx_o0, g.Nx_o1, g.Ny_o0, g.Ny_o1) && c;
+  auto cell = [&](auto fluid, unsigned bits) {
+    if (role == 0 && du) {
+      if constexpr (SPLIT) cell_assemble_u(g, fl, n, diff(), bits, S, own0, own1);
+      else cell_assemble_u(g, fl, n, diff(), bits, S, FLD(U_PR)[ij], FLD(RHO_U)[ij]);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (one equation's values in registers at a time)
+    if (role == (SPLIT ? 1 : 0) && dv) {
+      if constexpr (SPLIT) cell_assemble_v(g, fl, n, diff(), bits, S, own0, own1);
+      else cell_assemble_v(g, fl, n, diff(), bits, S, FLD(V_PR)[ij], FLD(RHO_V)[ij]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (role == (SPLIT ? 2 : 0) && en)
+      cell_energy_source<decltype(fluid)::value>(g, fl, n, bits, S, SPLIT ? own0 : FLD(P_PR)[ij]);
+  };
+  if (fluid) cell(std::true_type(), NB_ALL);
+  else cell(std::false_type(), nb);
 }
 
-// Tile of the loops' assembly: 64 x 8 cells at six waves per SIMD (78
-// registers; 51.6 KB of LDS, three workgroups per CU).
+// Tile of the loops' assembly: 64 x 8 cells at six waves per SIMD (80
+// registers; 51.8 KB of LDS, three workgroups per CU).  Its 172 bytes per cell
+// and its FP64 instructions take about as long (1920 x 384: 19 us at the rate
+// of a copy that fits the last-level cache, 12 us at four cycles per wave
+// instruction); what counts is that both overlap.  Waves without a wall in
+// reach take the form without masks, and every quotient whose divisor is the
+// mesh's is formed from a reciprocal (quot2): 33.2 -> 29.4 us at 1920 x 384, 19.7
+// -> 17.3 at 1280 x 256; 3840 x 768: 122 us, 4.2 TB/s.  Tiles of 64 x 4: 29.8 and
+// 16.4 us, 130 at 3840 x 768; 64 x 6: 34.0.
 constexpr int AX = 64, AY = 8;
 
-// HT1: launched for grids with rht_one.
-template <typename R, bool HT1>
+template <typename R>
 __global__ void __launch_bounds__(AX *AY) __attribute__((amdgpu_waves_per_eu(6, 8))) k_assemble_inl(KGridT<R> g, KFieldsT<R> fl, Gate gate) {
   if (gated_out(gate)) return;
   int i0, j0;
   tile_origin<AX, AY>(g.Nx, i0, j0);
-  assemble_inl_tile<R, AX, AY, HT1>(g, fl, i0, j0, (int)threadIdx.x, (int)threadIdx.y);
+  assemble_inl_tile<R, AX, AY>(g, fl, i0, j0, (int)threadIdx.x);
+}
+
+// Where the tiles of 64 x 2, or else 64 x 4, give at most a workgroup per CU, the
+// time is one cell's chain of instructions (10 us whatever the size): three
+// threads per cell.  240 x 48: 9.9 -> 6.7 us (64 x 4: 7.8), 301 x 95: 10.2 -> 7.0,
+// 512 x 128: 10.6 -> 7.7 (64 x 2, two workgroups per CU: 9.0); beyond, 777 x 211:
+// 13.4 us, but 14.3 and 16.5 with three threads.
+constexpr unsigned ASSEMBLE_SPLIT = 256;
+template <typename R, int TY>
+__global__ void __launch_bounds__(3 * AX *TY) k_assemble_split(KGridT<R> g, KFieldsT<R> fl, Gate gate) {
+  if (gated_out(gate)) return;
+  int i0, j0;
+  tile_origin<AX, TY>(g.Nx, i0, j0);
+  assemble_inl_tile<R, AX, TY, true>(g, fl, i0, j0, (int)threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2418,8 +2555,7 @@ __global__ void __launch_bounds__(TX *TY) kb_assemble(const BatchCase<R> *C, con
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
   if (gated_out(Gate{in_memory(c.ctrl), k}) || (k == 0 && !c.inline0)) return;
-  assemble_inl_tile<R, TX, TY>(grid_of(c), fields_at(c, par), t.x * TX, t.y * TY, (int)threadIdx.x % TX,
-                               (int)threadIdx.x / TX);
+  assemble_inl_tile<R, TX, TY>(grid_of(c), fields_at(c, par), t.x * TX, t.y * TY, (int)threadIdx.x);
 }
 
 template <typename R, int TX, int TY>
@@ -2624,10 +2760,12 @@ static inline dim3 grid_tiles(const KGridT<R> &g) {
 
 template <typename R>
 hipError_t launch_assemble(const KGridT<R> &g, const KFieldsT<R> &f, hipStream_t s, Gate gate, bool inline_diff) {
-  if (inline_diff && g.rht_one)
-    hipLaunchKernelGGL((k_assemble_inl<R, true>), (grid_tiles<AX, AY>(g)), dim3(AX, AY), 0, s, g, f, gate);
+  if (inline_diff && grid_tiles<AX, 2>(g).x <= ASSEMBLE_SPLIT)
+    hipLaunchKernelGGL((k_assemble_split<R, 2>), (grid_tiles<AX, 2>(g)), dim3(3 * AX * 2), 0, s, g, f, gate);
+  else if (inline_diff && grid_tiles<AX, 4>(g).x <= ASSEMBLE_SPLIT)
+    hipLaunchKernelGGL((k_assemble_split<R, 4>), (grid_tiles<AX, 4>(g)), dim3(3 * AX * 4), 0, s, g, f, gate);
   else if (inline_diff)
-    hipLaunchKernelGGL((k_assemble_inl<R, false>), (grid_tiles<AX, AY>(g)), dim3(AX, AY), 0, s, g, f, gate);
+    hipLaunchKernelGGL(k_assemble_inl<R>, (grid_tiles<AX, AY>(g)), dim3(AX * AY), 0, s, g, f, gate);
   else hipLaunchKernelGGL(k_assemble<R>, (grid_tiles<BX, BY>(g)), dim3(BX, BY), 0, s, g, f, gate);
   return hipGetLastError();
 }
