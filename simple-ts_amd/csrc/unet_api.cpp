@@ -57,8 +57,7 @@ struct sts_unet {
   u16 *x = nullptr, *act[NCONV] = {}, *pl[3] = {};
   u16 *gA = nullptr, *gB = nullptr, *gP = nullptr, *dc[3] = {};
   float *part = nullptr, *bpart = nullptr;  // partial sums of the parameter gradients
-  double *carry = nullptr;                  // and their running sums, where one part does not hold them all;
-  size_t carry_n = 0;                       // behind those, 2 zeros
+  u16 *zero = nullptr;                      // 16 bytes of zeros
   double *loss = nullptr;
   int *slots_dev = nullptr;
   // training set
@@ -87,7 +86,7 @@ void free_all(sts_unet *u) {
   }
   for (void *p : {(void *)u->P, (void *)u->G, (void *)u->Mo, (void *)u->Vo, (void *)u->xin, (void *)u->y,
                   (void *)u->dy, (void *)u->tg, (void *)u->mask, (void *)u->x, (void *)u->part,
-                  (void *)u->bpart, (void *)u->carry, (void *)u->gA,
+                  (void *)u->bpart, (void *)u->zero, (void *)u->gA,
                   (void *)u->gB, (void *)u->gP, (void *)u->loss, (void *)u->slots_dev, (void *)u->ds_x,
                   (void *)u->ds_t, (void *)u->ds_m})
     (void)hipFree(p);
@@ -115,7 +114,7 @@ int pack_weights(sts_unet *u) {
 
 int conv_fwd(sts_unet *u, int k, const u16 *X, int n, u16 *Y, const u16 *skip = nullptr, int Cb = 0) {
   const Conv &c = u->L[k];
-  ConvArgs a{X, c.Cx, n, u->h(c.level), u->w(c.level), 3, c.Wt, c.Kp, u->P + c.b_off, c.Cout, Y, 1, skip, Cb};
+  ConvArgs a{X, c.Cx, n, u->h(c.level), u->w(c.level), 3, c.Wt, c.Kp, u->P + c.b_off, c.Cout, Y, 1, u->zero, skip, Cb};
   U_OK(unet_conv(a, u->stream));
   return STS_OK;
 }
@@ -128,10 +127,10 @@ int conv_back(sts_unet *u, int k, const u16 *X, int n, const u16 *dz, u16 *dX, c
               const u16 *skip = nullptr, int Cb = 0) {
   const Conv &c = u->L[k];
   const int Hh = u->h(c.level), Ww = u->w(c.level);
-  U_OK(unet_wgrad(WgradArgs{X, c.Cx, c.Cin, n, Hh, Ww, dz, c.Cout, u->part, u->bpart, u->carry + u->carry_n, skip, Cb}, u->carry, u->G + c.w_off,
+  U_OK(unet_wgrad(WgradArgs{X, c.Cx, c.Cin, n, Hh, Ww, dz, c.Cout, u->part, u->bpart, u->zero, skip, Cb}, u->G + c.w_off,
                   u->G + c.b_off, u->stream));
   if (dX) {
-    ConvArgs a{dz, c.Cout, n, Hh, Ww, 3, c.Wb, c.Kpb, nullptr, c.Cx, dX, 0, nullptr, 0, act};
+    ConvArgs a{dz, c.Cout, n, Hh, Ww, 3, c.Wb, c.Kpb, nullptr, c.Cx, dX, 0, u->zero, nullptr, 0, act};
     U_OK(unet_conv(a, u->stream));
   }
   return STS_OK;
@@ -305,12 +304,11 @@ extern "C" int sts_unet_create(int cin, int cout, int base, int max_n, int H, in
     const size_t np = u->npix(max_n, c.level), P = (size_t)9 * c.Cin * c.Cout;
     part = std::max(part, std::max(P, std::min(UNET_PART_FLOATS, (np + 2047) / 2048 * P)));
     bpart = std::max(bpart, (np + 1023) / 1024 * (size_t)c.Cout);
-    u->carry_n = std::max(u->carry_n, (P + 1) / 2 * 2);
   }
   A_OK(hipMalloc(&u->part, sizeof(float) * part));
   A_OK(hipMalloc(&u->bpart, sizeof(float) * bpart));
-  A_OK(hipMalloc(&u->carry, sizeof(double) * (u->carry_n + 2)));
-  A_OK(hipMemsetAsync(u->carry + u->carry_n, 0, 2 * sizeof(double), u->stream));
+  A_OK(hipMalloc(&u->zero, 16));
+  A_OK(hipMemsetAsync(u->zero, 0, 16, u->stream));
   A_OK(hipMalloc(&u->gA, sizeof(u16) * big));
   A_OK(hipMalloc(&u->gB, sizeof(u16) * big));
   A_OK(hipMalloc(&u->gP, sizeof(u16) * big));

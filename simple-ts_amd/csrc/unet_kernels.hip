@@ -28,6 +28,10 @@ struct alignas(16) U16x8 {
   u16 v[8];
 };
 
+struct alignas(8) U16x4 {
+  u16 v[4];
+};
+
 __device__ __forceinline__ u16 f2bf(float f) {  // round to nearest even
   unsigned b = __float_as_uint(f);
   b += 0x7FFFu + ((b >> 16) & 1u);
@@ -41,13 +45,31 @@ __device__ __forceinline__ bf16x8 load8(const u16 *p) {
 }
 __device__ __forceinline__ bf16x8 zero8() { return __builtin_bit_cast(bf16x8, U16x8{}); }
 
+// Outputs of a convolution, channels co .. co + 3 (of a multiple of 4) of the
+// pixel at offset `at` of Y: bias, ReLU, the given ReLU's mask, rounding.
+__device__ __forceinline__ void conv_out(const ConvArgs &a, size_t at, int co, const floatx4 &acc) {
+  floatx4 bias = {0.f, 0.f, 0.f, 0.f};
+  if (a.bias) bias = *reinterpret_cast<const floatx4 *>(a.bias + co);
+  U16x4 act, out;
+  if (a.act) act = *reinterpret_cast<const U16x4 *>(a.act + at);
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    float v = acc[q] + bias[q];
+    if (a.relu) v = fmaxf(v, 0.f);
+    out.v[q] = a.act && !(bf2f(act.v[q]) > 0.f) ? (u16)0 : f2bf(v);
+  }
+  *reinterpret_cast<U16x4 *>(a.Y + at) = out;
+}
+
 // ---------------------------------------------------------------------------
-// Convolution (forward, and backward-data with flipped weights)
-// Block: 4 waves stacked along the pixels; a wave computes TM x TN tiles of
-// 16 pixels x 16 channels: pixels [p0, p0 + 16 TM) x channels
+// Convolution (forward, and backward-data with flipped weights) of any channel
+// stride.  Block: 4 waves stacked along the pixels; a wave computes TM x TN
+// tiles of 16 pixels x 16 channels: pixels [p0, p0 + 16 TM) x channels
 // [c0, c0 + 16 TN), p0 = (4 blockIdx.x + w) * 16 TM, c0 = 16 TN blockIdx.y.
 // Per 32-wide k chunk a lane loads TM + TN 16-byte fragments for TM * TN
-// MFMAs; every output sums its k chunks in the same order for any TM, TN.
+// MFMAs, those of the next chunk while they run (a fragment outside the image
+// from a.zero: no branch around a load); every output sums its k chunks in the
+// same order for any TM, TN.  D rows = channels: a lane stores 4 of a pixel.
 // ---------------------------------------------------------------------------
 template <int TM, int TN>
 __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
@@ -74,67 +96,75 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
   for (int x = 0; x < TM; x++)
 #pragma unroll
     for (int y = 0; y < TN; y++) acc[x][y] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int kc = 0; kc < a.Kp; kc += 32) {
+  const u16 *zero = (const u16 *)a.zero;
+  auto fetch = [&](int kc, bf16x8 (&A)[TM], bf16x8 (&B)[TN]) {
     const int k = kc + 8 * g;
     const int t = k / a.Cx, ci = k - t * a.Cx;
     const int dy = t / a.ks - rad, dx = t % a.ks - rad;
-    bf16x8 A[TM], B[TN];
+    // the tensor of channel ci: full size, or (u = 1) the half-size one
+    const int u = a.X2 && ci < a.Cb ? 1 : 0, Cs = !a.X2 ? a.Cx : u ? a.Cb : a.Cx - a.Cb;
+    const u16 *X = (a.X2 && !u ? a.X2 - a.Cb : a.X) + ci;
 #pragma unroll
     for (int s = 0; s < TM; s++) {
-      A[s] = zero8();
-      if (t < taps && pv[s]) {
-        const int jj = pj[s] + dy, ii = pi[s] + dx;
-        if (jj >= 0 && jj < a.H && ii >= 0 && ii < a.W) {
-          if (!a.X2)
-            A[s] = load8(a.X + ((size_t)(pn[s] * a.H + jj) * a.W + ii) * a.Cx + ci);
-          else if (ci < a.Cb)  // nearest-upsampled half-size tensor (channels [0, Cb))
-            A[s] = load8(a.X + ((size_t)(pn[s] * (a.H / 2) + jj / 2) * (a.W / 2) + ii / 2) * a.Cb + ci);
-          else  // skip tensor (channels [Cb, Cx))
-            A[s] = load8(a.X2 + ((size_t)(pn[s] * a.H + jj) * a.W + ii) * (a.Cx - a.Cb) + (ci - a.Cb));
-        }
-      }
+      const int jj = pj[s] + dy, ii = pi[s] + dx;
+      const u16 *at = X + ((size_t)(pn[s] * (a.H >> u) + (jj >> u)) * (a.W >> u) + (ii >> u)) * Cs;
+      A[s] = load8(t < taps && pv[s] && jj >= 0 && jj < a.H && ii >= 0 && ii < a.W ? at : zero);
     }
 #pragma unroll
     for (int s = 0; s < TN; s++) {
       const int co = c0 + 16 * s + r;
-      B[s] = (co < a.Cout) ? load8(a.Wt + (size_t)co * a.Kp + k) : zero8();
+      const u16 *at = a.Wt + (size_t)co * a.Kp + k;
+      B[s] = load8(co < a.Cout && kc < a.Kp ? at : zero);
     }
+  };
+  auto mul = [&](const bf16x8 (&A)[TM], const bf16x8 (&B)[TN]) {
 #pragma unroll
     for (int x = 0; x < TM; x++)
 #pragma unroll
-      for (int y = 0; y < TN; y++) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[x], B[y], acc[x][y], 0, 0, 0);
+      for (int y = 0; y < TN; y++) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[y], A[x], acc[x][y], 0, 0, 0);
+  };
+  bf16x8 A0[TM], B0[TN], A1[TM], B1[TN];
+  fetch(0, A0, B0);
+  for (int kc = 0; kc < a.Kp; kc += 64) {  // (beyond the end: zeros)
+    fetch(kc + 32, A1, B1);
+    mul(A0, B0);
+    fetch(kc + 64, A0, B0);
+    if (kc + 32 < a.Kp) mul(A1, B1);
   }
 #pragma unroll
   for (int y = 0; y < TN; y++) {
-    const int co = c0 + 16 * y + r;
+    const int co = c0 + 16 * y + 4 * g;
     if (co >= a.Cout) continue;
-    const float bias = a.bias ? a.bias[co] : 0.f;
 #pragma unroll
-    for (int x = 0; x < TM; x++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int p = p0 + 16 * x + 4 * g + q;
-        if (p >= npix) continue;
-        float v = acc[x][y][q] + bias;
-        if (a.relu) v = fmaxf(v, 0.f);
-        const size_t o = (size_t)p * a.Cout + co;
-        a.Y[o] = (a.act && !(bf2f(a.act[o]) > 0.f)) ? (u16)0 : f2bf(v);
-      }
+    for (int x = 0; x < TM; x++) {
+      const int p = p0 + 16 * x + r;
+      if (p < npix) conv_out(a, (size_t)p * a.Cout + co, co, acc[x][y]);
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
 // 3x3 convolution with its operands staged in LDS (input channel strides
-// that are multiples of 32).  A block computes a 4 RW x CONV_PW pixel tile
-// of one image (wave w: rows RW w .. RW w + RW - 1 of the tile, 4 sub-tiles
-// of 16 pixels each) for 16 TN output channels.  Per chunk of 32 input channels it stages the
-// input tile with a one-pixel halo (zeros outside the image) and the chunk's
-// weights of all 9 taps in LDS once; every wave then takes its A and B
-// fragments of the 9 taps from there, so an input value is read from memory
-// once per chunk instead of once per tap and the weights once per block
-// instead of once per wave.  Sums run over chunks, then taps.
+// that are multiples of 32).  Four waves, WP along the rows x WC along the
+// channels, compute a tile of R WP rows x 16 C pixels of one image for 16 TN WC
+// output channels; a wave R rows x 16 C pixels x 16 TN channels.  Per chunk of
+// 32 input channels the workgroup stages the input tile with a one-pixel halo
+// (zeros outside the image) and the chunk's weights of all 9 taps, AHEAD chunks
+// ahead in registers and NBUF of them in LDS.  A wave keeps the weights of the
+// 9 taps in registers and walks the rows of the input tile: a row is the lower
+// neighbour of one output row, the middle one of the next and the upper one of
+// the third, so it is read from LDS 3 times (once per dx), not 9, and every
+// output's sum still runs over the chunks, then the taps in order.
+//
+// Large images are bound by LDS reads and the chunks' loads in about equal parts
+// (1920 x 384: 32 -> 32 channels 61 -> 35 us, 94 MB; 96 -> 32 90 -> 59 us, 34 us of
+// MFMAs at the rate of a large product); small ones by the chain of a chunk
+// (512 x 128: 24 us per layer before, 6 .. 17 now): the tile shrinks until there
+// is a workgroup per CU, and two chunks are in flight.  Before, a lane's loads
+// stood behind the branches of the image's edge and were waited for one by one,
+// and a wave read every input fragment once per tap.
 // ---------------------------------------------------------------------------
-constexpr int CONV_PW = 64, CONV_CI = 32;
+constexpr int CONV_CI = 32;
 
 // LDS slot of 16-byte vector g (of 4) of the pixel or output channel at
 // position c: a pixel's 4 vectors are rotated by c / 2, so that the 8 lanes
@@ -143,112 +173,192 @@ constexpr int CONV_PW = 64, CONV_CI = 32;
 // positions puts them on 2 groups: 4-way conflicts).
 __device__ __forceinline__ int conv_slot(int c, int g) { return (g + (c >> 1)) & 3; }
 
-template <int TN, int RW>
-__global__ void __launch_bounds__(256) k_conv_lds(ConvArgs a) {
-  constexpr int CONV_PH = 4 * RW, TM = 4 * RW;
-  constexpr int NV = CONV_CI / 8;                               // 16-byte vectors per pixel per chunk
-  constexpr int NA = (CONV_PH + 2) * (CONV_PW + 2) * NV;        // input vectors per chunk
-  constexpr int NB = 9 * 16 * TN * NV;                          // weight vectors per chunk
-  constexpr int RA = (NA + 255) / 256, RB = (NB + 255) / 256;  // per thread
-  __shared__ u32x4 As[CONV_PH + 2][CONV_PW + 2][NV];
-  __shared__ u32x4 Bs[9][16 * TN][NV];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = threadIdx.x;
-  const int r = lane & 15, g = lane >> 4;
-  const int tiles_x = (a.W + CONV_PW - 1) / CONV_PW, tiles_y = (a.H + CONV_PH - 1) / CONV_PH;
+// Reads of one tensor from a workgroup-uniform address on, by byte offsets;
+// those not below 2^31 - 16 give zeros, without a branch around the load
+// (which would have to be waited for at the branch's end).
+constexpr unsigned BUF_NONE = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_from(const u16 *p) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, 0x7ffffff0, 0x00027000);
+}
+__device__ __forceinline__ u32x4 buf_load(__amdgpu_buffer_rsrc_t b, unsigned off, unsigned uniform) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, (int)off, (int)uniform, 0));
+}
+
+template <int WP, int WC, int R, int C, int TN, int NBUF, int AHEAD, bool CAT>
+__global__ void __launch_bounds__(256, NBUF == 1 ? 2 : 1) k_conv_lds(ConvArgs a) {
+  static_assert(WP * WC == 4 && AHEAD % NBUF == 0, "four waves");
+  constexpr int PH = R * WP, PW = 16 * C, CO = 16 * TN * WC, NV = CONV_CI / 8;
+  constexpr int NA = (PH + 2) * (PW + 2) * NV, NB = 9 * CO * NV;  // 16-byte vectors of a chunk
+  constexpr int RA = (NA + 255) / 256, RB = (NB + 255) / 256;    // per thread
+  __shared__ u32x4 As[NBUF][256 * RA], Bs[NBUF][256 * RB];        // (the rest of the last ones: not read)
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r = lane & 15, g = lane >> 4, wp = wave % WP, wc = wave / WP;
+  const int tiles_x = (a.W + PW - 1) / PW, tiles_y = (a.H + PH - 1) / PH;
   const int bx = blockIdx.x, n = bx / (tiles_x * tiles_y), ty = (bx / tiles_x) % tiles_y, tx = bx % tiles_x;
-  const int i0 = tx * CONV_PW, j0 = ty * CONV_PH, c0 = blockIdx.y * (16 * TN);
-  floatx4 acc[TM][TN];
+  const int i0 = tx * PW, j0 = ty * PH, c0 = blockIdx.y * CO;
+  floatx4 acc[R][C][TN];
 #pragma unroll
-  for (int x = 0; x < TM; x++)
+  for (int o = 0; o < R; o++)
 #pragma unroll
-    for (int y = 0; y < TN; y++) acc[x][y] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // the chunk at ci0 into registers: input tile (zeros outside the image) and weights
-  u32x4 qa[RA], qb[RB];
-  auto fetch = [&](int ci0) {
+    for (int c = 0; c < C; c++)
+#pragma unroll
+      for (int y = 0; y < TN; y++) acc[o][c][y] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // Offsets of the thread's vectors from the row above the tile (of the half-size
+  // image: from its row); the channel is a uniform offset.
+  const int jb = max(j0 - 1, 0), Cs = CAT ? a.Cx - a.Cb : a.Cx, H2 = a.H / 2, W2 = a.W / 2;
+  const __amdgpu_buffer_rsrc_t bufX = buf_from((CAT ? a.X2 : a.X) + ((size_t)n * a.H + jb) * a.W * Cs);
+  const __amdgpu_buffer_rsrc_t bufU = buf_from(CAT ? a.X + ((size_t)n * H2 + jb / 2) * W2 * a.Cb : a.X);
+  const __amdgpu_buffer_rsrc_t bufW = buf_from(a.Wt + (size_t)c0 * a.Kp);
+  unsigned oa[RA], ob[RB];
+  auto offsets = [&](bool up) {
 #pragma unroll
     for (int k = 0; k < RA; k++) {
-      const int e = t + 256 * k;
-      qa[k] = u32x4{0u, 0u, 0u, 0u};
-      if (e < NA) {
-        const int v = e % NV, pos = e / NV;
-        const int ii = i0 + pos % (CONV_PW + 2) - 1, jj = j0 + pos / (CONV_PW + 2) - 1, ci = ci0 + 8 * v;
-        if (ii >= 0 && ii < a.W && jj >= 0 && jj < a.H) {
-          const u16 *src;
-          if (!a.X2) src = a.X + ((size_t)(n * a.H + jj) * a.W + ii) * a.Cx + ci;
-          else if (ci < a.Cb)  // nearest-upsampled half-size tensor
-            src = a.X + ((size_t)(n * (a.H / 2) + jj / 2) * (a.W / 2) + ii / 2) * a.Cb + ci;
-          else  // skip tensor
-            src = a.X2 + ((size_t)(n * a.H + jj) * a.W + ii) * (a.Cx - a.Cb) + (ci - a.Cb);
-          qa[k] = *reinterpret_cast<const u32x4 *>(src);
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < RB; k++) {
-      const int e = t + 256 * k;
-      qb[k] = u32x4{0u, 0u, 0u, 0u};
-      if (e < NB) {
-        const int v = e % NV, col = (e / NV) % (16 * TN), tap = e / (NV * 16 * TN), co = c0 + col;
-        if (co < a.Cout) qb[k] = *reinterpret_cast<const u32x4 *>(a.Wt + (size_t)co * a.Kp + tap * a.Cx + ci0 + 8 * v);
-      }
+      const int e = t + 256 * k, pos = e / NV, col = pos % (PW + 2), v = (e % NV - (col >> 1)) & 3;
+      const int ii = i0 + col - 1, jj = j0 + pos / (PW + 2) - 1;
+      const unsigned px = up ? (unsigned)((jj / 2 - jb / 2) * W2 + ii / 2) * a.Cb : (unsigned)((jj - jb) * a.W + ii) * Cs;
+      oa[k] = e < NA && ii >= 0 && ii < a.W && jj >= 0 && jj < a.H ? 2 * (px + 8 * v) : BUF_NONE;
     }
   };
-  fetch(0);
-  for (int ci0 = 0; ci0 < a.Cx; ci0 += CONV_CI) {
 #pragma unroll
-    for (int k = 0; k < RA; k++) {
-      const int e = t + 256 * k;
-      if (e < NA) {
-        const int col = (e / NV) % (CONV_PW + 2);
-        As[(e / NV) / (CONV_PW + 2)][col][conv_slot(col, e % NV)] = qa[k];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < RB; k++) {
-      const int e = t + 256 * k;
-      if (e < NB) {
-        const int co = (e / NV) % (16 * TN);
-        Bs[e / (NV * 16 * TN)][co][conv_slot(co, e % NV)] = qb[k];
-      }
-    }
-    __syncthreads();
-    if (ci0 + CONV_CI < a.Cx) fetch(ci0 + CONV_CI);  // in flight while this chunk's MFMAs run
-#pragma unroll
-    for (int tap = 0; tap < 9; tap++) {
-      const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-      bf16x8 A[TM], B[TN];
-#pragma unroll
-      for (int s = 0; s < TM; s++) {
-        const int col = 16 * (s % 4) + r + 1 + dx;
-        A[s] = __builtin_bit_cast(bf16x8, As[RW * wave + s / 4 + 1 + dy][col][conv_slot(col, g)]);
-      }
-#pragma unroll
-      for (int s = 0; s < TN; s++) B[s] = __builtin_bit_cast(bf16x8, Bs[tap][16 * s + r][conv_slot(16 * s + r, g)]);
-#pragma unroll
-      for (int x = 0; x < TM; x++)
-#pragma unroll
-        for (int y = 0; y < TN; y++) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[x], B[y], acc[x][y], 0, 0, 0);
-    }
-    __syncthreads();
+  for (int k = 0; k < RB; k++) {
+    const int e = t + 256 * k, pos = e / NV, col = pos % CO, tap = pos / CO, v = (e % NV - (col >> 1)) & 3;
+    ob[k] = e < NB && c0 + col < a.Cout ? 2 * (unsigned)(col * a.Kp + tap * a.Cx + 8 * v) : BUF_NONE;
   }
+  offsets(CAT);
+  u32x4 qa[AHEAD][RA], qb[AHEAD][RB];
+  int cf = 0;  // the next chunk to fetch
+  auto fetch = [&](u32x4 (&x)[RA], u32x4 (&w)[RB]) {
+    if (CAT && cf == a.Cb) offsets(false);
+    const bool up = CAT && cf < a.Cb;
+    const __amdgpu_buffer_rsrc_t b = up ? bufU : bufX;
+    const unsigned ch = 2 * (unsigned)(CAT && !up ? cf - a.Cb : cf);
+#pragma unroll
+    for (int k = 0; k < RA; k++) x[k] = buf_load(b, oa[k], ch);
+#pragma unroll
+    for (int k = 0; k < RB; k++) w[k] = buf_load(bufW, ob[k], 2 * (unsigned)cf);
+    cf = min(cf + CONV_CI, a.Cx - CONV_CI);  // (at the end the last chunk again, not used)
+  };
+#pragma unroll
+  for (int k = 0; k < AHEAD; k++) fetch(qa[k], qb[k]);
+  for (int ci0 = 0; ci0 < a.Cx; ci0 += CONV_CI * AHEAD) {
+#pragma unroll
+    for (int h = 0; h < AHEAD; h++) {
+      if (AHEAD > 1 && ci0 + CONV_CI * h >= a.Cx) break;
+      const int buf = h % NBUF;
+      if (NBUF == 1) __syncthreads();  // the last chunk has been read
+#pragma unroll
+      for (int k = 0; k < RA; k++) As[buf][t + 256 * k] = qa[h][k];
+#pragma unroll
+      for (int k = 0; k < RB; k++) Bs[buf][t + 256 * k] = qb[h][k];
+      __syncthreads();
+      fetch(qa[h], qb[h]);  // in flight while this chunk's MFMAs run
+      bf16x8 B[9][TN];
+#pragma unroll
+      for (int tap = 0; tap < 9; tap++)
+#pragma unroll
+        for (int y = 0; y < TN; y++) {
+          const int col = 16 * (TN * wc + y) + r;
+          B[tap][y] = __builtin_bit_cast(bf16x8, Bs[buf][(tap * CO + col) * NV + conv_slot(col, g)]);
+        }
+#pragma unroll
+      for (int y = 0; y < R + 2; y++)  // input row R wp + y of the tile
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+          for (int c = 0; c < C; c++) {
+            const int col = 16 * c + r + dx;
+            const bf16x8 A = __builtin_bit_cast(
+                bf16x8, As[buf][((R * wp + y) * (PW + 2) + col) * NV + conv_slot(col, g)]);
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+              const int o = y - dy;
+              if (o < 0 || o >= R) continue;
+#pragma unroll
+              for (int q = 0; q < TN; q++)
+                acc[o][c][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[3 * dy + dx][q], A, acc[o][c][q], 0, 0, 0);
+            }
+          }
+    }
+  }
+  // D rows = channels 4 g .. 4 g + 3 of 16, column = pixel r of 16
 #pragma unroll
   for (int y = 0; y < TN; y++) {
-    const int co = c0 + 16 * y + r;
+    const int co = c0 + 16 * (TN * wc + y) + 4 * g;
     if (co >= a.Cout) continue;
-    const float bias = a.bias ? a.bias[co] : 0.f;
 #pragma unroll
-    for (int x = 0; x < TM; x++) {
-      const int j = j0 + RW * wave + x / 4;
+    for (int o = 0; o < R; o++) {
+      const int j = j0 + R * wp + o;
       if (j >= a.H) continue;
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int i = i0 + 16 * (x % 4) + 4 * g + q;
-        if (i >= a.W) continue;
-        float v = acc[x][y][q] + bias;
-        if (a.relu) v = fmaxf(v, 0.f);
-        const size_t o = ((size_t)(n * a.H + j) * a.W + i) * a.Cout + co;
-        a.Y[o] = (a.act && !(bf2f(a.act[o]) > 0.f)) ? (u16)0 : f2bf(v);
+      for (int c = 0; c < C; c++) {
+        const int i = i0 + 16 * c + r;
+        if (i < a.W) conv_out(a, ((size_t)(n * a.H + j) * a.W + i) * a.Cout + co, co, acc[o][c][y]);
       }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 3x3 convolution of few input channels (stride 8 CV, CV <= 3: the network's
+// first layer), whose 32-wide k chunks take several taps each.  A workgroup
+// computes PH rows x 64 pixels for 16 TN channels from the tile and its halo in
+// LDS; a lane's place in it for each chunk (its tap's shift and channel vector)
+// and the weights of all chunks stay in registers.  Same k order as k_conv, which
+// spends its time on addresses here: 1920 x 384, 9 .. 16 -> 32 channels 47 -> 26
+// us, 8 x 512 x 128, 8 -> 32 27 -> 16 us.
+// ---------------------------------------------------------------------------
+constexpr int FEW_PW = 64;
+
+template <int CV, int TN, int PH>
+__global__ void __launch_bounds__(256) k_conv_few(ConvArgs a) {
+  constexpr int NS = (72 * CV + 31) / 32;  // chunks
+  constexpr int NA = (PH + 2) * (FEW_PW + 2) * CV, RA = (NA + 255) / 256;
+  __shared__ u32x4 As[256 * RA + 1];  // the last one: zeros
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, r = lane & 15, g = lane >> 4;
+  const int tiles_x = (a.W + FEW_PW - 1) / FEW_PW, tiles_y = (a.H + PH - 1) / PH;
+  const int bx = blockIdx.x, n = bx / (tiles_x * tiles_y), ty = (bx / tiles_x) % tiles_y, tx = bx % tiles_x;
+  const int i0 = tx * FEW_PW, j0 = ty * PH, c0 = blockIdx.y * (16 * TN);
+  const u16 *zero = (const u16 *)a.zero;
+#pragma unroll
+  for (int k = 0; k < RA; k++) {
+    const int e = t + 256 * k, pos = e / CV, v = e % CV;
+    const int ii = i0 + pos % (FEW_PW + 2) - 1, jj = j0 + pos / (FEW_PW + 2) - 1;
+    const u16 *at = a.X + (((size_t)n * a.H + jj) * a.W + ii) * (8 * CV) + 8 * v;
+    As[e] = *reinterpret_cast<const u32x4 *>(ii >= 0 && ii < a.W && jj >= 0 && jj < a.H ? at : zero);
+  }
+  if (t == 0) As[256 * RA] = u32x4{0u, 0u, 0u, 0u};
+  bf16x8 B[NS][TN];
+  int off[NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    const int v = 4 * s + g, tap = v / CV;  // the lane's 16-byte vector of k
+    off[s] = tap < 9 ? ((tap / 3) * (FEW_PW + 2) + tap % 3) * CV + v % CV : -1;
+#pragma unroll
+    for (int y = 0; y < TN; y++) {
+      const int co = c0 + 16 * y + r;
+      const u16 *at = a.Wt + (size_t)co * a.Kp + 8 * v;
+      B[s][y] = load8(co < a.Cout ? at : zero);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PH; q++) {  // 4 tiles of 16 pixels per row, one of each per wave
+    const int px = 16 * wave + r, i = i0 + px, j = j0 + q;
+    floatx4 acc[TN];
+#pragma unroll
+    for (int y = 0; y < TN; y++) acc[y] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const int at = off[s] < 0 ? 256 * RA : (q * (FEW_PW + 2) + px) * CV + off[s];
+      const bf16x8 A = __builtin_bit_cast(bf16x8, As[at]);
+#pragma unroll
+      for (int y = 0; y < TN; y++) acc[y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[s][y], A, acc[y], 0, 0, 0);
+    }
+    if (j >= a.H || i >= a.W) continue;
+#pragma unroll
+    for (int y = 0; y < TN; y++) {
+      const int co = c0 + 16 * y + 4 * g;
+      if (co < a.Cout) conv_out(a, (((size_t)n * a.H + j) * a.W + i) * a.Cout + co, co, acc[y]);
     }
   }
 }
@@ -268,13 +378,13 @@ __global__ void __launch_bounds__(256) k_conv_lds(ConvArgs a) {
 // lane: ds_read_b64_tr_b16 reads them transposed (lane i of 16 gets channel i of
 // 4 pixels), and a tap's shift is then only another pixel address.  The workgroup
 // leaves its sums in its own slot of `part` (laid out as the gradient is);
-// k_sum_parts adds the slots in FP64: no atomics, and the same gradients on every
-// run.  The runs' length and the order within them, for the bias too, are those
+// k_sum_parts adds the slots in their order: no atomics, and the same gradients on
+// every run.  The runs' length and the order within them, for the bias too, are those
 // the sums always had: each slot holds the same bits as before.
 //
 // The bound is the chain of a step (LDS write, barrier, transposed reads, MFMA):
 // a layer with one workgroup per CU takes 27 us whatever its size.  At 8 x 512 x
-// 128, base 32: 590 us per training step for the 14 convolutions, biases
+// 128, base 32: 600 us per training step for the 14 convolutions, biases
 // included.  The kernels before took 3,484 us (one wave per 16 x 16 of one tap,
 // channel-strided 2-byte loads, atomics) and 2,958 us for the biases.  Loads
 // under an exec mask had to be waited for at each branch's end (73 us per layer);
@@ -460,66 +570,87 @@ __global__ void __launch_bounds__(128 * WCI * WCO, MT == 4 ? 2 : 4) k_wgrad(Wgra
   }
 }
 
-// Sums of slots of FP32 partial sums, in FP64 and a fixed order (each addition
-// of the many is then as good as exact): over part[s * P + e], s < S, for every
-// e < P (a multiple of 4) -- 8 runs of slots side by side, then the runs in
-// turn -- onto carry[e] unless `first`, into out[e] (rounded) if `last`, else
-// into carry[e].
-constexpr int SUM_RUNS = 8;
-typedef double doublex4 __attribute__((ext_vector_type(4)));
+// Sums of slots of FP32 partial sums, one slot after the other in FP32 (the
+// order in which the atomics they replaced mostly came): out[e] = sum of
+// part[q * P + e], q < S, onto out's own value unless `first`; P a multiple of 4.
+//
+// Many slots: a workgroup takes 256 consecutive e; wave y has slots SUM_SLOTS y ..
+// of SUM_WAVES * SUM_SLOTS at a time in registers, all loads in flight, and the
+// waves add theirs in turn.
+constexpr int SUM_WAVES = 8, SUM_SLOTS = 16;
 
-// The same for one e of few, by one wave: lane l adds slots l, l + 64, .., then
-// the lanes in a fixed tree.
-__device__ __forceinline__ void sum_row(const float *part, int S, int P, int e, float *out) {
-  const int lane = threadIdx.x & 63;
-  if (e >= P) return;
-  double v = 0.0;
-  for (int q = lane; q < S; q += 64) v += (double)part[(size_t)q * P + e];
+__device__ __forceinline__ void sum_turns(const float *part, int S, size_t P, bool first, float *out, int group) {
+  __shared__ floatx4 run[64];
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+  const size_t e = 4 * ((size_t)group * 64 + x);
+  const bool in = e < P;
+  if (y == 0) run[x] = in && !first ? *reinterpret_cast<const floatx4 *>(out + e) : (floatx4)0.f;
+  for (int q0 = 0; q0 < S; q0 += SUM_WAVES * SUM_SLOTS) {
+    floatx4 v[SUM_SLOTS];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if (lane == 0) out[e] = (float)v;
+    for (int k = 0; k < SUM_SLOTS; k++)
+      v[k] = *reinterpret_cast<const floatx4 *>(part + (size_t)min(q0 + SUM_SLOTS * y + k, S - 1) * P + (in ? e : 0));
+    for (int w = 0; w < SUM_WAVES; w++) {
+      __syncthreads();
+      if (w != y) continue;
+      floatx4 s = run[x];
+#pragma unroll
+      for (int k = 0; k < SUM_SLOTS; k++)
+        if (q0 + SUM_SLOTS * y + k < S) s += v[k];
+      run[x] = s;
+    }
+  }
+  __syncthreads();
+  if (y == 0 && in) *reinterpret_cast<floatx4 *>(out + e) = run[x];
 }
 
-__global__ void __launch_bounds__(256) k_sum_rows(const float *part, int S, int P, float *out) {
-  sum_row(part, S, P, (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), out);
+// Few slots: a thread takes 4 consecutive e, 8 slots' loads at a time.
+__device__ __forceinline__ void sum_each(const float *part, int S, size_t P, bool first, float *out, int group) {
+  const size_t e = 4 * ((size_t)group * (64 * SUM_WAVES) + threadIdx.x);
+  if (e >= P) return;
+  floatx4 s = first ? (floatx4)0.f : *reinterpret_cast<const floatx4 *>(out + e);
+  for (int q0 = 0; q0 < S; q0 += 8) {
+    floatx4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = *reinterpret_cast<const floatx4 *>(part + (size_t)min(q0 + k, S - 1) * P + e);
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      if (q0 + k < S) s += v[k];
+  }
+  *reinterpret_cast<floatx4 *>(out + e) = s;
 }
 
+// The weights' slots (each: by sum_each) and, by the workgroups past the first
+// `groups`, the bias's (rpart[rS][rP]).
 struct SumArgs {
   const float *part;
   int S;
   size_t P;
-  double *carry;
-  bool first, last;
+  bool each, first;
   float *out;
-  // workgroups past the first `groups`: rpart[rS][rP] by rows into rout
   int groups;
   const float *rpart;
   int rS, rP;
   float *rout;
 };
-__global__ void __launch_bounds__(64 * SUM_RUNS) k_sum_parts(SumArgs a) {
-  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
-  if ((int)blockIdx.x >= a.groups) {
-    sum_row(a.rpart, a.rS, a.rP, ((int)blockIdx.x - a.groups) * SUM_RUNS + y, a.rout);
-    return;
-  }
-  const size_t e = 4 * ((size_t)blockIdx.x * 64 + x);
-  const int per = (a.S + SUM_RUNS - 1) / SUM_RUNS, s1 = min(a.S, (y + 1) * per);
-  doublex4 v = {0.0, 0.0, 0.0, 0.0};
-  if (e < a.P) {
-#pragma unroll 4
-    for (int q = y * per; q < s1; q++)
-      v += __builtin_convertvector(*reinterpret_cast<const floatx4 *>(a.part + (size_t)q * a.P + e), doublex4);
-  }
-  __shared__ doublex4 sm[SUM_RUNS][64];
-  sm[y][x] = v;
-  __syncthreads();
-  if (y != 0 || e >= a.P) return;
-  if (!a.first) v += *reinterpret_cast<const doublex4 *>(a.carry + e);
+__global__ void __launch_bounds__(64 * SUM_WAVES) k_sum_parts(SumArgs a) {
+  const int q = (int)blockIdx.x - a.groups;
+  if (q >= 0) sum_turns(a.rpart, a.rS, a.rP, true, a.rout, q);
+  else if (a.each) sum_each(a.part, a.S, a.P, a.first, a.out, blockIdx.x);
+  else sum_turns(a.part, a.S, a.P, a.first, a.out, blockIdx.x);
+}
+
+// out[e] = sum of part[q * P + e], q < S, for few e, in FP64 (as good as exact):
+// one wave per e, lane l adds slots l, l + 64, .., then the lanes in a fixed tree.
+__global__ void __launch_bounds__(256) k_sum_rows(const float *part, int S, int P, float *out) {
+  const int e = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (e >= P) return;
+  double v = 0.0;
+#pragma unroll 8
+  for (int q = lane; q < S; q += 64) v += (double)part[(size_t)q * P + e];
 #pragma unroll
-  for (int q = 1; q < SUM_RUNS; q++) v += sm[q][x];
-  if (a.last) *reinterpret_cast<floatx4 *>(a.out + e) = __builtin_convertvector(v, floatx4);
-  else *reinterpret_cast<doublex4 *>(a.carry + e) = v;
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if (lane == 0) out[e] = (float)v;
 }
 
 // ---------------------------------------------------------------------------
@@ -598,33 +729,40 @@ __global__ void __launch_bounds__(256) k_pool_back_add(const u16 *P, const u16 *
 }
 
 // Head (1x1 conv, linear): Y[p][o] = sum_c X[p][c] * Wb[c][o] + b[o], FP32 out.
-// Co <= HEAD_MAX_CO; the sums are kept in registers (loops over a constant
-// bound, outputs past Co skipped).
-// The weights (C x Co <= HEAD_MAX_W) are read from LDS, one broadcast read
-// per weight and wavefront.
+// Co <= CO <= HEAD_MAX_CO; the sums are kept in registers.  The weights (C x Co
+// <= HEAD_MAX_W) are read from LDS, CO at a time, the pixel's channels 32 at a
+// time (16-byte loads, C is a multiple of 8).
 constexpr int HEAD_MAX_CO = 8, HEAD_MAX_W = 1024;
+template <int CO>
 __global__ void __launch_bounds__(256) k_head(const u16 *X, int C, const u16 *Wb, const float *b, int Co, int npix,
                                               float *Y) {
-  __shared__ float Ws[HEAD_MAX_W];
-  for (int e = threadIdx.x; e < C * Co; e += blockDim.x) Ws[e] = bf2f(Wb[e]);
+  __shared__ alignas(16) float Ws[CO * HEAD_MAX_W];  // [C][CO]
+  for (int e = threadIdx.x; e < C * CO; e += blockDim.x)
+    Ws[e] = e % CO < Co ? bf2f(Wb[e / CO * Co + e % CO]) : 0.f;
   __syncthreads();
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= npix) return;
-  float s[HEAD_MAX_CO];
+  float s[CO];
 #pragma unroll
-  for (int o = 0; o < HEAD_MAX_CO; o++) s[o] = 0.f;
-  for (int c0 = 0; c0 < C; c0 += 8) {  // C is a multiple of 8: 16-byte loads
-    const U16x8 x = *reinterpret_cast<const U16x8 *>(X + (size_t)p * C + c0);
+  for (int o = 0; o < CO; o++) s[o] = 0.f;
+  for (int c0 = 0; c0 < C; c0 += 32) {
+    U16x8 x[4];
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const float xv = bf2f(x.v[q]);
+    for (int v = 0; v < 4; v++)
+      x[v] = *reinterpret_cast<const U16x8 *>(X + (size_t)p * C + min(c0 + 8 * v, C - 8));
 #pragma unroll
-      for (int o = 0; o < HEAD_MAX_CO; o++)
-        if (o < Co) s[o] += xv * Ws[(c0 + q) * Co + o];
+    for (int v = 0; v < 4; v++) {
+      if (c0 + 8 * v >= C) break;
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const float xv = bf2f(x[v].v[q]);
+#pragma unroll
+        for (int o = 0; o < CO; o++) s[o] += xv * Ws[(c0 + 8 * v + q) * CO + o];
+      }
     }
   }
 #pragma unroll
-  for (int o = 0; o < HEAD_MAX_CO; o++)
+  for (int o = 0; o < CO; o++)
     if (o < Co) Y[(size_t)p * Co + o] = s[o] + b[o];
 }
 
@@ -883,7 +1021,8 @@ __global__ void k_gather(const u16 *Xs, const float *Ts, const uint8_t *Ms, cons
   if (e >= (size_t)n * npix) return;
   const int b = (int)(e / npix), q = (int)(e % npix);
   const size_t src = (size_t)slots[b] * npix + q;
-  for (int c = 0; c < Cx; c++) X[e * Cx + c] = Xs[src * Cx + c];
+  for (int c = 0; c < Cx; c += 8)  // Cx is a multiple of 8
+    *reinterpret_cast<U16x8 *>(X + e * Cx + c) = *reinterpret_cast<const U16x8 *>(Xs + src * Cx + c);
   for (int c = 0; c < Co; c++) Tg[e * Co + c] = Ts[src * Co + c];
   M[e] = Ms[src];
 }
@@ -895,14 +1034,60 @@ __global__ void k_gather(const u16 *Xs, const float *Ts, const uint8_t *Ms, cons
 // ---------------------------------------------------------------------------
 static inline unsigned nblk(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 
+// The largest tile of a class that gives a workgroup per CU.  64 channels: 4 rows
+// x 32 pixels (8 rows: 52 -> 57 us for 384 -> 128 at 480 x 96, 30 -> 31 for 64 -> 64
+// at 960 x 192), else 4 or 2 rows x 16 pixels with two chunks in flight (64 -> 64
+// at 256 x 64: 7.0 us, with 4 x 32 8.9, with 2 x 16 10; 256 -> 256 at 64 x 16: 9.9,
+// with 4 x 16 11, with 4 x 32 16).  32 channels: 8 rows x 32 pixels where that gives
+// two workgroups per CU (16 rows: 35 -> 41 us for 32 -> 32 at 1920 x 384), else 8 x
+// 16 (512 x 128: 7.1 -> 6.1 us).
+constexpr unsigned CONV_FULL = 256;
+
+template <int WP, int WC, int R, int C, int TN>
+static dim3 conv_grid(const ConvArgs &a) {
+  return dim3((unsigned)a.N * nblk(a.H, R * WP) * nblk(a.W, 16 * C), nblk(a.Cout, 16 * TN * WC));
+}
+template <int WP, int WC, int R, int C, int TN>
+static unsigned conv_groups(const ConvArgs &a) {
+  const dim3 g = conv_grid<WP, WC, R, C, TN>(a);
+  return g.x * g.y;
+}
+template <int WP, int WC, int R, int C, int TN, int NBUF, int AHEAD>
+static void launch_conv(const ConvArgs &a, hipStream_t s) {
+  const dim3 g = conv_grid<WP, WC, R, C, TN>(a);
+  if (a.X2) hipLaunchKernelGGL((k_conv_lds<WP, WC, R, C, TN, NBUF, AHEAD, true>), g, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((k_conv_lds<WP, WC, R, C, TN, NBUF, AHEAD, false>), g, dim3(256), 0, s, a);
+}
+
 hipError_t unet_conv(const ConvArgs &a, hipStream_t s) {
+  if (a.Cout % 4) return hipErrorInvalidValue;
   const size_t npix = (size_t)a.N * a.H * a.W;
-  if (a.ks == 3 && a.Cx % CONV_CI == 0 && (!a.X2 || a.Cb % CONV_CI == 0)) {
-    // 64 or 32 channels x 4 rows per block (32 channels x 8 rows, two rows per
-    // wave, needs 291 registers: one wave per SIMD, 45% slower)
-    const unsigned tiles = (unsigned)a.N * nblk(a.H, 4) * nblk(a.W, CONV_PW);
-    if (a.Cout >= 64) hipLaunchKernelGGL((k_conv_lds<4, 1>), dim3(tiles, nblk(a.Cout, 64)), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_conv_lds<2, 1>), dim3(tiles, nblk(a.Cout, 32)), dim3(256), 0, s, a);
+  // (offsets within a tile's rows are 32 bits)
+  const bool far = (size_t)20 * a.W * a.Cx >= ((size_t)1 << 30) || (size_t)64 * a.Kp >= ((size_t)1 << 30);
+  if (a.ks == 3 && a.Cx % CONV_CI == 0 && (!a.X2 || a.Cb % CONV_CI == 0) && !far) {
+    if (a.Cout % 64 == 0) {
+      if (conv_groups<2, 2, 2, 2, 2>(a) >= CONV_FULL) launch_conv<2, 2, 2, 2, 2, 1, 1>(a, s);
+      else if (conv_groups<1, 4, 4, 1, 1>(a) >= CONV_FULL) launch_conv<1, 4, 4, 1, 1, 2, 2>(a, s);
+      else launch_conv<1, 4, 2, 1, 1, 2, 2>(a, s);
+    } else {
+      if (conv_groups<4, 1, 2, 2, 2>(a) > 2 * CONV_FULL) launch_conv<4, 1, 2, 2, 2, 1, 1>(a, s);
+      else launch_conv<4, 1, 2, 1, 2, 1, 1>(a, s);
+    }
+    return hipGetLastError();
+  }
+  if (a.ks == 3 && a.Cx <= 24 && !a.X2) {
+    auto launch = [&](auto ph) {
+      constexpr int PH = decltype(ph)::value;
+      const dim3 g((unsigned)a.N * nblk(a.H, PH) * nblk(a.W, FEW_PW), nblk(a.Cout, 32));
+      if (a.Cx == 8) hipLaunchKernelGGL((k_conv_few<1, 2, PH>), g, dim3(256), 0, s, a);
+      else if (a.Cx == 16) hipLaunchKernelGGL((k_conv_few<2, 2, PH>), g, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL((k_conv_few<3, 2, PH>), g, dim3(256), 0, s, a);
+    };
+    // 8 rows where that gives two workgroups per CU (2 rows: 34 us instead of 26 at
+    // 1920 x 384, but 6.6 instead of 11 at 512 x 128)
+    if ((unsigned)a.N * nblk(a.H, 8) * nblk(a.W, FEW_PW) * nblk(a.Cout, 32) >= 2 * CONV_FULL)
+      launch(std::integral_constant<int, 8>());
+    else launch(std::integral_constant<int, 2>());
     return hipGetLastError();
   }
   // 4 pixel tiles per wave; 4 channel tiles where there are 64+ channels
@@ -917,8 +1102,9 @@ hipError_t unet_conv(const ConvArgs &a, hipStream_t s) {
 // 32 for a narrow input): a workgroup takes as long however few there are (64
 // workgroups of 64 x 64: 86 us per layer, 256 of 32 x 32: 27 us).
 constexpr long WGRAD_FULL = 256;
+constexpr int SUM_EACH = 32;
 
-hipError_t unet_wgrad(const WgradArgs &a, double *carry, float *dW, float *db, hipStream_t s) {
+hipError_t unet_wgrad(const WgradArgs &a, float *dW, float *db, hipStream_t s) {
   if (a.W % 8 || a.Cx % 8 || a.Cout % 8 || (a.X2 && a.Cb % 8)) return hipErrorInvalidValue;
   const int npix = a.N * a.H * a.W, S = (int)nblk(npix, WG_RUN);
   auto groups = [&](int CI, int CO) { return (long)nblk(a.Cx, CI) * nblk(a.Cout, CO) * S; };
@@ -928,7 +1114,9 @@ hipError_t unet_wgrad(const WgradArgs &a, double *carry, float *dW, float *db, h
   const size_t P = (size_t)9 * a.Cin * a.Cout;
   const int most = (int)std::min<size_t>(std::max<size_t>(1, UNET_PART_FLOATS / P), 65535);
   for (int q = 0; q < S; q += most) {
-    const int n = std::min(most, S - q), nsum = (int)nblk(P, 256);
+    const int n = std::min(most, S - q);
+    const bool each = n <= SUM_EACH;
+    const int nsum = (int)nblk(P, each ? 256 * SUM_WAVES : 256);
     const bool last = q + n == S;
     const dim3 gr(nblk(a.Cx, CI) + 1, nblk(a.Cout, CO), n);  // + the bias
     if (CI == 64 && a.X2) hipLaunchKernelGGL((k_wgrad<4, 1, 4, 2, true>), gr, dim3(512), 0, s, a, q);
@@ -938,8 +1126,8 @@ hipError_t unet_wgrad(const WgradArgs &a, double *carry, float *dW, float *db, h
     else if (a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, true>), gr, dim3(512), 0, s, a, q);
     else if (CI == 32) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, false>), gr, dim3(512), 0, s, a, q);
     else hipLaunchKernelGGL((k_wgrad<1, 2, 1, 4, false>), gr, dim3(256), 0, s, a, q);
-    const SumArgs b{a.part, n, P, carry, q == 0, last, dW, nsum, a.bpart, (int)nblk(npix, WG_BIAS), a.Cout, db};
-    hipLaunchKernelGGL(k_sum_parts, dim3(nsum + (last ? nblk(a.Cout, SUM_RUNS) : 0)), dim3(64 * SUM_RUNS), 0, s, b);
+    const SumArgs b{a.part, n, P, each, q == 0, dW, nsum, a.bpart, (int)nblk(npix, WG_BIAS), a.Cout, db};
+    hipLaunchKernelGGL(k_sum_parts, dim3(nsum + (last ? nblk(a.Cout, 256) : 0)), dim3(64 * SUM_WAVES), 0, s, b);
   }
   return hipGetLastError();
 }
@@ -963,7 +1151,9 @@ hipError_t unet_pool_back_add(const uint16_t *P, const uint16_t *Skip, int Cs, i
 hipError_t unet_head(const uint16_t *X, int C, const uint16_t *Wh, const float *b, int Co, int npix, float *Y,
                      hipStream_t s) {
   if (Co > HEAD_MAX_CO || C * Co > HEAD_MAX_W) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_head, dim3(nblk(npix, 256)), dim3(256), 0, s, X, C, Wh, b, Co, npix, Y);
+  if (Co <= 2) hipLaunchKernelGGL(k_head<2>, dim3(nblk(npix, 256)), dim3(256), 0, s, X, C, Wh, b, Co, npix, Y);
+  else if (Co <= 4) hipLaunchKernelGGL(k_head<4>, dim3(nblk(npix, 256)), dim3(256), 0, s, X, C, Wh, b, Co, npix, Y);
+  else hipLaunchKernelGGL(k_head<8>, dim3(nblk(npix, 256)), dim3(256), 0, s, X, C, Wh, b, Co, npix, Y);
   return hipGetLastError();
 }
 hipError_t unet_head_back(const float *dY, const uint16_t *X, int C, const uint16_t *Wh, int Co, int npix,

@@ -13,9 +13,10 @@ struct ConvArgs {
   const uint16_t *Wt;  // [Cout][Kp], k = tap*Cx + ci
   int Kp;              // multiple of 32, >= ks*ks*Cx
   const float *bias;   // [Cout] or null
-  int Cout;
+  int Cout;            // multiple of 4
   uint16_t *Y;  // [N][H][W][Cout], BF16
   int relu;
+  const void *zero;  // 16 bytes of zeros
   // Optional concatenated input read in place: channels [0, Cb) are X at
   // half resolution, nearest-upsampled; channels [Cb, Cx) are X2 (stride
   // Cx - Cb).  X2 == null: X is one tensor of stride Cx.
@@ -44,8 +45,7 @@ struct WgradArgs {
 constexpr size_t UNET_PART_FLOATS = (size_t)16 << 20;
 
 hipError_t unet_conv(const ConvArgs &a, hipStream_t s);
-// carry: 9 Cin Cout doubles.
-hipError_t unet_wgrad(const WgradArgs &a, double *carry, float *dW, float *db, hipStream_t s);
+hipError_t unet_wgrad(const WgradArgs &a, float *dW, float *db, hipStream_t s);
 hipError_t unet_pool(const uint16_t *X, int N, int H, int W, int C, uint16_t *Y, hipStream_t s);
 hipError_t unet_up_back(const uint16_t *D, int Cd, int Cu, const uint16_t *Act, int N, int H, int W, uint16_t *O,
                         hipStream_t s);
