@@ -15,6 +15,7 @@
 
 #include "simple_ts.h"
 #include "sts_device.h"
+#include "host_copy.h"
 #include "sts_internal.h"
 #include "sts_launch.h"
 
@@ -70,6 +71,7 @@ struct sts_ctx {
   bool mixed = false;
   KGridT<float> g32{};
   float *hx32 = nullptr, *hy32 = nullptr;
+  HostCopy copy;  // of fields
   float *f32[STS_NFIELDS] = {};
   float *p_alt32 = nullptr, *T_alt32 = nullptr;
   int last_iters32 = 0, last_iters64m = 0;
@@ -420,6 +422,7 @@ static int alloc_state(sts_ctx *c, const sts_grid *gi, const std::vector<uint8_t
   HIP_OK(hipHostMalloc(&c->h_red, sizeof(unsigned long long) * (NRED + 1), hipHostMallocDefault));
   HIP_OK(hipHostMalloc(&c->h_ctrl, sizeof(LoopCtrl), hipHostMallocDefault));
   HIP_OK(hipEventCreateWithFlags(&c->ev_ctrl, hipEventDisableTiming));
+  c->copy.reserve(bytes);
   HIP_OK(hipMemcpyAsync(c->hx, hx.data(), sizeof(double) * hx.size(), hipMemcpyHostToDevice, c->stream));
   HIP_OK(hipMemcpyAsync(c->hy, hy.data(), sizeof(double) * hy.size(), hipMemcpyHostToDevice, c->stream));
   HIP_OK(hipMemcpyAsync(c->m, mask.data(), Na, hipMemcpyHostToDevice, c->stream));
@@ -658,8 +661,7 @@ extern "C" int sts_set_field(sts_ctx *c, int field, const double *host) {
   c->pred_backoff = 1;
   c->pred_degree = -1;
   c->pred_wins = 0;
-  HIP_OK(hipMemcpyAsync(c->f[field], host, sizeof(double) * (size_t)c->Na, hipMemcpyHostToDevice, c->stream));
-  HIP_OK(hipStreamSynchronize(c->stream));
+  HIP_OK(c->copy.put(c->f[field], host, sizeof(double) * (size_t)c->Na, c->stream));
   return STS_OK;
 }
 
@@ -669,8 +671,7 @@ extern "C" int sts_get_field(sts_ctx *c, int field, double *host) {
     int rc = refresh_diff(c);
     if (rc) return rc;
   }
-  HIP_OK(hipMemcpyAsync(host, c->f[field], sizeof(double) * (size_t)c->Na, hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipStreamSynchronize(c->stream));
+  HIP_OK(c->copy.get(host, c->f[field], sizeof(double) * (size_t)c->Na, c->stream));
   return STS_OK;
 }
 

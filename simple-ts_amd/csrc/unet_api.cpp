@@ -8,6 +8,7 @@
 #include <string>
 #include <vector>
 
+#include "host_copy.h"
 #include "sts_internal.h"
 #include "sts_unet.h"
 #include "unet_launch.h"
@@ -59,6 +60,7 @@ struct sts_unet {
   float *part = nullptr, *bpart = nullptr;  // partial sums of the parameter gradients
   u16 *zero = nullptr;                      // 16 bytes of zeros
   double *loss = nullptr;
+  HostCopy copy;  // of inputs, outputs and parameters
   int *slots_dev = nullptr;
   // training set
   int ds_n = 0;
@@ -309,6 +311,7 @@ extern "C" int sts_unet_create(int cin, int cout, int base, int max_n, int H, in
   A_OK(hipMalloc(&u->bpart, sizeof(float) * bpart));
   A_OK(hipMalloc(&u->zero, 16));
   A_OK(hipMemsetAsync(u->zero, 0, 16, u->stream));
+  u->copy.reserve(sizeof(float) * std::max(n0 * (size_t)std::max(cin, cout), u->nparams));
   A_OK(hipMalloc(&u->gA, sizeof(u16) * big));
   A_OK(hipMalloc(&u->gB, sizeof(u16) * big));
   A_OK(hipMalloc(&u->gP, sizeof(u16) * big));
@@ -332,7 +335,7 @@ extern "C" long long sts_unet_param_count(const sts_unet *u) { return u ? (long 
 
 extern "C" int sts_unet_set_params(sts_unet *u, const float *host) {
   if (!u || !host) return ufail(STS_ERR_ARG, "null argument");
-  U_OK(hipMemcpyAsync(u->P, host, sizeof(float) * u->nparams, hipMemcpyHostToDevice, u->stream));
+  U_OK(u->copy.put(u->P, host, sizeof(float) * u->nparams, u->stream));
   int rc = pack_weights(u);
   if (rc) return rc;
   U_OK(hipStreamSynchronize(u->stream));
@@ -341,15 +344,13 @@ extern "C" int sts_unet_set_params(sts_unet *u, const float *host) {
 
 extern "C" int sts_unet_get_params(sts_unet *u, float *host) {
   if (!u || !host) return ufail(STS_ERR_ARG, "null argument");
-  U_OK(hipMemcpyAsync(host, u->P, sizeof(float) * u->nparams, hipMemcpyDeviceToHost, u->stream));
-  U_OK(hipStreamSynchronize(u->stream));
+  U_OK(u->copy.get(host, u->P, sizeof(float) * u->nparams, u->stream));
   return STS_OK;
 }
 
 extern "C" int sts_unet_get_grads(sts_unet *u, float *host) {
   if (!u || !host) return ufail(STS_ERR_ARG, "null argument");
-  U_OK(hipMemcpyAsync(host, u->G, sizeof(float) * u->nparams, hipMemcpyDeviceToHost, u->stream));
-  U_OK(hipStreamSynchronize(u->stream));
+  U_OK(u->copy.get(host, u->G, sizeof(float) * u->nparams, u->stream));
   return STS_OK;
 }
 
@@ -358,11 +359,10 @@ extern "C" int sts_unet_forward(sts_unet *u, int n, const float *x, float *y) {
   int rc = check_n(u, n);
   if (rc) return rc;
   const size_t np = u->npix(n, 0);
-  U_OK(hipMemcpyAsync(u->xin, x, sizeof(float) * np * u->cin, hipMemcpyHostToDevice, u->stream));
+  U_OK(u->copy.put(u->xin, x, sizeof(float) * np * u->cin, u->stream));
   U_OK(unet_to_bf16(u->xin, u->cin, u->Cx0, np, u->x, u->stream));
   if ((rc = forward_dev(u, n))) return rc;
-  U_OK(hipMemcpyAsync(y, u->y, sizeof(float) * np * u->cout, hipMemcpyDeviceToHost, u->stream));
-  U_OK(hipStreamSynchronize(u->stream));
+  U_OK(u->copy.get(y, u->y, sizeof(float) * np * u->cout, u->stream));
   return STS_OK;
 }
 
@@ -371,11 +371,10 @@ extern "C" int sts_unet_infer(sts_unet *u, int n, const float *x, float *y) {
   int rc = check_n(u, n);
   if (rc) return rc;
   const size_t np = u->npix(n, 0);
-  U_OK(hipMemcpyAsync(u->xin, x, sizeof(float) * np * u->cin, hipMemcpyHostToDevice, u->stream));
+  U_OK(u->copy.put(u->xin, x, sizeof(float) * np * u->cin, u->stream));
   U_OK(unet_to_bf16(u->xin, u->cin, u->Cx0, np, u->x, u->stream));
   if ((rc = forward_dev(u, n))) return rc;
-  U_OK(hipMemcpyAsync(y, u->y, sizeof(float) * np * u->cout, hipMemcpyDeviceToHost, u->stream));
-  U_OK(hipStreamSynchronize(u->stream));
+  U_OK(u->copy.get(y, u->y, sizeof(float) * np * u->cout, u->stream));
   return STS_OK;
 }
 
