@@ -1069,7 +1069,8 @@ struct CorrectIn {
   bool in, cu, cv;                    // cell in grid; u, v corrected
   bool mc, mw, ms;                    // fluid: cell, west, south
   R uf, vf, ups, vps, d12, d34, pc, pw, ps, Tc, Tw, Ts;
-  R hxi, hxw, hyj, hys, twu, twv;     // FLUX: mesh steps (cell, west; cell, south), wall temperatures
+  // FLUX: mesh steps (cell, west; cell, south), reciprocals of their sums (TileMesh), wall temperatures
+  R hxi, hxw, hyj, hys, rx, ry, twu, twv;
   __device__ __forceinline__ void load(const KGridT<R> &g, const KFieldsT<R> &fl, int i, int j, int do_correct) {
     in = i < g.Nx && j < g.Ny;
     if (!in) return;
@@ -1096,13 +1097,16 @@ struct CorrectIn {
     Tc = T[ij];
     Tw = T[i_1j];
     Ts = T[ij_1];
-    if (FLUX) {
-      hxi = g.hx[i];
-      hxw = g.hx[n.i_1];
-      hyj = g.hy[j];
-      hys = g.hy[j - 1 * (0 < j)];
-      load_walls(fl);
-    }
+    if (FLUX) load_flux(g, fl, i, j, n.i_1);
+  }
+  __device__ __forceinline__ void load_flux(const KGridT<R> &g, const KFieldsT<R> &fl, int i, int j, unsigned i_1) {
+    hxi = g.hx[i];
+    hxw = g.hx[i_1];
+    hyj = g.hy[j];
+    hys = g.hy[j - 1 * (0 < j)];
+    rx = g.hx[3 * g.Nx + i];
+    ry = g.hy[3 * g.Ny + j];
+    load_walls(fl);
   }
   // A wall temperature enters DTx (DTy) only where exactly one of the cell
   // and its west (south) neighbour is fluid: with both fluid its term is
@@ -1149,6 +1153,15 @@ struct CorrectIn {
     FLD(RHO_U)[ij] = ru;
     FLD(RHO_V)[ij] = rv;
     if (!FLUX) return;
+    // Waves without a wall: dtx's and dty's expressions with every mask 1 (the
+    // wall terms are + 0), the mesh's quotients from its reciprocals.
+    if (__all(mc && mw && ms)) {
+      FLD(FX)[ij] = hyj * ru * u;
+      FLD(FY)[ij] = hxi * rv * v;
+      FLD(DTX)[ij] = g.cT1 * quot2(hyj, R(0.5) * (hxi + hxw), R(2.0) * rx) * Hi(sw, sc, hxw, hxi);
+      FLD(DTY)[ij] = g.cT1 * quot2(hxi, R(0.5) * (hyj + hys), R(2.0) * ry) * Hi(ss, sc, hys, hyj);
+      return;
+    }
     FluxIn<R> f;
     f.in = true;
     f.ij = ij;
@@ -1172,25 +1185,21 @@ struct CorrectIn {
   }
 };
 
-// CORRECT_ROWS cells per thread, rows BY apart, all loads issued first.  Bound
-// by its memory traffic: with the fluxes it reads 8 arrays and writes 10 (107
-// MB at 1920x384: 20.0 us, 5.3 TB/s), where the correction and a flux pass of
-// its own took 15.7 + 11.8 us there and 5.5 + 4.4 us on 240x48 (now 7.0).
-constexpr int CORRECT_ROWS = 2;
-
+// One cell per thread.  Bound by its memory traffic on large grids: with the
+// fluxes it reads 8 arrays and writes 10 (107 MB at 1920x384: 19.3 us, 5.5 TB/s;
+// 3840x768: 81 us), by the chain of one cell on small ones: 240x48 4.9 us (6.9 with
+// two cells per thread and masks), 777x211 7.8 us (10.1), without the fluxes 4.7
+// and 7.1 us.
 template <typename R, bool FLUX>
 __global__ void __launch_bounds__(BX *BY) k_correct(KGridT<R> g, KFieldsT<R> fl, unsigned long long *red_u,
                                                     unsigned long long *red_v, int do_correct, Gate gate) {
   if (gated_out(gate)) return;
   unsigned long long r[2] = {0ull, 0ull};
   int i0, j0;
-  tile_origin<BX, BY * CORRECT_ROWS>(g.Nx, i0, j0);
-  CorrectIn<R, FLUX> c[CORRECT_ROWS];
-#pragma unroll
-  for (int q = 0; q < CORRECT_ROWS; q++)
-    c[q].load(g, fl, i0 + (int)threadIdx.x, j0 + (int)threadIdx.y + q * BY, do_correct);
-#pragma unroll
-  for (int q = 0; q < CORRECT_ROWS; q++) c[q].apply(g, fl, r);
+  tile_origin<BX, BY>(g.Nx, i0, j0);
+  CorrectIn<R, FLUX> c;
+  c.load(g, fl, i0 + (int)threadIdx.x, j0 + (int)threadIdx.y, do_correct);
+  c.apply(g, fl, r);
   if (do_correct) block_max_atomic<2, BX * BY>(r, MaxDst<2>{{red_u, red_v}, {}});
 }
 
@@ -1546,15 +1555,16 @@ __device__ __forceinline__ void edge_y(const KGridT<R> &g, R *a, int b0, int b1,
 }
 
 // The loop-2 test of iteration gate.k (S:4433-4437, Iter = k + 1 after the
-// increment), one wave: fold the slot copies of the six residual words,
+// increment), one wave (its last lane): fold the slot copies of the six residual words,
 // clear them, log the maxima, and end the loop by setting stop_at = k.  The
 // residuals stay in registers; the stagnation window's older log entries are
 // fetched alongside the slots.
 __device__ __forceinline__ void loop_test_wave(const Gate &gate, const LoopTest &lt) {
+  static_assert(NSLOT == 64, "one slot per lane");
   if (!lt.ctrl || threadIdx.x >= NSLOT) return;
   const bool stall = lt.stall_w > 0 && gate.k >= 2 * lt.stall_w;
   unsigned long long old[4] = {0ull, 0ull, 0ull, 0ull};
-  if (stall && threadIdx.x == 0) {
+  if (stall && threadIdx.x == NSLOT - 1) {
     const unsigned long long *lb = lt.log_k - 6 * lt.stall_w;
 #pragma unroll
     for (int q = 0; q < 4; q++) old[q] = lb[q];
@@ -1566,9 +1576,9 @@ __device__ __forceinline__ void loop_test_wave(const Gate &gate, const LoopTest 
 #pragma unroll
   for (int q = 0; q < 6; q++) {
     sl[q] = 0ull;
-    w[q] = wave_max(w[q]);
+    w[q] = wave_max_last(w[q]);
   }
-  if (threadIdx.x != 0) return;
+  if (threadIdx.x != NSLOT - 1) return;
 #pragma unroll
   for (int q = 0; q < 6; q++) lt.log_k[q] = w[q];
   double r[4];
@@ -1598,133 +1608,140 @@ __device__ __forceinline__ void loop_test_wave(const Gate &gate, const LoopTest 
   if (!cont) lt.ctrl->stop_at = gate.k;
 }
 
-constexpr int EDGE_GROUPS = 4;
+// The conditions of the two ends of a direction touch disjoint cells when the
+// box between them is not empty (b0 < b1): they run together, else one after
+// the other.
+template <typename R>
+__device__ __forceinline__ void edges_x(const KGridT<R> &g, R *a, int b0, int b1, bool lo, bool hi) {
+  if (!lo && !hi) return;
+  if (b0 < b1) edge_x(g, a, b0, b1, lo, hi);
+  else {
+    edge_x(g, a, b0, b1, lo, false);
+    __syncthreads();
+    edge_x(g, a, b0, b1, false, hi);
+  }
+  __syncthreads();
+}
+template <typename R>
+__device__ __forceinline__ void edges_y(const KGridT<R> &g, R *a, int b0, int b1, bool lo, bool hi) {
+  if (!lo && !hi) return;
+  if (b0 < b1) edge_y(g, a, b0, b1, lo, hi);
+  else {
+    edge_y(g, a, b0, b1, lo, false);
+    __syncthreads();
+    edge_y(g, a, b0, b1, false, hi);
+  }
+  __syncthreads();
+}
+
+// The conditions of u, v, temperature and pressure touch disjoint arrays (u and
+// v read rho and the face densities, which none of them writes; u reads v in one
+// kind), and the loop test reads only the residual words, so five workgroups run
+// them side by side: group 0 = u (after v where it reads v), 1 = temperature, 2 =
+// pressure and the probe, 3 = v, 4 = loop test.  Bound by the chain of a group's
+// phases, each a load, a store and a barrier: 240x48 4.3 -> 3.4 us, 1920x384 5.0
+// -> 4.1 us with u and v apart, the two ends of a direction together and no
+// barrier for a condition that is off.
+constexpr int EDGE_GROUPS = 5;
 
 template <typename R>
 __device__ void edges_block(const KGridT<R> &g, const KFieldsT<R> &fl, int parts, bool flux, double *probe,
                             const Gate &gate, const LoopTest &lt, int group) {
-  // The velocity, temperature and pressure conditions touch disjoint arrays
-  // (u, v read rho and the face densities, which none of them writes), and
-  // the loop test reads only the residual words, so four workgroups run them
-  // side by side: group 0 = velocities, 1 = temperature, 2 = pressure and the
-  // probe, 3 = loop test (group < 0: everything in one workgroup).
-  if (group == 3 || group < 0) loop_test_wave(gate, lt);
-  if (group == 3) return;
-  if (group == 1) parts &= STS_BC_TEMPERATURE;
-  if (group == 2) parts &= STS_BC_PRESSURE;
-  if (group == 0) parts &= STS_BC_VELOCITIES;
+  if (group == EDGE_GROUPS - 1) {
+    loop_test_wave(gate, lt);
+    return;
+  }
   // periodic about OX: the box-edge conditions are off (S:6795, S:7340, S:7655)
   if (g.px) parts &= ~(STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE);
-  if (group >= 0 && group != 2) probe = nullptr;
   const int Nx = g.Nx, Ny = g.Ny;
   const uint8_t *m = g.m;
   const unsigned bc = g.bc;
-  R *u = FLD(U), *v = FLD(V);
-  const R *rho = FLD(RHO), *rho_pr = FLD(RHO_PR), *rho_u = FLD(RHO_U), *rho_v = FLD(RHO_V);
   const R *hx = g.hx, *hy = g.hy;
-  if (parts & STS_BC_VELOCITIES) {
-    edge_x(g, v, g.Nx_v0, g.Nx_v1, bc & BC_DVDX_XB, false);
-    __syncthreads();
-    edge_x(g, v, g.Nx_v0, g.Nx_v1, false, bc & BC_DVDX_XE);
-    __syncthreads();
-    edge_y(g, v, g.Ny_v0, g.Ny_v1, bc & BC_DVDY_YB, false);
-    __syncthreads();
-    edge_y(g, v, g.Ny_v0, g.Ny_v1, false, bc & BC_DVDY_YE);
-    __syncthreads();
-    edge_x(g, u, g.Nx_u0, g.Nx_u1, bc & BC_DUDX_XB, false);
-    __syncthreads();
-    if (bc & BC_DURHODX_XB)
-      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-        int node = g.Nx_u0 - 1 + j * Nx;
-        if (m[node]) u[node] = (rho_u[node + 1] * u[node + 1]) / rho_u[node];
-      }
-    __syncthreads();
-    if (bc & BC_DRHODT_XB) {
-      const int i = g.Nx_u0 - 1;
-      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-        int node = i + j * Nx;
-        if (m[node] && j + 1 < Ny)
-          u[node] = ((rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
-                     + (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
-                     + rho_u[node + 1] * u[node + 1] * hy[j])
-                    / (rho_u[node] * hy[j]);
-      }
+  auto strip = [&](R *F, const R *rho_f, const R *vel, bool x, int c0, int c1, int r0, int r1) {
+    const int w = c1 - c0;
+    for (int t = threadIdx.x; t < w * (r1 - r0); t += EDGE_THREADS) {
+      const int dj = t / w, i = c0 + (t - dj * w), j = r0 + dj, k = i + j * Nx;
+      F[k] = (x ? hy[j] : hx[i]) * rho_f[k] * vel[k];
     }
-    __syncthreads();
-    edge_x(g, u, g.Nx_u0, g.Nx_u1, false, bc & BC_DUDX_XE);
-    __syncthreads();
-    if (bc & BC_DURHODX_XE)
-      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-        int node = g.Nx_u1 - 1 + j * Nx;
-        if (m[node]) u[node + 1] = (rho_u[node] * u[node]) / rho_u[node + 1];
-      }
-    __syncthreads();
-    if (bc & BC_DRHODT_XE) {
-      const int i = g.Nx_u1 - 1;
-      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-        int node = i + j * Nx;
-        if (m[node] && j + 1 < Ny)
-          u[node + 1] = (-(rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
-                         - (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
-                         + rho_u[node] * u[node] * hy[j])
-                        / (rho_u[node + 1] * hy[j]);
-      }
-    }
-    __syncthreads();
-    if (bc & BC_UMINMOUT_XE) {  // S:7031-7059 (serial build): the last row's rho_u
-      const R Min = rho_u[g.Nx_u0 + (Ny - 1) * Nx];
-      const R Mout = rho_u[g.Nx_u1 + (Ny - 1) * Nx];
-      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-        int node = g.Nx_u1 - 1 + j * Nx;
-        u[node + 1] = u[node] * Min / Mout;
-      }
-    }
-    __syncthreads();
-    edge_y(g, u, g.Ny_u0, g.Ny_u1, bc & BC_DUDY_YB, false);
-    __syncthreads();
-    edge_y(g, u, g.Ny_u0, g.Ny_u1, false, bc & BC_DUDY_YE);
-    __syncthreads();
-    if (flux) {  // the fluxes of the cells whose u, v the conditions above may have changed
-      auto strip = [&](R *F, const R *rho_f, const R *vel, bool x, int c0, int c1, int r0, int r1) {
-        const int w = c1 - c0;
-        for (int t = threadIdx.x; t < w * (r1 - r0); t += EDGE_THREADS) {
-          const int dj = t / w, i = c0 + (t - dj * w), j = r0 + dj, k = i + j * Nx;
-          F[k] = (x ? hy[j] : hx[i]) * rho_f[k] * vel[k];
-        }
-      };
-      R *Fx = FLD(FX), *Fy = FLD(FY);
-      if (bc & (BC_DUDX_XB | BC_DURHODX_XB | BC_DRHODT_XB)) strip(Fx, rho_u, u, true, 0, g.Nx_u0, 0, Ny);
-      if (bc & (BC_DUDX_XE | BC_DURHODX_XE | BC_DRHODT_XE | BC_UMINMOUT_XE))
-        strip(Fx, rho_u, u, true, g.Nx_u1, Nx, 0, Ny);
-      if (bc & BC_DUDY_YB) strip(Fx, rho_u, u, true, 0, Nx, 0, g.Ny_u0);
-      if (bc & BC_DUDY_YE) strip(Fx, rho_u, u, true, 0, Nx, g.Ny_u1, Ny);
+  };
+  const bool reads_v = bc & (BC_DRHODT_XB | BC_DRHODT_XE);
+  if ((parts & STS_BC_VELOCITIES) && group == (reads_v ? 0 : 3)) {
+    R *v = FLD(V);
+    edges_x(g, v, g.Nx_v0, g.Nx_v1, bc & BC_DVDX_XB, bc & BC_DVDX_XE);
+    edges_y(g, v, g.Ny_v0, g.Ny_v1, bc & BC_DVDY_YB, bc & BC_DVDY_YE);
+    if (flux) {  // the fluxes of the cells whose v the conditions above may have changed
+      R *Fy = FLD(FY);
+      const R *rho_v = FLD(RHO_V);
       if (bc & BC_DVDX_XB) strip(Fy, rho_v, v, false, 0, g.Nx_v0, 0, Ny);
       if (bc & BC_DVDX_XE) strip(Fy, rho_v, v, false, g.Nx_v1, Nx, 0, Ny);
       if (bc & BC_DVDY_YB) strip(Fy, rho_v, v, false, 0, Nx, 0, g.Ny_v0);
       if (bc & BC_DVDY_YE) strip(Fy, rho_v, v, false, 0, Nx, g.Ny_v1, Ny);
     }
   }
-  if (parts & STS_BC_TEMPERATURE) {
-    R *T = FLD(T);
-    edge_x(g, T, g.Nx_o0, g.Nx_o1, bc & BC_DTDX_XB, false);
-    __syncthreads();
-    edge_x(g, T, g.Nx_o0, g.Nx_o1, false, bc & BC_DTDX_XE);
-    __syncthreads();
-    edge_y(g, T, g.Ny_o0, g.Ny_o1, bc & BC_DTDY_YB, false);
-    __syncthreads();
-    edge_y(g, T, g.Ny_o0, g.Ny_o1, false, bc & BC_DTDY_YE);
-    __syncthreads();
+  if ((parts & STS_BC_VELOCITIES) && group == 0) {
+    R *u = FLD(U);
+    const R *v = FLD(V), *rho = FLD(RHO), *rho_pr = FLD(RHO_PR), *rho_u = FLD(RHO_U), *rho_v = FLD(RHO_V);
+    const bool apart = g.Nx_u0 < g.Nx_u1;  // (as edges_x)
+    for (int side = apart ? 2 : 0; side < (apart ? 3 : 2); side++) {  // 0 = XB, 1 = XE, 2 = both
+      const unsigned on = bc & ((side != 1 ? BC_DUDX_XB | BC_DURHODX_XB | BC_DRHODT_XB : 0u) |
+                                (side != 0 ? BC_DUDX_XE | BC_DURHODX_XE | BC_DRHODT_XE | BC_UMINMOUT_XE : 0u));
+      edges_x(g, u, g.Nx_u0, g.Nx_u1, on & BC_DUDX_XB, on & BC_DUDX_XE);
+      if (on & (BC_DURHODX_XB | BC_DURHODX_XE)) {
+        for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
+          int node = g.Nx_u0 - 1 + j * Nx;
+          if ((on & BC_DURHODX_XB) && m[node]) u[node] = (rho_u[node + 1] * u[node + 1]) / rho_u[node];
+          node = g.Nx_u1 - 1 + j * Nx;
+          if ((on & BC_DURHODX_XE) && m[node]) u[node + 1] = (rho_u[node] * u[node]) / rho_u[node + 1];
+        }
+        __syncthreads();
+      }
+      if (on & (BC_DRHODT_XB | BC_DRHODT_XE)) {
+        for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
+          int i = g.Nx_u0 - 1, node = i + j * Nx;
+          if ((on & BC_DRHODT_XB) && m[node] && j + 1 < Ny)
+            u[node] = ((rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
+                       + (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
+                       + rho_u[node + 1] * u[node + 1] * hy[j])
+                      / (rho_u[node] * hy[j]);
+          i = g.Nx_u1 - 1, node = i + j * Nx;
+          if ((on & BC_DRHODT_XE) && m[node] && j + 1 < Ny)
+            u[node + 1] = (-(rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
+                           - (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
+                           + rho_u[node] * u[node] * hy[j])
+                          / (rho_u[node + 1] * hy[j]);
+        }
+        __syncthreads();
+      }
+      if (on & BC_UMINMOUT_XE) {  // S:7031-7059 (serial build): the last row's rho_u
+        const R Min = rho_u[g.Nx_u0 + (Ny - 1) * Nx];
+        const R Mout = rho_u[g.Nx_u1 + (Ny - 1) * Nx];
+        for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
+          int node = g.Nx_u1 - 1 + j * Nx;
+          u[node + 1] = u[node] * Min / Mout;
+        }
+        __syncthreads();
+      }
+    }
+    edges_y(g, u, g.Ny_u0, g.Ny_u1, bc & BC_DUDY_YB, bc & BC_DUDY_YE);
+    if (flux) {  // likewise, u
+      R *Fx = FLD(FX);
+      if (bc & (BC_DUDX_XB | BC_DURHODX_XB | BC_DRHODT_XB)) strip(Fx, rho_u, u, true, 0, g.Nx_u0, 0, Ny);
+      if (bc & (BC_DUDX_XE | BC_DURHODX_XE | BC_DRHODT_XE | BC_UMINMOUT_XE))
+        strip(Fx, rho_u, u, true, g.Nx_u1, Nx, 0, Ny);
+      if (bc & BC_DUDY_YB) strip(Fx, rho_u, u, true, 0, Nx, 0, g.Ny_u0);
+      if (bc & BC_DUDY_YE) strip(Fx, rho_u, u, true, 0, Nx, g.Ny_u1, Ny);
+    }
   }
+  if ((parts & STS_BC_TEMPERATURE) && group == 1) {
+    R *T = FLD(T);
+    edges_x(g, T, g.Nx_o0, g.Nx_o1, bc & BC_DTDX_XB, bc & BC_DTDX_XE);
+    edges_y(g, T, g.Ny_o0, g.Ny_o1, bc & BC_DTDY_YB, bc & BC_DTDY_YE);
+  }
+  if (group != 2) return;
   if (parts & STS_BC_PRESSURE) {
     R *p = FLD(P);
-    edge_x(g, p, g.Nx_o0, g.Nx_o1, bc & BC_DPDX_XB, false);
-    __syncthreads();
-    edge_x(g, p, g.Nx_o0, g.Nx_o1, false, bc & BC_DPDX_XE);
-    __syncthreads();
-    edge_y(g, p, g.Ny_o0, g.Ny_o1, bc & BC_DPDY_YB, false);
-    __syncthreads();
-    edge_y(g, p, g.Ny_o0, g.Ny_o1, false, bc & BC_DPDY_YE);
-    __syncthreads();
+    edges_x(g, p, g.Nx_o0, g.Nx_o1, bc & BC_DPDX_XB, bc & BC_DPDX_XE);
+    edges_y(g, p, g.Ny_o0, g.Ny_o1, bc & BC_DPDY_YB, bc & BC_DPDY_YE);
   }
   if (probe && threadIdx.x == 0) {
     // S:7512-7513: the cell p_BC_xb is read from (not touched by the edge copies)
@@ -2293,11 +2310,7 @@ __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R
   ci.Tw = (R)sT[ty + 1][tx];
   ci.ps = (R)sp[ty][tx + 1];
   ci.Ts = (R)sT[ty][tx + 1];
-  ci.hxi = g.hx[i];
-  ci.hxw = g.hx[nb.i_1];
-  ci.hyj = g.hy[j];
-  ci.hys = g.hy[j - 1 * (0 < j)];
-  ci.load_walls(fl);
+  ci.load_flux(g, fl, i, j, nb.i_1);
   double d[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
@@ -2794,9 +2807,9 @@ hipError_t launch_sweep2(const KGridT<R> &g, const KFieldsT<R> &f, const R *Po, 
 template <typename R>
 hipError_t launch_correct(const KGridT<R> &g, const KFieldsT<R> &f, unsigned long long *ru, unsigned long long *rv,
                           int do_correct, bool flux, hipStream_t s, Gate gate) {
-  const dim3 gr = grid_tiles<BX, BY * CORRECT_ROWS>(g);
-  if (flux) hipLaunchKernelGGL((k_correct<R, true>), gr, dim3(BX, BY), 0, s, g, f, ru, rv, do_correct, gate);
-  else hipLaunchKernelGGL((k_correct<R, false>), gr, dim3(BX, BY), 0, s, g, f, ru, rv, do_correct, gate);
+  const dim3 gr = grid_tiles<BX, BY>(g), th(BX, BY);
+  if (flux) hipLaunchKernelGGL((k_correct<R, true>), gr, th, 0, s, g, f, ru, rv, do_correct, gate);
+  else hipLaunchKernelGGL((k_correct<R, false>), gr, th, 0, s, g, f, ru, rv, do_correct, gate);
   return hipGetLastError();
 }
 template <typename R>
