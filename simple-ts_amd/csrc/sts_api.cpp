@@ -1310,17 +1310,24 @@ static int copy_start(sts_ctx *c, hipStream_t s, bool back = false) {
   return STS_OK;
 }
 
-// After the prologue: loop 2 starts from the polynomial of degree `order`
-// (capped by the stored steps) through x^n and the previous converged steps
-// for u, v, p, T, and every field derived from them is rebuilt the way the
-// end of an outer iteration builds it.  The history then advances a step.
-static int extrapolate_start(sts_ctx *c, int order, hipStream_t s = nullptr, bool store_only = false,
-                             int degree_cap = MAX_EXTRAP, int *used = nullptr) {
-  if (!s) s = c->stream;
-  if (used) *used = 0;
+// The start of a step (S:3233-3239 and, with order > 0, the polynomial of degree
+// `order`, capped by the stored steps and degree_cap, through x^n and the previous
+// converged steps for u, v, p, T; store_only: stored, not used), and the
+// history's advance by it.
+static int plan_start(sts_ctx *c, int order, bool store_only, int degree_cap, BeginArgs *out) {
+  BeginArgs &a = *out;
+  a = BeginArgs{};
+  a.Nx = c->Nx;
+  a.Ny = c->Ny;
+  a.Nx_u0 = c->g.Nx_u0;
+  const int x[5] = {STS_U, STS_V, STS_P, STS_T, STS_RHO}, pr[5] = {STS_U_PR, STS_V_PR, STS_P_PR, STS_T_PR, STS_RHO_PR};
+  for (int q = 0; q < 5; q++) {
+    a.x[q] = c->f[x[q]];
+    a.pr[q] = c->f[pr[q]];
+  }
   if (order <= 0) {
     c->n_hist = 0;
-    return copy_start(c, s);
+    return STS_OK;
   }
   if (order > MAX_EXTRAP) return fail(STS_ERR_ARG, "extrapolation degree must be 0..5");
   const size_t bytes = sizeof(double) * (size_t)c->Na;
@@ -1329,20 +1336,29 @@ static int extrapolate_start(sts_ctx *c, int order, hipStream_t s = nullptr, boo
       for (double *&q : lv) HIP_OK(hipMalloc(&q, bytes));
   // `order` past steps are kept: x^n goes to a free level, or over the oldest
   // one, and that level becomes level 0 (the rest move down by renaming)
-  const int keep = std::min(c->n_hist, order), use = store_only ? 0 : std::min(keep, degree_cap);
-  const int slot = keep < order ? keep : order - 1;
-  const KFields kf = c->fields();
-  HIP_OK(launch_extrapolate(c->g, kf, c->hist, use, slot, s));
-  double *top[4];
-  for (int q = 0; q < 4; q++) top[q] = c->hist.f[slot][q];
+  const int keep = std::min(c->n_hist, order), slot = keep < order ? keep : order - 1;
+  a.order = store_only ? 0 : std::min(keep, degree_cap);
+  a.hist = c->hist;
+  for (int q = 0; q < 4; q++) a.to[q] = c->hist.f[slot][q];
   for (int h = slot; h > 0; h--)
     for (int q = 0; q < 4; q++) c->hist.f[h][q] = c->hist.f[h - 1][q];
-  for (int q = 0; q < 4; q++) c->hist.f[0][q] = top[q];
+  for (int q = 0; q < 4; q++) c->hist.f[0][q] = a.to[q];
   c->n_hist = std::min(keep + 1, order);
-  if (used) *used = use;
+  return STS_OK;
+}
+
+// The same, run: every field derived from a predicted start is rebuilt the way
+// the end of an outer iteration builds it.  *used: its degree.
+static int begin_step(sts_ctx *c, int order, bool store_only = false, int degree_cap = MAX_EXTRAP,
+                      int *used = nullptr) {
+  BeginArgs a;
   int rc;
-  if (use > 0 && (rc = rebuild_derived(c, s))) return rc;
-  return copy_start(c, s);
+  if (used) *used = 0;
+  if ((rc = plan_start(c, order, store_only, degree_cap, &a))) return rc;
+  HIP_OK(launch_begin(a, c->stream));
+  if (used) *used = a.order;
+  if (a.order > 0 && (rc = rebuild_derived(c, c->stream))) return rc;
+  return copy_start(c, c->stream);
 }
 
 // The first sweep's residual max(max|dp|/tol_p, max|dT|/tol_T) from the
@@ -1505,11 +1521,10 @@ extern "C" int sts_time_step_mixed(sts_ctx *c, const sts_loop_control *lc, const
   int rc;
   if ((rc = check_mixed(c, lc, mc))) return rc;
   if ((rc = ensure_loop_buffers(c, lc->N_I + mc->N_I32))) return rc;
-  if ((rc = sts_save_previous(c))) return rc;
   int n32 = 0, n64 = 0;
   if (mc->guard <= 0 || mc->extrapolate <= 0) {
     int used = 0;
-    if ((rc = extrapolate_start(c, mc->extrapolate, nullptr, false, MAX_EXTRAP, &used))) return rc;
+    if ((rc = begin_step(c, mc->extrapolate, false, MAX_EXTRAP, &used))) return rc;
     if (used > 0 && c->corr_net && (rc = corrector_refine(c, lc))) return rc;
     rc = run_phases(c, lc, mc, &n32, &n64);
     if (!rc && used > 0) corrector_outcome(c, n32 + n64, false);
@@ -1520,7 +1535,7 @@ extern "C" int sts_time_step_mixed(sts_ctx *c, const sts_loop_control *lc, const
     if (c->pred_degree < 0 || c->pred_degree > mc->extrapolate) c->pred_degree = mc->extrapolate;
     const bool predict = c->n_hist > 0 && c->plain_mean > 0.0 && c->pred_pause == 0;
     int used = 0;
-    if ((rc = extrapolate_start(c, mc->extrapolate, nullptr, !predict, c->pred_degree, &used))) return rc;
+    if ((rc = begin_step(c, mc->extrapolate, !predict, c->pred_degree, &used))) return rc;
     if (used > 0 && c->corr_net && (rc = corrector_refine(c, lc))) return rc;
     bool plain = !predict;
     if (predict) {
@@ -1670,8 +1685,7 @@ extern "C" int sts_time_step_ws(sts_ctx *c, sts_unet *net, const sts_unet_norm *
     HIP_OK(hipMalloc(&c->p_ws, sizeof(double) * (size_t)c->Na));
     HIP_OK(hipMalloc(&c->T_ws, sizeof(double) * (size_t)c->Na));
   }
-  if ((rc = sts_save_previous(c))) return rc;
-  if ((rc = extrapolate_start(c, mc ? mc->extrapolate : 0))) return rc;
+  if ((rc = begin_step(c, mc ? mc->extrapolate : 0))) return rc;
   StsView v;
   sts_internal_view(c, &v);
   if ((rc = sts_internal_unet_predict(net, v, nrm, c->p_ws, c->T_ws))) return rc;
@@ -1709,6 +1723,7 @@ struct sts_batch {
   std::vector<sts_ctx *> cs;
   hipStream_t stream = nullptr;
   BatchCase<double> *C64 = nullptr;
+  BeginArgs *begin = nullptr;
   BatchCase<float> *C32 = nullptr;
   LoopCtrl *ctrl = nullptr, *h_ctrl = nullptr;
   unsigned long long *lred = nullptr, *log = nullptr;
@@ -1731,7 +1746,7 @@ struct sts_batch {
 extern "C" int sts_batch_destroy(sts_batch *b) {
   if (!b) return STS_OK;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
-  for (void *p : {(void *)b->C64, (void *)b->C32, (void *)b->ctrl, (void *)b->lred, (void *)b->log}) (void)hipFree(p);
+  for (void *p : {(void *)b->C64, (void *)b->begin, (void *)b->C32, (void *)b->ctrl, (void *)b->lred, (void *)b->log}) (void)hipFree(p);
   if (b->h_ctrl) (void)hipHostFree(b->h_ctrl);
   for (int v = 0; v < NVARIANT; v++) {
     (void)hipFree(b->cell_t[v]);
@@ -1847,6 +1862,7 @@ extern "C" int sts_batch_create(sts_ctx *const *ctxs, int n, sts_batch **out) {
   } while (0)
   B_OK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
   B_OK(hipMalloc(&b->C64, sizeof(BatchCase<double>) * n));
+  B_OK(hipMalloc(&b->begin, sizeof(BeginArgs) * n));
   B_OK(hipMalloc(&b->C32, sizeof(BatchCase<float>) * n));
   B_OK(hipMalloc(&b->ctrl, sizeof(LoopCtrl) * n));
   B_OK(hipHostMalloc(&b->h_ctrl, sizeof(LoopCtrl) * n, hipHostMallocDefault));
@@ -2049,15 +2065,12 @@ extern "C" int sts_batch_time_step(sts_batch *b, const sts_loop_control *lc, con
     b->log_cap = cap;
   }
   hipStream_t s = b->stream;
-  for (sts_ctx *c : b->cs) {  // prologue S:3233-3239
-    const double *src[5] = {c->f[STS_P], c->f[STS_U], c->f[STS_V], c->f[STS_T], c->f[STS_RHO]};
-    double *dst[5] = {c->f[STS_P_PR], c->f[STS_U_PR], c->f[STS_V_PR], c->f[STS_T_PR], c->f[STS_RHO_PR]};
-    HIP_OK(launch_copy5(src, dst, c->Na, s));
-  }
   // predicted starts; with a guard, per case: a predicted step that needed
   // more outer iterations than the case's recent steps from x^n pauses its
   // prediction for 1, 2, 4, ... steps (no restart inside shared launches)
-  std::vector<char> predicted(n, 0);
+  std::vector<char> predicted(n, 0), from_xn(n, 1);
+  std::vector<BeginArgs> begin(n);
+  bool any = false;
   for (int i = 0; i < n; i++) {
     sts_ctx *c = b->cs[i];
     const int q = mc ? mc->extrapolate : 0;
@@ -2067,7 +2080,27 @@ extern "C" int sts_batch_time_step(sts_batch *b, const sts_loop_control *lc, con
       if (!pred && c->pred_pause > 0) c->pred_pause--;
     }
     predicted[i] = pred && c->n_hist > 0;
-    if ((rc = extrapolate_start(c, q, s, !pred))) return rc;
+    if ((rc = plan_start(c, q, !pred, MAX_EXTRAP, &begin[i]))) return rc;
+    if (begin[i].order > 0) {
+      from_xn[i] = 0;
+      any = true;
+    }
+  }
+  // the starts of all cases at once, and of the predicted ones the derived
+  // fields (rebuild_derived)
+  HIP_OK(hipMemcpyAsync(b->begin, begin.data(), sizeof(BeginArgs) * n, hipMemcpyHostToDevice, s));
+  const int cv = b->cell_v;
+  HIP_OK(launch_batch_begin(cv, b->begin, b->cell_t[cv], b->n_cell[cv], s));
+  if (any) {
+    if ((rc = upload_cases<double>(b, b->C64, 1, 0, 0, 0, 0, 0.0, 0, false, &from_xn))) return rc;
+    HIP_OK(launch_batch<double>(BK_DERIVE, cv, b->C64, n, b->cell_t[cv], b->n_cell[cv], 0, 0, 0, 0, s));
+    HIP_OK(launch_batch<double>(BK_WALL_OPS, 0, b->C64, n, b->wall_t, b->n_wall, -1, 0, 0, 0, s));
+    HIP_OK(launch_batch<double>(BK_EDGES, 0, b->C64, n, nullptr, 0, -1, 0,
+                                STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, 0, s));
+  }
+  for (int i = 0; i < n; i++) {
+    if (!from_xn[i]) b->cs[i]->diff_inline_ok = b->cs[i]->diff_stale = true;
+    if ((rc = copy_start(b->cs[i], s))) return rc;
   }
   std::vector<int> n32(n, 0), n64(n, 0);
   // cases the FP32 gate sends straight to FP64 sit the FP32 phase out

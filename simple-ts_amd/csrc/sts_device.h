@@ -170,6 +170,14 @@ constexpr int MAX_EXTRAP = 5;
 struct ExtrapHist {
   double *f[MAX_EXTRAP][4];  // [h][u, v, p, T]
 };
+// The start of a time step (begin_cell).
+struct BeginArgs {
+  int Nx, Ny, Nx_u0;
+  int order;             // degree of the predicted start (0: from x^n)
+  double *x[5], *pr[5];  // u, v, p, T, rho: the state, the previous step's fields
+  double *to[4];         // the history's level that takes x^n (null: none)
+  ExtrapHist hist;
+};
 
 // Anderson acceleration of loop 2 (Walker and Ni, SIAM J. Numer. Anal. 49,
 // 2011), in the difference form: the state is (u, v, p, T) of every cell, an

@@ -1870,32 +1870,39 @@ __device__ __forceinline__ double extrap(int order, const double (&x)[MAX_EXTRAP
   return s;
 }
 
-// Reads x^n and hist[0 .. order-1]; stores x^n into hist[slot] (the host then
-// rotates the level pointers, so no level is copied).
-__global__ void __launch_bounds__(BX *BY) k_extrapolate(KGrid g, KFields fl, ExtrapHist hist, int order, int slot) {
-  const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
-  if (i >= g.Nx || j >= g.Ny) return;
-  const unsigned k = (unsigned)i + (unsigned)j * (unsigned)g.Nx;
-  const int src[4] = {STS_U_PR, STS_V_PR, STS_P_PR, STS_T_PR}, dst[4] = {STS_U, STS_V, STS_P, STS_T};
+// One cell of a step's start: x^n (u, v, p, T, rho) into the previous-step
+// fields and u, v, p, T into the history's level `to` (the host then rotates
+// the level pointers, so no level is copied); with order > 0 the state becomes
+// the polynomial through x^n and hist[0 .. order-1].  30 arrays at degree 3: 31 us
+// at 1920x384, 36 in two passes with x^n read twice.
+__device__ __forceinline__ void begin_cell(const BeginArgs &a, int i, unsigned k) {
   // the inflow columns i < Nx_u0 hold the given velocity, which no kernel of
   // loop 2 rewrites and which the driver advances in time itself
   // (BoundaryConditions_function_of_time, S:8102-8144): u keeps x^n there
-  const bool given_u = i < g.Nx_u0;
+  const bool given_u = i < a.Nx_u0;
+  a.pr[4][k] = a.x[4][k];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     double x[MAX_EXTRAP + 1];
-    x[0] = fl.f[src[q]][k];
+    x[0] = a.x[q][k];
 #pragma unroll
-    for (int h = 0; h < MAX_EXTRAP; h++) x[h + 1] = (h < order) ? hist.f[h][q][k] : 0.0;
-    if (order > 0 && !(q == 0 && given_u)) {
+    for (int h = 0; h < MAX_EXTRAP; h++) x[h + 1] = (h < a.order) ? a.hist.f[h][q][k] : 0.0;
+    if (a.order > 0 && !(q == 0 && given_u)) {
       // a guess that is not finite, or a pressure or temperature that is not
       // positive, keeps the previous step's value in that cell
-      const double e = extrap(order, x);
+      const double e = extrap(a.order, x);
       const bool ok = isfinite(e) && (q < 2 || e > 0.0 || x[0] <= 0.0);
-      fl.f[dst[q]][k] = ok ? e : x[0];
+      if (ok) a.x[q][k] = e;
     }
-    hist.f[slot][q][k] = x[0];
+    a.pr[q][k] = x[0];
+    if (a.to[q]) a.to[q][k] = x[0];
   }
+}
+
+__global__ void __launch_bounds__(BX *BY) k_begin(BeginArgs a) {
+  const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
+  if (i >= a.Nx || j >= a.Ny) return;
+  begin_cell(a, i, (unsigned)i + (unsigned)j * (unsigned)a.Nx);
 }
 
 // ---------------------------------------------------------------------------
@@ -2649,7 +2656,7 @@ __global__ void __launch_bounds__(WALL_OPS_PER_TILE) kb_wall_ops(const BatchCase
                                                                  int par) {
   const BatchTile t = T[blockIdx.x];
   const BatchCase<R> &c = C[t.c];
-  if (gated_out(Gate{in_memory(c.ctrl), k})) return;
+  if (k < 0 ? c.skip != 0 : gated_out(Gate{in_memory(c.ctrl), k})) return;  // k < 0: after kb_derive
   const int q = t.x * WALL_OPS_PER_TILE + (int)threadIdx.x;
   if (q >= c.nwops) return;
   apply_wall_op<true>(grid_of(c), fields_at(c, par), in_memory(c.wops)[q]);
@@ -2735,14 +2742,48 @@ template <typename R>
 __global__ void __launch_bounds__(EDGE_THREADS) kb_edges(const BatchCase<R> *C, int k, int par, int parts) {
   const BatchCase<R> &c = C[blockIdx.x / EDGE_GROUPS];
   const Gate gate{c.ctrl, k};
-  if (gated_out(gate)) return;
+  if (k < 0 ? c.skip != 0 : gated_out(gate)) return;  // k < 0: after kb_derive
   const KFieldsT<R> f = fields_at(c, par);
-  const LoopTest lt{in_memory(c.ctrl), in_memory(c.lred), in_memory(c.log) + 6 * (size_t)k, c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w,
+  const LoopTest lt{in_memory(c.ctrl), in_memory(c.lred), in_memory(c.log) + 6 * (size_t)max(k, 0), c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w,
                     c.stall_ratio};
-  edges_block(grid_of(c), f, parts, true, in_memory(c.probe), gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
+  edges_block(grid_of(c), f, parts, true, k < 0 ? nullptr : in_memory(c.probe), gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
 }
 
 // Opens every case's loop 2: control, log (6 N_I words), slotted words.
+// The step's start of every case, and the fields derived from it of those that
+// do not skip (tiles of the cell variant in use).
+template <int TX, int TY>
+__global__ void __launch_bounds__(TX *TY) kb_begin(const BeginArgs *A, const BatchTile *T) {
+  const BatchTile t = T[blockIdx.x];
+  BeginArgs a = A[t.c];
+#pragma unroll
+  for (int q = 0; q < 5; q++) {
+    a.x[q] = in_memory(a.x[q]);
+    a.pr[q] = in_memory(a.pr[q]);
+    if (q < 4) a.to[q] = in_memory(a.to[q]);
+  }
+#pragma unroll
+  for (int h = 0; h < MAX_EXTRAP; h++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) a.hist.f[h][q] = in_memory(a.hist.f[h][q]);
+  const int i = t.x * TX + (int)threadIdx.x % TX, j = t.y * TY + (int)threadIdx.x / TX;
+  if (i >= a.Nx || j >= a.Ny) return;
+  begin_cell(a, i, (unsigned)i + (unsigned)j * (unsigned)a.Nx);
+}
+
+template <typename R, int TX, int TY>
+__global__ void __launch_bounds__(TX *TY) kb_derive(const BatchCase<R> *C, const BatchTile *T) {
+  const BatchTile t = T[blockIdx.x];
+  const BatchCase<R> &c = C[t.c];
+  if (c.skip) return;
+  unsigned long long r[2] = {0ull, 0ull};
+  const KFieldsT<R> f = fields_at(c, 0);
+  const KGridT<R> g = grid_of(c);
+  CorrectIn<R, true> x;
+  x.load(g, f, t.x * TX + (int)threadIdx.x % TX, t.y * TY + (int)threadIdx.x / TX, 0);
+  x.apply(g, f, r);
+}
+
 template <typename R>
 __global__ void __launch_bounds__(256) kb_loop_open(const BatchCase<R> *C) {
   const BatchCase<R> &c = C[blockIdx.x];
@@ -2888,9 +2929,8 @@ hipError_t launch_copy5(const double *const *src, double *const *dst, int n, hip
                      dst[3], dst[4], n);
   return hipGetLastError();
 }
-hipError_t launch_extrapolate(const KGrid &g, const KFields &f, const ExtrapHist &hist, int order, int slot,
-                              hipStream_t s) {
-  hipLaunchKernelGGL(k_extrapolate, grid2d(g), dim3(BX, BY), 0, s, g, f, hist, order, slot);
+hipError_t launch_begin(const BeginArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_begin, dim3((a.Nx + BX - 1) / BX, (a.Ny + BY - 1) / BY), dim3(BX, BY), 0, s, a);
   return hipGetLastError();
 }
 int aa_store_blocks(int Na) { return (Na + AA_THREADS * AA_STORE_CELLS - 1) / (AA_THREADS * AA_STORE_CELLS); }
@@ -3045,6 +3085,17 @@ hipError_t launch_batch_aa(int kernel, int variant, const BatchCase<double> *C, 
   return hipGetLastError();
 }
 
+hipError_t launch_batch_begin(int variant, const BeginArgs *A, const BatchTile *T, int ntiles, hipStream_t s) {
+  const dim3 gr(ntiles);
+  switch (variant) {
+    case 0: hipLaunchKernelGGL((kb_begin<64, 4>), gr, dim3(256), 0, s, A, T); break;
+    case 1: hipLaunchKernelGGL((kb_begin<64, 8>), gr, dim3(512), 0, s, A, T); break;
+    case 2: hipLaunchKernelGGL((kb_begin<128, 2>), gr, dim3(256), 0, s, A, T); break;
+    default: hipLaunchKernelGGL((kb_begin<32, 8>), gr, dim3(256), 0, s, A, T); break;
+  }
+  return hipGetLastError();
+}
+
 template <typename R>
 hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncases, const BatchTile *T, int ntiles,
                         int k, int par, int a, int b, hipStream_t s) {
@@ -3054,6 +3105,7 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
     case BK_ASSEMBLE_ARR: CELL_SWITCH(variant, kb_assemble_arr, C, T, k, par); break;
     case BK_SWEEP: CELL_SWITCH(variant, kb_sweep, C, T, k, par, a, b); break;
     case BK_CORRECT: CELL_SWITCH(variant, kb_correct, C, T, k, par); break;
+    case BK_DERIVE: CELL_SWITCH(variant, kb_derive, C, T); break;
     case BK_WALL_OPS:
       if (ntiles > 0)
         hipLaunchKernelGGL(kb_wall_ops<R>, dim3(ntiles), dim3(WALL_OPS_PER_TILE), 0, s, C, T, k, par);

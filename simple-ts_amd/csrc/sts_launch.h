@@ -51,10 +51,9 @@ hipError_t launch_apply_bodies(const KGrid &g, const KFields &f, hipStream_t s);
 hipError_t launch_jump_overwrite(const KGrid &g, const KFields &f, hipStream_t s);
 hipError_t launch_copy5(const double *const *src, double *const *dst, int n, hipStream_t s);
 hipError_t launch_set_inflow(const KGrid &g, const KFields &f, double u_in, hipStream_t s);
-// u, v, p, T extrapolated from x^n (the *_PR fields) and hist[h] = x^(n-1-h)
-// (h < order); x^n is stored into hist[slot]; order 0 only stores.
-hipError_t launch_extrapolate(const KGrid &g, const KFields &f, const ExtrapHist &hist, int order, int slot,
-                              hipStream_t s);
+// The start of a time step (BeginArgs): the previous step's fields, the history,
+// the predicted start from hist[h] = x^(n-1-h) (h < order).
+hipError_t launch_begin(const BeginArgs &a, hipStream_t s);
 // Anderson acceleration of loop 2.  launch_aa_begin at the loop start;
 // after an outer iteration's edge conditions, launch_aa_store (its
 // differences and their partial dot products), then, when sel.n > 0,
@@ -100,7 +99,8 @@ enum {
   BK_EDGES,
   BK_LOOP_OPEN,
   BK_WALL_OPS,
-  BK_ASSEMBLE_ARR
+  BK_ASSEMBLE_ARR,
+  BK_DERIVE
 };
 // BK_WALL_OPS: tile (c, x) = planned wall writes [x W, x W + W) of case c,
 // W = WALL_OPS_PER_TILE.
@@ -119,5 +119,9 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
 // partial slots.
 enum { BKA_BEGIN, BKA_STORE, BKA_SOLVE, BKA_MIX };
 int aa_case_tiles(int Nx, int Ny, int variant);
+// Starts of a step of all cases (A: one entry per case; cell tiles of
+// `variant`).  Then, for the cases of C that do not skip, BK_DERIVE and, with k =
+// -1, BK_WALL_OPS and BK_EDGES.
+hipError_t launch_batch_begin(int variant, const BeginArgs *A, const BatchTile *T, int ntiles, hipStream_t s);
 hipError_t launch_batch_aa(int kernel, int variant, const BatchCase<double> *C, int ncases, const BatchTile *T,
                            int ntiles, int k, int par, const AABatchSel &bs, hipStream_t s);
