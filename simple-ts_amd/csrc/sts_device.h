@@ -97,7 +97,12 @@ struct LoopTest {
   double tol_uv, tol_p, tol_T;
   int stall_w;         // > 0: also stop when the residuals stagnate (see k_edges)
   double stall_ratio;
+  // pinned host word (null: none) that the test of iteration k >= host_from, or
+  // of the last one, sets to k + 1 with LOOP_STOPPED and LOOP_NONFINITE
+  unsigned long long *host;
+  int host_from;
 };
+constexpr unsigned long long LOOP_STOPPED = 1ull << 32, LOOP_NONFINITE = 1ull << 33;
 
 // Clamped neighbour indices of cell (i, j).
 // Neighbour indices of cell (i, j): clamped at the grid edge (ij_function,

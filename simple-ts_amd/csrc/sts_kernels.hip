@@ -1606,6 +1606,10 @@ __device__ __forceinline__ void loop_test_wave(const Gate &gate, const LoopTest 
     cont = false;
   }
   if (!cont) lt.ctrl->stop_at = gate.k;
+  if (lt.host && (!cont || gate.k >= lt.host_from)) {
+    const unsigned long long w = (unsigned long long)(gate.k + 1) | (cont ? 0ull : LOOP_STOPPED) | (fin ? 0ull : LOOP_NONFINITE);
+    __hip_atomic_store(lt.host, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // The conditions of the two ends of a direction touch disjoint cells when the
@@ -2745,7 +2749,7 @@ __global__ void __launch_bounds__(EDGE_THREADS) kb_edges(const BatchCase<R> *C, 
   if (k < 0 ? c.skip != 0 : gated_out(gate)) return;  // k < 0: after kb_derive
   const KFieldsT<R> f = fields_at(c, par);
   const LoopTest lt{in_memory(c.ctrl), in_memory(c.lred), in_memory(c.log) + 6 * (size_t)max(k, 0), c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w,
-                    c.stall_ratio};
+                    c.stall_ratio, nullptr, 0};
   edges_block(grid_of(c), f, parts, true, k < 0 ? nullptr : in_memory(c.probe), gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
 }
 
