@@ -2121,8 +2121,8 @@ __global__ void __launch_bounds__(AA_THREADS) k_aa_store(AAFieldsT<R> s, AABuf a
 // matrix in LDS and two more barriers took 0.7 us longer of the mix's 13.0 on
 // 301x95).
 template <int NM, int NT>
-__device__ __forceinline__ void aa_solve_group(const AABuf &ab, const AASel &sel, double (&gam)[NM], bool leader) {
-  const int n = sel.n;
+__device__ __forceinline__ void aa_solve_group(const AABuf &ab, int n, const int (&slot)[MAX_AA], double (&gam)[NM],
+                                               bool leader) {
   double acc[2 * NM];
 #pragma unroll
   for (int j = 0; j < 2 * NM; j++) acc[j] = 0.0;
@@ -2145,20 +2145,20 @@ __device__ __forceinline__ void aa_solve_group(const AABuf &ab, const AASel &sel
       for (int j = 0; j < 2 * NM; j++) acc[j] += v[r][j];
   }
   double g00 = 0.0;  // two differences: the stored part of the Gram matrix
-  if (NM == 2 && n == 2) g00 = ab.gram[sel.slot[0] * MAX_AA + sel.slot[0]];
+  if (NM == 2 && n == 2) g00 = ab.gram[slot[0] * MAX_AA + slot[0]];
   __shared__ double A[NM][NM + 1];
   if (NM > 2 && (int)threadIdx.x < NM * NM) {
     const int a = (int)threadIdx.x / NM, b = (int)threadIdx.x % NM;
-    if (a < n - 1 && b < n - 1) A[a][b] = ab.gram[sel.slot[a] * MAX_AA + sel.slot[b]];
+    if (a < n - 1 && b < n - 1) A[a][b] = ab.gram[slot[a] * MAX_AA + slot[b]];
   }
   block_sums<2 * NM, NT>(acc, [n](int j) { return j % NM < n; });
   if (leader) {  // the newest row, kept for the next steps
-    const int kn = sel.slot[n - 1];
+    const int kn = slot[n - 1];
 #pragma unroll
     for (int j = 0; j < NM; j++)
       if (j < n && (int)threadIdx.x == j) {
-        ab.gram[sel.slot[j] * MAX_AA + kn] = acc[j];
-        ab.gram[kn * MAX_AA + sel.slot[j]] = acc[j];
+        ab.gram[slot[j] * MAX_AA + kn] = acc[j];
+        ab.gram[kn * MAX_AA + slot[j]] = acc[j];
       }
   }
   if constexpr (NM <= 2) {
@@ -2350,7 +2350,7 @@ __global__ void __launch_bounds__(AA_MIX_TX *AA_MIX_TY) k_aa_mix(KGridT<R> g, KF
                                                                  AABuf ab, AASel sel, Gate gate) {
   if (gated_out(gate)) return;
   double gam[NM];
-  aa_solve_group<NM, AA_MIX_TX * AA_MIX_TY>(ab, sel, gam, blockIdx.x == 0);
+  aa_solve_group<NM, AA_MIX_TX * AA_MIX_TY>(ab, sel.n, sel.slot, gam, blockIdx.x == 0);
   __shared__ double sp[AA_MIX_TY + 1][AA_MIX_TX + 1], sT[AA_MIX_TY + 1][AA_MIX_TX + 1],
       ss[AA_MIX_TY + 1][AA_MIX_TX + 1];
   const int ntx = (g.Nx + AA_MIX_TX - 1) / AA_MIX_TX, ntiles = ntx * ((g.Ny + AA_MIX_TY - 1) / AA_MIX_TY);
@@ -2723,7 +2723,7 @@ __global__ void __launch_bounds__(AA_SOLVE_THREADS) kb_aa_solve(const BatchCase<
   const BatchCase<double> &c = C[blockIdx.x];
   if (gated_out(Gate{in_memory(c.ctrl), k + 1})) return;
   double gam[NM];
-  aa_solve_group<NM, AA_SOLVE_THREADS>(aa_of(c), case_sel(c, bs), gam, true);
+  aa_solve_group<NM, AA_SOLVE_THREADS>(aa_of(c), bs.n, bs.slot, gam, true);
 }
 
 template <int TX, int TY, int NM>
