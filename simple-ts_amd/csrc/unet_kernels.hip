@@ -384,12 +384,13 @@ __global__ void __launch_bounds__(256) k_conv_few(ConvArgs a) {
 //
 // The bound is the chain of a step (LDS write, barrier, transposed reads, MFMA):
 // a layer with one workgroup per CU takes 27 us whatever its size.  At 8 x 512 x
-// 128, base 32: 600 us per training step for the 14 convolutions, biases
+// 128, base 32: 455 us per training step for the 14 convolutions, biases
 // included.  The kernels before took 3,484 us (one wave per 16 x 16 of one tap,
 // channel-strided 2-byte loads, atomics) and 2,958 us for the biases.  Loads
 // under an exec mask had to be waited for at each branch's end (73 us per layer);
 // the bias summed by a wave of the tile's own added 13 us to each layer: it has
-// workgroups of its own.  Pixel strides of 96 and 160 bytes put 4 pixels x 32
+// workgroups of its own, behind the others (between them they left every second
+// chiplet without a tile: 40 us).  Pixel strides of 96 and 160 bytes put 4 pixels x 32
 // bytes on distinct banks.
 // ---------------------------------------------------------------------------
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -408,7 +409,7 @@ __device__ __forceinline__ bf16x8 load_tr(const unsigned char *base, int stride)
 constexpr int WG_RUN = 2048, WG_BIAS = 1024;  // pixels per slot of the weights and of the bias
 
 template <int WCI, int WCO, int MT, int AHEAD, bool CAT>
-__global__ void __launch_bounds__(128 * WCI * WCO, MT == 4 ? 2 : 4) k_wgrad(WgradArgs a, int run0) {
+__global__ void __launch_bounds__(128 * WCI * WCO, MT == 4 ? 2 : 4) k_wgrad(WgradArgs a, int run0, int runs) {
   constexpr int NW = 2 * WCI * WCO, CI = 16 * WCI, CO = 16 * MT * WCO;
   static_assert((NW == 4 || NW == 8) && CI <= 64 && CO <= 64, "tile");
   constexpr int SX = CI == 64 ? 160 : 96, SZ = CO == 64 ? 160 : 96;  // bytes per pixel
@@ -423,9 +424,14 @@ __global__ void __launch_bounds__(128 * WCI * WCO, MT == 4 ? 2 : 4) k_wgrad(Wgra
   const int g = lane >> 4, r = lane & 15;
   const int wci = wave % WCI, wco = wave / WCI % WCO, wt = wave / (WCI * WCO);
   const int ci0 = blockIdx.x * CI, co0 = blockIdx.y * CO, H = a.H, W = a.W;
-  const int npix = a.N * H * W, run = run0 + (int)blockIdx.z;
+  const int npix = a.N * H * W;
+  // workgroups behind those of the runs: the biases' (not between them: a launch's
+  // workgroups go to the chiplets in turn, and every other one would be theirs)
+  const bool biased = (int)blockIdx.z >= runs;
+  const int run = run0 + (biased ? ((int)blockIdx.z - runs) * (int)gridDim.x + (int)blockIdx.x : (int)blockIdx.z);
   const int pbeg = run * WG_RUN, pend = min(npix, pbeg + WG_RUN);
-  if (blockIdx.x == gridDim.x - 1) {  // the bias: a lane takes a channel of one of the two runs
+  if (biased) {  // a lane takes a channel of one of the run's two halves
+    if (run >= run0 + runs) return;
     const int co = co0 + (int)threadIdx.x % CO, p0 = pbeg + (int)threadIdx.x / CO * WG_BIAS;
     const int p1 = min(npix, p0 + WG_BIAS);
     if ((int)threadIdx.x >= WG_RUN / WG_BIAS * CO || co >= a.Cout || p0 >= p1) return;
@@ -1098,10 +1104,11 @@ hipError_t unet_conv(const ConvArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 // Tiles of the weight gradient: the widest (64 x 64 channels; it reads least from
-// LDS per MFMA) that leaves a workgroup per CU, else 32 x 64, else 32 x 32 (16 x
-// 32 for a narrow input): a workgroup takes as long however few there are (64
-// workgroups of 64 x 64: 86 us per layer, 256 of 32 x 32: 27 us).
-constexpr long WGRAD_FULL = 256;
+// LDS per MFMA) that leaves 128 workgroups, else 32 x 64, else 32 x 32 (16 x 32
+// for a narrow input): a workgroup takes as long however few there are (64 -> 64
+// channels, 131,072 pixels: 64 workgroups of 64 x 64 44 us, 128 of 32 x 64 28, 256 of
+// 32 x 32, that read the pixels twice as often, 48).
+constexpr long WGRAD_FULL = 128;
 constexpr int SUM_EACH = 32;
 
 hipError_t unet_wgrad(const WgradArgs &a, float *dW, float *db, hipStream_t s) {
@@ -1112,20 +1119,21 @@ hipError_t unet_wgrad(const WgradArgs &a, float *dW, float *db, hipStream_t s) {
   const int CO = CI == 64 || (CI == 32 && a.Cout % 64 == 0 && groups(32, 64) >= WGRAD_FULL) ? 64 : 32;
   // as many slots at a time as the workspace holds
   const size_t P = (size_t)9 * a.Cin * a.Cout;
-  const int most = (int)std::min<size_t>(std::max<size_t>(1, UNET_PART_FLOATS / P), 65535);
+  const int most = (int)std::min<size_t>(std::max<size_t>(1, UNET_PART_FLOATS / P), 32767);
   for (int q = 0; q < S; q += most) {
     const int n = std::min(most, S - q);
     const bool each = n <= SUM_EACH;
     const int nsum = (int)nblk(P, each ? 256 * SUM_WAVES : 256);
     const bool last = q + n == S;
-    const dim3 gr(nblk(a.Cx, CI) + 1, nblk(a.Cout, CO), n);  // + the bias
-    if (CI == 64 && a.X2) hipLaunchKernelGGL((k_wgrad<4, 1, 4, 2, true>), gr, dim3(512), 0, s, a, q);
-    else if (CI == 64) hipLaunchKernelGGL((k_wgrad<4, 1, 4, 2, false>), gr, dim3(512), 0, s, a, q);
-    else if (CO == 64 && a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 2, 2, true>), gr, dim3(512), 0, s, a, q);
-    else if (CO == 64) hipLaunchKernelGGL((k_wgrad<2, 2, 2, 2, false>), gr, dim3(512), 0, s, a, q);
-    else if (a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, true>), gr, dim3(512), 0, s, a, q);
-    else if (CI == 32) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, false>), gr, dim3(512), 0, s, a, q);
-    else hipLaunchKernelGGL((k_wgrad<1, 2, 1, 4, false>), gr, dim3(256), 0, s, a, q);
+    const unsigned X = nblk(a.Cx, CI);
+    const dim3 gr(X, nblk(a.Cout, CO), n + (n + X - 1) / X);  // + the biases
+    if (CI == 64 && a.X2) hipLaunchKernelGGL((k_wgrad<4, 1, 4, 2, true>), gr, dim3(512), 0, s, a, q, n);
+    else if (CI == 64) hipLaunchKernelGGL((k_wgrad<4, 1, 4, 2, false>), gr, dim3(512), 0, s, a, q, n);
+    else if (CO == 64 && a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 2, 2, true>), gr, dim3(512), 0, s, a, q, n);
+    else if (CO == 64) hipLaunchKernelGGL((k_wgrad<2, 2, 2, 2, false>), gr, dim3(512), 0, s, a, q, n);
+    else if (a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, true>), gr, dim3(512), 0, s, a, q, n);
+    else if (CI == 32) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, false>), gr, dim3(512), 0, s, a, q, n);
+    else hipLaunchKernelGGL((k_wgrad<1, 2, 1, 4, false>), gr, dim3(256), 0, s, a, q, n);
     const SumArgs b{a.part, n, P, each, q == 0, dW, nsum, a.bpart, (int)nblk(npix, WG_BIAS), a.Cout, db};
     hipLaunchKernelGGL(k_sum_parts, dim3(nsum + (last ? nblk(a.Cout, 256) : 0)), dim3(64 * SUM_WAVES), 0, s, b);
   }
