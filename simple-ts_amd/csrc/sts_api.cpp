@@ -1010,6 +1010,9 @@ static int ensure_anderson(sts_ctx *c, int m) {
   return STS_OK;
 }
 
+// Whether the grid has conditions at the edges of its box at all.
+static bool edge_conditions(const KGrid &g) { return !g.px && g.bc != 0; }
+
 // Enqueues outer iteration k of the current loop 2; the p/T buffer parity at
 // its start follows the passes of the iterations before it.  The kernels
 // leave their residual maxima in the slotted words lred; the edge kernel folds
@@ -1064,14 +1067,20 @@ static int enqueue_outer(sts_ctx *c, const Loop2State<R> &st, int k, int n, Loop
   t = timed_begin(c, st.kid + STS_K_CORRECT, k);
   HIP_OK(launch_correct(g, kf, lr + 0, lr + 1, 1, flux, c->stream, gate));
   timed_end(c, t);
-  t = timed_begin(c, st.kid + STS_K_WALL, k);
-  HIP_OK(launch_wall_ops(g, kf, c->wall_ops, k == 0 ? c->n_wall_ops : c->n_wall_var, flux, c->stream, gate));
-  timed_end(c, t);
+  // the planned wall writes: in the edge conditions' launch where there are none of
+  // those (their order then does not matter), unless the launches are timed
+  const int nops = k == 0 ? c->n_wall_ops : c->n_wall_var;
+  const bool apart = edge_conditions(c->g) || c->timed;
+  if (apart) {
+    t = timed_begin(c, st.kid + STS_K_WALL, k);
+    HIP_OK(launch_wall_ops(g, kf, c->wall_ops, nops, flux, c->stream, gate));
+    timed_end(c, t);
+  }
   lt.lred = lr;
   lt.log_k += 6 * (size_t)k;
   t = timed_begin(c, st.kid + STS_K_EDGES, k);
   HIP_OK(launch_edges(g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, flux, c->probe, c->stream,
-                      gate, lt));
+                      gate, lt, c->wall_ops, apart ? 0 : nops));
   timed_end(c, t);
   return aa ? enqueue_anderson(c, st, kf, k, sel) : STS_OK;
 }
@@ -1306,8 +1315,10 @@ static constexpr unsigned long long WIDEN_MASK =
 static int rebuild_derived(sts_ctx *c, hipStream_t s) {
   const KFields kf = c->fields();
   HIP_OK(launch_correct(c->g, kf, nullptr, nullptr, 0, true, s));
-  HIP_OK(launch_wall_ops(c->g, kf, c->wall_ops, c->n_wall_ops, true, s));
-  HIP_OK(launch_edges(c->g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, true, nullptr, s));
+  const bool apart = edge_conditions(c->g);
+  if (apart) HIP_OK(launch_wall_ops(c->g, kf, c->wall_ops, c->n_wall_ops, true, s));
+  HIP_OK(launch_edges(c->g, kf, STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, true, nullptr, s,
+                      Gate{nullptr, 0}, LoopTest{}, c->wall_ops, apart ? 0 : c->n_wall_ops));
   c->diff_inline_ok = c->diff_stale = true;
   return STS_OK;
 }

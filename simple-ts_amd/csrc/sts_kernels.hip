@@ -1754,10 +1754,25 @@ __device__ void edges_block(const KGridT<R> &g, const KFieldsT<R> &fl, int parts
   }
 }
 
+// The workgroups past EDGE_GROUPS apply the planned wall writes of grids without
+// edge conditions: the rest of the launch then touches only the residual words and
+// the probed pressure, which no wall write reads or changes.  Both launches are
+// chains of a few loads, so together they take the longer one's time and not the
+// sum: a periodic 301x95 outer iteration 45.0 -> 41.5 us, a closed 640x320 box's
+// loop 3.31 -> 3.22 ms.
 template <typename R>
 __global__ void __launch_bounds__(EDGE_THREADS) k_edges(KGridT<R> g, KFieldsT<R> fl, int parts, bool flux,
-                                                        double *probe, Gate gate, LoopTest lt) {
+                                                        double *probe, Gate gate, LoopTest lt,
+                                                        const WallOp *__restrict__ ops, int nops) {
   if (gated_out(gate)) return;
+  if ((int)blockIdx.x >= EDGE_GROUPS) {
+    const int t = ((int)blockIdx.x - EDGE_GROUPS) * EDGE_THREADS + (int)threadIdx.x;
+    if (t >= nops) return;
+    const WallOp o = ops[t];
+    if (flux) apply_wall_op<true>(g, fl, o);
+    else apply_wall_op<false>(g, fl, o);
+    return;
+  }
   edges_block(g, fl, parts, flux, probe, gate, lt, (int)blockIdx.x);
 }
 
@@ -2871,9 +2886,10 @@ hipError_t launch_wall_ops(const KGridT<R> &g, const KFieldsT<R> &f, const WallO
 }
 template <typename R>
 hipError_t launch_edges(const KGridT<R> &g, const KFieldsT<R> &f, int parts, bool flux, double *probe, hipStream_t s,
-                        Gate gate, LoopTest lt) {
-  hipLaunchKernelGGL(k_edges<R>, dim3(lt.ctrl ? EDGE_GROUPS : EDGE_GROUPS - 1), dim3(EDGE_THREADS), 0, s, g, f, parts,
-                     flux, probe, gate, lt);
+                        Gate gate, LoopTest lt, const WallOp *ops, int nops) {
+  const int groups = nops > 0 ? EDGE_GROUPS + (nops + EDGE_THREADS - 1) / EDGE_THREADS
+                              : (lt.ctrl ? EDGE_GROUPS : EDGE_GROUPS - 1);
+  hipLaunchKernelGGL(k_edges<R>, dim3(groups), dim3(EDGE_THREADS), 0, s, g, f, parts, flux, probe, gate, lt, ops, nops);
   return hipGetLastError();
 }
 template <typename R>
@@ -2903,7 +2919,7 @@ hipError_t launch_flux_diff(const KGridT<R> &g, const KFieldsT<R> &f, hipStream_
   template hipError_t launch_wall_ops<R>(const KGridT<R> &, const KFieldsT<R> &, const WallOp *, int, bool,    \
                                          hipStream_t, Gate);                                                   \
   template hipError_t launch_edges<R>(const KGridT<R> &, const KFieldsT<R> &, int, bool, double *, hipStream_t, \
-                                      Gate, LoopTest);                                                         \
+                                      Gate, LoopTest, const WallOp *, int);                                    \
   template hipError_t launch_flux_diff<R>(const KGridT<R> &, const KFieldsT<R> &, hipStream_t, Gate, int);
 STS_INSTANTIATE(double)
 STS_INSTANTIATE(float)

@@ -38,7 +38,7 @@ hipError_t launch_wall_plan(const KGrid &g, const unsigned *cells, int n, WallOp
 template <typename R>
 hipError_t launch_edges(const KGridT<R> &g, const KFieldsT<R> &f, int parts, bool flux, double *probe, hipStream_t s,
                         Gate gate = Gate{nullptr, 0},
-                        LoopTest lt = LoopTest{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0});
+                        LoopTest lt = LoopTest{}, const WallOp *ops = nullptr, int nops = 0);
 // parts: FLUX_PART (Fx, Fy, DTx, DTy) and/or DIFF_PART (Gamma_*, D_*).
 template <typename R>
 hipError_t launch_flux_diff(const KGridT<R> &g, const KFieldsT<R> &f, hipStream_t s, Gate gate = Gate{nullptr, 0},

@@ -84,3 +84,23 @@ def test_anderson_mix_tiles(sts, size, depth, tmp_path):
         assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(a), k
     for r in runs:
         r.close()
+
+
+@pytest.mark.parametrize("size", [(9, 9), (65, 16), (245, 121), (700, 90)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_loop_without_edge_conditions(sts, oracle, size):
+    """No condition at any edge of the box: the wall writes then share the
+    launch of the loop test and the probe; a few of them and several
+    workgroups' worth."""
+    prob = channel_case(Nx=size[0], Ny=size[1], seed=5, bc={})
+    ctx, ora = sts.Context(prob), oracle.Oracle(prob)
+    for k, a in random_state(prob, seed=11).items():
+        ctx.set(k, a)
+        ora.set(k, a)
+    ctx.fluxes_diffusion()
+    ora.fluxes_diffusion()
+    it, log, _ = ctx.time_step(3, 2, 0.0, 0.0, 0.0)
+    ora.save_previous()
+    ro = np.array([ora.outer_iteration(2) for _ in range(3)])
+    bad = _same(sts, ctx, ora, sts.FIELDS)
+    ctx.close()
+    assert it == 3 and np.array_equal(log[:, :4], ro) and not bad, (log, ro, bad)
