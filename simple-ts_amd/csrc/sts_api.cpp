@@ -1755,8 +1755,10 @@ struct sts_batch {
   int log_cap = 0;
   BatchTile *cell_t[NVARIANT] = {}, *sweep_t[NVARIANT] = {};
   int n_cell[NVARIANT] = {}, n_sweep[NVARIANT] = {};
-  BatchTile *wall_t = nullptr;  // chunks of the cases' planned wall writes
-  int n_wall = 0;
+  // chunks of the cases' planned wall writes (wall_list): of all of them, then of the
+  // state-dependent ones, each first of the cases with edge conditions, then the rest
+  BatchTile *wall_t = nullptr;
+  int n_wall[2][2] = {};
   // tiles of the cases whose loop is still open (rebuilt as cases stop):
   // device lists for the cell, sweep and wall launches, and their pinned
   // host staging (rewritten only after the stream has passed the last copy)
@@ -1808,12 +1810,18 @@ static void tile_list(const sts_batch *b, int TX, int TY, const char *open, std:
   }
 }
 
-// Chunks of WALL_OPS_PER_TILE planned wall writes of the cases with open[c].
-static void wall_list(const sts_batch *b, const char *open, std::vector<BatchTile> &t) {
-  t.clear();
-  for (int c = 0; c < (int)b->cs.size(); c++)
-    if (!open || open[c])
-      for (int x = 0; x * WALL_OPS_PER_TILE < b->cs[c]->n_wall_ops; x++) t.push_back(BatchTile{c, x, 0});
+// Appends the chunks of WALL_OPS_PER_TILE planned wall writes (all of them, or
+// the state-dependent ones) of the cases with open[c]: n[0] of those with edge
+// conditions, then n[1] of those without.
+static void wall_list(const sts_batch *b, const char *open, bool all, std::vector<BatchTile> &t, int n[2]) {
+  for (int side = 0; side < 2; side++) {
+    const size_t at = t.size();
+    for (int c = 0; c < (int)b->cs.size(); c++)
+      if ((!open || open[c]) && edge_conditions(b->cs[c]->g) == (side == 0))
+        for (int x = 0; x * WALL_OPS_PER_TILE < (all ? b->cs[c]->n_wall_ops : b->cs[c]->n_wall_var); x++)
+          t.push_back(BatchTile{c, x, 0});
+    n[side] = (int)(t.size() - at);
+  }
 }
 
 static int build_tiles(sts_batch *b, const int (*shape)[2], BatchTile **out, int *count) {
@@ -1831,7 +1839,7 @@ static int build_tiles(sts_batch *b, const int (*shape)[2], BatchTile **out, int
 // Launch lists of one loop 2: the full lists, or those of the open cases.
 struct BatchLists {
   const BatchTile *cell, *sweep, *wall;
-  int n_cell, n_sweep, n_wall, n_open;
+  int n_cell, n_sweep, n_wall[2], n_open;  // (n_wall: wall_list)
 };
 
 // Rebuilds the active lists for the cases with open[c] and enqueues their
@@ -1843,7 +1851,7 @@ static int compact_lists(sts_batch *b, const std::vector<char> &open, BatchLists
   std::vector<BatchTile> t[3];
   tile_list(b, CELL_TILES[b->cell_v][0], CELL_TILES[b->cell_v][1], open.data(), t[0]);
   tile_list(b, SWEEP_TILES[b->sweep_v][0], SWEEP_TILES[b->sweep_v][1], open.data(), t[1]);
-  wall_list(b, open.data(), t[2]);
+  wall_list(b, open.data(), false, t[2], L.n_wall);
   size_t off = 0;
   for (int q = 0; q < 3; q++) {
     if ((int)t[q].size() > b->act_cap[q]) return fail(STS_ERR_ARG, "active tile list exceeds the full list");
@@ -1859,7 +1867,6 @@ static int compact_lists(sts_batch *b, const std::vector<char> &open, BatchLists
   L.wall = b->act_t[2];
   L.n_cell = (int)t[0].size();
   L.n_sweep = (int)t[1].size();
-  L.n_wall = (int)t[2].size();
   L.n_open = 0;
   for (char o : open) L.n_open += o ? 1 : 0;
   return STS_OK;
@@ -1901,8 +1908,8 @@ extern "C" int sts_batch_create(sts_ctx *const *ctxs, int n, sts_batch **out) {
     return bail(rc);
   {
     std::vector<BatchTile> wt;
-    wall_list(b, nullptr, wt);
-    b->n_wall = (int)wt.size();
+    wall_list(b, nullptr, true, wt, b->n_wall[0]);
+    wall_list(b, nullptr, false, wt, b->n_wall[1]);
     if (hipMalloc(&b->wall_t, sizeof(BatchTile) * (wt.empty() ? 1 : wt.size())) != hipSuccess ||
         (!wt.empty() && hipMemcpyAsync(b->wall_t, wt.data(), sizeof(BatchTile) * wt.size(), hipMemcpyHostToDevice,
                                        b->stream) != hipSuccess) ||
@@ -1911,7 +1918,7 @@ extern "C" int sts_batch_create(sts_ctx *const *ctxs, int n, sts_batch **out) {
   }
   b->act_cap[0] = *std::max_element(b->n_cell, b->n_cell + NVARIANT);
   b->act_cap[1] = *std::max_element(b->n_sweep, b->n_sweep + NVARIANT);
-  b->act_cap[2] = b->n_wall;
+  b->act_cap[2] = b->n_wall[1][0] + b->n_wall[1][1];
   for (int q = 0; q < 3; q++)
     if (hipMalloc(&b->act_t[q], sizeof(BatchTile) * std::max(1, b->act_cap[q])) != hipSuccess)
       return bail(fail(STS_ERR_HIP, "active tile lists"));
@@ -1963,6 +1970,7 @@ static int upload_cases(sts_batch *b, BatchCase<R> *dst, int N_I, double tol_uv,
     x.stall_ratio = stall_ratio;
     x.wops = c->wall_ops;
     x.nwops = c->n_wall_ops;
+    x.nwvar = c->n_wall_var;
     x.skip = skip ? (*skip)[i] : 0;
     x.inline0 = inline0 ? (*inline0)[i] : 0;
     x.aa = c->aa;
@@ -1986,7 +1994,9 @@ static int run_batch_loop2(sts_batch *b, BatchCase<R> *C, int n_pc, int N_I, int
   // launches cover the tiles of every case until the host has seen cases
   // stop; from then on only those of the open ones (a stopped case's tiles
   // would only read its control word and return)
-  BatchLists L{b->cell_t[cv], b->sweep_t[sv], b->wall_t, b->n_cell[cv], b->n_sweep[sv], b->n_wall, n};
+  const int n_wall_all = b->n_wall[0][0] + b->n_wall[0][1];
+  BatchLists L{b->cell_t[cv], b->sweep_t[sv], b->wall_t + n_wall_all, b->n_cell[cv], b->n_sweep[sv],
+               {b->n_wall[1][0], b->n_wall[1][1]}, n};
   std::vector<char> open_c(n, 1);
   HIP_OK(launch_batch<R>(BK_LOOP_OPEN, 0, C, n, nullptr, 0, 0, 0, 0, 0, s));
   if constexpr (sizeof(R) == sizeof(double))
@@ -2013,8 +2023,14 @@ static int run_batch_loop2(sts_batch *b, BatchCase<R> *C, int n_pc, int N_I, int
         par ^= 1;
       }
       HIP_OK(launch_batch<R>(BK_CORRECT, cv, C, n, L.cell, L.n_cell, k, par, 0, 0, s));
-      HIP_OK(launch_batch<R>(BK_WALL_OPS, 0, C, n, L.wall, L.n_wall, k, par, 0, 0, s));
-      HIP_OK(launch_batch<R>(BK_EDGES, 0, C, n, nullptr, 0, k, par,
+      // as in the single-context loop: constants once, and in the edges launch where a
+      // case has no edge conditions; of 12 cases, the half with edge conditions and
+      // constant wall values and the rest without, the wall launch goes after k = 0:
+      // 6.37 -> 6.25 ms per two steps
+      const BatchTile *wall = k == 0 ? b->wall_t : L.wall;
+      const int *n_wall = k == 0 ? b->n_wall[0] : L.n_wall;
+      HIP_OK(launch_batch<R>(BK_WALL_OPS, 0, C, n, wall, n_wall[0], k, par, 0, 0, s));
+      HIP_OK(launch_batch<R>(BK_EDGES, 0, C, n, wall + n_wall[0], n_wall[1], k, par,
                              STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, 0, s));
       if constexpr (sizeof(R) == sizeof(double))
         if (aa_m > 0 && (k + 1) % aa_every == 0) {  // as enqueue_anderson, for every case at once
@@ -2119,8 +2135,8 @@ extern "C" int sts_batch_time_step(sts_batch *b, const sts_loop_control *lc, con
   if (any) {
     if ((rc = upload_cases<double>(b, b->C64, 1, 0, 0, 0, 0, 0.0, 0, false, &from_xn))) return rc;
     HIP_OK(launch_batch<double>(BK_DERIVE, cv, b->C64, n, b->cell_t[cv], b->n_cell[cv], 0, 0, 0, 0, s));
-    HIP_OK(launch_batch<double>(BK_WALL_OPS, 0, b->C64, n, b->wall_t, b->n_wall, -1, 0, 0, 0, s));
-    HIP_OK(launch_batch<double>(BK_EDGES, 0, b->C64, n, nullptr, 0, -1, 0,
+    HIP_OK(launch_batch<double>(BK_WALL_OPS, 0, b->C64, n, b->wall_t, b->n_wall[0][0], -1, 0, 0, 0, s));
+    HIP_OK(launch_batch<double>(BK_EDGES, 0, b->C64, n, b->wall_t + b->n_wall[0][0], b->n_wall[0][1], -1, 0,
                                 STS_BC_VELOCITIES | STS_BC_TEMPERATURE | STS_BC_PRESSURE, 0, s));
   }
   for (int i = 0; i < n; i++) {

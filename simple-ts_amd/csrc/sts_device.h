@@ -242,7 +242,7 @@ struct BatchCase {
   int N_I, stall_w;
   double tol_uv, tol_p, tol_T, stall_ratio;
   const WallOp *wops;  // the case's planned wall writes
-  int nwops;
+  int nwops, nwvar;    // all of them, and the leading ones that depend on the state
   int skip;     // the case sits this loop out (its loop control opens closed)
   int inline0;  // the first outer iteration forms Gamma and D itself (else reads the arrays)
   // Anderson acceleration (FP64 loops): the case's vectors (aa.nb = its

@@ -2670,15 +2670,21 @@ __global__ void __launch_bounds__(TX *TY) kb_correct(const BatchCase<R> *C, cons
   block_max_atomic<2, TX * TY>(r, MaxDst<2>{{in_memory(c.lred), in_memory(c.lred) + 1}, {}});
 }
 
+// A chunk of a case's planned wall writes; after a loop's first iteration only the
+// state-dependent ones, which lead.
 template <typename R>
-__global__ void __launch_bounds__(WALL_OPS_PER_TILE) kb_wall_ops(const BatchCase<R> *C, const BatchTile *T, int k,
-                                                                 int par) {
-  const BatchTile t = T[blockIdx.x];
+__device__ __forceinline__ void batch_wall_chunk(const BatchCase<R> *C, const BatchTile t, int k, int par) {
   const BatchCase<R> &c = C[t.c];
   if (k < 0 ? c.skip != 0 : gated_out(Gate{in_memory(c.ctrl), k})) return;  // k < 0: after kb_derive
   const int q = t.x * WALL_OPS_PER_TILE + (int)threadIdx.x;
-  if (q >= c.nwops) return;
+  if ((int)threadIdx.x >= WALL_OPS_PER_TILE || q >= (k > 0 ? c.nwvar : c.nwops)) return;
   apply_wall_op<true>(grid_of(c), fields_at(c, par), in_memory(c.wops)[q]);
+}
+
+template <typename R>
+__global__ void __launch_bounds__(WALL_OPS_PER_TILE) kb_wall_ops(const BatchCase<R> *C, const BatchTile *T, int k,
+                                                                 int par) {
+  batch_wall_chunk(C, T[blockIdx.x], k, par);
 }
 
 // Batched Anderson steps (FP64): the single-context kernels' code per tile
@@ -2756,9 +2762,15 @@ __global__ void __launch_bounds__(TX *TY) kb_aa_mix(const BatchCase<double> *C, 
                           t.y * TY, (int)threadIdx.x % TX, (int)threadIdx.x / TX, sp, sT, ss);
 }
 
-// Edge conditions and the loop-2 test: one workgroup per case.
+// Edge conditions and the loop-2 test, EDGE_GROUPS workgroups per case; behind them
+// the wall writes of the cases without edge conditions (as k_edges).
 template <typename R>
-__global__ void __launch_bounds__(EDGE_THREADS) kb_edges(const BatchCase<R> *C, int k, int par, int parts) {
+__global__ void __launch_bounds__(EDGE_THREADS) kb_edges(const BatchCase<R> *C, const BatchTile *T, int ncases, int k,
+                                                         int par, int parts) {
+  if ((int)blockIdx.x >= ncases * EDGE_GROUPS) {
+    batch_wall_chunk(C, T[(int)blockIdx.x - ncases * EDGE_GROUPS], k, par);
+    return;
+  }
   const BatchCase<R> &c = C[blockIdx.x / EDGE_GROUPS];
   const Gate gate{c.ctrl, k};
   if (k < 0 ? c.skip != 0 : gated_out(gate)) return;  // k < 0: after kb_derive
@@ -3139,7 +3151,8 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
       }
       break;
     case BK_EDGES:
-      hipLaunchKernelGGL(kb_edges<R>, dim3(EDGE_GROUPS * ncases), dim3(EDGE_THREADS), 0, s, C, k, par, a);
+      hipLaunchKernelGGL(kb_edges<R>, dim3(EDGE_GROUPS * ncases + ntiles), dim3(EDGE_THREADS), 0, s, C, T, ncases, k,
+                         par, a);
       break;
     case BK_LOOP_OPEN: hipLaunchKernelGGL(kb_loop_open<R>, dim3(ncases), dim3(256), 0, s, C); break;
     default: return hipErrorInvalidValue;

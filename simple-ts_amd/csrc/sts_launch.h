@@ -88,7 +88,8 @@ hipError_t launch_continuity(const KGrid &g, const KFields &f, double *cs, doubl
 // Batched loop-2 launches over the tiles T[0..ntiles) of the cases
 // C[0..ncases).  kernel: BK_*; variant: index into CELL_TILES (cell
 // kernels) or SWEEP_TILES (BK_SWEEP2).  (a, b) = (first, last) for the
-// sweeps, a = parts for BK_EDGES.
+// sweeps, a = parts for BK_EDGES (its tiles: planned wall writes of the cases
+// without edge conditions, as those of BK_WALL_OPS).
 // BK_ASSEMBLE forms Gamma and D in the tile; BK_ASSEMBLE_ARR (first outer
 // iteration only) assembles the cases whose arrays are to be read instead.
 enum {
