@@ -1755,14 +1755,15 @@ struct sts_batch {
   int log_cap = 0;
   BatchTile *cell_t[NVARIANT] = {}, *sweep_t[NVARIANT] = {};
   int n_cell[NVARIANT] = {}, n_sweep[NVARIANT] = {};
-  // chunks of the cases' planned wall writes (wall_list): of all of them, then of the
+  // chunks of the cases' planned wall writes (wall_runs): of all of them, then of the
   // state-dependent ones, each first of the cases with edge conditions, then the rest
   BatchTile *wall_t = nullptr;
   int n_wall[2][2] = {};
-  // tiles of the cases whose loop is still open (rebuilt as cases stop):
-  // device lists for the cell, sweep and wall launches, and their pinned
-  // host staging (rewritten only after the stream has passed the last copy)
-  BatchTile *act_t[3] = {}, *h_act = nullptr;
+  // tiles of the cases whose loop is still open (rebuilt as cases stop): lists for
+  // the cell, sweep and wall launches; the runs they are made of (one per case and
+  // list) and their pinned host staging
+  BatchTile *act_t[3] = {};
+  TileRun *runs = nullptr, *h_runs = nullptr;
   int act_cap[3] = {};
   int cell_v = 0, sweep_v = 0;
   int last_iters32 = 0, last_iters64 = 0;
@@ -1781,7 +1782,8 @@ extern "C" int sts_batch_destroy(sts_batch *b) {
   }
   (void)hipFree(b->wall_t);
   for (BatchTile *p : b->act_t) (void)hipFree(p);
-  if (b->h_act) (void)hipHostFree(b->h_act);
+  (void)hipFree(b->runs);
+  if (b->h_runs) (void)hipHostFree(b->h_runs);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->ev_ctrl) (void)hipEventDestroy(b->ev_ctrl);
@@ -1790,48 +1792,80 @@ extern "C" int sts_batch_destroy(sts_batch *b) {
   return STS_OK;
 }
 
-// Tile list of the cases with open[c] (all when open is null) for tiles of
-// TX x TY cells, into t.  Workgroup b runs on chiplet b % 8 (round-robin
-// dispatch); every chiplet gets one contiguous run of the list (same order
-// as xcd_tile).
-static void tile_list(const sts_batch *b, int TX, int TY, const char *open, std::vector<BatchTile> &t) {
-  std::vector<BatchTile> lt;
+// The runs of the cases with open[c] (all when open is null) in the list of tiles
+// of TX x TY cells, to r; n[0] runs, n[1] tiles.
+static void tile_runs(const sts_batch *b, int TX, int TY, const char *open, TileRun *r, int n[2]) {
+  n[0] = n[1] = 0;
   for (int c = 0; c < (int)b->cs.size(); c++) {
     if (open && !open[c]) continue;
     const int nx = (b->cs[c]->Nx + TX - 1) / TX, ny = (b->cs[c]->Ny + TY - 1) / TY;
-    for (int y = 0; y < ny; y++)
-      for (int x = 0; x < nx; x++) lt.push_back(BatchTile{c, x, y});
-  }
-  const int nt = (int)lt.size(), per = nt / 8, rem = nt % 8;
-  t.resize(lt.size());
-  for (int bid = 0; bid < nt; bid++) {
-    const int x = bid % 8;
-    t[bid] = lt[x * per + std::min(x, rem) + bid / 8];
+    r[n[0]++] = TileRun{c, nx, n[1]};
+    n[1] += nx * ny;
   }
 }
 
-// Appends the chunks of WALL_OPS_PER_TILE planned wall writes (all of them, or
-// the state-dependent ones) of the cases with open[c]: n[0] of those with edge
-// conditions, then n[1] of those without.
-static void wall_list(const sts_batch *b, const char *open, bool all, std::vector<BatchTile> &t, int n[2]) {
-  for (int side = 0; side < 2; side++) {
-    const size_t at = t.size();
-    for (int c = 0; c < (int)b->cs.size(); c++)
-      if ((!open || open[c]) && edge_conditions(b->cs[c]->g) == (side == 0))
-        for (int x = 0; x * WALL_OPS_PER_TILE < (all ? b->cs[c]->n_wall_ops : b->cs[c]->n_wall_var); x++)
-          t.push_back(BatchTile{c, x, 0});
-    n[side] = (int)(t.size() - at);
+// Likewise of the list of their chunks of WALL_OPS_PER_TILE planned wall writes (all
+// of them, or the state-dependent ones): side[0] chunks of the cases with edge
+// conditions, then side[1] of those without.
+static void wall_runs(const sts_batch *b, const char *open, bool all, TileRun *r, int n[2], int side[2]) {
+  n[0] = n[1] = 0;
+  for (int q = 0; q < 2; q++) {
+    const int at = n[1];
+    for (int c = 0; c < (int)b->cs.size(); c++) {
+      const int ops = all ? b->cs[c]->n_wall_ops : b->cs[c]->n_wall_var;
+      if ((open && !open[c]) || edge_conditions(b->cs[c]->g) != (q == 0) || ops == 0) continue;
+      const int chunks = (ops + WALL_OPS_PER_TILE - 1) / WALL_OPS_PER_TILE;
+      r[n[0]++] = TileRun{c, chunks, n[1]};
+      n[1] += chunks;
+    }
+    side[q] = n[1] - at;
   }
 }
 
-static int build_tiles(sts_batch *b, const int (*shape)[2], BatchTile **out, int *count) {
+// Enqueues the lists of the runs in h_runs (n[q] = runs and tiles of list q) on the
+// batch stream.  The host has waited for what it enqueued here before, so the
+// staging is free.
+static int enqueue_lists(sts_batch *b, const int n[3][2], BatchTile *const out[3]) {
+  const int nc = (int)b->cs.size();
+  TileLists L{};
+  L.stride = nc;
+  for (int q = 0; q < 3; q++) {
+    L.out[q] = out[q];
+    L.nrun[q] = n[q][0];
+    L.ntiles[q] = n[q][1];
+  }
+  HIP_OK(hipMemcpyAsync(b->runs, b->h_runs, sizeof(TileRun) * 3 * (size_t)nc, hipMemcpyHostToDevice, b->stream));
+  HIP_OK(launch_tile_lists(b->runs, L, b->stream));
+  return STS_OK;
+}
+
+// The full lists of every tile variant, and of the wall writes.
+static int build_lists(sts_batch *b) {
+  const int nc = (int)b->cs.size();
   for (int v = 0; v < NVARIANT; v++) {
-    std::vector<BatchTile> t;
-    tile_list(b, shape[v][0], shape[v][1], nullptr, t);
-    HIP_OK(hipMalloc(&out[v], sizeof(BatchTile) * (t.empty() ? 1 : t.size())));
-    HIP_OK(hipMemcpyAsync(out[v], t.data(), sizeof(BatchTile) * t.size(), hipMemcpyHostToDevice, b->stream));
+    int n[3][2] = {};
+    tile_runs(b, CELL_TILES[v][0], CELL_TILES[v][1], nullptr, b->h_runs, n[0]);
+    tile_runs(b, SWEEP_TILES[v][0], SWEEP_TILES[v][1], nullptr, b->h_runs + nc, n[1]);
+    b->n_cell[v] = n[0][1];
+    b->n_sweep[v] = n[1][1];
+    HIP_OK(hipMalloc(&b->cell_t[v], sizeof(BatchTile) * std::max(1, n[0][1])));
+    HIP_OK(hipMalloc(&b->sweep_t[v], sizeof(BatchTile) * std::max(1, n[1][1])));
+    BatchTile *out[3] = {b->cell_t[v], b->sweep_t[v], nullptr};
+    int rc;
+    if ((rc = enqueue_lists(b, n, out))) return rc;
     HIP_OK(hipStreamSynchronize(b->stream));
-    count[v] = (int)t.size();
+  }
+  int n[2][2];
+  wall_runs(b, nullptr, true, b->h_runs, n[0], b->n_wall[0]);
+  wall_runs(b, nullptr, false, b->h_runs, n[1], b->n_wall[1]);
+  HIP_OK(hipMalloc(&b->wall_t, sizeof(BatchTile) * std::max(1, n[0][1] + n[1][1])));
+  for (int q = 0; q < 2; q++) {
+    int m[3][2] = {}, side[2];
+    BatchTile *out[3] = {nullptr, nullptr, b->wall_t + (q ? n[0][1] : 0)};
+    wall_runs(b, nullptr, q == 0, b->h_runs + 2 * nc, m[2], side);
+    int rc;
+    if ((rc = enqueue_lists(b, m, out))) return rc;
+    HIP_OK(hipStreamSynchronize(b->stream));
   }
   return STS_OK;
 }
@@ -1839,34 +1873,30 @@ static int build_tiles(sts_batch *b, const int (*shape)[2], BatchTile **out, int
 // Launch lists of one loop 2: the full lists, or those of the open cases.
 struct BatchLists {
   const BatchTile *cell, *sweep, *wall;
-  int n_cell, n_sweep, n_wall[2], n_open;  // (n_wall: wall_list)
+  int n_cell, n_sweep, n_wall[2], n_open;  // (n_wall: wall_runs)
 };
 
-// Rebuilds the active lists for the cases with open[c] and enqueues their
-// upload on the batch stream (kernels enqueued before it still read the
-// previous lists, which held a superset of these tiles).  Called only right
-// after the host waited for an event that follows the previous upload, so
-// the pinned staging is free.
+// Enqueues the active lists for the cases with open[c] (kernels enqueued before
+// still read the previous lists, which held a superset of these tiles).  Called
+// only right after the host waited for an event that follows the previous call's
+// work.  The host gives a few words per case and a kernel writes the tiles: with
+// the lists themselves built and copied here the device stood idle at each of the
+// ~4 times a step that cases stop (12 cases, two steps: 6.26 -> 6.17 ms).
 static int compact_lists(sts_batch *b, const std::vector<char> &open, BatchLists &L) {
-  std::vector<BatchTile> t[3];
-  tile_list(b, CELL_TILES[b->cell_v][0], CELL_TILES[b->cell_v][1], open.data(), t[0]);
-  tile_list(b, SWEEP_TILES[b->sweep_v][0], SWEEP_TILES[b->sweep_v][1], open.data(), t[1]);
-  wall_list(b, open.data(), false, t[2], L.n_wall);
-  size_t off = 0;
-  for (int q = 0; q < 3; q++) {
-    if ((int)t[q].size() > b->act_cap[q]) return fail(STS_ERR_ARG, "active tile list exceeds the full list");
-    if (!t[q].empty()) {
-      std::memcpy(b->h_act + off, t[q].data(), sizeof(BatchTile) * t[q].size());
-      HIP_OK(hipMemcpyAsync(b->act_t[q], b->h_act + off, sizeof(BatchTile) * t[q].size(), hipMemcpyHostToDevice,
-                            b->stream));
-    }
-    off += (size_t)b->act_cap[q];
-  }
+  const int nc = (int)b->cs.size();
+  int n[3][2];
+  tile_runs(b, CELL_TILES[b->cell_v][0], CELL_TILES[b->cell_v][1], open.data(), b->h_runs, n[0]);
+  tile_runs(b, SWEEP_TILES[b->sweep_v][0], SWEEP_TILES[b->sweep_v][1], open.data(), b->h_runs + nc, n[1]);
+  wall_runs(b, open.data(), false, b->h_runs + 2 * nc, n[2], L.n_wall);
+  for (int q = 0; q < 3; q++)
+    if (n[q][1] > b->act_cap[q]) return fail(STS_ERR_ARG, "active tile list exceeds the full list");
+  int rc;
+  if ((rc = enqueue_lists(b, n, b->act_t))) return rc;
   L.cell = b->act_t[0];
   L.sweep = b->act_t[1];
   L.wall = b->act_t[2];
-  L.n_cell = (int)t[0].size();
-  L.n_sweep = (int)t[1].size();
+  L.n_cell = n[0][1];
+  L.n_sweep = n[1][1];
   L.n_open = 0;
   for (char o : open) L.n_open += o ? 1 : 0;
   return STS_OK;
@@ -1899,32 +1929,21 @@ extern "C" int sts_batch_create(sts_ctx *const *ctxs, int n, sts_batch **out) {
   B_OK(hipMalloc(&b->ctrl, sizeof(LoopCtrl) * n));
   B_OK(hipHostMalloc(&b->h_ctrl, sizeof(LoopCtrl) * n, hipHostMallocDefault));
   B_OK(hipMalloc(&b->lred, sizeof(unsigned long long) * NSLOT * SLOT_STRIDE * (size_t)n));
+  B_OK(hipMalloc(&b->runs, sizeof(TileRun) * 3 * (size_t)n));
+  B_OK(hipHostMalloc(&b->h_runs, sizeof(TileRun) * 3 * (size_t)n, hipHostMallocDefault));
+  std::memset(b->h_runs, 0, sizeof(TileRun) * 3 * (size_t)n);
   B_OK(hipEventCreateWithFlags(&b->ev0, hipEventDisableSystemFence));
   B_OK(hipEventCreateWithFlags(&b->ev1, hipEventDisableSystemFence));
   B_OK(hipEventCreateWithFlags(&b->ev_ctrl, hipEventDisableTiming));
 #undef B_OK
   int rc;
-  if ((rc = build_tiles(b, CELL_TILES, b->cell_t, b->n_cell)) || (rc = build_tiles(b, SWEEP_TILES, b->sweep_t, b->n_sweep)))
-    return bail(rc);
-  {
-    std::vector<BatchTile> wt;
-    wall_list(b, nullptr, true, wt, b->n_wall[0]);
-    wall_list(b, nullptr, false, wt, b->n_wall[1]);
-    if (hipMalloc(&b->wall_t, sizeof(BatchTile) * (wt.empty() ? 1 : wt.size())) != hipSuccess ||
-        (!wt.empty() && hipMemcpyAsync(b->wall_t, wt.data(), sizeof(BatchTile) * wt.size(), hipMemcpyHostToDevice,
-                                       b->stream) != hipSuccess) ||
-        hipStreamSynchronize(b->stream) != hipSuccess)
-      return bail(fail(STS_ERR_HIP, "wall tiles"));
-  }
+  if ((rc = build_lists(b))) return bail(rc);
   b->act_cap[0] = *std::max_element(b->n_cell, b->n_cell + NVARIANT);
   b->act_cap[1] = *std::max_element(b->n_sweep, b->n_sweep + NVARIANT);
   b->act_cap[2] = b->n_wall[1][0] + b->n_wall[1][1];
   for (int q = 0; q < 3; q++)
     if (hipMalloc(&b->act_t[q], sizeof(BatchTile) * std::max(1, b->act_cap[q])) != hipSuccess)
       return bail(fail(STS_ERR_HIP, "active tile lists"));
-  if (hipHostMalloc(&b->h_act, sizeof(BatchTile) * std::max(1, b->act_cap[0] + b->act_cap[1] + b->act_cap[2]),
-                    hipHostMallocDefault) != hipSuccess)
-    return bail(fail(STS_ERR_HIP, "active tile staging"));
   if (hipStreamSynchronize(b->stream) != hipSuccess) return bail(fail(STS_ERR_HIP, "stream sync"));
   *out = b;
   return STS_OK;

@@ -265,3 +265,17 @@ struct AABatchSel {
 struct BatchTile {
   int c, x, y;
 };
+
+// A case's tiles in a launch list: row by row, nx to a row, from position `first`
+// of the list's plain order on (up to the next run's).
+struct TileRun {
+  int c, nx, first;
+};
+
+// Launch lists to write: list q from nrun[q] runs at q * stride, to out[q]; 0 and 1
+// so that every chiplet gets one stretch of the plain order (as xcd_tile), 2 (wall
+// writes) in the plain order.
+struct TileLists {
+  BatchTile *out[3];
+  int nrun[3], ntiles[3], stride;
+};

@@ -120,6 +120,8 @@ hipError_t launch_batch(int kernel, int variant, const BatchCase<R> *C, int ncas
 // partial slots.
 enum { BKA_BEGIN, BKA_STORE, BKA_SOLVE, BKA_MIX };
 int aa_case_tiles(int Nx, int Ny, int variant);
+// Writes the launch lists of L from their runs (device memory).
+hipError_t launch_tile_lists(const TileRun *runs, const TileLists &L, hipStream_t s);
 // Starts of a step of all cases (A: one entry per case; cell tiles of
 // `variant`).  Then, for the cases of C that do not skip, BK_DERIVE and, with k =
 // -1, BK_WALL_OPS and BK_EDGES.
