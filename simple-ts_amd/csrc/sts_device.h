@@ -261,6 +261,12 @@ struct AABatchSel {
   int slot[MAX_AA];
 };
 
+// Arrays copied together.
+struct CopySet {
+  const double *src[5];
+  double *dst[5];
+};
+
 // Work item of a batched launch: tile (x, y) of case c.
 struct BatchTile {
   int c, x, y;

@@ -28,5 +28,6 @@ void sts_internal_set_error(const std::string &msg);
 int sts_internal_unet_predict(sts_unet *u, const StsView &v, const sts_unet_norm *nrm, double *pw, double *Tw);
 // Corrector: from x^n (the *_PR fields) and the predicted start v.xe, the
 // corrected start written into out[4] (device u, v, p, T; may be the state
-// arrays themselves).
+// arrays themselves).  Enqueued in v.stream: the caller waits for that before
+// the network's other calls, also after an error.
 int sts_internal_unet_correct(sts_unet *u, const StsView &v, const sts_unet_corr_norm *nrm, double *const out[4]);

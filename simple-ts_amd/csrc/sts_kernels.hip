@@ -1851,16 +1851,17 @@ __global__ void __launch_bounds__(BX *BY) k_jump_overwrite(KGrid g, KFields fl) 
   else if (j >= 1 && m[k - Nx]) T[k] = FLD(TW_V)[k];
 }
 
-__global__ void __launch_bounds__(BX *BY) k_copy5(const double *a0, const double *a1, const double *a2,
-                                                  const double *a3, const double *a4, double *b0, double *b1,
-                                                  double *b2, double *b3, double *b4, int n) {
+// N arrays in one launch.  Bound by the launches where the arrays are small (four
+// copies of 512x128 as copy commands 25 us of a step, here 6).
+template <int N>
+__global__ void __launch_bounds__(BX *BY) k_copies(CopySet c, int n) {
   const int t = (blockIdx.x + blockIdx.y * gridDim.x) * (BX * BY) + threadIdx.x + threadIdx.y * BX;
   if (t >= n) return;
-  b0[t] = a0[t];
-  b1[t] = a1[t];
-  b2[t] = a2[t];
-  b3[t] = a3[t];
-  b4[t] = a4[t];
+  double x[N];
+#pragma unroll
+  for (int q = 0; q < N; q++) x[q] = c.src[q][t];
+#pragma unroll
+  for (int q = 0; q < N; q++) c.dst[q][t] = x[q];
 }
 
 // Start of loop 2 from a linear extrapolation in time: x = 2 x^n - x^(n-1)
@@ -2972,13 +2973,15 @@ hipError_t launch_jump_overwrite(const KGrid &g, const KFields &f, hipStream_t s
   hipLaunchKernelGGL(k_jump_overwrite, grid2d(g), dim3(BX, BY), 0, s, g, f);
   return hipGetLastError();
 }
-hipError_t launch_copy5(const double *const *src, double *const *dst, int n, hipStream_t s) {
+template <int N>
+hipError_t launch_copies(const CopySet &c, int n, hipStream_t s) {
   const int blocks = (n + BX * BY - 1) / (BX * BY);
   dim3 gr(blocks < 65535 ? blocks : 65535, (blocks + 65534) / 65535);
-  hipLaunchKernelGGL(k_copy5, gr, dim3(BX, BY), 0, s, src[0], src[1], src[2], src[3], src[4], dst[0], dst[1], dst[2],
-                     dst[3], dst[4], n);
+  hipLaunchKernelGGL(k_copies<N>, gr, dim3(BX, BY), 0, s, c, n);
   return hipGetLastError();
 }
+template hipError_t launch_copies<4>(const CopySet &, int, hipStream_t);
+template hipError_t launch_copies<5>(const CopySet &, int, hipStream_t);
 hipError_t launch_begin(const BeginArgs &a, hipStream_t s) {
   hipLaunchKernelGGL(k_begin, dim3((a.Nx + BX - 1) / BX, (a.Ny + BY - 1) / BY), dim3(BX, BY), 0, s, a);
   return hipGetLastError();

@@ -49,7 +49,9 @@ hipError_t launch_properties(const KGrid &g, const KFields &f, hipStream_t s);
 hipError_t launch_rho_mid(const KGrid &g, const KFields &f, hipStream_t s);
 hipError_t launch_apply_bodies(const KGrid &g, const KFields &f, hipStream_t s);
 hipError_t launch_jump_overwrite(const KGrid &g, const KFields &f, hipStream_t s);
-hipError_t launch_copy5(const double *const *src, double *const *dst, int n, hipStream_t s);
+// dst[q][0 .. n) = src[q][0 .. n), q < N (4 or 5).
+template <int N>
+hipError_t launch_copies(const CopySet &c, int n, hipStream_t s);
 hipError_t launch_set_inflow(const KGrid &g, const KFields &f, double u_in, hipStream_t s);
 // The start of a time step (BeginArgs): the previous step's fields, the history,
 // the predicted start from hist[h] = x^(n-1-h) (h < order).

@@ -114,10 +114,10 @@ int pack_weights(sts_unet *u) {
   return STS_OK;
 }
 
-int conv_fwd(sts_unet *u, int k, const u16 *X, int n, u16 *Y, const u16 *skip = nullptr, int Cb = 0) {
+int conv_fwd(sts_unet *u, hipStream_t s, int k, const u16 *X, int n, u16 *Y, const u16 *skip = nullptr, int Cb = 0) {
   const Conv &c = u->L[k];
   ConvArgs a{X, c.Cx, n, u->h(c.level), u->w(c.level), 3, c.Wt, c.Kp, u->P + c.b_off, c.Cout, Y, 1, u->zero, skip, Cb};
-  U_OK(unet_conv(a, u->stream));
+  U_OK(unet_conv(a, s));
   return STS_OK;
 }
 
@@ -138,33 +138,33 @@ int conv_back(sts_unet *u, int k, const u16 *X, int n, const u16 *dz, u16 *dX, c
   return STS_OK;
 }
 
-// Forward of the batch already in u->x; result in u->y.
-int forward_dev(sts_unet *u, int n) {
+// Forward, in stream s, of the batch already in u->x; result in u->y.
+int forward_dev(sts_unet *u, int n, hipStream_t s) {
   int rc;
   const int B = u->base;
-  if ((rc = conv_fwd(u, E1A, u->x, n, u->act[E1A])) || (rc = conv_fwd(u, E1B, u->act[E1A], n, u->act[E1B])))
+  if ((rc = conv_fwd(u, s, E1A, u->x, n, u->act[E1A])) || (rc = conv_fwd(u, s, E1B, u->act[E1A], n, u->act[E1B])))
     return rc;
-  U_OK(unet_pool(u->act[E1B], n, u->h(0), u->w(0), B, u->pl[0], u->stream));
-  if ((rc = conv_fwd(u, E2A, u->pl[0], n, u->act[E2A])) || (rc = conv_fwd(u, E2B, u->act[E2A], n, u->act[E2B])))
+  U_OK(unet_pool(u->act[E1B], n, u->h(0), u->w(0), B, u->pl[0], s));
+  if ((rc = conv_fwd(u, s, E2A, u->pl[0], n, u->act[E2A])) || (rc = conv_fwd(u, s, E2B, u->act[E2A], n, u->act[E2B])))
     return rc;
-  U_OK(unet_pool(u->act[E2B], n, u->h(1), u->w(1), 2 * B, u->pl[1], u->stream));
-  if ((rc = conv_fwd(u, E3A, u->pl[1], n, u->act[E3A])) || (rc = conv_fwd(u, E3B, u->act[E3A], n, u->act[E3B])))
+  U_OK(unet_pool(u->act[E2B], n, u->h(1), u->w(1), 2 * B, u->pl[1], s));
+  if ((rc = conv_fwd(u, s, E3A, u->pl[1], n, u->act[E3A])) || (rc = conv_fwd(u, s, E3B, u->act[E3A], n, u->act[E3B])))
     return rc;
-  U_OK(unet_pool(u->act[E3B], n, u->h(2), u->w(2), 4 * B, u->pl[2], u->stream));
-  if ((rc = conv_fwd(u, BA, u->pl[2], n, u->act[BA])) || (rc = conv_fwd(u, BB, u->act[BA], n, u->act[BB])))
+  U_OK(unet_pool(u->act[E3B], n, u->h(2), u->w(2), 4 * B, u->pl[2], s));
+  if ((rc = conv_fwd(u, s, BA, u->pl[2], n, u->act[BA])) || (rc = conv_fwd(u, s, BB, u->act[BA], n, u->act[BB])))
     return rc;
   // decoder convolutions on [nearest-up(half), skip], read in place
-  if ((rc = conv_fwd(u, D3A, u->act[BB], n, u->act[D3A], u->act[E3B], 8 * B)) ||
-      (rc = conv_fwd(u, D3B, u->act[D3A], n, u->act[D3B])))
+  if ((rc = conv_fwd(u, s, D3A, u->act[BB], n, u->act[D3A], u->act[E3B], 8 * B)) ||
+      (rc = conv_fwd(u, s, D3B, u->act[D3A], n, u->act[D3B])))
     return rc;
-  if ((rc = conv_fwd(u, D2A, u->act[D3B], n, u->act[D2A], u->act[E2B], 4 * B)) ||
-      (rc = conv_fwd(u, D2B, u->act[D2A], n, u->act[D2B])))
+  if ((rc = conv_fwd(u, s, D2A, u->act[D3B], n, u->act[D2A], u->act[E2B], 4 * B)) ||
+      (rc = conv_fwd(u, s, D2B, u->act[D2A], n, u->act[D2B])))
     return rc;
-  if ((rc = conv_fwd(u, D1A, u->act[D2B], n, u->act[D1A], u->act[E1B], 2 * B)) ||
-      (rc = conv_fwd(u, D1B, u->act[D1A], n, u->act[D1B])))
+  if ((rc = conv_fwd(u, s, D1A, u->act[D2B], n, u->act[D1A], u->act[E1B], 2 * B)) ||
+      (rc = conv_fwd(u, s, D1B, u->act[D1A], n, u->act[D1B])))
     return rc;
   const Conv &hd = u->L[HEAD];
-  U_OK(unet_head(u->act[D1B], B, hd.Wt, u->P + hd.b_off, u->cout, (int)u->npix(n, 0), u->y, u->stream));
+  U_OK(unet_head(u->act[D1B], B, hd.Wt, u->P + hd.b_off, u->cout, (int)u->npix(n, 0), u->y, s));
   return STS_OK;
 }
 
@@ -361,7 +361,7 @@ extern "C" int sts_unet_forward(sts_unet *u, int n, const float *x, float *y) {
   const size_t np = u->npix(n, 0);
   U_OK(u->copy.put(u->xin, x, sizeof(float) * np * u->cin, u->stream));
   U_OK(unet_to_bf16(u->xin, u->cin, u->Cx0, np, u->x, u->stream));
-  if ((rc = forward_dev(u, n))) return rc;
+  if ((rc = forward_dev(u, n, u->stream))) return rc;
   U_OK(u->copy.get(y, u->y, sizeof(float) * np * u->cout, u->stream));
   return STS_OK;
 }
@@ -373,7 +373,7 @@ extern "C" int sts_unet_infer(sts_unet *u, int n, const float *x, float *y) {
   const size_t np = u->npix(n, 0);
   U_OK(u->copy.put(u->xin, x, sizeof(float) * np * u->cin, u->stream));
   U_OK(unet_to_bf16(u->xin, u->cin, u->Cx0, np, u->x, u->stream));
-  if ((rc = forward_dev(u, n))) return rc;
+  if ((rc = forward_dev(u, n, u->stream))) return rc;
   U_OK(u->copy.get(y, u->y, sizeof(float) * np * u->cout, u->stream));
   return STS_OK;
 }
@@ -520,7 +520,7 @@ static int batch_loss(sts_unet *u, const int *slots, int n, double *loss, bool t
   const int np = u->H * u->W;
   U_OK(hipMemcpyAsync(u->slots_dev, slots, sizeof(int) * n, hipMemcpyHostToDevice, u->stream));
   U_OK(unet_gather(u->ds_x, u->ds_t, u->ds_m, u->slots_dev, n, np, u->Cx0, u->cout, u->x, u->tg, u->mask, u->stream));
-  if ((rc = forward_dev(u, n))) return rc;
+  if ((rc = forward_dev(u, n, u->stream))) return rc;
   return loss_backward_dev(u, n, count, loss, train, train ? &lr : nullptr);
 }
 
@@ -536,12 +536,12 @@ extern "C" int sts_unet_eval(sts_unet *u, const int *slots, int n, double *loss)
 int sts_internal_unet_correct(sts_unet *u, const StsView &v, const sts_unet_corr_norm *nrm, double *const out[4]) {
   int rc = check_corrector(u, v);
   if (rc) return rc;
-  U_OK(hipStreamSynchronize(v.stream));
+  U_OK(hipStreamSynchronize(u->stream));
   const int np = v.Nx * v.Ny;
   const CorrFields xe{{v.xe[0], v.xe[1], v.xe[2], v.xe[3]}};
   U_OK(unet_pack_corr_in(state_fields(v, true), xe, v.mask, np, u->Cx0, 1.0 / nrm->u_ref, 1.0 / nrm->p_ref,
-                         1.0 / nrm->step, u->x, u->stream));
-  if ((rc = forward_dev(u, 1))) return rc;
+                         1.0 / nrm->step, u->x, v.stream));
+  if ((rc = forward_dev(u, 1, v.stream))) return rc;
   CorrBoxes bx{v.Nx, v.px, {}, {}, {}};
   for (int q = 0; q < 4; q++) {
     bx.u[q] = v.box_u[q];
@@ -549,8 +549,7 @@ int sts_internal_unet_correct(sts_unet *u, const StsView &v, const sts_unet_corr
     bx.o[q] = v.box_o[q];
   }
   U_OK(unet_apply_corr(u->y, xe, v.mask, bx, np, nrm->u_ref * nrm->corr, nrm->p_ref * nrm->corr, nrm->corr,
-                       CorrOut{{out[0], out[1], out[2], out[3]}}, u->stream));
-  U_OK(hipStreamSynchronize(u->stream));
+                       CorrOut{{out[0], out[1], out[2], out[3]}}, v.stream));
   return STS_OK;
 }
 
@@ -563,7 +562,7 @@ int sts_internal_unet_predict(sts_unet *u, const StsView &v, const sts_unet_norm
   const double *const *f = v.f;
   U_OK(unet_pack_state(f[STS_U], f[STS_V], f[STS_P], f[STS_T], v.mask, np, u->Cx0, 1.0 / nrm->u_ref, 1.0 / nrm->p_ref,
                        u->x, u->stream));
-  if ((rc = forward_dev(u, 1))) return rc;
+  if ((rc = forward_dev(u, 1, u->stream))) return rc;
   U_OK(unet_apply_pred(u->y, f[STS_P], f[STS_T], v.mask, v.Nx, np, v.box_o, nrm->p_ref * nrm->dp_scale,
                        nrm->dT_scale, pw, Tw, u->stream));
   U_OK(hipStreamSynchronize(u->stream));
