@@ -173,22 +173,22 @@ typedef struct sts_loop_control {
   double tol_uv;      /* MaxError_Velocities */
   double tol_p;       /* MaxError_p_c */
   double tol_T;       /* MaxError_T */
-  int batch;          /* outer iterations in the first batch enqueued (the host reads the loop control one
-                         iteration before a batch ends); 0 = from the last step's count */
+  int batch;          /* outer iterations enqueued before the host follows the loop test (from one iteration
+                         before their end on, then one per report of it); 0 = from the last step's count */
 } sts_loop_control;
 
 /* One time step of loop 1 (S:3230-4608): the prologue S:3233-3239, then
    outer iterations (as sts_outer_iteration) until the reference's loop-2 test
    S:4433-4437 stops them or N_I is reached.  The test is evaluated on the GPU
-   after each outer iteration; iterations are enqueued in batches and those
-   past the stopping one exit without work, so the host waits about once per
-   step.  *iterations gets Iter; res_log (may be NULL) gets 6 doubles per outer
+   after each outer iteration; a first batch of iterations is enqueued at once,
+   then one for each that the test lets pass, and those past the stopping one
+   exit without work.  *iterations gets Iter; res_log (may be NULL) gets 6 doubles per outer
    iteration: max|du|, max|dv|, max|dp|, max|dT| (last sweep), max|dp|,
    max|dT| (first sweep).  p_probe as in sts_boundary_conditions, for the last
    outer iteration.  With res_log and p_probe both NULL the call returns as
    soon as the iteration count is known, without waiting for the step's last
-   launches (the flux pass of its last iteration, iterations gated out past
-   the stop); later calls on the context queue behind them, and every call
+   launches (an accelerated loop's flux pass, an iteration gated out past the
+   stop); later calls on the context queue behind them, and every call
    that hands device data back waits for them.  Returns STS_ERR_NONFINITE if
    a residual is not finite. */
 int sts_time_step(sts_ctx *ctx, const sts_loop_control *lc, int *iterations, double *res_log, double *p_probe);

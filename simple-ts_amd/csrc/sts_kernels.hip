@@ -1854,7 +1854,7 @@ __global__ void __launch_bounds__(BX *BY) k_jump_overwrite(KGrid g, KFields fl) 
 // N arrays in one launch.  Bound by the launches where the arrays are small (four
 // copies of 512x128 as copy commands 25 us of a step, here 6).
 template <int N>
-__global__ void __launch_bounds__(BX *BY) k_copies(CopySet c, int n) {
+__device__ __forceinline__ void copy_arrays(const CopySet &c, int n) {
   const int t = (blockIdx.x + blockIdx.y * gridDim.x) * (BX * BY) + threadIdx.x + threadIdx.y * BX;
   if (t >= n) return;
   double x[N];
@@ -1863,6 +1863,8 @@ __global__ void __launch_bounds__(BX *BY) k_copies(CopySet c, int n) {
 #pragma unroll
   for (int q = 0; q < N; q++) c.dst[q][t] = x[q];
 }
+__global__ void __launch_bounds__(BX *BY) k_copy4(CopySet c, int n) { copy_arrays<4>(c, n); }
+__global__ void __launch_bounds__(BX *BY) k_copy5(CopySet c, int n) { copy_arrays<5>(c, n); }
 
 // Start of loop 2 from a linear extrapolation in time: x = 2 x^n - x^(n-1)
 // for u, v, p, T on their update sets (x^n = the *_pr fields after the
@@ -2977,7 +2979,7 @@ template <int N>
 hipError_t launch_copies(const CopySet &c, int n, hipStream_t s) {
   const int blocks = (n + BX * BY - 1) / (BX * BY);
   dim3 gr(blocks < 65535 ? blocks : 65535, (blocks + 65534) / 65535);
-  hipLaunchKernelGGL(k_copies<N>, gr, dim3(BX, BY), 0, s, c, n);
+  hipLaunchKernelGGL(N == 4 ? k_copy4 : k_copy5, gr, dim3(BX, BY), 0, s, c, n);
   return hipGetLastError();
 }
 template hipError_t launch_copies<4>(const CopySet &, int, hipStream_t);
