@@ -2033,8 +2033,8 @@ static int run_batch_loop2(sts_batch *b, BatchCase<R> *C, int n_pc, int N_I, int
   HIP_OK(launch_batch<R>(BK_LOOP_OPEN, 0, C, n, nullptr, 0, 0, 0, 0, 0, s));
   if constexpr (sizeof(R) == sizeof(double))
     if (aa_m > 0) HIP_OK(launch_batch_aa(BKA_BEGIN, cv, C, n, L.cell, L.n_cell, 0, 0, AABatchSel{}, s));
-  // the loop control is read one iteration before a batch ends (as in the
-  // single-context loop), after the last one of a batch that ends at N_I
+  // the loop control is read one iteration before a batch ends, after the last one
+  // of a batch that ends at N_I
   constexpr int LOOKAHEAD = 1;
   int k = 0;
   while (true) {

@@ -1506,9 +1506,9 @@ __global__ void __launch_bounds__(256) k_wall_plan(KGrid g, const unsigned *cell
 // ---------------------------------------------------------------------------
 // A12 edge part: Neumann copies and inflow/outflow mass conditions at the
 // solve-box edges, S:6790-7096 (velocities), S:7650-7741 (temperature),
-// S:7335-7428 (pressure).  O(Nx+Ny) work whose phases read each other's
-// results, so one workgroup runs the phases in the reference's order with a
-// barrier between them.
+// S:7335-7428 (pressure).  O(Nx+Ny) work; the phases of one field read each
+// other's results, so a workgroup runs them in the reference's order with a
+// barrier between them (which fields side by side: edges_block).
 // ---------------------------------------------------------------------------
 constexpr int EDGE_THREADS = 1024;
 
@@ -1866,9 +1866,6 @@ __device__ __forceinline__ void copy_arrays(const CopySet &c, int n) {
 __global__ void __launch_bounds__(BX *BY) k_copy4(CopySet c, int n) { copy_arrays<4>(c, n); }
 __global__ void __launch_bounds__(BX *BY) k_copy5(CopySet c, int n) { copy_arrays<5>(c, n); }
 
-// Start of loop 2 from a linear extrapolation in time: x = 2 x^n - x^(n-1)
-// for u, v, p, T on their update sets (x^n = the *_pr fields after the
-// prologue); x^(n-1) (prev) then takes x^n.
 // Polynomial extrapolation in time of degree `order` through x^n and the
 // stored steps, as Newton's backward-difference sum x0 + D1 + ... + Dq
 // (D1 = x0 - x1, D(k+1) = Dk(x0) - Dk(x1)), so that a value constant in time
