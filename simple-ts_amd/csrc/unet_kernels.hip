@@ -576,16 +576,26 @@ __global__ void __launch_bounds__(128 * WCI * WCO, MT == 4 ? 2 : 4) k_wgrad(Wgra
   }
 }
 
-// Sums of slots of FP32 partial sums, one slot after the other in FP32 (the
-// order in which the atomics they replaced mostly came): out[e] = sum of
-// part[q * P + e], q < S, onto out's own value unless `first`; P a multiple of 4.
+// Sums of slots of FP32 partial sums, one slot after the other in FP32: out[e] =
+// sum of part[q * P + e], q < S, onto out's own value unless `first`; P a multiple
+// of 4.  The order is the one in which runs that start together end: a last run
+// of at most three quarters of the others' length first (`ragged`: its slot is the
+// last), then from the first one on.  Another order gives other last bits (1e-7 of
+// a gradient's norm), and an Adam step shows them.  FP32 parameters that differ after
+// one step from those of sums by atomics, in order of arrival: at 5 x 72 x 192 samples
+// and base 32 1,540 of 1.9 million (8,800 with the short run last; two runs of the
+// atomics 1,400), at 8 x 512 x 128 3,900 (3,800).
 //
 // Many slots: a workgroup takes 256 consecutive e; wave y has slots SUM_SLOTS y ..
 // of SUM_WAVES * SUM_SLOTS at a time in registers, all loads in flight, and the
 // waves add theirs in turn.
 constexpr int SUM_WAVES = 8, SUM_SLOTS = 16;
 
-__device__ __forceinline__ void sum_turns(const float *part, int S, size_t P, bool first, float *out, int group) {
+// The q-th slot of the sum's order.
+__device__ __forceinline__ int slot_at(int q, int S, bool ragged) { return !ragged ? q : q == 0 ? S - 1 : q - 1; }
+
+__device__ __forceinline__ void sum_turns(const float *part, int S, size_t P, bool first, bool ragged, float *out,
+                                          int group) {
   __shared__ floatx4 run[64];
   const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
   const size_t e = 4 * ((size_t)group * 64 + x);
@@ -595,7 +605,8 @@ __device__ __forceinline__ void sum_turns(const float *part, int S, size_t P, bo
     floatx4 v[SUM_SLOTS];
 #pragma unroll
     for (int k = 0; k < SUM_SLOTS; k++)
-      v[k] = *reinterpret_cast<const floatx4 *>(part + (size_t)min(q0 + SUM_SLOTS * y + k, S - 1) * P + (in ? e : 0));
+      v[k] = *reinterpret_cast<const floatx4 *>(
+          part + (size_t)slot_at(min(q0 + SUM_SLOTS * y + k, S - 1), S, ragged) * P + (in ? e : 0));
     for (int w = 0; w < SUM_WAVES; w++) {
       __syncthreads();
       if (w != y) continue;
@@ -611,14 +622,16 @@ __device__ __forceinline__ void sum_turns(const float *part, int S, size_t P, bo
 }
 
 // Few slots: a thread takes 4 consecutive e, 8 slots' loads at a time.
-__device__ __forceinline__ void sum_each(const float *part, int S, size_t P, bool first, float *out, int group) {
+__device__ __forceinline__ void sum_each(const float *part, int S, size_t P, bool first, bool ragged, float *out,
+                                         int group) {
   const size_t e = 4 * ((size_t)group * (64 * SUM_WAVES) + threadIdx.x);
   if (e >= P) return;
   floatx4 s = first ? (floatx4)0.f : *reinterpret_cast<const floatx4 *>(out + e);
   for (int q0 = 0; q0 < S; q0 += 8) {
     floatx4 v[8];
 #pragma unroll
-    for (int k = 0; k < 8; k++) v[k] = *reinterpret_cast<const floatx4 *>(part + (size_t)min(q0 + k, S - 1) * P + e);
+    for (int k = 0; k < 8; k++)
+      v[k] = *reinterpret_cast<const floatx4 *>(part + (size_t)slot_at(min(q0 + k, S - 1), S, ragged) * P + e);
 #pragma unroll
     for (int k = 0; k < 8; k++)
       if (q0 + k < S) s += v[k];
@@ -632,18 +645,19 @@ struct SumArgs {
   const float *part;
   int S;
   size_t P;
-  bool each, first;
+  bool each, first, ragged;
   float *out;
   int groups;
   const float *rpart;
   int rS, rP;
+  bool rragged;
   float *rout;
 };
 __global__ void __launch_bounds__(64 * SUM_WAVES) k_sum_parts(SumArgs a) {
   const int q = (int)blockIdx.x - a.groups;
-  if (q >= 0) sum_turns(a.rpart, a.rS, a.rP, true, a.rout, q);
-  else if (a.each) sum_each(a.part, a.S, a.P, a.first, a.out, blockIdx.x);
-  else sum_turns(a.part, a.S, a.P, a.first, a.out, blockIdx.x);
+  if (q >= 0) sum_turns(a.rpart, a.rS, a.rP, true, a.rragged, a.rout, q);
+  else if (a.each) sum_each(a.part, a.S, a.P, a.first, a.ragged, a.out, blockIdx.x);
+  else sum_turns(a.part, a.S, a.P, a.first, a.ragged, a.out, blockIdx.x);
 }
 
 // out[e] = sum of part[q * P + e], q < S, for few e, in FP64 (as good as exact):
@@ -1110,6 +1124,7 @@ hipError_t unet_conv(const ConvArgs &a, hipStream_t s) {
 // 32 x 32, that read the pixels twice as often, 48).
 constexpr long WGRAD_FULL = 128;
 constexpr int SUM_EACH = 32;
+static bool short_last(int npix, int run) { return npix % run != 0 && 4 * (npix % run) <= 3 * run; }
 
 hipError_t unet_wgrad(const WgradArgs &a, float *dW, float *db, hipStream_t s) {
   if (a.W % 8 || a.Cx % 8 || a.Cout % 8 || (a.X2 && a.Cb % 8)) return hipErrorInvalidValue;
@@ -1134,7 +1149,8 @@ hipError_t unet_wgrad(const WgradArgs &a, float *dW, float *db, hipStream_t s) {
     else if (a.X2) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, true>), gr, dim3(512), 0, s, a, q, n);
     else if (CI == 32) hipLaunchKernelGGL((k_wgrad<2, 2, 1, 2, false>), gr, dim3(512), 0, s, a, q, n);
     else hipLaunchKernelGGL((k_wgrad<1, 2, 1, 4, false>), gr, dim3(256), 0, s, a, q, n);
-    const SumArgs b{a.part, n, P, each, q == 0, dW, nsum, a.bpart, (int)nblk(npix, WG_BIAS), a.Cout, db};
+    const SumArgs b{a.part, n, P, each, q == 0, last && short_last(npix, WG_RUN), dW, nsum,
+                    a.bpart, (int)nblk(npix, WG_BIAS), a.Cout, short_last(npix, WG_BIAS), db};
     hipLaunchKernelGGL(k_sum_parts, dim3(nsum + (last ? nblk(a.Cout, 256) : 0)), dim3(64 * SUM_WAVES), 0, s, b);
   }
   return hipGetLastError();
