@@ -1126,17 +1126,18 @@ static int run_loop2(sts_ctx *c, Loop2State<R> &st, R *&p, R *&T, R *&p_alt, R *
   batch = std::min(batch, lt.N_I);
   lt.host_from = batch - 2;
   *(volatile unsigned long long *)c->h_loop = 0ull;
-  int rc;
+  int rc = STS_OK;
   unsigned long long word = 0;
-  for (int k = 0; k < lt.N_I && !(word & LOOP_STOPPED); k++) {
-    if (k >= batch && ((rc = wait_loop(c, k - 1, &word)) || (word & LOOP_STOPPED))) {
-      if (rc) return rc;
-      break;
-    }
-    if ((rc = enqueue_outer(c, st, k, n_pc, lt))) return rc;
+  for (int k = 0; k < lt.N_I && !rc; k++) {
+    if (k >= batch && ((rc = wait_loop(c, k - 1, &word)) || (word & LOOP_STOPPED))) break;
+    rc = enqueue_outer(c, st, k, n_pc, lt);
   }
-  if ((rc = wait_loop(c, lt.N_I, &word))) return rc;
-  if (!(word & LOOP_STOPPED)) return fail(STS_ERR_ARG, "loop 2 did not stop at N_I");  // the test always stops there
+  if (!rc) rc = wait_loop(c, lt.N_I, &word);
+  if (!rc && !(word & LOOP_STOPPED)) rc = fail(STS_ERR_ARG, "loop 2 did not stop at N_I");  // the test always stops there
+  if (rc) {
+    (void)hipStreamSynchronize(c->stream);  // iterations in flight would report to the next loop's word
+    return rc;
+  }
   const int stop = (int)(unsigned)word - 1;
   timed_loop_close(c, stop);
   *iters = stop + 1;
