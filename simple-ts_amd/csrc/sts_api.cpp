@@ -1340,8 +1340,8 @@ static int copy_start(sts_ctx *c, hipStream_t s, bool back = false) {
 
 // The start of a step (S:3233-3239 and, with order > 0, the polynomial of degree
 // `order`, capped by the stored steps and degree_cap, through x^n and the previous
-// converged steps for u, v, p, T; store_only: stored, not used), and the
-// history's advance by it.
+// converged steps for u, v, p, T; store_only: stored, not used).  Once its launch
+// has been accepted, advance_history makes the level that takes x^n level 0.
 static int plan_start(sts_ctx *c, int order, bool store_only, int degree_cap, BeginArgs *out) {
   BeginArgs &a = *out;
   a = BeginArgs{};
@@ -1353,26 +1353,29 @@ static int plan_start(sts_ctx *c, int order, bool store_only, int degree_cap, Be
     a.x[q] = c->f[x[q]];
     a.pr[q] = c->f[pr[q]];
   }
-  if (order <= 0) {
-    c->n_hist = 0;
-    return STS_OK;
-  }
+  if (order <= 0) return STS_OK;
   if (order > MAX_EXTRAP) return fail(STS_ERR_ARG, "extrapolation degree must be 0..5");
   const size_t bytes = sizeof(double) * (size_t)c->Na;
-  if (!c->hist.f[0][0])
-    for (auto &lv : c->hist.f)
-      for (double *&q : lv) HIP_OK(hipMalloc(&q, bytes));
-  // `order` past steps are kept: x^n goes to a free level, or over the oldest
-  // one, and that level becomes level 0 (the rest move down by renaming)
-  const int keep = std::min(c->n_hist, order), slot = keep < order ? keep : order - 1;
+  for (auto &lv : c->hist.f)
+    for (double *&q : lv)
+      if (!q) HIP_OK(hipMalloc(&q, bytes));
+  // `order` past steps are kept: x^n goes to a free level, or over the oldest one
+  const int keep = std::min(c->n_hist, order);
   a.order = store_only ? 0 : std::min(keep, degree_cap);
   a.hist = c->hist;
-  for (int q = 0; q < 4; q++) a.to[q] = c->hist.f[slot][q];
-  for (int h = slot; h > 0; h--)
-    for (int q = 0; q < 4; q++) c->hist.f[h][q] = c->hist.f[h - 1][q];
-  for (int q = 0; q < 4; q++) c->hist.f[0][q] = a.to[q];
-  c->n_hist = std::min(keep + 1, order);
+  for (int q = 0; q < 4; q++) a.to[q] = c->hist.f[std::min(keep, order - 1)][q];
   return STS_OK;
+}
+
+// The level that took x^n becomes level 0, the rest move down by renaming.
+static void advance_history(sts_ctx *c, int order) {
+  const int keep = order > 0 ? std::min(c->n_hist, order) : 0, slot = std::min(keep, order - 1);
+  for (int q = 0; q < 4 && slot >= 0; q++) {
+    double *const to = c->hist.f[slot][q];
+    for (int h = slot; h > 0; h--) c->hist.f[h][q] = c->hist.f[h - 1][q];
+    c->hist.f[0][q] = to;
+  }
+  c->n_hist = order > 0 ? std::min(keep + 1, order) : 0;
 }
 
 // The same, run: every field derived from a predicted start is rebuilt the way
@@ -1384,6 +1387,7 @@ static int begin_step(sts_ctx *c, int order, bool store_only = false, int degree
   if (used) *used = 0;
   if ((rc = plan_start(c, order, store_only, degree_cap, &a))) return rc;
   HIP_OK(launch_begin(a, c->stream));
+  advance_history(c, order);
   if (used) *used = a.order;
   if (a.order > 0 && (rc = rebuild_derived(c, c->stream))) return rc;
   return copy_start(c, c->stream);
@@ -2165,6 +2169,7 @@ extern "C" int sts_batch_time_step(sts_batch *b, const sts_loop_control *lc, con
   HIP_OK(hipMemcpyAsync(b->begin, begin.data(), sizeof(BeginArgs) * n, hipMemcpyHostToDevice, s));
   const int cv = b->cell_v;
   HIP_OK(launch_batch_begin(cv, b->begin, b->cell_t[cv], b->n_cell[cv], s));
+  for (sts_ctx *c : b->cs) advance_history(c, mc ? mc->extrapolate : 0);
   if (any) {
     if ((rc = upload_cases<double>(b, b->C64, 1, 0, 0, 0, 0, 0.0, 0, false, &from_xn))) return rc;
     HIP_OK(launch_batch<double>(BK_DERIVE, cv, b->C64, n, b->cell_t[cv], b->n_cell[cv], 0, 0, 0, 0, s));

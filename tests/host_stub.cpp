@@ -47,8 +47,16 @@ void stub_fail(const char *name, int n) { fails[name] = n; }
 void stub_clear() { fails.clear(), begins.clear(); }
 void stub_stop(int iterations) { stop_after = iterations; }
 int stub_begins() { return (int)begins.size(); }
-int stub_order(int q) { return begins[q].order; }                                 // degree of the q-th start
-int stub_kept(int q) { return begins[q].to[0] == begins[q].hist.f[0][0] ? 0 : 1; }  // level that takes x^n
+int stub_order(int q) { return begins[q].order; }  // degree of the q-th start
+int stub_whole(int q) {                            // its levels are there, the one that takes x^n and those it reads
+  const BeginArgs &a = begins[q];
+  for (int f = 0; f < 4; f++) {
+    if (!a.to[f]) return 0;
+    for (int h = 0; h < a.order; h++)
+      if (!a.hist.f[h][f]) return 0;
+  }
+  return 1;
+}
 
 hipError_t hipMalloc(void **p, size_t n) {
   hipError_t e = call("hipMalloc");

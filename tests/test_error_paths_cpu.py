@@ -63,3 +63,43 @@ def test_loop_after_a_failed_one(stub, gpu, call):
         step()
     gpu.stub_stop(6)
     assert step() == 6
+
+
+def starts(gpu, step, n):
+    """The degrees of the starts of n steps."""
+    first = gpu.stub_begins()
+    for _ in range(n):
+        step()
+    assert all(gpu.stub_whole(q) for q in range(first, gpu.stub_begins()))
+    return [gpu.stub_order(q) for q in range(first, gpu.stub_begins())]
+
+
+@pytest.mark.parametrize("call,n", [("launch_begin", 1), ("hipMalloc", 6)])
+def test_predicted_start_after_a_failed_one(stub, gpu, call, n):
+    """A start that was not made counts for no step of the history, and an
+    allocation that failed is made good."""
+    ctx = context(stub)
+
+    def step(degree=3):
+        ctx.time_step_mixed(20, 2, *TOL, 0, TOL, extrapolate=degree, wait=False)
+
+    step(0)  # the loops' own buffers
+    gpu.stub_fail(call.encode(), n)
+    with pytest.raises(stub.StsError):
+        step()
+    assert starts(gpu, step, 5) == [0, 1, 2, 3, 3]
+
+
+@pytest.mark.parametrize("call,n", [("launch_batch_begin", 1), ("hipMalloc", 26)])
+def test_batched_starts_after_a_failed_one(stub, gpu, call, n):
+    """As above for two cases; the 26th allocation is one of the second case's."""
+    batch = stub.Batch([context(stub) for _ in range(2)])
+
+    def step(degree=3):
+        batch.time_step(20, 2, *TOL, mixed=(0, TOL, 0, 0.95, degree))
+
+    step(0)
+    gpu.stub_fail(call.encode(), n)
+    with pytest.raises(stub.StsError):
+        step()
+    assert starts(gpu, step, 5) == [0, 0, 1, 1, 2, 2, 3, 3, 3, 3]
