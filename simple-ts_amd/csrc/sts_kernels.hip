@@ -2775,8 +2775,9 @@ __global__ void __launch_bounds__(EDGE_THREADS) kb_edges(const BatchCase<R> *C, 
   const Gate gate{c.ctrl, k};
   if (k < 0 ? c.skip != 0 : gated_out(gate)) return;  // k < 0: after kb_derive
   const KFieldsT<R> f = fields_at(c, par);
-  const LoopTest lt{in_memory(c.ctrl), in_memory(c.lred), in_memory(c.log) + 6 * (size_t)max(k, 0), c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w,
-                    c.stall_ratio, nullptr, 0};
+  // (no loop is open after kb_derive: no test of it)
+  const LoopTest lt{k < 0 ? nullptr : in_memory(c.ctrl), in_memory(c.lred), in_memory(c.log) + 6 * (size_t)max(k, 0),
+                    c.N_I, c.tol_uv, c.tol_p, c.tol_T, c.stall_w, c.stall_ratio, nullptr, 0};
   edges_block(grid_of(c), f, parts, true, k < 0 ? nullptr : in_memory(c.probe), gate, lt, (int)(blockIdx.x % EDGE_GROUPS));
 }
 
