@@ -1612,29 +1612,18 @@ __device__ __forceinline__ void loop_test_wave(const Gate &gate, const LoopTest 
   }
 }
 
-// The conditions of the two ends of a direction touch disjoint cells when the
-// box between them is not empty (b0 < b1): they run together, else one after
-// the other.
+// The conditions of the two ends of a direction together: the box between them is
+// not empty (sts_create), so they touch disjoint cells.
 template <typename R>
 __device__ __forceinline__ void edges_x(const KGridT<R> &g, R *a, int b0, int b1, bool lo, bool hi) {
   if (!lo && !hi) return;
-  if (b0 < b1) edge_x(g, a, b0, b1, lo, hi);
-  else {
-    edge_x(g, a, b0, b1, lo, false);
-    __syncthreads();
-    edge_x(g, a, b0, b1, false, hi);
-  }
+  edge_x(g, a, b0, b1, lo, hi);
   __syncthreads();
 }
 template <typename R>
 __device__ __forceinline__ void edges_y(const KGridT<R> &g, R *a, int b0, int b1, bool lo, bool hi) {
   if (!lo && !hi) return;
-  if (b0 < b1) edge_y(g, a, b0, b1, lo, hi);
-  else {
-    edge_y(g, a, b0, b1, lo, false);
-    __syncthreads();
-    edge_y(g, a, b0, b1, false, hi);
-  }
+  edge_y(g, a, b0, b1, lo, hi);
   __syncthreads();
 }
 
@@ -1685,46 +1674,41 @@ __device__ void edges_block(const KGridT<R> &g, const KFieldsT<R> &fl, int parts
   if ((parts & STS_BC_VELOCITIES) && group == 0) {
     R *u = FLD(U);
     const R *v = FLD(V), *rho = FLD(RHO), *rho_pr = FLD(RHO_PR), *rho_u = FLD(RHO_U), *rho_v = FLD(RHO_V);
-    const bool apart = g.Nx_u0 < g.Nx_u1;  // (as edges_x)
-    for (int side = apart ? 2 : 0; side < (apart ? 3 : 2); side++) {  // 0 = XB, 1 = XE, 2 = both
-      const unsigned on = bc & ((side != 1 ? BC_DUDX_XB | BC_DURHODX_XB | BC_DRHODT_XB : 0u) |
-                                (side != 0 ? BC_DUDX_XE | BC_DURHODX_XE | BC_DRHODT_XE | BC_UMINMOUT_XE : 0u));
-      edges_x(g, u, g.Nx_u0, g.Nx_u1, on & BC_DUDX_XB, on & BC_DUDX_XE);
-      if (on & (BC_DURHODX_XB | BC_DURHODX_XE)) {
-        for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-          int node = g.Nx_u0 - 1 + j * Nx;
-          if ((on & BC_DURHODX_XB) && m[node]) u[node] = (rho_u[node + 1] * u[node + 1]) / rho_u[node];
-          node = g.Nx_u1 - 1 + j * Nx;
-          if ((on & BC_DURHODX_XE) && m[node]) u[node + 1] = (rho_u[node] * u[node]) / rho_u[node + 1];
-        }
-        __syncthreads();
+    edges_x(g, u, g.Nx_u0, g.Nx_u1, bc & BC_DUDX_XB, bc & BC_DUDX_XE);
+    if (bc & (BC_DURHODX_XB | BC_DURHODX_XE)) {
+      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
+        int node = g.Nx_u0 - 1 + j * Nx;
+        if ((bc & BC_DURHODX_XB) && m[node]) u[node] = (rho_u[node + 1] * u[node + 1]) / rho_u[node];
+        node = g.Nx_u1 - 1 + j * Nx;
+        if ((bc & BC_DURHODX_XE) && m[node]) u[node + 1] = (rho_u[node] * u[node]) / rho_u[node + 1];
       }
-      if (on & (BC_DRHODT_XB | BC_DRHODT_XE)) {
-        for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-          int i = g.Nx_u0 - 1, node = i + j * Nx;
-          if ((on & BC_DRHODT_XB) && m[node] && j + 1 < Ny)
-            u[node] = ((rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
-                       + (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
-                       + rho_u[node + 1] * u[node + 1] * hy[j])
-                      / (rho_u[node] * hy[j]);
-          i = g.Nx_u1 - 1, node = i + j * Nx;
-          if ((on & BC_DRHODT_XE) && m[node] && j + 1 < Ny)
-            u[node + 1] = (-(rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
-                           - (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
-                           + rho_u[node] * u[node] * hy[j])
-                          / (rho_u[node + 1] * hy[j]);
-        }
-        __syncthreads();
+      __syncthreads();
+    }
+    if (bc & (BC_DRHODT_XB | BC_DRHODT_XE)) {
+      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
+        int i = g.Nx_u0 - 1, node = i + j * Nx;
+        if ((bc & BC_DRHODT_XB) && m[node] && j + 1 < Ny)
+          u[node] = ((rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
+                     + (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
+                     + rho_u[node + 1] * u[node + 1] * hy[j])
+                    / (rho_u[node] * hy[j]);
+        i = g.Nx_u1 - 1, node = i + j * Nx;
+        if ((bc & BC_DRHODT_XE) && m[node] && j + 1 < Ny)
+          u[node + 1] = (-(rho[node] - rho_pr[node]) * hx[i] * hy[j] / g.ht
+                         - (rho_v[node + Nx] * v[node + Nx] - rho_v[node] * v[node]) * hx[i]
+                         + rho_u[node] * u[node] * hy[j])
+                        / (rho_u[node + 1] * hy[j]);
       }
-      if (on & BC_UMINMOUT_XE) {  // S:7031-7059 (serial build): the last row's rho_u
-        const R Min = rho_u[g.Nx_u0 + (Ny - 1) * Nx];
-        const R Mout = rho_u[g.Nx_u1 + (Ny - 1) * Nx];
-        for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
-          int node = g.Nx_u1 - 1 + j * Nx;
-          u[node + 1] = u[node] * Min / Mout;
-        }
-        __syncthreads();
+      __syncthreads();
+    }
+    if (bc & BC_UMINMOUT_XE) {  // S:7031-7059 (serial build): the last row's rho_u
+      const R Min = rho_u[g.Nx_u0 + (Ny - 1) * Nx];
+      const R Mout = rho_u[g.Nx_u1 + (Ny - 1) * Nx];
+      for (int j = threadIdx.x; j < Ny; j += EDGE_THREADS) {
+        int node = g.Nx_u1 - 1 + j * Nx;
+        u[node + 1] = u[node] * Min / Mout;
       }
+      __syncthreads();
     }
     edges_y(g, u, g.Ny_u0, g.Ny_u1, bc & BC_DUDY_YB, bc & BC_DUDY_YE);
     if (flux) {  // likewise, u
