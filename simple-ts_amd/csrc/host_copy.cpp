@@ -57,6 +57,15 @@ void populate(void *p, size_t bytes) {
 #endif
 }
 
+// Whether the runtime knows the array (pinned, managed or device memory): its own
+// copy is then one transfer, at the rate of one into pinned_.
+bool known(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Helper threads on the pieces, joined when it goes out of scope (their pieces
 // are then copied); fewer when the system gives fewer.
 struct Helpers {
@@ -105,7 +114,7 @@ void HostCopy::release() {
 hipError_t HostCopy::get(void *host, const void *dev, size_t bytes, hipStream_t s) {
   std::lock_guard<std::mutex> hold(lock_);
   hipError_t e = hipSuccess;
-  if (!pinned_) {
+  if (!pinned_ || known(host)) {
     e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
@@ -140,7 +149,7 @@ hipError_t HostCopy::get(void *host, const void *dev, size_t bytes, hipStream_t 
 hipError_t HostCopy::put(void *dev, const void *host, size_t bytes, hipStream_t s) {
   std::lock_guard<std::mutex> hold(lock_);
   hipError_t e = hipSuccess;
-  if (!pinned_) {
+  if (!pinned_ || known(host)) {
     e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }

@@ -1,5 +1,6 @@
-// Copies between device memory and a caller's pageable host arrays, through
-// pinned memory that the object owning the stream keeps (host_copy.cpp).
+// Copies between device memory and a caller's host arrays: pageable ones through
+// pinned memory that the object owning the stream keeps (host_copy.cpp), others
+// as they are.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
