@@ -10,6 +10,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -1085,12 +1086,17 @@ static int enqueue_outer(sts_ctx *c, const Loop2State<R> &st, int k, int n, Loop
   return aa ? enqueue_anderson(c, st, kf, k, sel) : STS_OK;
 }
 
-// Waits until the loop test has reported `done` iterations or the loop's end.
+// Waits until the loop test has reported `done` iterations or the loop's end:
+// looks at the word, lets another thread have the processor after every 64 looks
+// (other contexts' loops wait and enqueue too), and asks for the stream's state
+// after 65536.
 static int wait_loop(sts_ctx *c, int done, unsigned long long *word) {
   volatile unsigned long long *w = c->h_loop;
   for (unsigned spin = 1;; spin++) {
     *word = *w;
     if ((*word & LOOP_STOPPED) || (int)(unsigned)*word >= done) return STS_OK;
+    __builtin_ia32_pause();
+    if (spin % 64 == 0) std::this_thread::yield();
     if (spin % 65536) continue;
     const hipError_t e = hipStreamQuery(c->stream);  // a failed stream reports nothing more
     if (e == hipErrorNotReady) {
