@@ -2868,10 +2868,12 @@ template <typename R>
 hipError_t launch_sweep2(const KGridT<R> &g, const KFieldsT<R> &f, const R *Po, const R *To, R *Pn, R *Tn,
                          unsigned long long *r1p, unsigned long long *r1T, unsigned long long *r2p,
                          unsigned long long *r2T, hipStream_t s, Gate gate) {
-  // 6 rows per tile; 2 where that leaves most of the 256 CUs without a
-  // workgroup (240x48, 32 tiles of 6 rows: 5.7 against 6.6 us; 301x95, 96
-  // tiles: 6.3 against 6.6; 512x128, 198 tiles: 7.3 against 6.6)
-  if (grid_tiles<SWEEP_X, 6>(g).x < 64)
+  // 6 rows per tile; 2 while those give at most two workgroups to each of the 256
+  // CUs, where a tile's chain counts and not what it reads twice (kernel trace, 2
+  // against 6 rows: 240x48 5.7 and 6.9 us, 301x95 6.7 and 7.0, 360x96 6.6 and 6.8,
+  // 480x120, 480 tiles of 2 rows, 6.75 and 6.9; 512x128, 576 tiles, 7.7 and 7.0,
+  // 600x140 7.85 and 6.9)
+  if (grid_tiles<SWEEP_X, 2>(g).x <= 512)
     hipLaunchKernelGGL((k_sweep2<R, 2>), (grid_tiles<SWEEP_X, 2>(g)), dim3(SweepTile<2>::THREADS), 0, s, g, f, Po, To,
                        Pn, Tn, r1p, r1T, r2p, r2T, gate);
   else
