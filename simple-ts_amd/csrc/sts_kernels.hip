@@ -1056,8 +1056,8 @@ __global__ void __launch_bounds__((SweepTile<SR>::THREADS)) __attribute__((amdgp
 // ij needs rho of the west/south cell; it is recomputed here from p and T
 // with the same operations, so no second pass is needed.
 // ---------------------------------------------------------------------------
-// The pass in two phases, so that a thread can issue the loads of several
-// cells before it computes any of them.  FLUX: with it the fluxes and thermal
+// The pass in two phases, a cell's loads before what is computed from them (the
+// second also runs on an Anderson mix's values).  FLUX: with it the fluxes and thermal
 // diffusion coefficients (S:10440-10618) of the corrected state, whose
 // inputs at the cell and its west and south neighbours are all here.  What
 // the wall and edge conditions change after it (u, v at wall faces and box
@@ -1853,8 +1853,7 @@ __global__ void __launch_bounds__(BX *BY) k_copy5(CopySet c, int n) { copy_array
 // Polynomial extrapolation in time of degree `order` through x^n and the
 // stored steps, as Newton's backward-difference sum x0 + D1 + ... + Dq
 // (D1 = x0 - x1, D(k+1) = Dk(x0) - Dk(x1)), so that a value constant in time
-// (fixed inflow, outflow pressure, body values) is kept exactly; then the
-// history shifts (keep = number of levels stored).  Every cell is
+// (fixed inflow, outflow pressure, body values) is kept exactly.  Every cell is
 // extrapolated: besides the update sets, the cells the boundary conditions
 // copy into (e.g. the inflow pressure, which sets the inflow density) carry
 // the step's slowest-converging change.
