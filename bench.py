@@ -49,14 +49,14 @@ L2 error against the fp64 path after the W + K steps are reported beside it.
 
 roofline (plain FP64 program, timed steps only): the kernel with the largest
 share of the outer iteration's time, the coefficient assembly of the loops
-(k_assemble_inl: u and v pseudo-velocities and the energy source), at the
-reference-formula bytes of A2 + A3 + A4, 128 + 128 + 40 = 296 B per cell
-(12 + 12 + 4 arrays read, 4 + 4 + 1 written, 8 B each, shared arrays counted
-once per equation) over all Nx*Ny cells, divided by its average launch
-duration from HIP events around every launch in the timed region that did
-work (launches that the device-side loop gates out past its stop are not
-counted), against the 8 TB/s HBM peak.  Beside it, frac_measured: the bytes
-one launch really moves (traffic) over the same duration.  traffic comes from
+(k_assemble_inl: u and v pseudo-velocities and the energy source), at 170 B per
+cell, each distinct array of its three equations once (12 arrays read, 9
+written, 8 B each, and a 2-byte word of neighbour bits), over all Nx*Ny cells,
+divided by its average launch duration from HIP events around every launch in
+the timed region that did work (launches that the device-side loop gates out
+past its stop are not counted), against the 8 TB/s HBM peak.  Beside it,
+frac_measured: the bytes one launch really moves (traffic) over the same
+duration.  traffic comes from
 two rocprofv3 counter passes over a 3-step run of the same case (FETCH_SIZE,
 then WRITE_SIZE, median KiB per working launch), each scaled by what the
 counter reports for the 5-array copy of the time-step prologue (k_copy5, 5 x
@@ -94,10 +94,11 @@ NX, NY = 1920, 384
 RE, KN = 1415.0, 0.00283
 DT_OVER_TIN = 0.01 * 240 / NX
 HBM_PEAK_GBS = 8000.0
-# FP64 reference-formula bytes per cell: assembly A2 + A3 + A4; the fused
-# pass of two p/T sweeps reads Fx Fy DTx DTy T_old p_old u v ScT1 rho apx apy
+# FP64 bytes per cell, each distinct array once: the loops' assembly reads Fx Fy
+# u v sqrt_T rho rho_pr u_pr v_pr p_pr rho_u rho_v and the neighbour bits and
+# writes its 9 results; the fused pass of two p/T sweeps reads Fx Fy DTx DTy T_old p_old u v ScT1 rho apx apy
 # bpx bpy p_pr T_pr once and writes T p once
-ASSEMBLE_BYTES_PER_CELL = 128 + 128 + 40
+ASSEMBLE_BYTES_PER_CELL = 8 * (12 + 9) + 2
 SWEEP2_BYTES_PER_CELL = 144
 CPU_STEPS = 2  # steps of the CPU sample (after one restart step)
 WEIGHTS = os.path.join(ROOT, "simple-ts_amd", "unet_corr_b32.npz")
