@@ -770,7 +770,7 @@ __device__ __forceinline__ void assemble_inl_tile(const KGridT<R> &g, const KFie
 }
 
 // Tile of the loops' assembly: 64 x 8 cells at six waves per SIMD (80
-// registers; 51.8 KB of LDS, three workgroups per CU).  Its 172 bytes per cell
+// registers; 51.8 KB of LDS, three workgroups per CU).  Its 170 bytes per cell
 // and its FP64 instructions take about as long (1920 x 384: 19 us at the rate
 // of a copy that fits the last-level cache, 12 us at four cycles per wave
 // instruction); what counts is that both overlap.  Waves without a wall in
@@ -953,8 +953,8 @@ __global__ void __launch_bounds__(BX *BY) k_sweep(KGridT<R> g, KFieldsT<R> fl, c
 // issues 25 (34 with every neighbour loaded), all waves in one phase, where a
 // workgroup of whole-tile threads ran the halo ring first and its own cells
 // after it; each cell's factors stay in registers for the second sweep.
-// Tile of 6 rows at seven waves per SIMD (72 registers), k_sweep2 with the
-// ring phase before: 1920x384 28.8 -> 23.2 us, 3840x768 141.7 -> 118.6,
+// Tile of 6 rows at seven waves per SIMD (72 registers), against tiles with such a
+// ring phase: 1920x384 28.8 -> 23.2 us, 3840x768 141.7 -> 118.6,
 // 1500x375 24.7 -> 19.5, 1280x256 17.6 -> 13.4, 961x193 13.3 -> 10.5, 301x95
 // 9.0 -> 6.6.  Other heights at 1920x384: 2 rows 26.7, 4 26.8, 5 24.9, 8 27.1, 10
 // 24.3, 14 29.4; 64 registers (eight waves) spill, 33.2.
@@ -1632,9 +1632,9 @@ __device__ __forceinline__ void edges_y(const KGridT<R> &g, R *a, int b0, int b1
 // kind), and the loop test reads only the residual words, so five workgroups run
 // them side by side: group 0 = u (after v where it reads v), 1 = temperature, 2 =
 // pressure and the probe, 3 = v, 4 = loop test.  Bound by the chain of a group's
-// phases, each a load, a store and a barrier: 240x48 4.3 -> 3.4 us, 1920x384 5.0
-// -> 4.1 us with u and v apart, the two ends of a direction together and no
-// barrier for a condition that is off.
+// phases, each a load, a store and a barrier: 240x48 4.3 -> 3.2 us with u and v
+// apart, the two ends of a direction together and no barrier for a condition that
+// is off; 1920x384 5.0 us either way (there the loop test is the longest group).
 constexpr int EDGE_GROUPS = 5;
 
 template <typename R>
@@ -2337,7 +2337,7 @@ __device__ __forceinline__ void aa_mix_tile(const KGridT<R> &g, const KFieldsT<R
 constexpr int AA_MIX_TX = 64, AA_MIX_TY = 8;
 // Tiles per workgroup: one while the tiles fit the workgroups the GPU holds at
 // once (256 CUs x 3), so that small grids spread over the CUs and no tile
-// waits for another (three tiles each before: 301x95 12.4 against 6.6 us,
+// waits for another (with three tiles each: 301x95 12.4 against 6.6 us,
 // 961x193 14.8 against 10.5); then as few as give about one such round, at
 // most 4, to fold the partial sums less often (1920x384, 1440 tiles: 21.6,
 // 21.4, 22.0 us with 1, 2, 3, at depth 2 27.6 against 30.4 with 2 and 3;

@@ -157,12 +157,11 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
 // output's sum still runs over the chunks, then the taps in order.
 //
 // Large images are bound by LDS reads and the chunks' loads in about equal parts
-// (1920 x 384: 32 -> 32 channels 61 -> 35 us, 94 MB; 96 -> 32 90 -> 59 us, 34 us of
-// MFMAs at the rate of a large product); small ones by the chain of a chunk
-// (512 x 128: 24 us per layer before, 6 .. 17 now): the tile shrinks until there
-// is a workgroup per CU, and two chunks are in flight.  Before, a lane's loads
-// stood behind the branches of the image's edge and were waited for one by one,
-// and a wave read every input fragment once per tap.
+// (1920 x 384: 32 -> 32 channels 35 us, 94 MB; 96 -> 32 59 us, 34 us of MFMAs at
+// the rate of a large product); small ones by the chain of a chunk (512 x 128: 6 ..
+// 17 us per layer): the tile shrinks until there is a workgroup per CU, and two
+// chunks are in flight.  With loads behind branches at the image's edge, which are
+// waited for one by one, and every input fragment read once per tap: 61, 90 and 24 us.
 // ---------------------------------------------------------------------------
 constexpr int CONV_CI = 32;
 
@@ -379,14 +378,13 @@ __global__ void __launch_bounds__(256) k_conv_few(ConvArgs a) {
 // 4 pixels), and a tap's shift is then only another pixel address.  The workgroup
 // leaves its sums in its own slot of `part` (laid out as the gradient is);
 // k_sum_parts adds the slots in their order: no atomics, and the same gradients on
-// every run.  The runs' length and the order within them, for the bias too, are those
-// the sums always had: each slot holds the same bits as before.
+// every run.
 //
 // The bound is the chain of a step (LDS write, barrier, transposed reads, MFMA):
 // a layer with one workgroup per CU takes 27 us whatever its size.  At 8 x 512 x
 // 128, base 32: 455 us per training step for the 14 convolutions, biases
-// included.  The kernels before took 3,484 us (one wave per 16 x 16 of one tap,
-// channel-strided 2-byte loads, atomics) and 2,958 us for the biases.  Loads
+// included; with one wave per 16 x 16 of one tap, channel-strided 2-byte loads and
+// atomics 3,484 us, and 2,958 for the biases in kernels of their own.  Loads
 // under an exec mask had to be waited for at each branch's end (73 us per layer);
 // the bias summed by a wave of the tile's own added 13 us to each layer: it has
 // workgroups of its own, behind the others (between them they left every second
@@ -685,7 +683,7 @@ __device__ __forceinline__ void load8f(const u16 *p, float (&v)[8]) {
 }
 
 // Sum of the 2x2 children (row pitch W) of output pixel (n, j, i), channels
-// c .. c + 7 of a tensor of stride C: (00 + 01) + (10 + 11), as before.
+// c .. c + 7 of a tensor of stride C: (00 + 01) + (10 + 11).
 __device__ __forceinline__ void sum4(const u16 *X, int H, int W, int C, int n, int j, int i, int c, float (&s)[8]) {
   const size_t b = ((size_t)(n * H + 2 * j) * W + 2 * i) * C + c;
   float x[4][8];
